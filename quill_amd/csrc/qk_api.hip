@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "quillk.h"
+#include "qk_drain.h"
 #include "qk_kernels.h"
 
 using namespace qk;
@@ -178,6 +179,11 @@ struct qk_ctx {
     void *d_fill = nullptr;
     size_t fill_cap = 0;
     Tape tape;
+    // read-backs: pinned slots on the way to the caller's arrays, and the
+    // scanned live counts of the species being read
+    Drain drain;
+    int *d_live = nullptr;
+    size_t live_cap = 0;            // runs that fit
     // laser sources at an x plane, per side (0: x-min, 1: x-max)
     InjSide inj[2];
     int window_shifts = 0;          // qk_moving_window calls so far
@@ -1104,18 +1110,130 @@ int upload3(qk_ctx *c, const double *aos, void *d0, void *d1, void *d2)
     return QK_OK;
 }
 
-int download3(qk_ctx *c, double *aos, const void *d0, const void *d1, const void *d2)
+// widen n numbers of the region's precision to FP64
+void widen(const qk_ctx *c, const void *src, int64_t n, double *dst)
+{
+    if (c->rsize == 8) {
+        std::memcpy(dst, src, (size_t)n * sizeof(double));
+        return;
+    }
+    const float *f = (const float *)src;
+    for (int64_t m = 0; m < n; ++m) dst[m] = f[m];
+}
+
+// up to four fields (three component arrays each) into interleaved FP64 arrays
+int download_fields(qk_ctx *c, int nf, double *const *aos, void *const (*comp)[3])
 {
     const int64_t n = c->g.ncell;
-    const size_t bytes = (size_t)n * c->rsize;
-    std::vector<char> buf(bytes * 3);
-    HIP_TRY(hipMemcpy(buf.data(), d0, bytes, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(buf.data() + bytes, d1, bytes, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(buf.data() + 2 * bytes, d2, bytes, hipMemcpyDeviceToHost));
-    for (int64_t m = 0; m < n; ++m)
-        for (int a = 0; a < 3; ++a)
-            aos[3 * m + a] = c->rsize == 4 ? (double)((const float *)buf.data())[a * n + m]
-                                           : ((const double *)buf.data())[a * n + m];
+    const size_t node = 3 * c->rsize, total = (size_t)nf * n * node;
+    const int64_t per = (int64_t)(Drain::slot_bytes(total) / node);   // nodes per block
+    const int64_t nb = (n + per - 1) / per;                            // blocks per field
+    auto launch = [&](int64_t b, void *slot) {
+        void *const *s = comp[b / nb];
+        const int64_t first = b % nb * per;
+        const int m = (int)std::min(per, n - first);
+        return c->rsize == 4 ? launch_pack_fields<float>(c->stream, (const float *)s[0], (const float *)s[1],
+                                                         (const float *)s[2], first, m, (float *)slot)
+                             : launch_pack_fields<double>(c->stream, (const double *)s[0], (const double *)s[1],
+                                                          (const double *)s[2], first, m, (double *)slot);
+    };
+    auto take = [&](int64_t b, const void *slot) {
+        const int64_t first = b % nb * per;
+        widen(c, slot, 3 * std::min(per, n - first), aos[b / nb] + 3 * first);
+    };
+    HIP_TRY(c->drain.run(c->p.device, c->stream, total, nf * nb, launch, take));
+    return QK_OK;
+}
+
+// the live count of each run of slots of species b, scanned, in d_live:
+// entry r is the row of run r's first live slot; `live` the total
+int scan_live(qk_ctx *c, const SpeciesBuf &b, int64_t &live, std::vector<int> *offs)
+{
+    const int64_t runs = (b.n + kLiveRun - 1) / kLiveRun;
+    const size_t row = ((size_t)runs + 64) & ~(size_t)63;   // counts, then offsets, then scan scratch
+    if (c->live_cap < (size_t)runs) {
+        if (c->d_live) HIP_TRY(hipFree(c->d_live));
+        c->d_live = nullptr;
+        c->live_cap = 0;
+        HIP_TRY(hipMalloc(&c->d_live, (2 * row + scan_scratch_ints(row)) * sizeof(int)));
+        c->live_cap = (size_t)runs;
+    }
+    int *counts = c->d_live + row;
+    HIP_TRY(launch_count_live(c->stream, b.buf[b.cur].cell, b.n, counts));
+    HIP_TRY(launch_fill_int(c->stream, counts + runs, 1, 0));
+    HIP_TRY(launch_exclusive_scan(c->stream, counts, c->d_live, (int)runs, c->d_live + 2 * row));
+    int total = 0;
+    if (offs) {
+        offs->resize((size_t)runs + 1);
+        HIP_TRY(hipMemcpyAsync(offs->data(), c->d_live, ((size_t)runs + 1) * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    } else {
+        HIP_TRY(hipMemcpyAsync(&total, c->d_live + runs, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    }
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    live = offs ? offs->back() : total;
+    return QK_OK;
+}
+
+// the records of species b's live slots, in slot order, as qk_get_particles
+// gives them
+template <typename real>
+int download_particles(qk_ctx *c, const SpeciesBuf &b, const std::vector<int> &offs, double *rec, int32_t *ids)
+{
+    const SoA &src = b.buf[b.cur];
+    const Species<real> v = view<real>(src);
+    const int nreal = src.a[7] ? 8 : 7;
+    const bool has_id = src.id != nullptr;
+    const size_t row = 4 + (size_t)nreal * sizeof(real) + (has_id ? 4 : 0), total = (size_t)offs.back() * row;
+    const int64_t per = (int64_t)(Drain::slot_bytes(total) / row) / kLiveRun * kLiveRun;   // slots per block
+    const int64_t nb = (b.n + per - 1) / per;
+    // a slot holds `per` rows: the reals first (aligned), then cells and ids
+    auto reals = [&](void *slot) { return (real *)slot; };
+    auto cells = [&](void *slot) { return (int *)((char *)slot + (size_t)per * nreal * sizeof(real)); };
+    auto launch = [&](int64_t k, void *slot) {
+        return launch_pack_live<real>(c->stream, v, k * per, std::min(b.n, (k + 1) * per), c->d_live, (int)per,
+                                      cells(slot), reals(slot), cells(slot) + per);
+    };
+    const double cmr = b.cmr;
+    const bool photon = b.kind == 1;
+    auto take = [&](int64_t k, void *slot) {
+        const size_t run0 = (size_t)(k * per / kLiveRun), run1 = std::min((size_t)((k + 1) * per / kLiveRun), offs.size() - 1);
+        const int64_t at = offs[run0], m1 = offs[run1] - at;
+        const real *x = reals(slot);
+        const int *cc = cells(slot), *id = cc + per;
+        for (int64_t m = 0; m < m1; ++m) {
+            double *w = rec + 10 * (at + m);
+            w[0] = cell_i(cc[m]) + (double)x[m];
+            w[1] = cell_j(cc[m]) + (double)x[per + m];
+            w[2] = cell_k(cc[m]) + (double)x[2 * per + m];
+            w[3] = (double)x[3 * per + m];
+            w[4] = (double)x[4 * per + m];
+            w[5] = (double)x[5 * per + m];
+            const double u2 = w[3] * w[3] + w[4] * w[4] + w[5] * w[5];
+            w[6] = photon ? std::sqrt(u2) : std::sqrt(1 + u2);
+            w[7] = (double)x[6 * per + m];
+            w[8] = cmr;
+            w[9] = nreal == 8 ? (double)x[7 * per + m] : 0.0;
+        }
+        if (ids) {
+            if (has_id) std::memcpy(ids + at, id, (size_t)m1 * sizeof(int));
+            else std::fill(ids + at, ids + at + m1, 0);
+        }
+    };
+    HIP_TRY(c->drain.run(c->p.device, c->stream, total, nb, launch, take));
+    return QK_OK;
+}
+
+// n doubles from device memory
+int download_doubles(qk_ctx *c, double *dst, const double *src, int64_t n)
+{
+    const size_t total = (size_t)n * sizeof(double);
+    const int64_t per = (int64_t)(Drain::slot_bytes(total) / sizeof(double));
+    auto count = [&](int64_t b) { return (size_t)std::min(per, n - b * per) * sizeof(double); };
+    auto launch = [&](int64_t b, void *slot) {
+        return hipMemcpyAsync(slot, src + b * per, count(b), hipMemcpyDeviceToHost, c->stream);
+    };
+    auto take = [&](int64_t b, const void *slot) { std::memcpy(dst + b * per, slot, count(b)); };
+    HIP_TRY(c->drain.run(c->p.device, c->stream, total, (n + per - 1) / per, launch, take));
     return QK_OK;
 }
 
@@ -1272,6 +1390,8 @@ int qk_destroy(qk_ctx *c)
     if (c->d_fill) note(hipFree(c->d_fill));
     for (auto &side : c->inj)
         if (side.mem) note(hipFree(side.mem));
+    if (c->d_live) note(hipFree(c->d_live));
+    note(c->drain.release());
     for (auto e : c->ev) note(hipEventDestroy(e));
     if (c->stream) note(hipStreamDestroy(c->stream));
     delete c;
@@ -1292,14 +1412,21 @@ int qk_set_fields(qk_ctx *c, const double *E, const double *B)
 int qk_get_fields(qk_ctx *c, double *E, double *B, double *J, double *Be)
 {
     if (!c) return fail(QK_ERR_INVALID, "null context");
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    if (E) QK_TRY(download3(c, E, c->F[0], c->F[1], c->F[2]));
-    if (B) QK_TRY(download3(c, B, c->F[3], c->F[4], c->F[5]));
-    if (Be) QK_TRY(download3(c, Be, c->F[6], c->F[7], c->F[8]));
-    if (J) {
-        const int w = c->have_step ? (c->jcur ^ 1) : c->jcur;   // buffer of the last step
-        QK_TRY(download3(c, J, c->F[9 + 3 * w], c->F[10 + 3 * w], c->F[11 + 3 * w]));
+    const int w = c->have_step ? (c->jcur ^ 1) : c->jcur;   // current buffer of the last step
+    double *const out[4] = {E, B, J, Be};
+    const int at[4] = {0, 3, 9 + 3 * w, 6};
+    double *aos[4];
+    void *comp[4][3];
+    int nf = 0;
+    for (int k = 0; k < 4; ++k) {
+        if (!out[k]) continue;
+        aos[nf] = out[k];
+        for (int a = 0; a < 3; ++a) comp[nf][a] = c->F[at[k] + a];
+        ++nf;
     }
+    const DeviceScope on(c->p.device);
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    if (nf > 0) QK_TRY(download_fields(c, nf, aos, comp));
     return QK_OK;
 }
 
@@ -1429,12 +1556,8 @@ int qk_particle_count(qk_ctx *c, int s, int64_t *n)
     SpeciesBuf &b = c->sp[s];
     *n = 0;
     if (b.n == 0) return QK_OK;
-    std::vector<int> cell((size_t)b.n);
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    HIP_TRY(hipMemcpy(cell.data(), b.buf[b.cur].cell, (size_t)b.n * 4, hipMemcpyDeviceToHost));
-    int64_t live = 0;
-    for (int v : cell) live += v >= 0;
-    *n = live;
+    const DeviceScope on(c->p.device);
+    QK_TRY(scan_live(c, b, *n, nullptr));
     return QK_OK;
 }
 
@@ -1446,46 +1569,22 @@ int qk_get_particles(qk_ctx *c, int s, int64_t cap, double *rec, int32_t *ids, i
     *n_out = 0;
     if (b.n == 0) return QK_OK;
     if (!rec) return fail(QK_ERR_INVALID, "null output buffer");
-    const SoA &src = b.buf[b.cur];
-    const size_t r = c->rsize;
-    const int64_t n = b.n;
-    std::vector<int> cell((size_t)n), id((size_t)n);
-    std::vector<char> buf((size_t)n * r * 8, 0);
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    HIP_TRY(hipMemcpy(cell.data(), src.cell, (size_t)n * 4, hipMemcpyDeviceToHost));
-    for (int a = 0; a < 8; ++a)
-        if (src.a[a]) HIP_TRY(hipMemcpy(buf.data() + (size_t)a * n * r, src.a[a], (size_t)n * r, hipMemcpyDeviceToHost));
-    if (src.id) HIP_TRY(hipMemcpy(id.data(), src.id, (size_t)n * 4, hipMemcpyDeviceToHost));
-    auto get = [&](int a, int64_t m) {
-        return r == 4 ? (double)((const float *)buf.data())[(size_t)a * n + m] : ((const double *)buf.data())[(size_t)a * n + m];
-    };
-    int64_t o = 0;
-    for (int64_t m = 0; m < n; ++m) {
-        const int cc = cell[(size_t)m];
-        if (cc < 0) continue;
-        if (o >= cap) return fail(QK_ERR_CAPACITY, "output buffer too small");
-        double *w = rec + 10 * o;
-        w[0] = cell_i(cc) + get(0, m);
-        w[1] = cell_j(cc) + get(1, m);
-        w[2] = cell_k(cc) + get(2, m);
-        w[3] = get(3, m);
-        w[4] = get(4, m);
-        w[5] = get(5, m);
-        const double u2 = w[3] * w[3] + w[4] * w[4] + w[5] * w[5];
-        w[6] = b.kind == 1 ? std::sqrt(u2) : std::sqrt(1 + u2);
-        w[7] = get(6, m);
-        w[8] = b.cmr;
-        w[9] = get(7, m);
-        if (ids) ids[o] = src.id ? id[(size_t)m] : 0;
-        ++o;
-    }
-    *n_out = o;
+    const DeviceScope on(c->p.device);
+    std::vector<int> offs;
+    int64_t live = 0;
+    QK_TRY(scan_live(c, b, live, &offs));
+    if (live > cap) return fail(QK_ERR_CAPACITY, "output buffer too small");
+    if (live > 0)
+        QK_TRY(c->rsize == 4 ? download_particles<float>(c, b, offs, rec, ids)
+                             : download_particles<double>(c, b, offs, rec, ids));
+    *n_out = live;
     return QK_OK;
 }
 
 int qk_compute_rho(qk_ctx *c, double *rho)
 {
     if (!c || !rho) return fail(QK_ERR_INVALID, "null argument");
+    const DeviceScope on(c->p.device);
     const size_t bytes = (size_t)c->g.ncell * 3 * sizeof(double);
     double *d = nullptr;
     HIP_TRY(hipMalloc(&d, bytes));
@@ -1498,9 +1597,10 @@ int qk_compute_rho(qk_ctx *c, double *rho)
                           : launch_compute_rho<double>(c->stream, c->g, view<double>(b.buf[b.cur]), b.n, d, t);
     }
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (e == hipSuccess) e = hipMemcpy(rho, d, bytes, hipMemcpyDeviceToHost);
+    const int rc = e == hipSuccess ? download_doubles(c, rho, d, 3 * (int64_t)c->g.ncell) : QK_OK;
     const hipError_t ef = hipFree(d);
     HIP_TRY(e);
+    QK_TRY(rc);
     HIP_TRY(ef);
     return QK_OK;
 }

@@ -207,6 +207,22 @@ hipError_t launch_load_uniform(hipStream_t st, const Grid &g, const Species<real
 template <typename real>
 hipError_t launch_compute_rho(hipStream_t st, const Grid &g, const Species<real> &s, int64_t n, double *rho, int slot);
 
+// ---- results for the host (into pinned memory) ------------------------------
+
+// slots per run of the live-particle counts
+constexpr int kLiveRun = 1024;
+// out[3 m + c] = component c at node first + m, m in [0, n)
+template <typename real>
+hipError_t launch_pack_fields(hipStream_t st, const real *a, const real *b, const real *c, int64_t first, int n,
+                              real *out);
+// counts[r] = live particles of slots [r kLiveRun, (r + 1) kLiveRun) below n
+hipError_t launch_count_live(hipStream_t st, const int *cell, int64_t n, int *counts);
+// the live slots of [first, end) (first a multiple of kLiveRun) in slot order,
+// one array per record entry, `stride` entries apart; offs: scanned counts
+template <typename real>
+hipError_t launch_pack_live(hipStream_t st, const Species<real> &s, int64_t first, int64_t end, const int *offs,
+                            int stride, int *cell_out, real *real_out, int *id_out);
+
 // ---- cell-tile counting sort ----------------------------------------------
 
 // scratch for the exclusive scan of n ints: at most scan_scratch_ints(n) ints
