@@ -126,17 +126,13 @@ struct Tape {
     double *tpart = nullptr;      // 7 record tangents per species (x y z ux uy uz q)
 };
 
-// the laser sources of one side of the box (qk_add_laser_source) and the
-// stack their corrections run on
+// the laser sources of one side of the box (qk_add_laser_source)
 struct InjSide {
     int nsrc = 0;
     int plane = 0;
-    int W = 0;                    // planes per slab
     LaserFrame src[kMaxSources];
     uint32_t t0[kMaxSources] = {};   // step index at which each source was added
     int shifts0[kMaxSources] = {};   // window shifts at that time
-    void *mem = nullptr;          // 6 field + 6 current arrays of the stack
-    Grid gs{};
 };
 
 }  // namespace
@@ -844,22 +840,7 @@ void tangent_records(const qk_ctx *c, int s, double *out[7])
     for (int a = 0; a < 7; ++a) out[a] = m + (size_t)a * c->tape.n[s];
 }
 
-// views of a side's stack: fields (ex..bz; no Be) and two current sets
-template <typename real>
-void stack_views(const InjSide &side, Fields<real> &f, Current<real> &j0, Current<real> &j1)
-{
-    const size_t n = ((size_t)side.gs.ncell * sizeof(real) + 255) & ~(size_t)255;
-    char *m = (char *)side.mem;
-    real *a[12];
-    for (int k = 0; k < 12; ++k) a[k] = (real *)(m + k * n);
-    f.ex = a[0]; f.ey = a[1]; f.ez = a[2];
-    f.bx = a[3]; f.by = a[4]; f.bz = a[5];
-    f.bex = f.bey = f.bez = nullptr;
-    j0.jx = a[6]; j0.jy = a[7]; j0.jz = a[8];
-    j1.jx = a[9]; j1.jy = a[10]; j1.jz = a[11];
-}
-
-// Whether any pulse of the side can be nonzero on its stack planes after
+// Whether any pulse of the side can be nonzero near its plane after
 // travelling shift[n]: the envelope is |x| < xs along the propagation axis,
 // and x is linear in position, so the slab's corner points bound it.
 bool side_active(const qk_ctx *c, const InjSide &side, const InjectArgs &a)
@@ -888,27 +869,24 @@ bool side_active(const qk_ctx *c, const InjSide &side, const InjectArgs &a)
 template <typename real>
 int inject_impl(qk_ctx *c, int b_field, double frac)
 {
+    InjectArgs a[2];
+    int n = 0;
     for (int sd = 0; sd < 2; ++sd) {
-        InjSide &side = c->inj[sd];
+        const InjSide &side = c->inj[sd];
         if (side.nsrc == 0) continue;
-        InjectArgs a{};
-        a.nsrc = side.nsrc;
-        for (int n = 0; n < side.nsrc; ++n) {
-            a.src[n] = side.src[n];
-            a.shift[n] = ((double)(c->step_index - side.t0[n]) + frac) * c->g.dt;
-            a.ishift[n] = c->window_shifts - side.shifts0[n];
+        InjectArgs &s = a[n];
+        s = InjectArgs{};
+        s.nsrc = side.nsrc;
+        for (int m = 0; m < side.nsrc; ++m) {
+            s.src[m] = side.src[m];
+            s.shift[m] = ((double)(c->step_index - side.t0[m]) + frac) * c->g.dt;
+            s.ishift[m] = c->window_shifts - side.shifts0[m];
         }
-        a.side = sd;
-        a.plane = side.plane;
-        a.W = side.W;
-        a.main_lo = sd == 0 ? 0 : c->g.nx - side.W;
-        a.b_field = b_field;
-        if (!side_active(c, side, a)) continue;
-        Fields<real> st;
-        Current<real> j0, j1;
-        stack_views<real>(side, st, j0, j1);
-        HIP_TRY(launch_inject<real>(c->stream, c->p.solver, c->g, c->coef, fields_of<real>(c), side.gs, st, j0, j1, a));
+        s.side = sd;
+        s.plane = side.plane;
+        n += side_active(c, side, s);
     }
+    HIP_TRY(launch_inject<real>(c->stream, c->p.solver, c->g, c->coef, fields_of<real>(c), b_field, n, a));
     return QK_OK;
 }
 
@@ -1388,8 +1366,6 @@ int qk_destroy(qk_ctx *c)
     if (c->d_maxw) note(hipFree(c->d_maxw));
     if (c->h_maxw) note(hipHostFree(c->h_maxw));
     if (c->d_fill) note(hipFree(c->d_fill));
-    for (auto &side : c->inj)
-        if (side.mem) note(hipFree(side.mem));
     if (c->d_live) note(hipFree(c->d_live));
     note(c->drain.release());
     for (auto e : c->ev) note(hipEventDestroy(e));
@@ -1642,16 +1618,7 @@ int qk_add_laser_source(qk_ctx *c, const double L[16], int side, int plane)
     if (sd.nsrc > 0 && sd.plane != plane) return fail(QK_ERR_INVALID, "the sources of one side share one plane");
     LaserFrame F;
     if (!laser_frame(c->g, L, F)) return fail(QK_ERR_INVALID, "laser source: x1, y0, z0 all zero");
-    if (!sd.mem) {
-        sd.W = side == 0 ? plane + 6 : nx - plane + 6;
-        sd.gs = c->g;
-        sd.gs.nx = 2 * sd.W + kInjGap;
-        sd.gs.ncell = sd.gs.nx * c->g.sx;
-        const size_t n = ((size_t)sd.gs.ncell * c->rsize + 255) & ~(size_t)255;
-        HIP_TRY(hipMalloc(&sd.mem, 12 * n));
-        HIP_TRY(hipMemset(sd.mem, 0, 12 * n));   // the current sets stay zero
-        sd.plane = plane;
-    }
+    sd.plane = plane;
     sd.src[sd.nsrc] = F;
     sd.t0[sd.nsrc] = c->step_index;
     sd.shifts0[sd.nsrc] = c->window_shifts;

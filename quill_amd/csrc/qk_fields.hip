@@ -6,6 +6,8 @@
 // Fields are structure-of-arrays, one array per component, [nx][ny][nz] with
 // k fastest; a thread owns one cell and consecutive lanes walk k, so every
 // stencil load of a wavefront is a coalesced run.
+#include <cstdlib>
+
 #include "qk_kernels.h"
 
 namespace qk {
@@ -423,82 +425,128 @@ __global__ void __launch_bounds__(kBX * kBY) k_laser_cos(Grid g, Fields<real> f,
 // across the plane is corrected by the same update applied to the incident
 // field on the far side: + L(inc on the scattered side) at total nodes,
 // - L(inc on the total side) at scattered nodes, L being the solver's own
-// update (k_maxwell_b / k_maxwell_e) with its boundary-plane sets.  Both
-// passes run as one launch on a stack of two copies of the W planes next to
-// the source's wall, separated by kInjGap empty planes: the copy whose
-// outputs are read at scattered nodes sits at the wall's end of the stack,
-// so its planes near the wall see the grid's own boundary-plane sets.  The
-// incident field is sampled where each component lives on the staggered
-// grid (E_a a half cell along a, B_a a half cell across a).
+// update with its boundary-plane sets.  The incident field is sampled where
+// each component lives on the staggered grid (E_a a half cell along a, B_a a
+// half cell across a).
+//
+// The stencils reach kInjReach planes across, so only 2 kInjReach planes
+// matter.  A workgroup evaluates the incident field of its rows of 64 columns
+// (and, for NDFX, the rim its transverse smoothing reads) there into LDS, its
+// threads sharing the points, and applies the masked update to the grid, a
+// wavefront per plane and row: one launch per sub-step for both sides.  Only differences along x cross the plane, and NDFX's smoothing of
+// the x component along x: component x is needed there only, and neither it
+// nor its own update is ever corrected.
+// Bound by the FP64 pulse (three sines and cosines per point and the
+// transverse ones).  Before, the pulse was evaluated on 18 planes of a stack
+// that the solver then swept whole, three launches per side and sub-step: a
+// sub-step took 66 us for two sides of 128 x 128 columns (five-point), now
+// 9.4 us; 17.6 us for one of 32 x 32 (FDTD), now 5.1 us.  With 64 x 4 columns
+// per workgroup (six points in turn per thread instead of at most two) it was
+// 21.7 us and 6.6 us.
+template <int S>
+constexpr int kInjReach = S == 2 ? 2 : 1;
 
-// the slab of the stack at plane l: 0 low, 1 high, -1 gap; sets the grid plane
-__device__ inline int stack_slab(const InjectArgs &a, int l, int &i)
+// whether the corrections of a sub-step read component c of the incident
+// field in plane m of the 2 kInjReach (m = kInjReach is the source plane);
+// BF: B half step (forward differences of E), else E step (backward, of B)
+template <int S, bool BF>
+constexpr bool inj_reads(int c, int m)
 {
-    if (l < a.W) { i = a.main_lo + l; return 0; }
-    if (l >= a.W + kInjGap) { i = a.main_lo + l - a.W - kInjGap; return 1; }
-    return -1;
+    if (c == 0) return S == 1;
+    if (S == 2) return BF ? m >= 1 : m <= 2;
+    return BF ? m == 1 : m == 0;
 }
 
-__device__ inline bool total_side(const InjectArgs &a, int i) { return a.side == 0 ? i >= a.plane : i < a.plane; }
+struct InjectSides {
+    InjectArgs s[2];
+};
 
-// fill the stack's input component (E for a B half step, B for an E step)
-// with the incident field of every source, masked per slab, and clear the
-// output components
-template <typename real>
-__global__ void __launch_bounds__(kBX * kBY) k_inject_prepare(Grid gs, Fields<real> st, InjectArgs a)
+template <int S, bool BF, typename real>
+__global__ void __launch_bounds__(kBX * kBY) k_inject(Grid g, Coef<real> cf, Fields<real> f, InjectSides sides)
 {
-    const int k = blockIdx.x * kBX + threadIdx.x;
-    const int j = blockIdx.y * kBY + threadIdx.y;
-    const int l = blockIdx.z;
-    if (k >= gs.nz || j >= gs.ny) return;
-    const int id = l * gs.sx + j * gs.sy + k;
-    real *in[3] = {a.b_field ? st.ex : st.bx, a.b_field ? st.ey : st.by, a.b_field ? st.ez : st.bz};
-    real *out[3] = {a.b_field ? st.bx : st.ex, a.b_field ? st.by : st.ey, a.b_field ? st.bz : st.ez};
-    int i = 0;
-    const int slab = stack_slab(a, l, i);
-    // the low slab holds the pass read at scattered nodes when the wall is
-    // at x-min, the pass read at total nodes when it is at x-max
-    const bool reads_at_total = (slab == 1) == (a.side == 0);
-    // pass read at total nodes: incident field on scattered nodes, and back
-    const bool fill = slab >= 0 && abs(i - a.plane) <= 4 && total_side(a, i) != reads_at_total;
-    double v[3] = {0, 0, 0};
-    if (fill) {
-        for (int n = 0; n < a.nsrc; ++n)
-            for (int c = 0; c < 3; ++c) {
-                // staggered position of component c of the input field
-                double h[3];
-                for (int m = 0; m < 3; ++m) h[m] = (a.b_field ? m == c : m != c) ? 0.5 : 0.0;
+    constexpr int R = kInjReach<S>, M = S == 1 ? 1 : 0;   // planes per side, rim
+    constexpr int kRows = kBY / (2 * R);                   // rows of columns: a thread owns one node of one plane
+    constexpr int W = kBX + 2 * M, H = kRows + 2 * M;
+    constexpr int kPairs = S == 0 ? 2 : (S == 1 ? 4 : 6);  // (component, plane) pairs read: see inj_reads
+    __shared__ real inc[3][2 * R][H][W];
+    const InjectArgs &a = sides.s[blockIdx.z];
+    const int k0 = blockIdx.x * kBX, j0 = blockIdx.y * kRows, i0 = a.plane - R;
+    for (int e = threadIdx.y * kBX + threadIdx.x; e < kPairs * H * W; e += kBX * kBY) {
+        const int pair = e / (H * W), rq = e - pair * H * W, r = rq / W, q = rq - r * W;
+        const int c = S == 0 ? 1 + pair : (S == 1 ? (pair < 2 ? 0 : pair - 1) : 1 + pair / 3);
+        const int m = S == 2 ? pair % 3 + BF : (S == 1 && pair < 2 ? pair : (int)BF);
+        const int i = i0 + m, j = j0 + r - M, k = k0 + q - M;
+        // staggered position of component c of the input field
+        const double hx = (BF ? c == 0 : c != 0) ? 0.5 : 0.0, hy = (BF ? c == 1 : c != 1) ? 0.5 : 0.0,
+                     hz = (BF ? c == 2 : c != 2) ? 0.5 : 0.0;
+        double v = 0;
+        if ((unsigned)i < (unsigned)g.nx && (unsigned)j < (unsigned)g.ny && (unsigned)k < (unsigned)g.nz)
+            for (int n = 0; n < a.nsrc; ++n) {
                 double ev[3], bv[3];
-                if (pulse_at(a.src[n], (i + a.ishift[n] + h[0]) * gs.dx, (j + h[1]) * gs.dy, (k + h[2]) * gs.dz,
-                             a.shift[n], ev, bv))
-                    v[c] += a.b_field ? ev[c] : bv[c];
+                if (pulse_at(a.src[n], (i + a.ishift[n] + hx) * g.dx, (j + hy) * g.dy, (k + hz) * g.dz, a.shift[n], ev, bv)) {
+                    const double *p = BF ? ev : bv;
+                    v += c == 0 ? p[0] : (c == 1 ? p[1] : p[2]);
+                }
             }
+        inc[c][m][r][q] = (real)v;
     }
-    for (int c = 0; c < 3; ++c) {
-        in[c][id] = (real)v[c];
-        out[c][id] = real(0);
-    }
-}
-
-// add the stack's corrections to the grid's planes within 3 of the source plane
-template <typename real>
-__global__ void __launch_bounds__(kBX * kBY) k_inject_apply(Grid g, Fields<real> f, Grid gs, Fields<real> st,
-                                                            InjectArgs a)
-{
-    const int k = blockIdx.x * kBX + threadIdx.x;
-    const int j = blockIdx.y * kBY + threadIdx.y;
-    const int i = a.plane - 3 + (int)blockIdx.z;
-    if (k >= g.nz || j >= g.ny || i < 0 || i >= g.nx) return;
-    const bool tot = total_side(a, i);
-    // the slab read here: at total nodes the high slab for an x-min wall
-    const bool high = tot == (a.side == 0);
-    const int l = (i - a.main_lo) + (high ? a.W + kInjGap : 0);
-    const int id = i * g.sx + j * g.sy + k, ls = l * gs.sx + j * gs.sy + k;
-    real *dst[3] = {a.b_field ? f.bx : f.ex, a.b_field ? f.by : f.ey, a.b_field ? f.bz : f.ez};
-    const real *src[3] = {a.b_field ? st.bx : st.ex, a.b_field ? st.by : st.ey, a.b_field ? st.bz : st.ez};
-    for (int c = 0; c < 3; ++c) {
-        const real d = src[c][ls];
-        dst[c][id] = tot ? dst[c][id] + d : dst[c][id] - d;
+    __syncthreads();
+    const int row = threadIdx.y / (2 * R), j = j0 + row, k = k0 + threadIdx.x;
+    if (j >= g.ny || k >= g.nz) return;
+    const int r = row + M, q = threadIdx.x + M;
+#pragma unroll
+    for (int m = 0; m < 2 * R; ++m) {
+        if (m != (int)threadIdx.y % (2 * R)) continue;   // uniform over the wavefront
+        const int i = i0 + m;
+        if (i < 0 || i >= g.nx) continue;
+        const bool low = m < R;
+        // the incident field on the node's far side, zero on its own
+        auto in = [&](int c, int mm, int dj, int dk) -> real {
+            if (mm < 0 || mm >= 2 * R || (mm < R) == low || !inj_reads<S, BF>(c, mm)) return real(0);
+            return inc[c][mm][r + dj][q + dk];
+        };
+        // difference along x of component c (1 or 2)
+        auto dx = [&](int c) -> real {
+            const int lo = BF ? m : m - 1;
+            if (S == 0) return in(c, lo + 1, 0, 0) - in(c, lo, 0, 0);
+            if (S == 1) {   // smoothed along the component's own axis
+                const int uj = c == 1, uk = c == 2;
+                return cf.b[c] * (in(c, lo + 1, 0, 0) - in(c, lo, 0, 0)) +
+                       cf.a[c] * ((in(c, lo + 1, uj, uk) - in(c, lo, uj, uk)) +
+                                  (in(c, lo + 1, -uj, -uk) - in(c, lo, -uj, -uk)));
+            }
+            const real fm = in(c, lo - 1, 0, 0), f0 = in(c, lo, 0, 0), f1 = in(c, lo + 1, 0, 0), f2 = in(c, lo + 2, 0, 0);
+            return cf.b[0] * (f1 - f0) + cf.a[0] * (f2 - f1 + f0 - fm);
+        };
+        // difference along y or z of component x: NDFX's smoothing along x
+        auto dt = [&](int axis) -> real {
+            if (S != 1) return real(0);
+            const int uj = axis == 1, uk = axis == 2, s = BF ? 0 : -1;
+            auto d = [&](int mm) { return in(0, mm, (s + 1) * uj, (s + 1) * uk) - in(0, mm, s * uj, s * uk); };
+            return cf.a[0] * (d(m + 1) + d(m - 1));
+        };
+        const bool tot = low == (a.side == 1);
+        const int id = i * g.sx + j * g.sy + k;
+        if (BF) {
+            const real h = real(0.5);
+            if (b_updates<S, 1>(g, i, j, k)) {
+                const real d = h * (cf.dtd[0] * dx(2) - cf.dtd[2] * dt(2));
+                f.by[id] = tot ? f.by[id] + d : f.by[id] - d;
+            }
+            if (b_updates<S, 2>(g, i, j, k)) {
+                const real d = h * (cf.dtd[1] * dt(1) - cf.dtd[0] * dx(1));
+                f.bz[id] = tot ? f.bz[id] + d : f.bz[id] - d;
+            }
+        } else {
+            if (e_updates<S, 1>(g, i, j, k)) {
+                const real d = -cf.dtd[0] * dx(2) + cf.dtd[2] * dt(2);
+                f.ey[id] = tot ? f.ey[id] + d : f.ey[id] - d;
+            }
+            if (e_updates<S, 2>(g, i, j, k)) {
+                const real d = cf.dtd[0] * dx(1) - cf.dtd[1] * dt(1);
+                f.ez[id] = tot ? f.ez[id] + d : f.ez[id] - d;
+            }
+        }
     }
 }
 
@@ -626,18 +674,32 @@ hipError_t launch_laser_cos(hipStream_t st, const Grid &g, const Fields<real> &f
 
 template <typename real>
 hipError_t launch_inject(hipStream_t st, int solver, const Grid &g, const SolverCoef &c, const Fields<real> &f,
-                         const Grid &gs, const Fields<real> &stack, const Current<real> &j0, const Current<real> &j1,
-                         const InjectArgs &a)
+                         int b_field, int nsides, const InjectArgs *a)
 {
-    k_inject_prepare<real><<<cell_grid(gs), dim3(kBX, kBY), 0, st>>>(gs, stack, a);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    e = a.b_field ? launch_maxwell_b<real>(st, solver, gs, c, stack, nullptr)
-                  : launch_maxwell_e<real>(st, solver, gs, c, stack, j0, j1);
-    if (e != hipSuccess) return e;
-    const dim3 grid((g.nz + kBX - 1) / kBX, (g.ny + kBY - 1) / kBY, 7);   // planes plane-3 .. plane+3
-    k_inject_apply<real><<<grid, dim3(kBX, kBY), 0, st>>>(g, f, gs, stack, a);
-    return hipGetLastError();
+    if (nsides <= 0) return hipSuccess;
+    const Coef<real> cf = make_coef<real>(g, c);
+    const dim3 block(kBX, kBY);
+    const int rows = solver == 2 ? 1 : 2;   // k_inject's kRows
+    dim3 grid((g.nz + kBX - 1) / kBX, (g.ny + rows - 1) / rows, nsides);
+    auto one = [&](const InjectArgs &a0, const InjectArgs &a1) {
+        const InjectSides sides{{a0, a1}};
+#define QK_INJ(S)                                                                              \
+    if (b_field) k_inject<S, true, real><<<grid, block, 0, st>>>(g, cf, f, sides);             \
+    else k_inject<S, false, real><<<grid, block, 0, st>>>(g, cf, f, sides)
+        if (solver == 0) { QK_INJ(0); }
+        else if (solver == 1) { QK_INJ(1); }
+        else { QK_INJ(2); }
+#undef QK_INJ
+        return hipGetLastError();
+    };
+    // sides whose planes lie closer than the corrections reach follow each
+    // other: in one launch they would update the same nodes
+    if (nsides == 2 && std::abs(a[0].plane - a[1].plane) < 2 * 2) {
+        grid.z = 1;
+        const hipError_t e = one(a[0], a[0]);
+        return e != hipSuccess ? e : one(a[1], a[1]);
+    }
+    return one(a[0], a[nsides - 1]);
 }
 
 #define QK_INST(real)                                                                                            \
@@ -649,8 +711,7 @@ hipError_t launch_inject(hipStream_t st, int solver, const Grid &g, const Solver
     template hipError_t launch_init_boundaries<real>(hipStream_t, int, const Grid &, const Fields<real> &);     \
     template hipError_t launch_laser_cos<real>(hipStream_t, const Grid &, const Fields<real> &, const double *); \
     template hipError_t launch_inject<real>(hipStream_t, int, const Grid &, const SolverCoef &, const Fields<real> &, \
-                                            const Grid &, const Fields<real> &, const Current<real> &,           \
-                                            const Current<real> &, const InjectArgs &);
+                                            int, int, const InjectArgs *);
 QK_INST(float)
 QK_INST(double)
 #undef QK_INST
