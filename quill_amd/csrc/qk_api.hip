@@ -147,13 +147,15 @@ struct qk_ctx {
     void *fmem = nullptr;           // all field arrays
     void *F[15] = {};               // ex ey ez bx by bz bex bey bez j0x j0y j0z j1x j1y j1z
     int jcur = 0;                   // current buffer deposited this step
+    bool j_zero[2] = {true, true};  // which current buffers are known to be zero
     bool have_step = false;
     SpeciesBuf sp[QK_MAX_SPECIES];
     // shared sort buffers (allocated at the first sort)
     int *s_counts = nullptr, *s_imm = nullptr, *s_offsets = nullptr, *s_tile_start = nullptr, *s_tile_mult = nullptr,
         *s_chunk_n = nullptr, *s_chunk_off = nullptr, *s_scratch = nullptr;
     int *h_sortinfo = nullptr;      // pinned: [live count, chunk count]
-    double *d_diag = nullptr;       // [QK_MAX_SPECIES][kDiagPerSpecies] + field energy
+    double *d_diag = nullptr;       // two rows (steps alternate) of [QK_MAX_SPECIES][kDiagPerSpecies] + field energy
+    double *diag_row = nullptr;     // the current step's
     double *h_diag = nullptr;       // pinned per-step copies of the accumulators
     size_t h_diag_cap = 0;          // steps that fit in h_diag
     std::vector<hipEvent_t> ev;     // timing events
@@ -523,7 +525,7 @@ int qed_particle_phase(qk_ctx *c, const Fields<real> &f, const Current<real> &jc
         t.count = c->d_count + s;
         t.cap = (int)b.cap;
         t.overflow = c->d_count + QK_MAX_SPECIES;
-        t.diag = c->d_diag + s * kDiagPerSpecies;
+        t.diag = c->diag_row + s * kDiagPerSpecies;
         return t;
     };
     const int64_t ninner = std::max<int64_t>(0, (int64_t)(c->p.nx - 4) * (c->p.ny - 4) * (c->p.nz - 4));
@@ -548,9 +550,9 @@ int qed_particle_phase(qk_ctx *c, const Fields<real> &f, const Current<real> &jc
         a.kind = b.kind;
         a.cmr = b.cmr;
         a.external_bz = c->p.external_bz;
-        a.diag = c->d_diag + s * kDiagPerSpecies;
+        a.diag = c->diag_row + s * kDiagPerSpecies;
         a.energy_mode = b.energy_mode;
-        a.nonfinite = c->d_diag + kNonfiniteSlot;
+        a.nonfinite = c->diag_row + kNonfiniteSlot;
         a.first = 0;
         a.n = b.n;
         const Species<real> v = view<real>(b.buf[b.cur]);
@@ -566,9 +568,9 @@ int qed_particle_phase(qk_ctx *c, const Fields<real> &f, const Current<real> &jc
         a.kind = 1;
         a.cmr = 0;
         a.external_bz = c->p.external_bz;
-        a.diag = c->d_diag + QK_PHOTON * kDiagPerSpecies;
+        a.diag = c->diag_row + QK_PHOTON * kDiagPerSpecies;
         a.energy_mode = 1;
-        a.nonfinite = c->d_diag + kNonfiniteSlot;
+        a.nonfinite = c->diag_row + kNonfiniteSlot;
         a.first = 0;
         a.n = n_ph0;
         HIP_TRY(launch_photon_qed<real>(c->stream, c->g, f, jc, view<real>(bph.buf[bph.cur]), a, qa,
@@ -809,6 +811,7 @@ int adjoint_impl(qk_ctx *c, const double *lam_E, const double *lam_B, const doub
     QK_TRY(tape_load(c, t.fin));
     c->jcur = jcur_end;
     c->step_index = step_end;
+    c->j_zero[0] = c->j_zero[1] = false;   // the replayed steps' bookkeeping
     HIP_TRY(hipStreamSynchronize(c->stream));
     return QK_OK;
 }
@@ -894,7 +897,7 @@ template <typename real>
 int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
 {
     const Fields<real> f = fields_of<real>(c);
-    // three events per step: before the particle phase, between phases, after the field phase
+    // three events per step: before the particle phase (see `start`), between phases, after the field phase
     QK_TRY(ensure_events(c, 3 * (size_t)nsteps));
     if (c->h_diag_cap < (size_t)nsteps) {
         if (c->h_diag) HIP_TRY(hipHostFree(c->h_diag));
@@ -906,21 +909,38 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
     const bool qed = c->p.qed != 0;
     // the QED kernels deposit through global atomics
     const bool tiled = c->p.deposit == QK_DEPOSIT_TILED && !qed;
+    Tape &tp = c->tape;
+    // Without charged particles nothing reads Be or B between two steps: Be
+    // is interpolated once, at the end, and the second half step of B runs
+    // with the next step's first one.  (Photons fly straight.  A laser source
+    // corrects each half step by itself; the tape keeps the state of every
+    // step.)
+    bool charged = qed || tp.active;
+    for (const SpeciesBuf &b : c->sp) charged = charged || (b.active && b.n > 0 && b.kind == 0);
+    const bool fuse_b = !charged && c->inj[0].nsrc == 0 && c->inj[1].nsrc == 0;
+    // the event that marks the start of each step's particle phase: the end
+    // of the step before unless something ran in between
+    std::vector<int> start((size_t)nsteps);
+    HIP_TRY(launch_zero(c->stream, c->d_diag, 2 * kDiagLen));
     for (int l = 0; l < nsteps; ++l) {
-        Tape &tp = c->tape;
+        bool between = l == 0;
+        c->diag_row = c->d_diag + (l & 1) * kDiagLen;
         if (tp.active && !tp.replay) {
-            if (tp.steps > 0 && tp.steps % tp.every == 0) QK_TRY(tape_snapshot(c));
+            if (tp.steps > 0 && tp.steps % tp.every == 0) {
+                QK_TRY(tape_snapshot(c));
+                between = true;
+            }
             ++tp.steps;
         }
-        // The window fallback of step l - 2: once step l - 1 has begun its
-        // particle phase, step l - 2 and its diagnostics copy are done, and
-        // the GPU still has step l - 1 queued while the host decides.  The
+        // The window fallback of step l - 2: once that step has ended, its
+        // diagnostics are here, and the GPU still has step l - 1 queued while
+        // the host decides.  The
         // first two steps of a call use the last step of the previous call
         // (kept per species), so the rule holds for callers that step one
         // step per call.
         bool fb_high[QK_MAX_SPECIES] = {};
         if (tiled && c->p.sort_fallback > 0 && l >= 2) {
-            HIP_TRY(hipEventSynchronize(c->ev[3 * (l - 1)]));
+            HIP_TRY(hipEventSynchronize(c->ev[3 * (l - 2) + 2]));
             const double *h = hd + (size_t)(l - 2) * kDiagLen;
             for (int s = 0; s < QK_MAX_SPECIES; ++s) {
                 const double live = h[s * kDiagPerSpecies + 2], fb = h[s * kDiagPerSpecies + 3];
@@ -940,20 +960,24 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
             const bool due = (c->p.sort_every > 0 && b.steps_since_sort >= c->p.sort_every) ||
                              (fb_high[s] && b.steps_since_sort >= 2);
             const bool tail = tiled && (b.n_sorted == 0 || (b.n - b.n_sorted) * 16 > b.n_sorted);
-            if (tail || due) QK_TRY(sort_species<real>(c, s));
+            if (tail || due) {
+                QK_TRY(sort_species<real>(c, s));
+                between = true;
+            }
         }
         // a merge decided after the previous step runs first (pmerging before
         // birth_from_vacuum, src/main.cpp:2321-2322)
         if (c->merge_due) {
             QK_TRY(merge_impl<real>(c, c->p.merging, c->merge_ppd));
             c->merge_due = false;
+            between = true;
         }
         const Current<real> jc = current_of<real>(c, c->jcur), jn = current_of<real>(c, c->jcur ^ 1);
-        HIP_TRY(launch_zero(c->stream, c->d_diag, kDiagLen));
         // padvance (src/advance.cpp:90-387); the push kernels erase the
         // particles p_boundary (src/plist.cpp:73-102) would: those outside
         // is_inside, which only a moving-window shift leaves behind
-        HIP_TRY(hipEventRecord(c->ev[3 * l], c->stream));
+        if (between) HIP_TRY(hipEventRecord(c->ev[3 * l], c->stream));
+        start[l] = between ? 3 * l : 3 * (l - 1) + 2;
         if (qed) QK_TRY(qed_particle_phase<real>(c, f, jc));
         for (int s = 0; s < QK_MAX_SPECIES && !qed; ++s) {
             SpeciesBuf &b = c->sp[s];
@@ -963,9 +987,9 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
             a.kind = b.kind;
             a.cmr = b.cmr;
             a.external_bz = c->p.external_bz;
-            a.diag = c->d_diag + s * kDiagPerSpecies;
+            a.diag = c->diag_row + s * kDiagPerSpecies;
             a.energy_mode = b.energy_mode;
-            a.nonfinite = c->d_diag + kNonfiniteSlot;
+            a.nonfinite = c->diag_row + kNonfiniteSlot;
             const Species<real> v = view<real>(b.buf[b.cur]);
             if (tp.tangent && !tp.replay && b.kind == 0 && tp.n[s] > 0) {
                 // the tangent of this push, from the state before it
@@ -995,28 +1019,38 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
         // fadvance (src/advance.cpp:13-18): B half, E, B half, interpolate_be.  The
         // first half step also sums compute_energy's field term, which sees the
         // fields before fadvance (src/main.cpp:2327)
-        HIP_TRY(launch_maxwell_b<real>(c->stream, c->p.solver, c->g, c->coef, f,
-                                       c->d_diag + QK_MAX_SPECIES * kDiagPerSpecies));
-        QK_TRY(inject_impl<real>(c, 1, 0.0));
-        HIP_TRY(launch_maxwell_e<real>(c->stream, c->p.solver, c->g, c->coef, f, jc, jn));
+        if (charged) c->j_zero[c->jcur] = false;
+        const bool no_j = !charged && c->j_zero[0] && c->j_zero[1], last = l + 1 == nsteps;
+        constexpr size_t en = QK_MAX_SPECIES * kDiagPerSpecies;
+        if (!fuse_b || l == 0) {
+            HIP_TRY(launch_maxwell_b<real>(c->stream, c->p.solver, c->g, c->coef, f, c->diag_row + en));
+            QK_TRY(inject_impl<real>(c, 1, 0.0));
+        }
+        const DiagDrain dd{c->diag_row, hd + (size_t)l * kDiagLen, (int)kDiagLen};
+        HIP_TRY(launch_maxwell_e<real>(c->stream, c->p.solver, c->g, c->coef, f, no_j ? nullptr : &jc,
+                                       no_j ? nullptr : &jn, dd));
+        c->j_zero[c->jcur ^ 1] = true;
         QK_TRY(inject_impl<real>(c, 0, 0.5));
-        HIP_TRY(launch_maxwell_b<real>(c->stream, c->p.solver, c->g, c->coef, f, nullptr));
-        QK_TRY(inject_impl<real>(c, 1, 1.0));
-        HIP_TRY(launch_interpolate_be<real>(c->stream, c->g, f));
+        if (fuse_b && !last) {
+            HIP_TRY(launch_maxwell_b<real>(c->stream, c->p.solver, c->g, c->coef, f,
+                                           c->d_diag + ((l + 1) & 1) * kDiagLen + en, true));
+        } else {
+            HIP_TRY(launch_maxwell_b<real>(c->stream, c->p.solver, c->g, c->coef, f, nullptr));
+            QK_TRY(inject_impl<real>(c, 1, 1.0));
+        }
+        if (charged || last) HIP_TRY(launch_interpolate_be<real>(c->stream, c->g, f));
         if (tp.tangent && !tp.replay) {
             // the tangent fields advance with the same (linear) field step
             const Fields<double> tf = tangent_fields(c);
             const Current<double> tjc = tangent_current(c, tp.tjcur), tjn = tangent_current(c, tp.tjcur ^ 1);
             HIP_TRY(launch_maxwell_b<double>(c->stream, c->p.solver, c->g, c->coef, tf, nullptr));
-            HIP_TRY(launch_maxwell_e<double>(c->stream, c->p.solver, c->g, c->coef, tf, tjc, tjn));
+            HIP_TRY(launch_maxwell_e<double>(c->stream, c->p.solver, c->g, c->coef, tf, &tjc, &tjn));
             HIP_TRY(launch_maxwell_b<double>(c->stream, c->p.solver, c->g, c->coef, tf, nullptr));
             HIP_TRY(launch_interpolate_be<double>(c->stream, c->g, tf));
             tp.tjcur ^= 1;
         }
         HIP_TRY(hipEventRecord(c->ev[3 * l + 2], c->stream));
         c->jcur ^= 1;
-        HIP_TRY(hipMemcpyAsync(hd + (size_t)l * kDiagLen, c->d_diag, kDiagLen * sizeof(double), hipMemcpyDeviceToHost,
-                               c->stream));
         if (qed) QK_TRY(qed_download_counts(c));
         if (c->p.merging) {
             HIP_TRY(hipStreamSynchronize(c->stream));
@@ -1028,7 +1062,7 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
     float t_part = 0, t_field = 0, t_tot = 0;
     for (int l = 0; l < nsteps; ++l) {
         float a = 0, b = 0;
-        HIP_TRY(hipEventElapsedTime(&a, c->ev[3 * l], c->ev[3 * l + 1]));
+        HIP_TRY(hipEventElapsedTime(&a, c->ev[start[l]], c->ev[3 * l + 1]));
         HIP_TRY(hipEventElapsedTime(&b, c->ev[3 * l + 1], c->ev[3 * l + 2]));
         t_part += a;
         t_field += b;
@@ -1316,7 +1350,7 @@ int qk_create(const qk_params *params, qk_ctx **out)
         return bail(fail(QK_ERR_HIP, std::string("field allocation: ") + hipGetErrorString(e)));
     if ((e = hipMemset(c->fmem, 0, fbytes * 15)) != hipSuccess) return bail(fail(QK_ERR_HIP, hipGetErrorString(e)));
     for (int a = 0; a < 15; ++a) c->F[a] = (char *)c->fmem + a * fbytes;
-    if ((e = hipMalloc(&c->d_diag, kDiagLen * sizeof(double))) != hipSuccess)
+    if ((e = hipMalloc(&c->d_diag, 2 * kDiagLen * sizeof(double))) != hipSuccess)
         return bail(fail(QK_ERR_HIP, hipGetErrorString(e)));
     if (p.qed) {
         if ((e = hipMalloc(&c->d_count, (QK_MAX_SPECIES + 1) * sizeof(int))) != hipSuccess ||

@@ -37,6 +37,46 @@ __device__ inline dim3 band_block()
     return dim3((unsigned)(vin % gridDim.x), (unsigned)(vin / gridDim.x), (unsigned)(l / q));
 }
 
+// The Maxwell sweeps take a plane's cells as one run (j, k flattened), in
+// blocks of kSweep, so that no lane is idle whatever nz is (64-column blocks
+// left 22 % of them idle at nz = 199, 45 % at 71 and half at 32).  Planes of
+// at least kBandMin blocks are dealt to the XCDs in bands as above, the
+// blocks per plane rounded up to a multiple of 8 (under 12 % empty blocks);
+// smaller ones in launch order.  Bound by HBM (3.0 -> 4.2 TB/s at 301x203x199,
+// where a plain copy reaches 4.8): B 145 -> 102 us there, 13.4 -> 10.2 us at
+// 135x75x71 (NDFX), 285 -> 277 us at 512x256x256, 35.6 -> 37.1 us at
+// 256x128x128 (NDFX; the division per cell).
+constexpr int kSweep = 256, kBandMin = 64;
+
+struct SweepPlan {
+    int per;      // blocks per plane, empty ones included
+    bool banded;
+};
+
+inline SweepPlan sweep_plan(const Grid &g)
+{
+    const int P = (g.sx + kSweep - 1) / kSweep;
+    return P >= kBandMin ? SweepPlan{(P + 7) / 8 * 8, true} : SweepPlan{P, false};
+}
+
+// this thread's cell; false past the plane's end
+__device__ inline bool sweep_cell(const Grid &g, const SweepPlan &sw, int &i, int &j, int &k)
+{
+    int vin;
+    if (sw.banded) {
+        const int q = sw.per / 8, l = blockIdx.x / 8;
+        i = l / q;
+        vin = (int)(blockIdx.x % 8) * q + l % q;
+    } else {
+        i = blockIdx.x / sw.per;
+        vin = blockIdx.x % sw.per;
+    }
+    const int t = vin * kSweep + (int)threadIdx.x;
+    j = t / g.nz;
+    k = t - j * g.nz;
+    return t < g.sx;
+}
+
 __device__ inline bool in(int v, int lo, int hi) { return v >= lo && v <= hi; }
 
 // which cells get component C of B updated
@@ -136,73 +176,97 @@ __device__ inline real diff(const Grid &g, const Coef<real> &cf, const real *__r
 // energy != null the first half step also sums E^2 + B^2 of the fields it
 // starts from, in FP64: compute_energy's field term, which the reference takes
 // between padvance and fadvance (src/fout.cpp:102, src/main.cpp:2327-2331).
-template <int S, typename real>
-__global__ void __launch_bounds__(kBX * kBY) k_maxwell_b(Grid g, Coef<real> cf, const real *__restrict__ ex,
-                                                         const real *__restrict__ ey, const real *__restrict__ ez,
-                                                         real *__restrict__ bx, real *__restrict__ by,
-                                                         real *__restrict__ bz, double *energy)
+//
+// TWICE: the second half step of one step and the first of the next, which
+// use the same E when nothing reads B in between; the energy is that of the
+// fields between the two.  36 instead of 72 B per cell: 104 us at 301x203x199,
+// against 102 us for each half step.
+template <int S, bool TWICE, typename real>
+__global__ void __launch_bounds__(kSweep) k_maxwell_b(Grid g, SweepPlan sw, Coef<real> cf, const real *__restrict__ ex,
+                                                      const real *__restrict__ ey, const real *__restrict__ ez,
+                                                      real *__restrict__ bx, real *__restrict__ by,
+                                                      real *__restrict__ bz, double *energy)
 {
-    __shared__ double part[kBX * kBY / 64];
-    const dim3 vb = band_block();
-    const int k = vb.x * kBX + threadIdx.x;
-    const int j = vb.y * kBY + threadIdx.y;
-    const int i = vb.z;
+    __shared__ double part[kSweep / 64];
+    int i, j, k;
     double en = 0;
-    if (k < g.nz && j < g.ny) {
+    if (sweep_cell(g, sw, i, j, k)) {
         const int id = i * g.sx + j * g.sy + k;
         const real h = real(0.5);
-        const real b0 = bx[id], b1 = by[id], b2 = bz[id];
-        if (energy) {
+        real b0 = bx[id], b1 = by[id], b2 = bz[id];
+        auto add_energy = [&] {
             const double e0 = ex[id], e1 = ey[id], e2 = ez[id];
             en = e0 * e0 + e1 * e1 + e2 * e2 + (double)b0 * b0 + (double)b1 * b1 + (double)b2 * b2;
+        };
+        if (energy && !TWICE) add_energy();
+        const bool u0 = b_updates<S, 0>(g, i, j, k), u1 = b_updates<S, 1>(g, i, j, k), u2 = b_updates<S, 2>(g, i, j, k);
+        real d0 = real(0), d1 = real(0), d2 = real(0);
+        if (u0) d0 = -cf.dtd[1] * diff<S, 2, 1, true>(g, cf, ez, i, j, k) + cf.dtd[2] * diff<S, 1, 2, true>(g, cf, ey, i, j, k);
+        if (u1) d1 = cf.dtd[0] * diff<S, 2, 0, true>(g, cf, ez, i, j, k) - cf.dtd[2] * diff<S, 0, 2, true>(g, cf, ex, i, j, k);
+        if (u2) d2 = cf.dtd[1] * diff<S, 0, 1, true>(g, cf, ex, i, j, k) - cf.dtd[0] * diff<S, 1, 0, true>(g, cf, ey, i, j, k);
+        if (u0) b0 += h * d0;
+        if (u1) b1 += h * d1;
+        if (u2) b2 += h * d2;
+        if (TWICE) {
+            if (energy) add_energy();
+            if (u0) b0 += h * d0;
+            if (u1) b1 += h * d1;
+            if (u2) b2 += h * d2;
         }
-        if (b_updates<S, 0>(g, i, j, k))
-            bx[id] = b0 + h * (-cf.dtd[1] * diff<S, 2, 1, true>(g, cf, ez, i, j, k) + cf.dtd[2] * diff<S, 1, 2, true>(g, cf, ey, i, j, k));
-        if (b_updates<S, 1>(g, i, j, k))
-            by[id] = b1 + h * (cf.dtd[0] * diff<S, 2, 0, true>(g, cf, ez, i, j, k) - cf.dtd[2] * diff<S, 0, 2, true>(g, cf, ex, i, j, k));
-        if (b_updates<S, 2>(g, i, j, k))
-            bz[id] = b2 + h * (cf.dtd[1] * diff<S, 0, 1, true>(g, cf, ex, i, j, k) - cf.dtd[0] * diff<S, 1, 0, true>(g, cf, ey, i, j, k));
+        if (u0) bx[id] = b0;
+        if (u1) by[id] = b1;
+        if (u2) bz[id] = b2;
     }
     if (energy) {   // uniform across the launch
         en = wave_sum(en);
-        const int t = threadIdx.y * kBX + threadIdx.x;
+        const int t = threadIdx.x;
         if ((t & 63) == 0) part[t >> 6] = en;
         __syncthreads();
         if (t == 0) {
             double s = 0;
-            for (int w = 0; w < kBX * kBY / 64; ++w) s += part[w];
-            const int slot = (int)((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) % kEnergySlots;
-            atomicAdd(energy + slot, s);
+            for (int w = 0; w < kSweep / 64; ++w) s += part[w];
+            atomicAdd(energy + blockIdx.x % kEnergySlots, s);
         }
     }
 }
 
 // E step with the current of this step; also clears the other current
 // buffer, which the next step deposits into (replaces the J reset of
-// src/advance.cpp:112-123 without a separate pass)
-template <int S, typename real>
-__global__ void __launch_bounds__(kBX * kBY) k_maxwell_e(Grid g, Coef<real> cf, real *__restrict__ ex, real *__restrict__ ey,
-                                                         real *__restrict__ ez, const real *__restrict__ bx,
-                                                         const real *__restrict__ by, const real *__restrict__ bz,
-                                                         const real *__restrict__ jx, const real *__restrict__ jy,
-                                                         const real *__restrict__ jz, real *__restrict__ njx,
-                                                         real *__restrict__ njy, real *__restrict__ njz)
+// src/advance.cpp:112-123 without a separate pass).  CUR false: both current
+// buffers are known to be zero (no charged particles), 36 instead of 60 B per
+// cell (92 us instead of 200 at 301x203x199, the sweep order included).  The last workgroup also hands the step's diagnostics over, complete
+// by now: the accumulators go to pinned host memory and are cleared for the
+// step after next.
+template <int S, bool CUR, typename real>
+__global__ void __launch_bounds__(kSweep) k_maxwell_e(Grid g, SweepPlan sw, Coef<real> cf, real *__restrict__ ex,
+                                                      real *__restrict__ ey, real *__restrict__ ez,
+                                                      const real *__restrict__ bx, const real *__restrict__ by,
+                                                      const real *__restrict__ bz, const real *__restrict__ jx,
+                                                      const real *__restrict__ jy, const real *__restrict__ jz,
+                                                      real *__restrict__ njx, real *__restrict__ njy,
+                                                      real *__restrict__ njz, DiagDrain dd)
 {
-    const dim3 vb = band_block();
-    const int k = vb.x * kBX + threadIdx.x;
-    const int j = vb.y * kBY + threadIdx.y;
-    const int i = vb.z;
-    if (k >= g.nz || j >= g.ny) return;
+    if (dd.n > 0 && blockIdx.x == gridDim.x - 1)
+        for (int t = threadIdx.x; t < dd.n; t += kSweep) {
+            dd.host[t] = dd.acc[t];
+            dd.acc[t] = 0.0;
+        }
+    int i, j, k;
+    if (!sweep_cell(g, sw, i, j, k)) return;
     const int id = i * g.sx + j * g.sy + k;
+    const real c0 = CUR ? jx[id] * cf.d[0] : real(0), c1 = CUR ? jy[id] * cf.d[1] : real(0),
+               c2 = CUR ? jz[id] * cf.d[2] : real(0);
     if (e_updates<S, 0>(g, i, j, k))
-        ex[id] += cf.dtd[1] * diff<S, 2, 1, false>(g, cf, bz, i, j, k) - cf.dtd[2] * diff<S, 1, 2, false>(g, cf, by, i, j, k) - jx[id] * cf.d[0];
+        ex[id] += cf.dtd[1] * diff<S, 2, 1, false>(g, cf, bz, i, j, k) - cf.dtd[2] * diff<S, 1, 2, false>(g, cf, by, i, j, k) - c0;
     if (e_updates<S, 1>(g, i, j, k))
-        ey[id] += -cf.dtd[0] * diff<S, 2, 0, false>(g, cf, bz, i, j, k) + cf.dtd[2] * diff<S, 0, 2, false>(g, cf, bx, i, j, k) - jy[id] * cf.d[1];
+        ey[id] += -cf.dtd[0] * diff<S, 2, 0, false>(g, cf, bz, i, j, k) + cf.dtd[2] * diff<S, 0, 2, false>(g, cf, bx, i, j, k) - c1;
     if (e_updates<S, 2>(g, i, j, k))
-        ez[id] += cf.dtd[0] * diff<S, 1, 0, false>(g, cf, by, i, j, k) - cf.dtd[1] * diff<S, 0, 1, false>(g, cf, bx, i, j, k) - jz[id] * cf.d[2];
-    njx[id] = real(0);
-    njy[id] = real(0);
-    njz[id] = real(0);
+        ez[id] += cf.dtd[0] * diff<S, 1, 0, false>(g, cf, by, i, j, k) - cf.dtd[1] * diff<S, 0, 1, false>(g, cf, bx, i, j, k) - c2;
+    if (CUR) {
+        njx[id] = real(0);
+        njy[id] = real(0);
+        njz[id] = real(0);
+    }
 }
 
 // Be = B averaged to E positions (src/advance.cpp:20-83): each component is
@@ -581,27 +645,33 @@ hipError_t launch_zero(hipStream_t st, double *p, size_t n)
 
 template <typename real>
 hipError_t launch_maxwell_b(hipStream_t st, int solver, const Grid &g, const SolverCoef &c, const Fields<real> &f,
-                            double *energy)
+                            double *energy, bool twice)
 {
     const Coef<real> cf = make_coef<real>(g, c);
-    const dim3 grid = cell_grid(g), block(kBX, kBY);
-    if (solver == 0) k_maxwell_b<0, real><<<grid, block, 0, st>>>(g, cf, f.ex, f.ey, f.ez, f.bx, f.by, f.bz, energy);
-    else if (solver == 1) k_maxwell_b<1, real><<<grid, block, 0, st>>>(g, cf, f.ex, f.ey, f.ez, f.bx, f.by, f.bz, energy);
-    else k_maxwell_b<2, real><<<grid, block, 0, st>>>(g, cf, f.ex, f.ey, f.ez, f.bx, f.by, f.bz, energy);
+    const SweepPlan sw = sweep_plan(g);
+    const dim3 grid((unsigned)(sw.per * g.nx));
+#define QK_B(S, T) k_maxwell_b<S, T, real><<<grid, kSweep, 0, st>>>(g, sw, cf, f.ex, f.ey, f.ez, f.bx, f.by, f.bz, energy)
+    if (solver == 0) { if (twice) QK_B(0, true); else QK_B(0, false); }
+    else if (solver == 1) { if (twice) QK_B(1, true); else QK_B(1, false); }
+    else { if (twice) QK_B(2, true); else QK_B(2, false); }
+#undef QK_B
     return hipGetLastError();
 }
 
 template <typename real>
 hipError_t launch_maxwell_e(hipStream_t st, int solver, const Grid &g, const SolverCoef &c, const Fields<real> &f,
-                            const Current<real> &j, const Current<real> &jn)
+                            const Current<real> *j, const Current<real> *jn, const DiagDrain &dd)
 {
     const Coef<real> cf = make_coef<real>(g, c);
-    const dim3 grid = cell_grid(g), block(kBX, kBY);
-#define QK_E_ARGS g, cf, f.ex, f.ey, f.ez, f.bx, f.by, f.bz, j.jx, j.jy, j.jz, jn.jx, jn.jy, jn.jz
-    if (solver == 0) k_maxwell_e<0, real><<<grid, block, 0, st>>>(QK_E_ARGS);
-    else if (solver == 1) k_maxwell_e<1, real><<<grid, block, 0, st>>>(QK_E_ARGS);
-    else k_maxwell_e<2, real><<<grid, block, 0, st>>>(QK_E_ARGS);
-#undef QK_E_ARGS
+    const SweepPlan sw = sweep_plan(g);
+    const dim3 grid((unsigned)(sw.per * g.nx));
+    const Current<real> none{nullptr, nullptr, nullptr}, a = j ? *j : none, b = j ? *jn : none;
+#define QK_E(S, C) k_maxwell_e<S, C, real><<<grid, kSweep, 0, st>>>(g, sw, cf, f.ex, f.ey, f.ez, f.bx, f.by, f.bz, a.jx, \
+                                                                   a.jy, a.jz, b.jx, b.jy, b.jz, dd)
+    if (solver == 0) { if (j) QK_E(0, true); else QK_E(0, false); }
+    else if (solver == 1) { if (j) QK_E(1, true); else QK_E(1, false); }
+    else { if (j) QK_E(2, true); else QK_E(2, false); }
+#undef QK_E
     return hipGetLastError();
 }
 
@@ -704,9 +774,9 @@ hipError_t launch_inject(hipStream_t st, int solver, const Grid &g, const Solver
 
 #define QK_INST(real)                                                                                            \
     template hipError_t launch_maxwell_b<real>(hipStream_t, int, const Grid &, const SolverCoef &, const Fields<real> &, \
-                                               double *);                                                       \
+                                               double *, bool);                                                 \
     template hipError_t launch_maxwell_e<real>(hipStream_t, int, const Grid &, const SolverCoef &, const Fields<real> &, \
-                                               const Current<real> &, const Current<real> &);                   \
+                                               const Current<real> *, const Current<real> *, const DiagDrain &); \
     template hipError_t launch_interpolate_be<real>(hipStream_t, const Grid &, const Fields<real> &);           \
     template hipError_t launch_init_boundaries<real>(hipStream_t, int, const Grid &, const Fields<real> &);     \
     template hipError_t launch_laser_cos<real>(hipStream_t, const Grid &, const Fields<real> &, const double *); \

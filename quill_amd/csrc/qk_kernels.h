@@ -156,13 +156,21 @@ hipError_t launch_adj_particles(hipStream_t st, const Grid &g, const Fields<real
 constexpr int kEnergySlots = 256;
 
 // half step of B; with energy != null also accumulates sum(E^2 + B^2) of the
-// incoming fields into energy[0 .. kEnergySlots) (FP64)
+// incoming fields into energy[0 .. kEnergySlots) (FP64).  twice: two half
+// steps with the same E, the energy taken between them.
 template <typename real>
 hipError_t launch_maxwell_b(hipStream_t st, int solver, const Grid &g, const SolverCoef &c, const Fields<real> &f,
-                            double *energy);
+                            double *energy, bool twice = false);
+// n accumulators that the E step copies to pinned host memory and clears
+struct DiagDrain {
+    double *acc = nullptr, *host = nullptr;
+    int n = 0;
+};
+// E step; j (may be null: both buffers are zero) the step's current, jn the
+// buffer to clear for the next
 template <typename real>
 hipError_t launch_maxwell_e(hipStream_t st, int solver, const Grid &g, const SolverCoef &c, const Fields<real> &f,
-                            const Current<real> &j, const Current<real> &j_next);
+                            const Current<real> *j, const Current<real> *jn, const DiagDrain &dd = DiagDrain());
 template <typename real>
 hipError_t launch_interpolate_be(hipStream_t st, const Grid &g, const Fields<real> &f);
 template <typename real>
