@@ -1140,14 +1140,14 @@ int download_fields(qk_ctx *c, int nf, double *const *aos, void *const (*comp)[3
     const size_t node = 3 * c->rsize, total = (size_t)nf * n * node;
     const int64_t per = (int64_t)(Drain::slot_bytes(total) / node);   // nodes per block
     const int64_t nb = (n + per - 1) / per;                            // blocks per field
-    auto launch = [&](int64_t b, void *slot) {
+    auto launch = [&](int64_t b, void *slot, const ReadDone &done) {
         void *const *s = comp[b / nb];
         const int64_t first = b % nb * per;
         const int m = (int)std::min(per, n - first);
         return c->rsize == 4 ? launch_pack_fields<float>(c->stream, (const float *)s[0], (const float *)s[1],
-                                                         (const float *)s[2], first, m, (float *)slot)
+                                                         (const float *)s[2], first, m, (float *)slot, done)
                              : launch_pack_fields<double>(c->stream, (const double *)s[0], (const double *)s[1],
-                                                          (const double *)s[2], first, m, (double *)slot);
+                                                          (const double *)s[2], first, m, (double *)slot, done);
     };
     auto take = [&](int64_t b, const void *slot) {
         const int64_t first = b % nb * per;
@@ -1201,9 +1201,9 @@ int download_particles(qk_ctx *c, const SpeciesBuf &b, const std::vector<int> &o
     // a slot holds `per` rows: the reals first (aligned), then cells and ids
     auto reals = [&](void *slot) { return (real *)slot; };
     auto cells = [&](void *slot) { return (int *)((char *)slot + (size_t)per * nreal * sizeof(real)); };
-    auto launch = [&](int64_t k, void *slot) {
+    auto launch = [&](int64_t k, void *slot, const ReadDone &done) {
         return launch_pack_live<real>(c->stream, v, k * per, std::min(b.n, (k + 1) * per), c->d_live, (int)per,
-                                      cells(slot), reals(slot), cells(slot) + per);
+                                      cells(slot), reals(slot), cells(slot) + per, done);
     };
     const double cmr = b.cmr;
     const bool photon = b.kind == 1;
@@ -1240,11 +1240,11 @@ int download_doubles(qk_ctx *c, double *dst, const double *src, int64_t n)
 {
     const size_t total = (size_t)n * sizeof(double);
     const int64_t per = (int64_t)(Drain::slot_bytes(total) / sizeof(double));
-    auto count = [&](int64_t b) { return (size_t)std::min(per, n - b * per) * sizeof(double); };
-    auto launch = [&](int64_t b, void *slot) {
-        return hipMemcpyAsync(slot, src + b * per, count(b), hipMemcpyDeviceToHost, c->stream);
+    auto count = [&](int64_t b) { return (size_t)std::min(per, n - b * per); };
+    auto launch = [&](int64_t b, void *slot, const ReadDone &done) {
+        return launch_copy_out(c->stream, src + b * per, (int)count(b), (double *)slot, done);
     };
-    auto take = [&](int64_t b, const void *slot) { std::memcpy(dst + b * per, slot, count(b)); };
+    auto take = [&](int64_t b, const void *slot) { std::memcpy(dst + b * per, slot, count(b) * sizeof(double)); };
     HIP_TRY(c->drain.run(c->p.device, c->stream, total, (n + per - 1) / per, launch, take));
     return QK_OK;
 }

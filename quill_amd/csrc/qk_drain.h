@@ -1,22 +1,28 @@
 // qk_drain.h -- results on their way to the caller's arrays (host side).
 //
-// A read-back is a list of blocks.  For each, `launch` enqueues a kernel (or
-// copy) that writes the block into a pinned slot, and `take` moves the slot
-// into the caller's array (widening FP32 to FP64).  Every worker owns two
-// slots and has its next block on the stream while it takes the previous
-// one, so the link, the conversion and the page faults of a fresh array
-// overlap.  A single-threaded conversion from pageable copies took 564 ms
-// for the four fields of 512x256x256 cells (3.2 GB in FP64): most of it the
-// first touch of the caller's pages, which threads share.
+// A read-back is a list of blocks.  For each, `launch` enqueues a kernel that
+// writes the block into a pinned slot and then the slot's flag, and `take`
+// moves the slot into the caller's array (widening FP32 to FP64).  Every
+// worker owns two slots and has its next block on the stream while it takes
+// the previous one, so the link, the conversion and the page faults of a
+// fresh array overlap; the workers are the calling thread and the context's
+// helpers.  A single-threaded conversion from pageable copies took 564 ms
+// for the four fields of 512x256x256 cells (3.2 GB in FP64), most of it the
+// first touch of the caller's pages, which threads share: 46 ms.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <exception>
+#include <functional>
+#include <mutex>
 #include <thread>
 #include <vector>
+
+#include "qk_kernels.h"
 
 namespace qk {
 
@@ -46,33 +52,47 @@ public:
     // 96 GB/s (16: 104), against 110 GB/s of widened numbers from the link.
     static constexpr size_t kSlot = (size_t)2 << 20;
     static constexpr int kWorkers = 8;
-    // Reads below kSmall take slots of kSmallSlot: pinned allocations up to
+    // A read of less than kShare is taken by the calling thread alone, and no
+    // read waits for a helper that has not woken up yet: with the caller's own
+    // thread pool still spinning (torch after a parallel region) a new thread
+    // got a CPU only after 3 ms, against 0.4 ms for the whole read of
+    // 64x32x32 cells.  It has one slot, a small one (pinned allocations up to
     // 1 MiB cost 20 us, larger ones 340 us or more, and a short run reads
-    // its fields once.
-    static constexpr size_t kSmall = (size_t)12 << 20, kSmallSlot = (size_t)256 << 10;
+    // once), and sleeps in the stream's synchronization instead of polling.
+    static constexpr size_t kShare = (size_t)8 << 20, kAloneSlot = (size_t)960 << 10;
 
-    static size_t slot_bytes(size_t total) { return total < kSmall ? kSmallSlot : kSlot; }
+    static size_t slot_bytes(size_t total) { return total < kShare ? kAloneSlot : kSlot; }
 
-    // launch(block, slot) -> hipError_t; take(block, slot).  `total` is the
-    // size of the whole read in the slots' format; `device` is current in the
-    // calling thread.  On return the stream has no work left that writes a
-    // slot.
+    // launch(block, slot, done) -> hipError_t; take(block, slot).  `total` is
+    // the size of the whole read in the slots' format; `device` is current in
+    // the calling thread.  On return the stream is idle.
     template <class Launch, class Take>
     hipError_t run(int device, hipStream_t st, size_t total, int64_t nblocks, Launch &&launch, Take &&take)
     {
         if (nblocks <= 0) return hipSuccess;
         const size_t slot = slot_bytes(total);
-        // a worker for every two blocks, at least 1 MiB each
-        int nw = (int)std::min<int64_t>(std::min<int64_t>(kWorkers, (nblocks + 1) / 2), (int64_t)(total >> 20) + 1);
-        nw = std::max(1, std::min(nw, (int)std::max(1u, std::thread::hardware_concurrency())));
-        if (hipError_t e = reserve(slot * 2 * nw, 2 * nw)) return e;
+        if (total < kShare) {
+            if (hipError_t e = reserve(st, slot)) return e;
+            void *at = pin_ + kFlagBytes;
+            for (int64_t b = 0; b < nblocks; ++b) {
+                if (hipError_t e = launch(b, at, ReadDone{arrived_, flag(0), ++seq_[0]})) return e;
+                if (hipError_t e = hipStreamSynchronize(st)) return e;
+                take(b, at);
+            }
+            return hipSuccess;
+        }
+        // a worker for every two blocks
+        int nw = (int)std::min<int64_t>(kWorkers, (nblocks + 1) / 2);
+        nw = std::max(1, std::min(nw, (int)std::thread::hardware_concurrency()));
+        if (hipError_t e = reserve(st, slot * 2 * nw)) return e;
         std::atomic<int64_t> next{0};
         std::atomic<int> err{hipSuccess};
         auto work = [&](int w) {
             hipError_t e = w > 0 ? hipSetDevice(device) : hipSuccess;   // a new thread starts on device 0
+            auto at = [&](int h) { return pin_ + kFlagBytes + slot * (2 * w + h); };
             auto start = [&](int64_t b, int h) {
-                if (e == hipSuccess) e = launch(b, pin_ + slot * (2 * w + h));
-                if (e == hipSuccess) e = hipEventRecord(ev_[2 * w + h], st);
+                const int s = 2 * w + h;
+                if (e == hipSuccess) e = launch(b, (void *)at(h), ReadDone{arrived_ + s, flag(s), ++seq_[s]});
             };
             int64_t b = next++;
             int h = 0;
@@ -80,43 +100,114 @@ public:
             while (b < nblocks && e == hipSuccess && err.load() == hipSuccess) {
                 const int64_t b2 = next++;
                 if (b2 < nblocks) start(b2, h ^ 1);
-                if (e == hipSuccess) e = hipEventSynchronize(ev_[2 * w + h]);
-                if (e == hipSuccess) take(b, pin_ + slot * (2 * w + h));
+                if (e == hipSuccess) e = wait(st, 2 * w + h);
+                if (e == hipSuccess) take(b, (void *)at(h));
                 b = b2;
                 h ^= 1;
             }
             if (e != hipSuccess) err.store((int)e);
         };
-        std::vector<std::thread> helpers;
-        try {
-            helpers.reserve((size_t)nw);
-            for (int w = 1; w < nw; ++w) helpers.emplace_back(work, w);
-        } catch (const std::exception &) {
-            // fewer workers than asked for: the ones that started and this
-            // thread take all blocks
-        }
+        open_job(nw, work);
         work(0);
-        for (auto &t : helpers) t.join();
+        close_job();
         const hipError_t e = hipStreamSynchronize(st);
         return err.load() != hipSuccess ? (hipError_t)err.load() : e;
     }
 
     hipError_t release()
     {
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            stop_ = true;
+        }
+        wake_.notify_all();
+        for (auto &t : helpers_) t.join();
+        helpers_.clear();
         hipError_t first = pin_ ? hipHostFree(pin_) : hipSuccess;
-        pin_ = nullptr;
-        cap_ = 0;
-        for (hipEvent_t ev : ev_) {
-            const hipError_t e = hipEventDestroy(ev);
+        if (arrived_) {
+            const hipError_t e = hipFree(arrived_);
             if (first == hipSuccess) first = e;
         }
-        ev_.clear();
+        pin_ = nullptr;
+        arrived_ = nullptr;
+        cap_ = 0;
         return first;
     }
 
 private:
-    hipError_t reserve(size_t bytes, int events)
+    // each slot's flag in a cache line of its own, before the slots
+    static constexpr size_t kFlagLine = 128, kFlagBytes = kFlagLine * 2 * kWorkers;
+    unsigned *flag(int s) const { return (unsigned *)(pin_ + kFlagLine * s); }
+
+    // until slot s holds its block.  The flag comes with the launch; should
+    // the stream end without it, the launch failed.
+    hipError_t wait(hipStream_t st, int s)
     {
+        const std::atomic<unsigned> *f = (const std::atomic<unsigned> *)flag(s);
+        const unsigned want = seq_[s];
+        for (unsigned spins = 1; f->load(std::memory_order_acquire) != want; ++spins) {
+            if (spins % 65536 == 0) {
+                const hipError_t e = hipStreamQuery(st);
+                if (e == hipErrorNotReady) continue;
+                if (e != hipSuccess) return e;
+                return f->load(std::memory_order_acquire) == want ? hipSuccess : hipErrorLaunchFailure;
+            }
+#if defined(__x86_64__)
+            __builtin_ia32_pause();
+#endif
+        }
+        return hipSuccess;
+    }
+
+    // helpers sleep between reads and live as long as the context
+    void open_job(int nw, std::function<void(int)> work)
+    {
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            work_ = std::move(work);
+            want_ = nw;
+            index_ = 1;   // worker 0 is the calling thread
+        }
+        try {
+            while ((int)helpers_.size() < nw - 1) helpers_.emplace_back([this] { help(); });
+        } catch (const std::exception &) {
+            // fewer helpers than asked for: those that started and the
+            // calling thread take all blocks
+        }
+        wake_.notify_all();
+    }
+
+    void close_job()
+    {
+        std::unique_lock<std::mutex> lock(mu_);
+        want_ = 0;
+        idle_.wait(lock, [this] { return busy_ == 0; });
+    }
+
+    void help()
+    {
+        std::unique_lock<std::mutex> lock(mu_);
+        for (;;) {
+            wake_.wait(lock, [this] { return stop_ || index_ < want_; });
+            if (stop_) return;
+            const int w = index_++;
+            ++busy_;
+            lock.unlock();
+            work_(w);
+            lock.lock();
+            if (--busy_ == 0) idle_.notify_one();
+        }
+    }
+
+    hipError_t reserve(hipStream_t st, size_t slots)
+    {
+        if (!arrived_) {
+            void *p = nullptr;
+            if (hipError_t e = hipMalloc(&p, 2 * kWorkers * sizeof(unsigned))) return e;
+            arrived_ = (unsigned *)p;
+            if (hipError_t e = launch_fill_int(st, (int *)arrived_, 2 * kWorkers, 0)) return e;
+        }
+        const size_t bytes = kFlagBytes + slots;
         if (cap_ < bytes) {
             if (pin_) {
                 if (hipError_t e = hipHostFree(pin_)) return e;
@@ -127,18 +218,24 @@ private:
             if (hipError_t e = hipHostMalloc(&p, bytes)) return e;
             pin_ = (char *)p;
             cap_ = bytes;
-        }
-        while ((int)ev_.size() < events) {
-            hipEvent_t ev;
-            if (hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) return e;
-            ev_.push_back(ev);
+            for (int s = 0; s < 2 * kWorkers; ++s) {
+                seq_[s] = 0;
+                *flag(s) = 0;
+            }
         }
         return hipSuccess;
     }
 
-    char *pin_ = nullptr;   // the workers' slots
+    char *pin_ = nullptr;   // flags, then the workers' slots
     size_t cap_ = 0;
-    std::vector<hipEvent_t> ev_;
+    unsigned *arrived_ = nullptr;   // workgroups of each slot's launch that are done
+    unsigned seq_[2 * kWorkers] = {};
+    std::mutex mu_;
+    std::condition_variable wake_, idle_;
+    std::vector<std::thread> helpers_;
+    std::function<void(int)> work_;
+    int want_ = 0, index_ = 0, busy_ = 0;   // workers of the open read, the next one's index, those at work
+    bool stop_ = false;
 };
 
 }  // namespace qk

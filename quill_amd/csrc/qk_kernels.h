@@ -214,17 +214,26 @@ hipError_t launch_compute_rho(hipStream_t st, const Grid &g, const Species<real>
 
 // slots per run of the live-particle counts
 constexpr int kLiveRun = 1024;
-// out[3 m + c] = component c at node first + m, m in [0, n)
+// how a pack kernel tells the host that its block is complete: the last of
+// its workgroups (counted in arrived, left at zero) stores seq to flag
+struct ReadDone {
+    unsigned *arrived;   // device memory
+    unsigned *flag;      // pinned host memory
+    unsigned seq;
+};
+// out[3 m + c] = component c at node first + m, m in [0, n), n > 0
 template <typename real>
 hipError_t launch_pack_fields(hipStream_t st, const real *a, const real *b, const real *c, int64_t first, int n,
-                              real *out);
+                              real *out, const ReadDone &done);
+// out[m] = src[m], m in [0, n), n > 0
+hipError_t launch_copy_out(hipStream_t st, const double *src, int n, double *out, const ReadDone &done);
 // counts[r] = live particles of slots [r kLiveRun, (r + 1) kLiveRun) below n
 hipError_t launch_count_live(hipStream_t st, const int *cell, int64_t n, int *counts);
-// the live slots of [first, end) (first a multiple of kLiveRun) in slot order,
+// the live slots of [first, end) (not empty, first a multiple of kLiveRun) in slot order,
 // one array per record entry, `stride` entries apart; offs: scanned counts
 template <typename real>
 hipError_t launch_pack_live(hipStream_t st, const Species<real> &s, int64_t first, int64_t end, const int *offs,
-                            int stride, int *cell_out, real *real_out, int *id_out);
+                            int stride, int *cell_out, real *real_out, int *id_out, const ReadDone &done);
 
 // ---- cell-tile counting sort ----------------------------------------------
 
