@@ -292,7 +292,7 @@ int reserve(qk_ctx *c, int s, int64_t cap)
     b.cur = 0;
     b.cap = cap;
     // work list capacity: every tile may end in a partial chunk
-    const int64_t mc = (int64_t)c->tg.ntiles + cap / kChunk + 1;
+    const int64_t mc = (int64_t)c->tg.ntiles + cap / kMinChunk + 1;
     if (b.chunks) HIP_TRY(hipFree(b.chunks));
     b.chunks = nullptr;
     HIP_TRY(hipMalloc(&b.chunks, (size_t)mc * sizeof(int4)));
@@ -345,6 +345,26 @@ int ensure_sort_buffers(qk_ctx *c)
     return QK_OK;
 }
 
+// Most particles per workgroup of the tiled push.  With at least half as many
+// tiles as the chip has CUs a tile is one chunk (kChunk).  Fewer tiles leave
+// CUs idle and run their particles in long serial rounds, so they are cut
+// into as many parts as give one workgroup per CU: 1.3 covers the tiles at
+// the box's faces, which hold less than the inner ones.  A second workgroup
+// per CU (FP32 only: two fit) pays for its own staging and flush, some four
+// rounds' time, only where the parts stay above half of kChunk.  Particle
+// phase at 128 tiles, 8 per cell: 36.8 -> 26.5 us (33.9 with four parts per
+// tile, 31.9 with 4096 per part), FP64 45.6 -> 30.3; 27 per cell: 57.0 ->
+// 47.1 us (51.9 at three parts, 62.5 at six); 27 tiles: 32.7 -> 15.4 us.  At
+// 432 tiles halves take 70 us against 61.
+int chunk_size(const qk_ctx *c, int64_t n)
+{
+    constexpr int kCU = 256;
+    if (c->tg.ntiles > kCU / 2) return kChunk;
+    int64_t chunk = (13 * n / 10 + kCU - 1) / kCU;
+    if (c->rsize == 4 && chunk > kChunk / 2) chunk = (chunk + 1) / 2;
+    return (int)std::min<int64_t>(std::max<int64_t>(chunk, kMinChunk), kChunk);
+}
+
 // sort species s by (tile, cell), compacting free slots; builds its work list
 template <typename real>
 int sort_species(qk_ctx *c, int s)
@@ -365,6 +385,7 @@ int sort_species(qk_ctx *c, int s)
     sb.chunks = b.chunks;
     sb.scratch = c->s_scratch;
     sb.max_chunks = b.max_chunks;
+    sb.chunk = chunk_size(c, b.n);
     HIP_TRY(launch_sort<real>(c->stream, c->tg, view<real>(b.buf[b.cur]), view<real>(b.buf[b.cur ^ 1]), b.n, sb));
     HIP_TRY(hipMemcpyAsync(b.d_nchunks, c->s_chunk_off + c->tg.ntiles, sizeof(int), hipMemcpyDeviceToDevice, c->stream));
     HIP_TRY(hipMemcpyAsync(b.tile_start, c->s_tile_start, ((size_t)c->tg.ntiles + 1) * sizeof(int),

@@ -22,8 +22,9 @@ constexpr int kDiagPerSpecies = 4;
 // most particles per workgroup of the tiled kernel (a chunk never spans two
 // tiles; a tile is cut into equal chunks).  Twice the mean tile population at
 // 8 per cell, so a uniform plasma's tile is one chunk: 4096 measured 15 %
-// slower on the push, 2048 30 %, from staging tiles more than once
-constexpr int kChunk = 8192;
+// slower on the push, 2048 30 %, from staging tiles more than once.  A grid of
+// few tiles takes smaller chunks, at least kMinChunk (see chunk_size)
+constexpr int kChunk = 8192, kMinChunk = 512;
 
 struct PushArgs {
     int pusher;              // 0 Vay, 1 Boris
@@ -253,6 +254,7 @@ struct SortBuffers {
     int4 *chunks;     // max_chunks
     int *scratch;     // scan scratch
     int max_chunks;
+    int chunk;        // most particles per chunk
     const int *old_start;   // ntiles + 1: the tiles of the source's slots [0, n_sorted), or null
     int64_t n_sorted;
 };

@@ -4,7 +4,7 @@
 //
 //   1. count live particles per (tile, cell) key
 //   2. exclusive scan of the counts -> first slot of every key
-//   3. per tile: the number of kChunk-particle chunks and the spread
+//   3. per tile: the number of its chunks and the spread
 //      multiplier of its storage order
 //   4. scatter every live particle to the next position of its key in the
 //      other buffer, stored at its tile's spread slot (free slots are
@@ -248,7 +248,7 @@ __global__ void k_sum_counts(const int *__restrict__ stay, int *imm, int n)
 // re-sort, layout: tile_start = scan of stay + imm (done by the caller);
 // the movers' counters start after each tile's stayers; the chunk counts
 __global__ void k_keep_layout(const int *__restrict__ tile_start, const int *__restrict__ stay, int ntiles, int *cur,
-                              int *chunk_n, int *tile_mult)
+                              int *chunk_n, int *tile_mult, int chunk)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t > ntiles) return;
@@ -258,7 +258,7 @@ __global__ void k_keep_layout(const int *__restrict__ tile_start, const int *__r
     }
     cur[t] = tile_start[t] + stay[t];
     const int cnt = tile_start[t + 1] - tile_start[t];
-    chunk_n[t] = (cnt + kChunk - 1) / kChunk;
+    chunk_n[t] = (cnt + chunk - 1) / chunk;
     tile_mult[t] = 1;
 }
 
@@ -383,7 +383,7 @@ __device__ inline int mod_inverse(int a, int n)
 }
 
 __global__ void k_tile_chunks(const int *__restrict__ offsets, int ntiles, int *tile_start, int *chunk_n,
-                              int *tile_mult)
+                              int *tile_mult, int chunk)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t > ntiles) return;
@@ -391,7 +391,7 @@ __global__ void k_tile_chunks(const int *__restrict__ offsets, int ntiles, int *
     tile_start[t] = s;
     if (t < ntiles) {
         const int cnt = offsets[(t + 1) * kTileCells] - s;
-        chunk_n[t] = (cnt + kChunk - 1) / kChunk;
+        chunk_n[t] = (cnt + chunk - 1) / chunk;
         int m = 1;   // identity if every spread shares a factor with cnt
         for (int a : kSpread)
             if (cnt > 1 && cnt % a != 0) {
@@ -405,14 +405,14 @@ __global__ void k_tile_chunks(const int *__restrict__ offsets, int ntiles, int *
 }
 
 __global__ void k_write_chunks(const int *__restrict__ tile_start, const int *__restrict__ chunk_off, int ntiles,
-                               int4 *chunks, int max_chunks)
+                               int4 *chunks, int max_chunks, int chunk)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ntiles) return;
     const int s = tile_start[t], e = tile_start[t + 1];
-    const int nc = (e - s + kChunk - 1) / kChunk;
+    const int nc = (e - s + chunk - 1) / chunk;
     if (nc == 0) return;
-    // equal parts: a tile a little over kChunk gives two halves, not a full
+    // equal parts: a tile a little over `chunk` gives two halves, not a full
     // chunk and a nearly empty one that pays the tile's staging again
     const int sz = (e - s + nc - 1) / nc;
     const int o = chunk_off[t];
@@ -486,7 +486,7 @@ hipError_t launch_sort(hipStream_t st, const TileGeom &tg, const Species<real> &
         if ((e = hipGetLastError()) != hipSuccess) return e;
         if ((e = launch_exclusive_scan(st, b.imm, b.tile_start, tg.ntiles, b.scratch)) != hipSuccess) return e;
         k_keep_layout<<<nblocks((size_t)tg.ntiles + 1, 256), 256, 0, st>>>(b.tile_start, b.counts, tg.ntiles, b.imm,
-                                                                           b.chunk_n, b.tile_mult);
+                                                                           b.chunk_n, b.tile_mult, b.chunk);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         k_scatter_keep<real><<<tg.ntiles, kSortBlock, 0, st>>>(src, dst, b.old_start, tg, b.tile_start, b.imm);
         if ((e = hipGetLastError()) != hipSuccess) return e;
@@ -503,7 +503,7 @@ hipError_t launch_sort(hipStream_t st, const TileGeom &tg, const Species<real> &
         }
         if ((e = launch_exclusive_scan(st, b.counts, b.offsets, tg.nkeys, b.scratch)) != hipSuccess) return e;
         k_tile_chunks<<<nblocks((size_t)tg.ntiles + 1, 256), 256, 0, st>>>(b.offsets, tg.ntiles, b.tile_start,
-                                                                           b.chunk_n, b.tile_mult);
+                                                                           b.chunk_n, b.tile_mult, b.chunk);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         if (n > 0) {
             k_scatter<real><<<nblocks((size_t)n, 256), 256, 0, st>>>(src, dst, 0, n, tg, b.offsets, b.tile_start,
@@ -513,7 +513,7 @@ hipError_t launch_sort(hipStream_t st, const TileGeom &tg, const Species<real> &
     }
     if ((e = launch_exclusive_scan(st, b.chunk_n, b.chunk_off, tg.ntiles, b.scratch)) != hipSuccess) return e;
     k_write_chunks<<<nblocks((size_t)tg.ntiles, 256), 256, 0, st>>>(b.tile_start, b.chunk_off, tg.ntiles, b.chunks,
-                                                                    b.max_chunks);
+                                                                    b.max_chunks, b.chunk);
     return hipGetLastError();
 }
 
