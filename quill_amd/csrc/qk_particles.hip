@@ -215,10 +215,20 @@ __global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<
     __shared__ real stage[2 * kFStage];
     __shared__ uint32_t listed[kDefer];
     __shared__ int nlisted;
-    // chunks in launch order: the round-robin deal of workgroups to the XCDs
-    // spreads neighbouring tiles over all eight, which measured faster here
-    // than grouping them on one XCD (unlike the scatter, see qk_sort.hip)
-    const int vb = (int)blockIdx.x;
+    // Chunks in groups of kXcdGroup per XCD.  Workgroups are dealt to the
+    // XCDs round-robin; a line of the field arrays spans four tiles along k,
+    // and neighbouring tiles share their halos, so with neighbours on
+    // different XCDs each L2 fetches (and, for the current's flush, merges)
+    // its own copy.  The groups leave the set of chunks in flight as it is.
+    // Push 4.72 -> 4.40 ms at 512x256x256 and 0.615 -> 0.60 ms at 256x128x128;
+    // groups of 2, 4, 8: 4.64, 4.59, 4.53 ms; 32 to 512: 4.37-4.45 ms but
+    // 95-97 us at 128x64x64, against 93; one range per XCD: 4.48 ms.
+    constexpr int kXcdGroup = 16;
+    int vb = (int)blockIdx.x;
+    if (vb < (int)gridDim.x / (8 * kXcdGroup) * (8 * kXcdGroup)) {
+        const int xcd = vb % 8, l = vb / 8;
+        vb = (l / kXcdGroup * 8 + xcd) * kXcdGroup + l % kXcdGroup;
+    }
     // the work-list entry loads together with the count (the list has an
     // entry for every launched workgroup; those past the count are unused)
     const int4 ch = chunks[vb];
