@@ -264,24 +264,26 @@ template <typename real, class Acc>
 __device__ inline void deposit_path(Acc &acc, real q, real p[3], const real d[3])
 {
     int c2[3];
-    real t[3];
-    int ax[3] = {0, 1, 2};
 #pragma unroll
-    for (int m = 0; m < 3; ++m) {
-        c2[m] = (int)floor(p[m] + d[m]);
-        // non-crossing axes sort after every crossing one
-        t[m] = c2[m] != 0 ? (real(c2[m] > 0 ? 1 : 0) - p[m]) * qk_rcp(d[m]) : real(2);
-    }
+    for (int m = 0; m < 3; ++m) c2[m] = (int)floor(p[m] + d[m]);
     const int nc = (c2[0] != 0) + (c2[1] != 0) + (c2[2] != 0);
-    auto cswap = [&](int a, int b) {
-        if (t[a] > t[b]) {
-            const real tt = t[a]; t[a] = t[b]; t[b] = tt;
-            const int ta = ax[a]; ax[a] = ax[b]; ax[b] = ta;
-        }
-    };
-    cswap(0, 1);
-    cswap(1, 2);
-    cswap(0, 1);
+    real t[3] = {real(1), real(1), real(1)};
+    int ax[3] = {0, 1, 2};
+    // a wavefront without a crossing lane skips the fractions
+    if (nc > 0) {
+#pragma unroll
+        for (int m = 0; m < 3; ++m)   // non-crossing axes sort after every crossing one
+            t[m] = c2[m] != 0 ? (real(c2[m] > 0 ? 1 : 0) - p[m]) * qk_rcp(d[m]) : real(2);
+        auto cswap = [&](int a, int b) {
+            if (t[a] > t[b]) {
+                const real tt = t[a]; t[a] = t[b]; t[b] = tt;
+                const int ta = ax[a]; ax[a] = ax[b]; ax[b] = ta;
+            }
+        };
+        cswap(0, 1);
+        cswap(1, 2);
+        cswap(0, 1);
+    }
     int w[3] = {0, 0, 0};
     real done = real(0);
 #pragma unroll

@@ -61,7 +61,7 @@ constexpr int kJWin = jsize(0) + jsize(1) + jsize(2);
 __host__ __device__ constexpr int fdim(int c, int a) { return kT[a] + 2 * kHalo + (a == c ? 0 : 1); }
 __host__ __device__ constexpr int fsize(int c) { return fdim(c, 0) * fdim(c, 1) * fdim(c, 2); }
 __host__ __device__ constexpr int foff(int c) { return c == 0 ? 0 : (c == 1 ? fsize(0) : fsize(0) + fsize(1)); }
-constexpr int kFStage = fsize(0) + fsize(1) + fsize(2);   // per field (E or Be)
+constexpr int kFStage = fsize(0) + fsize(1) + fsize(2);
 
 // contributions go to the workgroup's LDS current window (one block per
 // component, dims jdim).  The window is FP64 for both particle precisions:
@@ -91,28 +91,37 @@ struct LdsAcc {
     }
 };
 
-// Corner nodes of a window particle from the field stage (E then Be, one
-// block per component, dims fdim); the same squares as load_corners.
+// E and Be of one node and component side by side in the field stage: one
+// 8-byte LDS read takes 5.6 clocks per wavefront and CU at random cells, two
+// 4-byte reads 10.4.  With the integer counters of DiagAcc and the crossing
+// fractions taken only where a lane crosses (deposit_path): push 95.1 -> 92.5
+// us at 128x64x64, 4.48 -> 4.38 ms at 512x256x256
 template <typename real>
-__device__ inline void load_corners_stage(const real *st, int ri, int rj, int rk, Corners<real> &c)
+struct alignas(2 * sizeof(real)) EB {
+    real e, b;
+};
+
+// Corner nodes of a window particle from the field stage (one block per
+// component, dims fdim); the same squares as load_corners.
+template <typename real>
+__device__ inline void load_corners_stage(const EB<real> *st, int ri, int rj, int rk, Corners<real> &c)
 {
     int b[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a)
         b[a] = foff(a) + ((ri + kHalo) * fdim(a, 1) + (rj + kHalo)) * fdim(a, 2) + (rk + kHalo);
     const int sx0 = fdim(0, 2), sx1 = fdim(1, 1) * fdim(1, 2), sy2 = fdim(2, 1) * fdim(2, 2), sz2 = fdim(2, 2);
-    const int ox[4] = {0, sx0, 1, sx0 + 1};          // x components: (j, k) square
-    const int oy[4] = {0, sx1, 1, sx1 + 1};          // y components: (i, k) square
-    const int oz[4] = {0, sy2, sz2, sy2 + sz2};      // z components: (i, j) square
+    const int o[3][4] = {{0, sx0, 1, sx0 + 1},          // x components: (j, k) square
+                         {0, sx1, 1, sx1 + 1},          // y components: (i, k) square
+                         {0, sy2, sz2, sy2 + sz2}};     // z components: (i, j) square
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        c.e[0][m] = st[b[0] + ox[m]];
-        c.e[1][m] = st[b[1] + oy[m]];
-        c.e[2][m] = st[b[2] + oz[m]];
-        c.b[0][m] = st[kFStage + b[0] + ox[m]];
-        c.b[1][m] = st[kFStage + b[1] + oy[m]];
-        c.b[2][m] = st[kFStage + b[2] + oz[m]];
-    }
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const EB<real> v = st[b[a] + o[a][m]];
+            c.e[a][m] = v.e;
+            c.b[a][m] = v.b;
+        }
 }
 
 // Component C of one field into its stage block, in two passes over a
@@ -142,12 +151,12 @@ __device__ inline void load_component(real (&v)[kStageIt], const real *__restric
 }
 
 template <int C, typename real>
-__device__ inline void store_component(real *dst, const real (&v)[kStageIt])
+__device__ inline void store_component(EB<real> *dst, const real (&e)[kStageIt], const real (&b)[kStageIt])
 {
 #pragma unroll
     for (int m = 0; m < kStageIt; ++m) {
         const int w = threadIdx.x + m * kTBlock;
-        if (w < fsize(C)) dst[foff(C) + w] = v[m];
+        if (w < fsize(C)) dst[foff(C) + w] = EB<real>{e[m], b[m]};
     }
 }
 
@@ -212,7 +221,7 @@ __global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<
                                                        const int *__restrict__ nchunks, TileGeom tg, double *diag)
 {
     __shared__ double win[kJWin];
-    __shared__ real stage[2 * kFStage];
+    __shared__ EB<real> stage[kFStage];
     __shared__ uint32_t listed[kDefer];
     __shared__ int nlisted;
     // Chunks in groups of kXcdGroup per XCD.  Workgroups are dealt to the
@@ -270,12 +279,9 @@ __global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<
         load_component<0>(v[3], f.bex, g, si, sj, sk);
         load_component<1>(v[4], f.bey, g, si, sj, sk);
         load_component<2>(v[5], f.bez, g, si, sj, sk);
-        store_component<0>(stage, v[0]);
-        store_component<1>(stage, v[1]);
-        store_component<2>(stage, v[2]);
-        store_component<0>(stage + kFStage, v[3]);
-        store_component<1>(stage + kFStage, v[4]);
-        store_component<2>(stage + kFStage, v[5]);
+        store_component<0>(stage, v[0], v[3]);
+        store_component<1>(stage, v[1], v[4]);
+        store_component<2>(stage, v[2], v[5]);
     }
     __syncthreads();
 

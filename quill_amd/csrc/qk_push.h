@@ -90,7 +90,8 @@ __device__ inline void block_accumulate(double *dst, double v0, double v1, doubl
 }
 
 struct DiagAcc {
-    double q = 0, e = 0, n = 0, fallback = 0;
+    double q = 0, e = 0;
+    int n = 0, fallback = 0;
 };
 
 // one particle in registers
