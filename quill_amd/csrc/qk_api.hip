@@ -9,6 +9,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "quillk.h"
@@ -90,7 +91,6 @@ struct SpeciesBuf {
     SoA buf[2];             // current and sort target
     int cur = 0;
     int4 *chunks = nullptr; // tiled-kernel work list
-    int *d_nchunks = nullptr;
     int max_chunks = 0;     // capacity of chunks
     int nchunks = 0;        // host copy after the last sort
     int steps_since_sort = 0;
@@ -297,7 +297,6 @@ int reserve(qk_ctx *c, int s, int64_t cap)
     b.chunks = nullptr;
     HIP_TRY(hipMalloc(&b.chunks, (size_t)mc * sizeof(int4)));
     b.max_chunks = (int)mc;
-    if (!b.d_nchunks) HIP_TRY(hipMalloc(&b.d_nchunks, sizeof(int)));
     b.n_sorted = 0;   // the work list refers to the old buffers
     b.nchunks = 0;
     return QK_OK;
@@ -386,13 +385,10 @@ int sort_species(qk_ctx *c, int s)
     sb.scratch = c->s_scratch;
     sb.max_chunks = b.max_chunks;
     sb.chunk = chunk_size(c, b.n);
+    sb.info = c->h_sortinfo;
     HIP_TRY(launch_sort<real>(c->stream, c->tg, view<real>(b.buf[b.cur]), view<real>(b.buf[b.cur ^ 1]), b.n, sb));
-    HIP_TRY(hipMemcpyAsync(b.d_nchunks, c->s_chunk_off + c->tg.ntiles, sizeof(int), hipMemcpyDeviceToDevice, c->stream));
-    HIP_TRY(hipMemcpyAsync(b.tile_start, c->s_tile_start, ((size_t)c->tg.ntiles + 1) * sizeof(int),
-                           hipMemcpyDeviceToDevice, c->stream));
-    HIP_TRY(hipMemcpyAsync(c->h_sortinfo, c->s_tile_start + c->tg.ntiles, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipMemcpyAsync(c->h_sortinfo + 1, c->s_chunk_off + c->tg.ntiles, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
+    std::swap(b.tile_start, c->s_tile_start);   // the next sort's source
     b.cur ^= 1;
     b.n = c->h_sortinfo[0];
     b.n_sorted = b.n;
@@ -1000,6 +996,11 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
         if (between) HIP_TRY(hipEventRecord(c->ev[3 * l], c->stream));
         start[l] = between ? 3 * l : 3 * (l - 1) + 2;
         if (qed) QK_TRY(qed_particle_phase<real>(c, f, jc));
+        // the sorted slots of every charged species go in one tiled launch, the
+        // rest (photons, unsorted tails, the global deposit) one by one
+        Species<real> ts[kMaxTiled];
+        PushArgs ta[kMaxTiled];
+        int nt = 0;
         for (int s = 0; s < QK_MAX_SPECIES && !qed; ++s) {
             SpeciesBuf &b = c->sp[s];
             if (!b.active || b.n == 0) continue;
@@ -1022,11 +1023,10 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
             }
             if (tiled && b.kind == 0) {
                 a.chunks = b.chunks;
-                a.nchunks = b.d_nchunks;
-                a.max_chunks = b.nchunks;
-                a.tg = c->tg;
-                a.tg.ishift = b.ishift;
-                HIP_TRY(launch_push_tiled<real>(c->stream, c->g, f, jc, v, a));
+                a.nchunks = b.nchunks;
+                a.ishift = b.ishift;
+                ts[nt] = v;
+                ta[nt++] = a;
                 a.first = b.n_sorted;   // the unsorted tail, if any
                 a.n = b.n - b.n_sorted;
             } else {
@@ -1036,6 +1036,7 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
             HIP_TRY(launch_push_global<real>(c->stream, c->g, f, jc, v, a));
             ++b.steps_since_sort;
         }
+        if (nt > 0) HIP_TRY(launch_push_tiled<real>(c->stream, c->g, f, jc, c->tg, nt, ts, ta));
         HIP_TRY(hipEventRecord(c->ev[3 * l + 1], c->stream));
         // fadvance (src/advance.cpp:13-18): B half, E, B half, interpolate_be.  The
         // first half step also sums compute_energy's field term, which sees the
@@ -1337,7 +1338,6 @@ int qk_create(const qk_params *params, qk_ctx **out)
     c->tg.ntz = (p.nz + kTz - 1) / kTz;
     c->tg.ntiles = c->tg.ntx * c->tg.nty * c->tg.ntz;
     c->tg.nkeys = c->tg.ntiles * kTileCells;
-    c->tg.ishift = 0;
     c->rsize = p.precision == QK_FP64 ? 8 : 4;
     // solver coefficients (src/maxwell.cpp:24-33, 238-249)
     for (int a = 0; a < 3; ++a) {
@@ -1398,7 +1398,6 @@ int qk_destroy(qk_ctx *c)
         for (auto &k : b.buf)
             if (k.mem) note(hipFree(k.mem));
         if (b.chunks) note(hipFree(b.chunks));
-        if (b.d_nchunks) note(hipFree(b.d_nchunks));
         if (b.tile_start) note(hipFree(b.tile_start));
     }
     int *sb[8] = {c->s_counts, c->s_imm, c->s_offsets, c->s_tile_start, c->s_tile_mult, c->s_chunk_n, c->s_chunk_off,

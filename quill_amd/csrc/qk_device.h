@@ -42,7 +42,6 @@ struct TileGeom {
     int ntx, nty, ntz;   // tiles per axis
     int ntiles;
     int nkeys;           // sort keys: ntiles * kTileCells
-    int ishift;          // moving-window shifts since the sort: a tile's cells now start at i = 8 ti - ishift
 };
 
 __host__ __device__ inline int tile_of(const TileGeom &t, int i, int j, int k)

@@ -37,9 +37,8 @@ struct PushArgs {
     double *nonfinite;       // FP64 count of particles dropped for a non-finite momentum (may be null)
     // tiled kernel: work list of (tile, first slot, count) chunks
     const int4 *chunks;
-    const int *nchunks;      // device counter
-    int max_chunks;          // launch size (upper bound of *nchunks)
-    TileGeom tg;
+    int nchunks;
+    int ishift;              // moving-window shifts since the species' sort
 };
 
 // clear n doubles / ints with a kernel (kept out of hipMemsetAsync so the
@@ -52,10 +51,12 @@ template <typename real>
 hipError_t launch_push_global(hipStream_t st, const Grid &g, const Fields<real> &f, const Current<real> &j,
                               const Species<real> &s, const PushArgs &a);
 // one workgroup per chunk of a cell tile: the current is accumulated in an
-// LDS window around the tile and flushed to global memory once
+// LDS window around the tile and flushed to global memory once; the chunks
+// of all ns species (at most kMaxTiled, one pusher) in one launch
+constexpr int kMaxTiled = 6;
 template <typename real>
 hipError_t launch_push_tiled(hipStream_t st, const Grid &g, const Fields<real> &f, const Current<real> &j,
-                             const Species<real> &s, const PushArgs &a);
+                             const TileGeom &tg, int ns, const Species<real> *s, const PushArgs *a);
 
 // ---- QED -------------------------------------------------------------------
 
@@ -255,6 +256,7 @@ struct SortBuffers {
     int *scratch;     // scan scratch
     int max_chunks;
     int chunk;        // most particles per chunk
+    int *info;        // pinned host memory: [live count, chunk count]
     const int *old_start;   // ntiles + 1: the tiles of the source's slots [0, n_sorted), or null
     int64_t n_sorted;
 };

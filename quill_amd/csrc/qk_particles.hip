@@ -215,10 +215,31 @@ __global__ void __launch_bounds__(kBlock) k_push_global(Grid g, Fields<real> f, 
 // it; listed, they run densely (the push measured 3.8 % faster at
 // 512x256x256, where they gather in the laser's wake, and 1.5 % slower at
 // 256x128x128, where a few per chunk make a short serial tail).
+//
+// The chunks of all species follow each other in one launch: a launch takes
+// some 20 us to fill the chip and to drain it, with every workgroup staging
+// and flushing at once in between.  Particle phase 303 -> 252 us for three
+// species at 135x75x71 (3 per cell), 54 -> 39 us for two at 64x32x32, FP64 175
+// -> 152 us for two at 97x61x53; one species as before.
+template <typename real>
+struct TiledSpecies {
+    Species<real> s;
+    StepConst<real> sc;
+    const int4 *chunks;
+    double *diag;
+    int first;     // workgroup of the species' first chunk
+    int ishift;    // a tile's cells now start at i = 8 ti - ishift
+};
+
+template <typename real>
+struct TiledArgs {
+    TiledSpecies<real> sp[kMaxTiled];
+    int ns;
+};
+
 template <typename real, int PUSHER>
-__global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<real> f, Current<real> cur, Species<real> s,
-                                                       StepConst<real> sc, const int4 *__restrict__ chunks,
-                                                       const int *__restrict__ nchunks, TileGeom tg, double *diag)
+__global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<real> f, Current<real> cur, TileGeom tg,
+                                                                TiledArgs<real> args)
 {
     __shared__ double win[kJWin];
     __shared__ EB<real> stage[kFStage];
@@ -238,14 +259,16 @@ __global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<
         const int xcd = vb % 8, l = vb / 8;
         vb = (l / kXcdGroup * 8 + xcd) * kXcdGroup + l % kXcdGroup;
     }
-    // the work-list entry loads together with the count (the list has an
-    // entry for every launched workgroup; those past the count are unused)
-    const int4 ch = chunks[vb];
-    if (vb >= *nchunks) return;   // whole workgroup leaves together
+    int m = 0;
+    while (m + 1 < args.ns && vb >= args.sp[m + 1].first) ++m;
+    const TiledSpecies<real> &sp = args.sp[m];
+    const Species<real> s = sp.s;
+    const StepConst<real> sc = sp.sc;
+    const int4 ch = sp.chunks[vb - sp.first];
     const int tile = ch.x;
     const int tk = tile % tg.ntz, t2 = tile / tg.ntz;
     const int tj = t2 % tg.nty, ti = t2 / tg.nty;
-    const int i0 = ti * kTx - tg.ishift, j0 = tj * kTy, k0 = tk * kTz;
+    const int i0 = ti * kTx - sp.ishift, j0 = tj * kTy, k0 = tk * kTz;
     // Slots as 32-bit indices: the record arrays are addressed as scalar
     // base + one shared 32-bit byte offset (capacity keeps slot * size below
     // 2^32).  The first two rounds' records load while the tile is staged.
@@ -413,7 +436,7 @@ __global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<
         flush_component<1>(cur.jy, v[1], g, wi0, wj0, wk0);
         flush_component<2>(cur.jz, v[2], g, wi0, wj0, wk0);
     }
-    block_accumulate(diag, da.q, da.e, da.n, da.fallback);
+    block_accumulate(sp.diag, da.q, da.e, da.n, da.fallback);
 }
 
 // Photons with QED off move on straight lines (src/advance.cpp:173-183) and
@@ -599,14 +622,24 @@ hipError_t launch_push_global(hipStream_t st, const Grid &g, const Fields<real> 
 
 template <typename real>
 hipError_t launch_push_tiled(hipStream_t st, const Grid &g, const Fields<real> &f, const Current<real> &j,
-                             const Species<real> &s, const PushArgs &a)
+                             const TileGeom &tg, int ns, const Species<real> *s, const PushArgs *a)
 {
-    if (a.max_chunks <= 0) return hipSuccess;
-    const StepConst<real> sc = step_const<real>(g, a);
-    if (a.pusher == 1)
-        k_push_tiled<real, 1><<<a.max_chunks, kTBlock, 0, st>>>(g, f, j, s, sc, a.chunks, a.nchunks, a.tg, a.diag);
-    else
-        k_push_tiled<real, 0><<<a.max_chunks, kTBlock, 0, st>>>(g, f, j, s, sc, a.chunks, a.nchunks, a.tg, a.diag);
+    TiledArgs<real> args{};
+    int total = 0;
+    for (int m = 0; m < ns; ++m) {
+        if (a[m].nchunks <= 0) continue;
+        TiledSpecies<real> &t = args.sp[args.ns++];
+        t.s = s[m];
+        t.sc = step_const<real>(g, a[m]);
+        t.chunks = a[m].chunks;
+        t.diag = a[m].diag;
+        t.first = total;
+        t.ishift = a[m].ishift;
+        total += a[m].nchunks;
+    }
+    if (total == 0) return hipSuccess;
+    if (a[0].pusher == 1) k_push_tiled<real, 1><<<total, kTBlock, 0, st>>>(g, f, j, tg, args);
+    else k_push_tiled<real, 0><<<total, kTBlock, 0, st>>>(g, f, j, tg, args);
     return hipGetLastError();
 }
 
@@ -657,7 +690,8 @@ hipError_t launch_scale_charge(hipStream_t st, const Species<real> &s, int64_t n
     template hipError_t launch_push_global<real>(hipStream_t, const Grid &, const Fields<real> &,               \
                                                  const Current<real> &, const Species<real> &, const PushArgs &); \
     template hipError_t launch_push_tiled<real>(hipStream_t, const Grid &, const Fields<real> &,                \
-                                                const Current<real> &, const Species<real> &, const PushArgs &); \
+                                                const Current<real> &, const TileGeom &, int,                   \
+                                                const Species<real> *, const PushArgs *);                       \
     template hipError_t launch_load_uniform<real>(hipStream_t, const Grid &, const Species<real> &, int64_t, int, \
                                                   double, double, uint64_t, int, int);                           \
     template hipError_t launch_compute_rho<real>(hipStream_t, const Grid &, const Species<real> &, int64_t,       \

@@ -405,9 +405,13 @@ __global__ void k_tile_chunks(const int *__restrict__ offsets, int ntiles, int *
 }
 
 __global__ void k_write_chunks(const int *__restrict__ tile_start, const int *__restrict__ chunk_off, int ntiles,
-                               int4 *chunks, int max_chunks, int chunk)
+                               int4 *chunks, int max_chunks, int chunk, int *info)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t == 0) {
+        info[0] = tile_start[ntiles];
+        info[1] = chunk_off[ntiles];
+    }
     if (t >= ntiles) return;
     const int s = tile_start[t], e = tile_start[t + 1];
     const int nc = (e - s + chunk - 1) / chunk;
@@ -513,7 +517,7 @@ hipError_t launch_sort(hipStream_t st, const TileGeom &tg, const Species<real> &
     }
     if ((e = launch_exclusive_scan(st, b.chunk_n, b.chunk_off, tg.ntiles, b.scratch)) != hipSuccess) return e;
     k_write_chunks<<<nblocks((size_t)tg.ntiles, 256), 256, 0, st>>>(b.tile_start, b.chunk_off, tg.ntiles, b.chunks,
-                                                                    b.max_chunks, b.chunk);
+                                                                    b.max_chunks, b.chunk, b.info);
     return hipGetLastError();
 }
 
