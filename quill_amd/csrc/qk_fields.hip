@@ -137,12 +137,16 @@ __device__ inline int stride(const Grid &g)
     return A == 0 ? g.sx : (A == 1 ? g.sy : 1);
 }
 
-// zero outside the grid; used by the five-point planes at n-1 (src/maxwell.cpp:52-84)
-template <typename real>
-__device__ inline real rd0(const Grid &g, const real *F, int i, int j, int k)
+// F at offset `off` along axis A from the cell (index c of n along A, linear
+// index id), zero outside the grid; used by the five-point planes at n-1
+// (src/maxwell.cpp:52-84).  The load is unconditional, its index clamped, so
+// that the loads of a cell are in flight together.
+template <int A, typename real>
+__device__ inline real rd0(const Grid &g, const real *__restrict__ F, int id, int c, int n, int off)
 {
-    if ((unsigned)i >= (unsigned)g.nx || (unsigned)j >= (unsigned)g.ny || (unsigned)k >= (unsigned)g.nz) return real(0);
-    return F[i * g.sx + j * g.sy + k];
+    const int at = min(max(c + off, 0), n - 1);
+    const real v = F[id + (at - c) * (A == 0 ? g.sx : (A == 1 ? g.sy : 1))];
+    return (unsigned)(c + off) < (unsigned)n ? v : real(0);
 }
 
 // Difference of component C (stored in F) along axis A at cell (i,j,k);
@@ -164,10 +168,10 @@ __device__ inline real diff(const Grid &g, const Coef<real> &cf, const real *__r
         const int sC = stride<C>(g);
         return cf.b[C] * (F[hi] - F[lo]) + cf.a[C] * ((F[hi + sC] - F[lo + sC]) + (F[hi - sC] - F[lo - sC]));
     } else {
-        const real fm = rd0(g, F, li - ua, lj - va, lk - wa);
-        const real f0 = rd0(g, F, li, lj, lk);
-        const real f1 = rd0(g, F, li + ua, lj + va, lk + wa);
-        const real f2 = rd0(g, F, li + 2 * ua, lj + 2 * va, lk + 2 * wa);
+        const int id = i * g.sx + j * g.sy + k, c = A == 0 ? i : (A == 1 ? j : k);
+        const int n = A == 0 ? g.nx : (A == 1 ? g.ny : g.nz), s = FWD ? 0 : -1;
+        const real fm = rd0<A>(g, F, id, c, n, s - 1), f0 = rd0<A>(g, F, id, c, n, s);
+        const real f1 = rd0<A>(g, F, id, c, n, s + 1), f2 = rd0<A>(g, F, id, c, n, s + 2);
         return cf.b[A] * (f1 - f0) + cf.a[A] * (f2 - f1 + f0 - fm);
     }
 }
@@ -275,55 +279,57 @@ __global__ void __launch_bounds__(kSweep) k_maxwell_e(Grid g, SweepPlan sw, Coef
 // the half that leaves the grid is dropped (4-point mean); cells on two or
 // more boundary planes keep their value.
 //
-// A workgroup owns a kBeK x kBeJ block of (j, k) columns over a run of
-// planes.  It loads B of its block plus the one-column rim each component's
-// square reaches (Bx: rows j-1, columns k-1; By: rows j+1, columns k-1; Bz:
-// rows j-1, columns k+1), on the run's planes plus one (Bx one plane ahead,
-// By and Bz one behind), with every load issued before the first LDS write
-// and unconditional (indices clamped into the grid, entries outside it set
-// to zero), then takes each cell's sums from LDS in the order and with the
-// entries of a sum over the grid.  Each B value is loaded about 1.4 times
-// instead of the thirteen L1 reads per cell of a thread summing its own
-// squares from global memory (field phase 1.28 -> 1.18 ms at 512x256x256).
+// Two forms with the same sums in the same order.  In FP32, and in FP64 up to
+// kDirectBe cells, a thread of the flattened sweep takes its cell's squares
+// from global memory.  Above that, FP64 stages B in LDS: field phase 126
+// against 133 us at 128x128x128 and 321 against 334 us at 256x128x128
+// (five-point; the direct form's eight cache lines per value).  The direct
+// form is the faster one below (73.5 -> 69.3 us at 135x75x71 in FP64) and in
+// FP32 (23.0 -> 17.8 us at 64x32x32, where the staged kernel has 64
+// workgroups, 48.3 -> 41.3 at 135x75x71, 109.5 -> 101.2 at 251x97x89, 138.9 ->
+// 131.6 at 256x128x128; equal at 512x256x256).
+//
+// Staged: a workgroup owns a kBeK x kBeJ block of (j, k) columns over a run
+// of planes.  It loads B of its block plus the one-column rim each
+// component's square reaches (Bx: rows j-1, columns k-1; By: rows j+1,
+// columns k-1; Bz: rows j-1, columns k+1), on the run's planes plus one (Bx
+// one plane ahead, By and Bz one behind), with every load issued before the
+// first LDS write and unconditional (indices clamped into the grid, entries
+// outside it set to zero), then takes each cell's sums from LDS.
+constexpr int kDirectBe = 1 << 20;
 constexpr int kBeK = 64, kBeJ = 8;
 constexpr int kBeW = kBeK + 1, kBeH = kBeJ + 1;   // rim-extended block, per component
 constexpr int kBeCols = kBeW * kBeH;
-// planes per run; the LDS holds the run plus one plane of three components
-template <typename real>
-struct BeRun {
-    static constexpr int n = sizeof(real) == 4 ? 4 : 2;
-};
+constexpr int kBeRun = 2;   // planes per run; the LDS holds the run plus one plane of three components
 
 // 2x2 sum of the LDS plane P (kBeH rows of kBeW) at (r, c) with the
 // neighbour row r + dr (when vj) and column c + dc (when vk)
-template <typename real>
-__device__ inline real lds_sum(const real *P, int r, int c, int dr, int dc, bool vj, bool vk)
+__device__ inline double lds_sum(const double *P, int r, int c, int dr, int dc, bool vj, bool vk)
 {
-    real s = P[r * kBeW + c];
+    double s = P[r * kBeW + c];
     if (vk) s += P[r * kBeW + c + dc];
     if (vj) s += P[(r + dr) * kBeW + c];
     if (vj && vk) s += P[(r + dr) * kBeW + c + dc];
     return s;
 }
 
-template <typename real>
-__global__ void __launch_bounds__(kBeK * kBeJ) k_interpolate_be(Grid g, const real *__restrict__ bx,
-                                                                const real *__restrict__ by,
-                                                                const real *__restrict__ bz, real *__restrict__ bex,
-                                                                real *__restrict__ bey, real *__restrict__ bez)
+__global__ void __launch_bounds__(kBeK * kBeJ) k_interpolate_be(Grid g, const double *__restrict__ bx,
+                                                                const double *__restrict__ by,
+                                                                const double *__restrict__ bz, double *__restrict__ bex,
+                                                                double *__restrict__ bey, double *__restrict__ bez)
 {
-    constexpr int R = BeRun<real>::n;
+    constexpr int R = kBeRun;
     constexpr int kN = (R + 1) * kBeCols;   // LDS entries per component
     constexpr int kIt = (kN + kBeK * kBeJ - 1) / (kBeK * kBeJ);
     // [plane][component][row][column]: plane m holds Bx at x = i0 + m and By,
     // Bz at x = i0 - 1 + m; component c's (row, column) is (j, k) =
     // (j0 - 1 + row, k0 - 1 + col) for Bx, (j0 + row, k0 - 1 + col) for By,
     // (j0 - 1 + row, k0 + col) for Bz
-    __shared__ real L[R + 1][3][kBeCols];
+    __shared__ double L[R + 1][3][kBeCols];
     const dim3 vb = band_block();
     const int k0 = vb.x * kBeK, j0 = vb.y * kBeJ, i0 = vb.z * R;
     const int tid = threadIdx.y * kBeK + threadIdx.x;
-    real v[3][kIt];
+    double v[3][kIt];
 #pragma unroll
     for (int it = 0; it < kIt; ++it) {
         const int w = tid + it * kBeK * kBeJ;
@@ -338,12 +344,12 @@ __global__ void __launch_bounds__(kBeK * kBeJ) k_interpolate_be(Grid g, const re
         const int cpx = min(px, g.nx - 1), cpyz = max(min(pyz, g.nx - 1), 0);
         const int cjx = max(min(jx, g.ny - 1), 0), cjy = min(jy, g.ny - 1);
         const int ckx = max(min(kx, g.nz - 1), 0), ckz = min(kz, g.nz - 1);
-        const real ax = bx[cpx * g.sx + cjx * g.sy + ckx];
-        const real ay = by[cpyz * g.sx + cjy * g.sy + ckx];
-        const real az = bz[cpyz * g.sx + cjx * g.sy + ckz];
-        v[0][it] = inx ? ax : real(0);
-        v[1][it] = iny ? ay : real(0);
-        v[2][it] = inz ? az : real(0);
+        const double ax = bx[cpx * g.sx + cjx * g.sy + ckx];
+        const double ay = by[cpyz * g.sx + cjy * g.sy + ckx];
+        const double az = bz[cpyz * g.sx + cjx * g.sy + ckz];
+        v[0][it] = inx ? ax : double(0);
+        v[1][it] = iny ? ay : double(0);
+        v[2][it] = inz ? az : double(0);
     }
 #pragma unroll
     for (int it = 0; it < kIt; ++it) {
@@ -372,18 +378,49 @@ __global__ void __launch_bounds__(kBeK * kBeJ) k_interpolate_be(Grid g, const re
         const int i = i0 + m;
         if (i < g.nx && nbjk + (i == 0 || i == g.nx - 1) < 2) {
             const bool up = i + 1 < g.nx;
-            const real sx0 = lds_sum(L[m][0], ty + 1, tx + 1, -1, -1, xvj, xvk);
-            const real px1 = up ? lds_sum(L[m + 1][0], ty + 1, tx + 1, -1, -1, xvj, xvk) : real(0);
-            const real qy = i > 0 ? lds_sum(L[m][1], ty, tx + 1, 1, -1, yvj, yvk) : real(0);
-            const real sy1 = lds_sum(L[m + 1][1], ty, tx + 1, 1, -1, yvj, yvk);
-            const real rz = i > 0 ? lds_sum(L[m][2], ty + 1, tx, -1, 1, zvj, zvk) : real(0);
-            const real sz1 = lds_sum(L[m + 1][2], ty + 1, tx, -1, 1, zvj, zvk);
+            const double sx0 = lds_sum(L[m][0], ty + 1, tx + 1, -1, -1, xvj, xvk);
+            const double px1 = up ? lds_sum(L[m + 1][0], ty + 1, tx + 1, -1, -1, xvj, xvk) : double(0);
+            const double qy = i > 0 ? lds_sum(L[m][1], ty, tx + 1, 1, -1, yvj, yvk) : double(0);
+            const double sy1 = lds_sum(L[m + 1][1], ty, tx + 1, 1, -1, yvj, yvk);
+            const double rz = i > 0 ? lds_sum(L[m][2], ty + 1, tx, -1, 1, zvj, zvk) : double(0);
+            const double sz1 = lds_sum(L[m + 1][2], ty + 1, tx, -1, 1, zvj, zvk);
             const int id = i * g.sx + j * g.sy + k;
-            bex[id] = (sx0 + px1) * (cx * (1 + up) == 8 ? real(0.125) : real(0.25));
-            bey[id] = (qy + sy1) * (cy * (1 + (i > 0)) == 8 ? real(0.125) : real(0.25));
-            bez[id] = (rz + sz1) * (cz * (1 + (i > 0)) == 8 ? real(0.125) : real(0.25));
+            bex[id] = (sx0 + px1) * (cx * (1 + up) == 8 ? double(0.125) : double(0.25));
+            bey[id] = (qy + sy1) * (cy * (1 + (i > 0)) == 8 ? double(0.125) : double(0.25));
+            bez[id] = (rz + sz1) * (cz * (1 + (i > 0)) == 8 ? double(0.125) : double(0.25));
         }
     }
+}
+
+template <typename real>
+__global__ void __launch_bounds__(kSweep) k_interpolate_be_direct(Grid g, SweepPlan sw, const real *__restrict__ bx,
+                                                                  const real *__restrict__ by,
+                                                                  const real *__restrict__ bz, real *__restrict__ bex,
+                                                                  real *__restrict__ bey, real *__restrict__ bez)
+{
+    int i, j, k;
+    if (!sweep_cell(g, sw, i, j, k)) return;
+    if ((i == 0 || i == g.nx - 1) + (j == 0 || j == g.ny - 1) + (k == 0 || k == g.nz - 1) >= 2) return;
+    const int id = i * g.sx + j * g.sy + k;
+    // neighbours on each axis, clamped to the cell itself where they leave the grid
+    const bool il = i > 0, iu = i + 1 < g.nx, jl = j > 0, ju = j + 1 < g.ny, kl = k > 0, ku = k + 1 < g.nz;
+    const int ml = il ? -g.sx : 0, mu = iu ? g.sx : 0, nl = jl ? -g.sy : 0, nu = ju ? g.sy : 0, ol = kl ? -1 : 0,
+              ou = ku ? 1 : 0;
+    auto sum = [&](const real *__restrict__ F, int at, int dj, int dk, bool vj, bool vk) {
+        const real a = F[at], b = F[at + dk], c = F[at + dj], d = F[at + dj + dk];
+        real s = a;
+        s += vk ? b : real(0);
+        s += vj ? c : real(0);
+        s += vj && vk ? d : real(0);
+        return s;
+    };
+    const real x0 = sum(bx, id, nl, ol, jl, kl), x1 = sum(bx, id + mu, nl, ol, jl, kl);
+    const real y0 = sum(by, id + ml, nu, ol, ju, kl), y1 = sum(by, id, nu, ol, ju, kl);
+    const real z0 = sum(bz, id + ml, nl, ou, jl, ku), z1 = sum(bz, id, nl, ou, jl, ku);
+    const int cx = (1 + jl) * (1 + kl) * (1 + iu), cy = (1 + ju) * (1 + kl) * (1 + il), cz = (1 + jl) * (1 + ku) * (1 + il);
+    bex[id] = (x0 + (iu ? x1 : real(0))) * (cx == 8 ? real(0.125) : real(0.25));
+    bey[id] = ((il ? y0 : real(0)) + y1) * (cy == 8 ? real(0.125) : real(0.25));
+    bez[id] = ((il ? z0 : real(0)) + z1) * (cz == 8 ? real(0.125) : real(0.25));
 }
 
 // init_boundaries: zero components on boundary planes, transverse indices in
@@ -676,11 +713,17 @@ hipError_t launch_maxwell_e(hipStream_t st, int solver, const Grid &g, const Sol
 }
 
 template <typename real>
-hipError_t launch_interpolate_be(hipStream_t st, const Grid &g, const Fields<real> &f)
+hipError_t launch_interpolate_be(hipStream_t st, const Grid &g, const Fields<real> &f, const real *const *b)
 {
-    constexpr int R = BeRun<real>::n;
-    const dim3 grid((g.nz + kBeK - 1) / kBeK, (g.ny + kBeJ - 1) / kBeJ, (g.nx + R - 1) / R);
-    k_interpolate_be<real><<<grid, dim3(kBeK, kBeJ), 0, st>>>(g, f.bx, f.by, f.bz, f.bex, f.bey, f.bez);
+    const real *bx = b ? b[0] : f.bx, *by = b ? b[1] : f.by, *bz = b ? b[2] : f.bz;
+    if (sizeof(real) == 4 || g.ncell <= kDirectBe) {
+        const SweepPlan sw = sweep_plan(g);
+        k_interpolate_be_direct<real><<<(unsigned)(sw.per * g.nx), kSweep, 0, st>>>(g, sw, bx, by, bz, f.bex, f.bey, f.bez);
+    } else {
+        const dim3 grid((g.nz + kBeK - 1) / kBeK, (g.ny + kBeJ - 1) / kBeJ, (g.nx + kBeRun - 1) / kBeRun);
+        k_interpolate_be<<<grid, dim3(kBeK, kBeJ), 0, st>>>(g, (const double *)bx, (const double *)by, (const double *)bz,
+                                                            (double *)f.bex, (double *)f.bey, (double *)f.bez);
+    }
     return hipGetLastError();
 }
 
@@ -777,7 +820,7 @@ hipError_t launch_inject(hipStream_t st, int solver, const Grid &g, const Solver
                                                double *, bool);                                                 \
     template hipError_t launch_maxwell_e<real>(hipStream_t, int, const Grid &, const SolverCoef &, const Fields<real> &, \
                                                const Current<real> *, const Current<real> *, const DiagDrain &); \
-    template hipError_t launch_interpolate_be<real>(hipStream_t, const Grid &, const Fields<real> &);           \
+    template hipError_t launch_interpolate_be<real>(hipStream_t, const Grid &, const Fields<real> &, const real *const *); \
     template hipError_t launch_init_boundaries<real>(hipStream_t, int, const Grid &, const Fields<real> &);     \
     template hipError_t launch_laser_cos<real>(hipStream_t, const Grid &, const Fields<real> &, const double *); \
     template hipError_t launch_inject<real>(hipStream_t, int, const Grid &, const SolverCoef &, const Fields<real> &, \

@@ -173,8 +173,9 @@ struct DiagDrain {
 template <typename real>
 hipError_t launch_maxwell_e(hipStream_t st, int solver, const Grid &g, const SolverCoef &c, const Fields<real> &f,
                             const Current<real> *j, const Current<real> *jn, const DiagDrain &dd = DiagDrain());
+// Be from B, or from the three arrays b
 template <typename real>
-hipError_t launch_interpolate_be(hipStream_t st, const Grid &g, const Fields<real> &f);
+hipError_t launch_interpolate_be(hipStream_t st, const Grid &g, const Fields<real> &f, const real *const *b = nullptr);
 template <typename real>
 hipError_t launch_init_boundaries(hipStream_t st, int solver, const Grid &g, const Fields<real> &f);
 template <typename real>
