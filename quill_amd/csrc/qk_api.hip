@@ -145,6 +145,8 @@ struct qk_ctx {
     hipStream_t stream = nullptr;
     size_t rsize = 4;               // bytes per real
     void *fmem = nullptr;           // all field arrays
+    void *mid = nullptr;            // B at the step's end while the grid's B is half a step ahead (three arrays)
+    bool no_mid = false;            // the memory for it is not there
     void *F[15] = {};               // ex ey ez bx by bz bex bey bez j0x j0y j0z j1x j1y j1z
     int jcur = 0;                   // current buffer deposited this step
     bool j_zero[2] = {true, true};  // which current buffers are known to be zero
@@ -887,7 +889,7 @@ bool side_active(const qk_ctx *c, const InjSide &side, const InjectArgs &a)
 // the laser sources' corrections of one sub-step of fadvance: b_field = 1
 // after a B half step at time (step + frac) dt, 0 after the E step
 template <typename real>
-int inject_impl(qk_ctx *c, int b_field, double frac)
+int inject_impl(qk_ctx *c, int b_field, double frac, real *const *mid = nullptr, double *energy = nullptr)
 {
     InjectArgs a[2];
     int n = 0;
@@ -906,7 +908,7 @@ int inject_impl(qk_ctx *c, int b_field, double frac)
         s.plane = side.plane;
         n += side_active(c, side, s);
     }
-    HIP_TRY(launch_inject<real>(c->stream, c->p.solver, c->g, c->coef, fields_of<real>(c), b_field, n, a));
+    HIP_TRY(launch_inject<real>(c->stream, c->p.solver, c->g, c->coef, fields_of<real>(c), b_field, n, a, mid, energy));
     return QK_OK;
 }
 
@@ -927,14 +929,32 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
     // the QED kernels deposit through global atomics
     const bool tiled = c->p.deposit == QK_DEPOSIT_TILED && !qed;
     Tape &tp = c->tape;
-    // Without charged particles nothing reads Be or B between two steps: Be
-    // is interpolated once, at the end, and the second half step of B runs
-    // with the next step's first one.  (Photons fly straight.  A laser source
-    // corrects each half step by itself; the tape keeps the state of every
-    // step.)
+    // Within a call the second half step of B runs together with the next
+    // step's first one, which uses the same E: 72 instead of 96 B per cell for
+    // B and Be (field phase 1.11 -> 0.99 ms per step at 512x256x256, 130 -> 117
+    // us at 256x128x128 and 29.6 -> 22.5 us at 128x64x64 in calls of four
+    // steps; 64x32x32 with a laser source, 73 -> 60 us per step).  The B
+    // between the two, at the step's end, is what Be, the laser sources'
+    // corrections and the field energy want: it is kept in `mid`.  Without
+    // charged particles nothing reads Be between two steps, and without a
+    // laser source nothing needs mid either (photons fly straight).  The tape
+    // keeps the state of every step, so there each half step runs by itself.
     bool charged = qed || tp.active;
     for (const SpeciesBuf &b : c->sp) charged = charged || (b.active && b.n > 0 && b.kind == 0);
-    const bool fuse_b = !charged && c->inj[0].nsrc == 0 && c->inj[1].nsrc == 0;
+    const bool need_mid = charged || c->inj[0].nsrc > 0 || c->inj[1].nsrc > 0;
+    bool fuse_b = !tp.active;
+    real *mid_b[3] = {};
+    if (fuse_b && need_mid && nsteps > 1) {
+        const size_t fb = ((size_t)c->g.ncell * sizeof(real) + 255) & ~(size_t)255;
+        if (!c->mid && !c->no_mid && hipMalloc(&c->mid, 3 * fb) != hipSuccess) {
+            (void)hipGetLastError();   // the steps run without it
+            c->mid = nullptr;
+            c->no_mid = true;
+        }
+        fuse_b = c->mid != nullptr;
+        for (int a = 0; a < 3; ++a) mid_b[a] = (real *)((char *)c->mid + a * fb);
+    }
+    real *const *mid = need_mid ? mid_b : nullptr;
     // the event that marks the start of each step's particle phase: the end
     // of the step before unless something ran in between
     std::vector<int> start((size_t)nsteps);
@@ -1054,13 +1074,15 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
         c->j_zero[c->jcur ^ 1] = true;
         QK_TRY(inject_impl<real>(c, 0, 0.5));
         if (fuse_b && !last) {
-            HIP_TRY(launch_maxwell_b<real>(c->stream, c->p.solver, c->g, c->coef, f,
-                                           c->d_diag + ((l + 1) & 1) * kDiagLen + en, true));
+            double *next_en = c->d_diag + ((l + 1) & 1) * kDiagLen + en;
+            HIP_TRY(launch_maxwell_b<real>(c->stream, c->p.solver, c->g, c->coef, f, next_en, true, mid));
+            if (mid) QK_TRY(inject_impl<real>(c, 1, 1.0, mid, next_en));
         } else {
             HIP_TRY(launch_maxwell_b<real>(c->stream, c->p.solver, c->g, c->coef, f, nullptr));
             QK_TRY(inject_impl<real>(c, 1, 1.0));
         }
-        if (charged || last) HIP_TRY(launch_interpolate_be<real>(c->stream, c->g, f));
+        if (charged || last)
+            HIP_TRY(launch_interpolate_be<real>(c->stream, c->g, f, fuse_b && !last ? mid_b : nullptr));
         if (tp.tangent && !tp.replay) {
             // the tangent fields advance with the same (linear) field step
             const Fields<double> tf = tangent_fields(c);
@@ -1406,6 +1428,7 @@ int qk_destroy(qk_ctx *c)
         if (p) note(hipFree(p));
     if (c->h_sortinfo) note(hipHostFree(c->h_sortinfo));
     if (c->fmem) note(hipFree(c->fmem));
+    if (c->mid) note(hipFree(c->mid));
     if (c->d_diag) note(hipFree(c->d_diag));
     if (c->h_diag) note(hipHostFree(c->h_diag));
     if (c->d_count) note(hipFree(c->d_count));

@@ -176,6 +176,12 @@ __device__ inline real diff(const Grid &g, const Coef<real> &cf, const real *__r
     }
 }
 
+// B at the step's end, between two half steps taken together
+template <typename real>
+struct Mid {
+    real *b[3];
+};
+
 // half step of B (maxwell_solver::advance_b, src/maxwell.cpp:10-22).  With
 // energy != null the first half step also sums E^2 + B^2 of the fields it
 // starts from, in FP64: compute_energy's field term, which the reference takes
@@ -184,12 +190,13 @@ __device__ inline real diff(const Grid &g, const Coef<real> &cf, const real *__r
 // TWICE: the second half step of one step and the first of the next, which
 // use the same E when nothing reads B in between; the energy is that of the
 // fields between the two.  36 instead of 72 B per cell: 104 us at 301x203x199,
-// against 102 us for each half step.
-template <int S, bool TWICE, typename real>
+// against 102 us for each half step.  HELD: the B between the two also goes
+// to mid, for interpolate_be and the laser sources' corrections.
+template <int S, bool TWICE, bool HELD, typename real>
 __global__ void __launch_bounds__(kSweep) k_maxwell_b(Grid g, SweepPlan sw, Coef<real> cf, const real *__restrict__ ex,
                                                       const real *__restrict__ ey, const real *__restrict__ ez,
                                                       real *__restrict__ bx, real *__restrict__ by,
-                                                      real *__restrict__ bz, double *energy)
+                                                      real *__restrict__ bz, double *energy, Mid<real> mid)
 {
     __shared__ double part[kSweep / 64];
     int i, j, k;
@@ -213,6 +220,11 @@ __global__ void __launch_bounds__(kSweep) k_maxwell_b(Grid g, SweepPlan sw, Coef
         if (u2) b2 += h * d2;
         if (TWICE) {
             if (energy) add_energy();
+            if (HELD) {
+                mid.b[0][id] = b0;
+                mid.b[1][id] = b1;
+                mid.b[2][id] = b2;
+            }
             if (u0) b0 += h * d0;
             if (u1) b1 += h * d1;
             if (u2) b2 += h * d2;
@@ -562,8 +574,13 @@ struct InjectSides {
     InjectArgs s[2];
 };
 
-template <int S, bool BF, typename real>
-__global__ void __launch_bounds__(kBX * kBY) k_inject(Grid g, Coef<real> cf, Fields<real> f, InjectSides sides)
+// TURN: the corrections of a half step of B and of the next step's first one
+// (the same incident field) where both were taken together: the grid's B takes
+// them twice, mid once, and the energy of the fields between the two changes
+// with mid.
+template <int S, bool BF, bool TURN, typename real>
+__global__ void __launch_bounds__(kBX * kBY) k_inject(Grid g, Coef<real> cf, Fields<real> f, InjectSides sides,
+                                                      Mid<real> mid, double *energy)
 {
     constexpr int R = kInjReach<S>, M = S == 1 ? 1 : 0;   // planes per side, rim
     constexpr int kRows = kBY / (2 * R);                   // rows of columns: a thread owns one node of one plane
@@ -593,11 +610,11 @@ __global__ void __launch_bounds__(kBX * kBY) k_inject(Grid g, Coef<real> cf, Fie
     }
     __syncthreads();
     const int row = threadIdx.y / (2 * R), j = j0 + row, k = k0 + threadIdx.x;
-    if (j >= g.ny || k >= g.nz) return;
     const int r = row + M, q = threadIdx.x + M;
+    double en = 0;
 #pragma unroll
     for (int m = 0; m < 2 * R; ++m) {
-        if (m != (int)threadIdx.y % (2 * R)) continue;   // uniform over the wavefront
+        if (m != (int)threadIdx.y % (2 * R) || j >= g.ny || k >= g.nz) continue;   // the plane is uniform over the wavefront
         const int i = i0 + m;
         if (i < 0 || i >= g.nx) continue;
         const bool low = m < R;
@@ -630,14 +647,19 @@ __global__ void __launch_bounds__(kBX * kBY) k_inject(Grid g, Coef<real> cf, Fie
         const int id = i * g.sx + j * g.sy + k;
         if (BF) {
             const real h = real(0.5);
-            if (b_updates<S, 1>(g, i, j, k)) {
-                const real d = h * (cf.dtd[0] * dx(2) - cf.dtd[2] * dt(2));
-                f.by[id] = tot ? f.by[id] + d : f.by[id] - d;
-            }
-            if (b_updates<S, 2>(g, i, j, k)) {
-                const real d = h * (cf.dtd[1] * dt(1) - cf.dtd[0] * dx(1));
-                f.bz[id] = tot ? f.bz[id] + d : f.bz[id] - d;
-            }
+            auto correct = [&](real *F, real *at_mid, real d) {
+                if (!tot) d = -d;
+                real v = F[id] + d;
+                if (TURN) {
+                    v += d;
+                    const real o = at_mid[id], w = o + d;
+                    at_mid[id] = w;
+                    en += (double)w * w - (double)o * o;
+                }
+                F[id] = v;
+            };
+            if (b_updates<S, 1>(g, i, j, k)) correct(f.by, mid.b[1], h * (cf.dtd[0] * dx(2) - cf.dtd[2] * dt(2)));
+            if (b_updates<S, 2>(g, i, j, k)) correct(f.bz, mid.b[2], h * (cf.dtd[1] * dt(1) - cf.dtd[0] * dx(1)));
         } else {
             if (e_updates<S, 1>(g, i, j, k)) {
                 const real d = -cf.dtd[0] * dx(2) + cf.dtd[2] * dt(2);
@@ -648,6 +670,11 @@ __global__ void __launch_bounds__(kBX * kBY) k_inject(Grid g, Coef<real> cf, Fie
                 f.ez[id] = tot ? f.ez[id] + d : f.ez[id] - d;
             }
         }
+    }
+    if (TURN) {
+        en = wave_sum(en);
+        if (threadIdx.x == 0 && en != 0)
+            atomicAdd(energy + (blockIdx.y * gridDim.x + blockIdx.x) % kEnergySlots, en);
     }
 }
 
@@ -682,15 +709,22 @@ hipError_t launch_zero(hipStream_t st, double *p, size_t n)
 
 template <typename real>
 hipError_t launch_maxwell_b(hipStream_t st, int solver, const Grid &g, const SolverCoef &c, const Fields<real> &f,
-                            double *energy, bool twice)
+                            double *energy, bool twice, real *const *mid)
 {
     const Coef<real> cf = make_coef<real>(g, c);
     const SweepPlan sw = sweep_plan(g);
     const dim3 grid((unsigned)(sw.per * g.nx));
-#define QK_B(S, T) k_maxwell_b<S, T, real><<<grid, kSweep, 0, st>>>(g, sw, cf, f.ex, f.ey, f.ez, f.bx, f.by, f.bz, energy)
-    if (solver == 0) { if (twice) QK_B(0, true); else QK_B(0, false); }
-    else if (solver == 1) { if (twice) QK_B(1, true); else QK_B(1, false); }
-    else { if (twice) QK_B(2, true); else QK_B(2, false); }
+    Mid<real> md{};
+    for (int a = 0; a < 3 && mid; ++a) md.b[a] = mid[a];
+#define QK_B(S, T, H) k_maxwell_b<S, T, H, real><<<grid, kSweep, 0, st>>>(g, sw, cf, f.ex, f.ey, f.ez, f.bx, f.by, f.bz, energy, md)
+#define QK_BS(S)                              \
+    if (twice && mid) QK_B(S, true, true);    \
+    else if (twice) QK_B(S, true, false);     \
+    else QK_B(S, false, false)
+    if (solver == 0) { QK_BS(0); }
+    else if (solver == 1) { QK_BS(1); }
+    else { QK_BS(2); }
+#undef QK_BS
 #undef QK_B
     return hipGetLastError();
 }
@@ -787,18 +821,21 @@ hipError_t launch_laser_cos(hipStream_t st, const Grid &g, const Fields<real> &f
 
 template <typename real>
 hipError_t launch_inject(hipStream_t st, int solver, const Grid &g, const SolverCoef &c, const Fields<real> &f,
-                         int b_field, int nsides, const InjectArgs *a)
+                         int b_field, int nsides, const InjectArgs *a, real *const *mid, double *energy)
 {
     if (nsides <= 0) return hipSuccess;
     const Coef<real> cf = make_coef<real>(g, c);
+    Mid<real> md{};
+    for (int x = 0; x < 3 && mid; ++x) md.b[x] = mid[x];
     const dim3 block(kBX, kBY);
     const int rows = solver == 2 ? 1 : 2;   // k_inject's kRows
     dim3 grid((g.nz + kBX - 1) / kBX, (g.ny + rows - 1) / rows, nsides);
     auto one = [&](const InjectArgs &a0, const InjectArgs &a1) {
         const InjectSides sides{{a0, a1}};
-#define QK_INJ(S)                                                                              \
-    if (b_field) k_inject<S, true, real><<<grid, block, 0, st>>>(g, cf, f, sides);             \
-    else k_inject<S, false, real><<<grid, block, 0, st>>>(g, cf, f, sides)
+#define QK_INJ(S)                                                                                              \
+    if (b_field && mid) k_inject<S, true, true, real><<<grid, block, 0, st>>>(g, cf, f, sides, md, energy);    \
+    else if (b_field) k_inject<S, true, false, real><<<grid, block, 0, st>>>(g, cf, f, sides, md, nullptr);    \
+    else k_inject<S, false, false, real><<<grid, block, 0, st>>>(g, cf, f, sides, md, nullptr)
         if (solver == 0) { QK_INJ(0); }
         else if (solver == 1) { QK_INJ(1); }
         else { QK_INJ(2); }
@@ -817,14 +854,14 @@ hipError_t launch_inject(hipStream_t st, int solver, const Grid &g, const Solver
 
 #define QK_INST(real)                                                                                            \
     template hipError_t launch_maxwell_b<real>(hipStream_t, int, const Grid &, const SolverCoef &, const Fields<real> &, \
-                                               double *, bool);                                                 \
+                                               double *, bool, real *const *);                                  \
     template hipError_t launch_maxwell_e<real>(hipStream_t, int, const Grid &, const SolverCoef &, const Fields<real> &, \
                                                const Current<real> *, const Current<real> *, const DiagDrain &); \
     template hipError_t launch_interpolate_be<real>(hipStream_t, const Grid &, const Fields<real> &, const real *const *); \
     template hipError_t launch_init_boundaries<real>(hipStream_t, int, const Grid &, const Fields<real> &);     \
     template hipError_t launch_laser_cos<real>(hipStream_t, const Grid &, const Fields<real> &, const double *); \
     template hipError_t launch_inject<real>(hipStream_t, int, const Grid &, const SolverCoef &, const Fields<real> &, \
-                                            int, int, const InjectArgs *);
+                                            int, int, const InjectArgs *, real *const *, double *);
 QK_INST(float)
 QK_INST(double)
 #undef QK_INST

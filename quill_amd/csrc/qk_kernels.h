@@ -159,10 +159,11 @@ constexpr int kEnergySlots = 256;
 
 // half step of B; with energy != null also accumulates sum(E^2 + B^2) of the
 // incoming fields into energy[0 .. kEnergySlots) (FP64).  twice: two half
-// steps with the same E, the energy taken between them.
+// steps with the same E, the energy taken between them and, with mid, the B
+// there stored to its three arrays.
 template <typename real>
 hipError_t launch_maxwell_b(hipStream_t st, int solver, const Grid &g, const SolverCoef &c, const Fields<real> &f,
-                            double *energy, bool twice = false);
+                            double *energy, bool twice = false, real *const *mid = nullptr);
 // n accumulators that the E step copies to pinned host memory and clears
 struct DiagDrain {
     double *acc = nullptr, *host = nullptr;
@@ -203,10 +204,13 @@ struct InjectArgs {
     int plane;
 };
 // the corrections of one sub-step for nsides (1 or 2) sides: b_field = 1 after
-// a B half step (from E_inc), 0 after the E step (from B_inc)
+// a B half step (from E_inc), 0 after the E step (from B_inc).  With mid, after
+// two half steps taken together (launch_maxwell_b): B is corrected for both,
+// mid for the first, and energy for the change of mid.
 template <typename real>
 hipError_t launch_inject(hipStream_t st, int solver, const Grid &g, const SolverCoef &c, const Fields<real> &f,
-                         int b_field, int nsides, const InjectArgs *a);
+                         int b_field, int nsides, const InjectArgs *a, real *const *mid = nullptr,
+                         double *energy = nullptr);
 template <typename real>
 hipError_t launch_load_uniform(hipStream_t st, const Grid &g, const Species<real> &s, int64_t first, int ppc,
                                double q, double sigma, uint64_t seed, int ilo, int ihi);

@@ -49,3 +49,31 @@ def test_source_planes_match_oracle(solver, shape, planes):
         err = np.abs(a - b).max() / np.abs(b).max()
         print(f"{name}: {err:.2e}", flush=True)
         assert err < 1e-10, name
+
+
+@pytest.mark.parametrize("plasma", [False, True])
+@pytest.mark.parametrize("solver", sorted(SOLVERS))
+def test_one_call_equals_single_steps(solver, plasma):
+    """Half steps of B taken in pairs inside a call, with the sources' corrections
+    and the field energy in between, against calls of one step: FP64, sums of
+    the same terms in another order."""
+    shape = (24, 11, 66)
+    dtf = SOLVERS[solver][1]
+    rec, ids = oracle.synth_plasma(*shape, 1, 0.02, 0.1, 17)
+    out = []
+    for calls in ((1,) * 14, (14,), (3, 11)):
+        print(f"calls {solver} plasma {plasma} {calls}", flush=True)
+        with qa.Region(*shape, DX, DX, DX, dtf * DX, solver=solver, pusher="vay", precision="fp64", sort_every=4) as r:
+            if plasma:
+                r.add_records(rec)
+            for side, plane in ((0, 3), (1, 19)):
+                L = pulse(plane * DX, -1.0 if side == 0 else 1.0, 0.15, 0.4)
+                r.add_laser_source(side, plane, *L[:11], phi=L[12])
+            r.init_boundaries()
+            en = [d["energy_f"] for n in calls for d in r.step(n, diag=True)]
+            out.append((r.get_fields(), en))
+    assert out[0][1][-1] > 10 * out[0][1][1] > 0
+    for f, en in out[1:]:
+        np.testing.assert_allclose(en, out[0][1], rtol=1e-12)
+        for a, b in zip(f, out[0][0]):
+            assert np.abs(a - b).max() <= 1e-12 * np.abs(b).max()
