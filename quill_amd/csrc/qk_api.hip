@@ -169,7 +169,7 @@ struct qk_ctx {
     int *s_counts = nullptr, *s_imm = nullptr, *s_offsets = nullptr, *s_tile_start = nullptr, *s_tile_mult = nullptr,
         *s_chunk_n = nullptr, *s_chunk_off = nullptr, *s_scratch = nullptr;
     int *h_sortinfo = nullptr;      // pinned: [live count, chunk count], workgroups of the joint push
-    double *d_diag = nullptr;       // two rows (steps alternate) of [QK_MAX_SPECIES][kDiagPerSpecies] + field energy
+    double *d_diag = nullptr;       // two rows (steps alternate) of kDiagRow
     double *diag_row = nullptr;     // the current step's
     double *h_diag = nullptr;       // pinned per-step copies of the accumulators
     size_t h_diag_cap = 0;          // steps that fit in h_diag
@@ -204,10 +204,16 @@ struct qk_ctx {
 
 namespace {
 
-// per-species accumulators, then the field-energy slots
-constexpr size_t kDiagLen = QK_MAX_SPECIES * kDiagPerSpecies + kEnergySlots + 1;
-// the last slot counts particles dropped for a non-finite momentum
+// a step's results: per-species accumulators, then the field-energy slots and
+// the count of particles dropped for a non-finite momentum
+constexpr size_t kSpeciesLen = QK_MAX_SPECIES * kDiagPerSpecies;
+constexpr size_t kDiagLen = kSpeciesLen + kEnergySlots + 1;
 constexpr size_t kNonfiniteSlot = kDiagLen - 1;
+// and where they are accumulated: the copies of the species' accumulators first
+constexpr size_t kRowEnergy = (size_t)kDiagSlots * kDiagStride;
+constexpr size_t kRowNonfinite = kRowEnergy + kEnergySlots;
+constexpr size_t kDiagRow = kRowNonfinite + 1;
+static_assert(kSpeciesLen <= (size_t)kDiagStride, "one copy holds every species");
 
 template <typename real>
 Fields<real> fields_of(qk_ctx *c)
@@ -495,7 +501,7 @@ void unpack_diag(const qk_ctx *c, const double *h, qk_diag &d)
         d.energy_ion += d.energy_ions[s - QK_ION0];
     }
     double ef_sum = 0;
-    for (int m = 0; m < kEnergySlots; ++m) ef_sum += h[QK_MAX_SPECIES * kDiagPerSpecies + m];
+    for (int m = 0; m < kEnergySlots; ++m) ef_sum += h[kSpeciesLen + m];
     d.energy_f = ef_sum * ef;
     d.n_nonfinite = (int64_t)h[kNonfiniteSlot];
 }
@@ -643,7 +649,7 @@ int qed_particle_phase(qk_ctx *c, const Fields<real> &f, const Current<real> &jc
         a.external_bz = c->p.external_bz;
         a.diag = c->diag_row + s * kDiagPerSpecies;
         a.energy_mode = b.energy_mode;
-        a.nonfinite = c->diag_row + kNonfiniteSlot;
+        a.nonfinite = c->diag_row + kRowNonfinite;
         a.first = 0;
         a.n = b.n;
         const Species<real> v = view<real>(b.buf[b.cur]);
@@ -661,7 +667,7 @@ int qed_particle_phase(qk_ctx *c, const Fields<real> &f, const Current<real> &jc
         a.external_bz = c->p.external_bz;
         a.diag = c->diag_row + QK_PHOTON * kDiagPerSpecies;
         a.energy_mode = 1;
-        a.nonfinite = c->diag_row + kNonfiniteSlot;
+        a.nonfinite = c->diag_row + kRowNonfinite;
         a.first = 0;
         a.n = n_ph0;
         HIP_TRY(launch_photon_qed<real>(c->stream, c->g, f, jc, view<real>(bph.buf[bph.cur]), a, qa,
@@ -1030,10 +1036,10 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
     // the event that marks the start of each step's particle phase: the end
     // of the step before unless something ran in between
     std::vector<int> start((size_t)nsteps);
-    HIP_TRY(launch_zero(c->stream, c->d_diag, 2 * kDiagLen));
+    HIP_TRY(launch_zero(c->stream, c->d_diag, 2 * kDiagRow));
     for (int l = 0; l < nsteps; ++l) {
         bool between = l == 0;
-        c->diag_row = c->d_diag + (l & 1) * kDiagLen;
+        c->diag_row = c->d_diag + (l & 1) * kDiagRow;
         if (tp.active && !tp.replay) {
             if (tp.steps > 0 && tp.steps % tp.every == 0) {
                 QK_TRY(tape_snapshot(c));
@@ -1110,7 +1116,7 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
             a.external_bz = c->p.external_bz;
             a.diag = c->diag_row + s * kDiagPerSpecies;
             a.energy_mode = b.energy_mode;
-            a.nonfinite = c->diag_row + kNonfiniteSlot;
+            a.nonfinite = c->diag_row + kRowNonfinite;
             const Species<real> v = view<real>(b.buf[b.cur]);
             if (tp.tangent && !tp.replay && b.kind == 0 && tp.n[s] > 0) {
                 // the tangent of this push, from the state before it
@@ -1143,18 +1149,17 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
         // fields before fadvance (src/main.cpp:2327)
         if (charged) c->j_zero[c->jcur] = false;
         const bool no_j = !charged && c->j_zero[0] && c->j_zero[1], last = l + 1 == nsteps;
-        constexpr size_t en = QK_MAX_SPECIES * kDiagPerSpecies;
         if (!fuse_b || l == 0) {
-            HIP_TRY(launch_maxwell_b<real>(c->stream, c->p.solver, c->g, c->coef, f, c->diag_row + en));
+            HIP_TRY(launch_maxwell_b<real>(c->stream, c->p.solver, c->g, c->coef, f, c->diag_row + kRowEnergy));
             QK_TRY(inject_impl<real>(c, 1, 0.0));
         }
-        const DiagDrain dd{c->diag_row, hd + (size_t)l * kDiagLen, (int)kDiagLen};
+        const DiagDrain dd{c->diag_row, hd + (size_t)l * kDiagLen, (int)kSpeciesLen, (int)(kDiagLen - kSpeciesLen)};
         HIP_TRY(launch_maxwell_e<real>(c->stream, c->p.solver, c->g, c->coef, f, no_j ? nullptr : &jc,
                                        no_j ? nullptr : &jn, dd));
         c->j_zero[c->jcur ^ 1] = true;
         QK_TRY(inject_impl<real>(c, 0, 0.5));
         if (fuse_b && !last) {
-            double *next_en = c->d_diag + ((l + 1) & 1) * kDiagLen + en;
+            double *next_en = c->d_diag + ((l + 1) & 1) * kDiagRow + kRowEnergy;
             HIP_TRY(launch_maxwell_b<real>(c->stream, c->p.solver, c->g, c->coef, f, next_en, true, mid));
             if (mid) QK_TRY(inject_impl<real>(c, 1, 1.0, mid, next_en));
         } else {
@@ -1473,7 +1478,7 @@ int qk_create(const qk_params *params, qk_ctx **out)
         return bail(fail(QK_ERR_HIP, std::string("field allocation: ") + hipGetErrorString(e)));
     if ((e = hipMemset(c->fmem, 0, fbytes * 15)) != hipSuccess) return bail(fail(QK_ERR_HIP, hipGetErrorString(e)));
     for (int a = 0; a < 15; ++a) c->F[a] = (char *)c->fmem + a * fbytes;
-    if ((e = hipMalloc(&c->d_diag, 2 * kDiagLen * sizeof(double))) != hipSuccess)
+    if ((e = hipMalloc(&c->d_diag, 2 * kDiagRow * sizeof(double))) != hipSuccess)
         return bail(fail(QK_ERR_HIP, hipGetErrorString(e)));
     if (p.qed) {
         if ((e = hipMalloc(&c->d_count, (QK_MAX_SPECIES + 1) * sizeof(int))) != hipSuccess ||

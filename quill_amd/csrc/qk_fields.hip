@@ -262,11 +262,27 @@ __global__ void __launch_bounds__(kSweep) k_maxwell_e(Grid g, SweepPlan sw, Coef
                                                       real *__restrict__ njx, real *__restrict__ njy,
                                                       real *__restrict__ njz, DiagDrain dd)
 {
-    if (dd.n > 0 && blockIdx.x == gridDim.x - 1)
-        for (int t = threadIdx.x; t < dd.n; t += kSweep) {
-            dd.host[t] = dd.acc[t];
-            dd.acc[t] = 0.0;
+    if (dd.n > 0 && blockIdx.x == gridDim.x - 1) {
+        // eight threads per accumulator, each summing every eighth copy
+        static_assert(kSweep == 8 * kDiagStride && kDiagSlots % 8 == 0, "a thread per accumulator and eighth of the copies");
+        const int a = threadIdx.x / 8, p = threadIdx.x % 8;
+        double v[kDiagSlots / 8], sum = 0;
+#pragma unroll
+        for (int m = 0; m < kDiagSlots / 8; ++m) {
+            double *s = dd.acc + (p + 8 * m) * kDiagStride + a;
+            v[m] = *s;
+            *s = 0.0;
         }
+#pragma unroll
+        for (int m = 0; m < kDiagSlots / 8; ++m) sum += v[m];
+        for (int o = 4; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+        if (p == 0 && a < dd.nspread) dd.host[a] = sum;
+        double *rest = dd.acc + kDiagSlots * kDiagStride;
+        for (int t = threadIdx.x; t < dd.n; t += kSweep) {
+            dd.host[dd.nspread + t] = rest[t];
+            rest[t] = 0.0;
+        }
+    }
     int i, j, k;
     if (!sweep_cell(g, sw, i, j, k)) return;
     const int id = i * g.sx + j * g.sy + k;

@@ -18,6 +18,13 @@ struct SolverCoef {
 // [0] sum q, [1] sum energy, [2] live count, [3] particles deposited through
 // the global fallback of the tiled kernel
 constexpr int kDiagPerSpecies = 4;
+// The accumulators of all species stand kDiagSlots times, kDiagStride doubles
+// apart, and a workgroup adds to the copy blockIdx mod kDiagSlots; the E step
+// sums the copies (DiagDrain).  FP64 atomics to one address take some 6 ns each
+// whatever else runs, those of 8192 workgroups 0.2 ms: particle phase 426 ->
+// 237 us at 256x128x128 with 1 per cell, 608 -> 595 us with 8 (NDFX, Vay), 27.7
+// -> 22.1 us at 64x32x32.  The workgroups of a copy are all of one XCD.
+constexpr int kDiagSlots = 64, kDiagStride = 32;
 
 // most particles per workgroup of the tiled kernel (a chunk never spans two
 // tiles; a tile is cut into equal chunks).  Twice the mean tile population at
@@ -32,7 +39,7 @@ struct PushArgs {
     double cmr;              // charge-to-mass ratio
     double external_bz;
     int64_t first, n;        // slots [first, first + n) (global kernel)
-    double *diag;            // kDiagPerSpecies doubles, accumulated atomically
+    double *diag;            // kDiagPerSpecies doubles of the first copy, accumulated atomically
     int energy_mode;         // 0: (g-1) q ; 1: g q (photons) ; 2: (g-1) q / cmr (ions)
     double *nonfinite;       // FP64 count of particles dropped for a non-finite momentum (may be null)
     // tiled kernel: work list of (tile, first slot, count) chunks
@@ -85,7 +92,7 @@ struct AppendTarget {
     int *count;
     int cap;
     int *overflow;
-    double *diag;        // kDiagPerSpecies accumulators of the target species
+    double *diag;        // kDiagPerSpecies accumulators of the target species (first copy)
 };
 
 // electrons / positrons with photon emission (src/advance.cpp:253-359);
@@ -173,10 +180,12 @@ constexpr int kEnergySlots = 256;
 template <typename real>
 hipError_t launch_maxwell_b(hipStream_t st, int solver, const Grid &g, const SolverCoef &c, const Fields<real> &f,
                             double *energy, bool twice = false, real *const *mid = nullptr);
-// n accumulators that the E step copies to pinned host memory and clears
+// accumulators that the E step hands to pinned host memory and clears: nspread
+// (at most kDiagStride) summed over their kDiagSlots copies, then the n that
+// follow those
 struct DiagDrain {
     double *acc = nullptr, *host = nullptr;
-    int n = 0;
+    int nspread = 0, n = 0;
 };
 // E step; j (may be null: both buffers are zero) the step's current, jn the
 // buffer to clear for the next

@@ -200,7 +200,7 @@ __global__ void __launch_bounds__(kBlock) k_push_global(Grid g, Fields<real> f, 
             store_rec(s, p, r);
         }
     }
-    block_accumulate(diag, da.q, da.e, da.n, da.fallback);
+    diag_accumulate(diag, da.q, da.e, da.n, da.fallback);
 }
 
 
@@ -505,7 +505,7 @@ __global__ void __launch_bounds__(kTBlock, sizeof(real) == 4 ? 4 : 2) k_push_til
         flush_component<2>(cur.jz, v[2], g, wi0, wj0, wk0);
     }
     if (!JOINT) {
-        block_accumulate(args.sp[m].diag, da.q, da.e, da.n, da.fallback);
+        diag_accumulate(args.sp[m].diag, da.q, da.e, da.n, da.fallback);
         return;
     }
     __syncthreads();
@@ -517,7 +517,7 @@ __global__ void __launch_bounds__(kTBlock, sizeof(real) == 4 ? 4 : 2) k_push_til
         v += o[a];
         n += o[2] + o[3];
     }
-    if (n != 0) atomicAdd(args.sp[r].diag + a, v);
+    if (n != 0) atomicAdd(args.sp[r].diag + blockIdx.x % kDiagSlots * kDiagStride + a, v);
 }
 
 // The runs of the joint launch: tile t = blockIdx.x * kBlock + threadIdx.x of
@@ -600,7 +600,7 @@ __global__ void __launch_bounds__(kBlock) k_photon_move(Grid g, Species<real> s,
             }
         }
     }
-    block_accumulate(diag, da.q, da.e, da.n, 0.0);
+    diag_accumulate(diag, da.q, da.e, da.n, 0.0);
 }
 
 // Uniform thermal plasma: ppc particles per is_inside cell with ilo <= i < ihi,

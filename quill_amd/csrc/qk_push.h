@@ -89,6 +89,12 @@ __device__ inline void block_accumulate(double *dst, double v0, double v1, doubl
     }
 }
 
+// the same into this workgroup's copy of a species' accumulators
+__device__ inline void diag_accumulate(double *diag, double v0, double v1, double v2, double v3)
+{
+    block_accumulate(diag + blockIdx.x % kDiagSlots * kDiagStride, v0, v1, v2, v3);
+}
+
 struct DiagAcc {
     double q = 0, e = 0;
     int n = 0, fallback = 0;

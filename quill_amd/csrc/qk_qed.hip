@@ -183,8 +183,8 @@ __global__ void __launch_bounds__(kBlock) k_push_qed_lepton(Grid g, Fields<real>
             s.cell[p] = -1;
         }
     }
-    block_accumulate(diag, da.q, da.e, da.n, 0.0);
-    block_accumulate(ph.diag, dph.q, dph.e, dph.n, 0.0);
+    diag_accumulate(diag, da.q, da.e, da.n, 0.0);
+    diag_accumulate(ph.diag, dph.q, dph.e, dph.n, 0.0);
 }
 
 // One lepton of a Breit-Wheeler pair (bear_particle, src/mc.cpp:118-139,
@@ -270,9 +270,9 @@ __global__ void __launch_bounds__(kBlock) k_photon_qed(Grid g, Fields<real> f, C
             s.cell[p] = -1;
         }
     }
-    block_accumulate(diag, da.q, da.e, da.n, 0.0);
-    block_accumulate(el.diag, de.q, de.e, de.n, 0.0);
-    block_accumulate(po.diag, dp.q, dp.e, dp.n, 0.0);
+    diag_accumulate(diag, da.q, da.e, da.n, 0.0);
+    diag_accumulate(el.diag, de.q, de.e, de.n, 0.0);
+    diag_accumulate(po.diag, dp.q, dp.e, dp.n, 0.0);
 }
 
 template <typename real, int PUSHER>
