@@ -97,17 +97,6 @@ struct SpeciesBuf {
     double fb_last = -1;    // window-fallback fraction of the last finished step (-1: unknown or re-sorted since)
     int ishift = 0;         // moving-window shifts since the last sort
     int *tile_start = nullptr;   // ntiles + 1: the tiles of slots [0, n_sorted) (the next sort's source)
-    uint64_t layout = 0;    // changes with tile_start and the slots it refers to
-};
-
-// the joint work list of the species pushed together (launch_joint_runs), and
-// the layouts it was made from
-struct JointList {
-    int ns = 0, n = 0;
-    int sp[kMaxTiled] = {};
-    uint64_t layout[kMaxTiled] = {};
-    int4 *runs = nullptr;
-    size_t cap = 0;         // entries
 };
 
 // The recorded trajectory of qk_tape_begin: snapshots of the whole device
@@ -163,12 +152,10 @@ struct qk_ctx {
     bool j_zero[2] = {true, true};  // which current buffers are known to be zero
     bool have_step = false;
     SpeciesBuf sp[QK_MAX_SPECIES];
-    uint64_t layouts = 0;           // last value given to a SpeciesBuf::layout
-    JointList joint;
     // shared sort buffers (allocated at the first sort)
     int *s_counts = nullptr, *s_imm = nullptr, *s_offsets = nullptr, *s_tile_start = nullptr, *s_tile_mult = nullptr,
         *s_chunk_n = nullptr, *s_chunk_off = nullptr, *s_scratch = nullptr;
-    int *h_sortinfo = nullptr;      // pinned: [live count, chunk count], workgroups of the joint push
+    int *h_sortinfo = nullptr;      // pinned: [live count, chunk count]
     double *d_diag = nullptr;       // two rows (steps alternate) of kDiagRow
     double *diag_row = nullptr;     // the current step's
     double *h_diag = nullptr;       // pinned per-step copies of the accumulators
@@ -320,7 +307,6 @@ int reserve(qk_ctx *c, int s, int64_t cap)
     b.max_chunks = (int)mc;
     b.n_sorted = 0;   // the work list refers to the old buffers
     b.nchunks = 0;
-    b.layout = ++c->layouts;
     return QK_OK;
 }
 
@@ -362,7 +348,7 @@ int ensure_sort_buffers(qk_ctx *c)
     HIP_TRY(hipMalloc(&c->s_chunk_n, nt * sizeof(int)));
     HIP_TRY(hipMalloc(&c->s_chunk_off, nt * sizeof(int)));
     HIP_TRY(hipMalloc(&c->s_scratch, scan_scratch_ints(std::max(nk, nt)) * sizeof(int)));
-    HIP_TRY(hipHostMalloc((void **)&c->h_sortinfo, 3 * sizeof(int)));
+    HIP_TRY(hipHostMalloc((void **)&c->h_sortinfo, 2 * sizeof(int)));
     return QK_OK;
 }
 
@@ -415,68 +401,10 @@ int sort_species(qk_ctx *c, int s)
     b.n = c->h_sortinfo[0];
     b.n_sorted = b.n;
     b.nchunks = c->h_sortinfo[1];
-    b.layout = ++c->layouts;
     b.steps_since_sort = 0;
     b.fb_last = -1;
     b.ishift = 0;
     if (b.nchunks > b.max_chunks) return fail(QK_ERR_STATE, "tile work list overflow");
-    return QK_OK;
-}
-
-// The joint work list of ns species, made again when one of them was sorted.
-// joint stays false where each species is better pushed on its own, or where
-// their tiles do not lie alike (a species sorted since a window shift that
-// another has not been sorted after).
-//
-// A species' chunk costs about five rounds of 512 particles to stage and to
-// flush; a tile taken jointly pays that once, but its rounds run 5 % slower
-// (the species loop's registers).  Particle phase, apart and jointly: two
-// species at 256x128x128, 1 and 4 per cell, 789 -> 408 us and 944 -> 686 us;
-// three at 135x75x71, 3 per cell, 258 -> 165 us; two in FP64 at 97x61x53, 8 per
-// cell (a mean of 2995 per tile), 156 -> 153 us; but two at 128x64x64, 8 and
-// (at 128x96x64) 16 per cell, 154 -> 160 us and 371 -> 387 us, and three of 27
-// per cell 440 -> 470 us.
-constexpr int kJointMean = 3072;   // most particles per tile and species, in the mean
-
-int joint_list(qk_ctx *c, int ns, const int *sp, bool &joint, bool &made)
-{
-    JointList &j = c->joint;
-    joint = false;
-    bool same = j.ns == ns;
-    int64_t n = 0;
-    for (int m = 0; m < ns; ++m) {
-        const SpeciesBuf &b = c->sp[sp[m]];
-        if (b.n_sorted <= 0 || b.ishift != c->sp[sp[0]].ishift) return QK_OK;
-        same = same && j.sp[m] == sp[m] && j.layout[m] == b.layout;
-        n += b.n_sorted;
-    }
-    if (n > (int64_t)kJointMean * ns * c->tg.ntiles) return QK_OK;
-    joint = true;
-    if (same) return QK_OK;
-    made = true;
-    j.ns = 0;
-    const int per = chunk_size(c, n), chunk = per == kChunk ? ns * kChunk : per;
-    const int64_t items = c->tg.ntiles + n / chunk + 1;
-    const size_t need = (size_t)items * ns;
-    if (need > j.cap) {
-        if (j.runs) HIP_TRY(hipFree(j.runs));
-        j.runs = nullptr;
-        j.cap = 0;
-        HIP_TRY(hipMalloc(&j.runs, need * sizeof(int4)));
-        j.cap = need;
-    }
-    const int *start[kMaxTiled];
-    for (int m = 0; m < ns; ++m) start[m] = c->sp[sp[m]].tile_start;
-    HIP_TRY(launch_joint_runs(c->stream, ns, start, c->tg.ntiles, chunk, c->s_chunk_n, c->s_chunk_off, c->s_scratch,
-                              j.runs, (int)items, c->h_sortinfo + 2));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    j.n = c->h_sortinfo[2];
-    if (j.n > items) return fail(QK_ERR_STATE, "joint work list overflow");
-    j.ns = ns;
-    for (int m = 0; m < ns; ++m) {
-        j.sp[m] = sp[m];
-        j.layout[m] = c->sp[sp[m]].layout;
-    }
     return QK_OK;
 }
 
@@ -1087,13 +1015,6 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
             c->merge_due = false;
             between = true;
         }
-        bool joint = false;
-        if (tiled) {
-            int tsp[kMaxTiled], nt = 0;
-            for (int s = 0; s < QK_MAX_SPECIES; ++s)
-                if (c->sp[s].active && c->sp[s].n > 0 && c->sp[s].kind == 0) tsp[nt++] = s;
-            if (nt > 1) QK_TRY(joint_list(c, nt, tsp, joint, between));
-        }
         const Current<real> jc = current_of<real>(c, c->jcur), jn = current_of<real>(c, c->jcur ^ 1);
         // padvance (src/advance.cpp:90-387); the push kernels erase the
         // particles p_boundary (src/plist.cpp:73-102) would: those outside
@@ -1141,8 +1062,7 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
             HIP_TRY(launch_push_global<real>(c->stream, c->g, f, jc, v, a));
             ++b.steps_since_sort;
         }
-        if (nt > 0) HIP_TRY(launch_push_tiled<real>(c->stream, c->g, f, jc, c->tg, nt, ts, ta,
-                                                     joint ? c->joint.runs : nullptr, c->joint.n));
+        if (nt > 0) HIP_TRY(launch_push_tiled<real>(c->stream, c->g, f, jc, c->tg, nt, ts, ta));
         HIP_TRY(hipEventRecord(c->ev[3 * l + 1], c->stream));
         // fadvance (src/advance.cpp:13-18): B half, E, B half, interpolate_be.  The
         // first half step also sums compute_energy's field term, which sees the
@@ -1512,7 +1432,6 @@ int qk_destroy(qk_ctx *c)
     for (int *p : sb)
         if (p) note(hipFree(p));
     if (c->h_sortinfo) note(hipHostFree(c->h_sortinfo));
-    if (c->joint.runs) note(hipFree(c->joint.runs));
     if (c->fmem) note(hipFree(c->fmem));
     if (c->mid) note(hipFree(c->mid));
     if (c->d_diag) note(hipFree(c->d_diag));

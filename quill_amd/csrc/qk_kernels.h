@@ -59,20 +59,11 @@ hipError_t launch_push_global(hipStream_t st, const Grid &g, const Fields<real> 
                               const Species<real> &s, const PushArgs &a);
 // one workgroup per chunk of a cell tile: the current is accumulated in an
 // LDS window around the tile and flushed to global memory once; the chunks
-// of all ns species (at most kMaxTiled, one pusher) in one launch; with runs,
-// nruns workgroups that each take every species' part of a tile
+// of all ns species (at most kMaxTiled, one pusher) in one launch
 constexpr int kMaxTiled = 6;
 template <typename real>
 hipError_t launch_push_tiled(hipStream_t st, const Grid &g, const Fields<real> &f, const Current<real> &j,
-                             const TileGeom &tg, int ns, const Species<real> *s, const PushArgs *a,
-                             const int4 *runs = nullptr, int nruns = 0);
-// the runs of ns species sorted into the same tiles (start[m]: ntiles + 1 first
-// slots): ns entries (tile, first slot, count) for each of *n workgroups, a
-// tile cut into parts of about `chunk` particles of all species.  parts, off:
-// ntiles + 1 ints each; scratch as for the scan; n: pinned host memory; at most
-// max_items workgroups are written.
-hipError_t launch_joint_runs(hipStream_t st, int ns, const int *const *start, int ntiles, int chunk, int *parts,
-                             int *off, int *scratch, int4 *runs, int max_items, int *n);
+                             const TileGeom &tg, int ns, const Species<real> *s, const PushArgs *a);
 
 // ---- QED -------------------------------------------------------------------
 

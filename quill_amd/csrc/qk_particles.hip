@@ -34,11 +34,15 @@ constexpr int kT[3] = {kTx, kTy, kTz};
 #ifndef QK_TBLOCK
 #define QK_TBLOCK 512
 #endif
+#ifdef QK_TWAVES_EU
+#define QK_TATTR __attribute__((amdgpu_waves_per_eu(QK_TWAVES_EU)))
+#else
+#define QK_TATTR
+#endif
 constexpr int kTBlock = QK_TBLOCK;
 // out-of-window particles listed per workgroup and pushed after its rounds:
 // at most this many per chunk, the rest inline
 constexpr int kDefer = 512;
-constexpr int kWaveSums = kTBlock / 64 * 4;   // doubles
 
 // Current window, FP64, one block per component.  A deposit from start cell
 // r touches cells r-1 .. r+1 (one face crossing per axis at most) and, for
@@ -204,41 +208,6 @@ __global__ void __launch_bounds__(kBlock) k_push_global(Grid g, Fields<real> f, 
 }
 
 
-// sum over the wavefront, in its last lane, by DPP moves: no lane indices to
-// keep in registers through the push loop, as a shuffle's would be
-template <int CTRL, int ROWS>
-__device__ inline double add_moved(double v)
-{
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, true);
-    return v + __hiloint2double(hi, lo);
-}
-
-__device__ inline double last_lane_sum(double v)
-{
-    v = add_moved<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8: sums of 16 lanes in lanes 15, 31, 47, 63
-    v = add_moved<0x112, 0xf>(v);
-    v = add_moved<0x114, 0xf>(v);
-    v = add_moved<0x118, 0xf>(v);
-    v = add_moved<0x142, 0xa>(v);   // lane 15 to row 1, lane 47 to row 3
-    return add_moved<0x143, 0xc>(v);   // lane 31 to rows 2 and 3
-}
-
-// a wavefront's diagnostics added to its four sums in LDS; every lane takes part
-__device__ inline void add_sums(double *sums, const DiagAcc &da)
-{
-    const bool last = (threadIdx.x & 63) == 63;
-    double *w = sums + threadIdx.x / 64 * 4;
-    double v = last_lane_sum(da.q);
-    if (last) w[0] += v;
-    v = last_lane_sum(da.e);
-    if (last) w[1] += v;
-    v = last_lane_sum((double)da.n);
-    if (last) w[2] += v;
-    v = last_lane_sum((double)da.fallback);
-    if (last) w[3] += v;
-}
-
 // A particle that starts outside the window is not pushed in its round but
 // listed (its slot) in LDS, and the workgroup pushes the listed particles
 // after its rounds, one per thread, through global memory.  Inline, every
@@ -262,29 +231,20 @@ struct TiledSpecies {
     int ishift;    // a tile's cells now start at i = 8 ti - ishift
 };
 
-// Two launch forms.  JOINT: one workgroup takes every species' particles of
-// its tile in turn, so the tile is staged and its current flushed once, not
-// once per species; runs holds ns entries (tile, first slot, count) per
-// workgroup, one per species, some empty (launch_joint_runs).  Otherwise each
-// workgroup takes one chunk of one species.  joint_list chooses, where the
-// measurements stand.
 template <typename real>
 struct TiledArgs {
     TiledSpecies<real> sp[kMaxTiled];
     int ns;
-    const int4 *runs;
 };
 
-template <typename real, int PUSHER, bool JOINT>
-__global__ void __launch_bounds__(kTBlock, sizeof(real) == 4 ? 4 : 2) k_push_tiled(Grid g, Fields<real> f, Current<real> cur, TileGeom tg,
+template <typename real, int PUSHER>
+__global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<real> f, Current<real> cur, TileGeom tg,
                                                                 TiledArgs<real> args)
 {
     __shared__ double win[kJWin];
     __shared__ EB<real> stage[kFStage];
     __shared__ uint32_t listed[kDefer];
     __shared__ int nlisted;
-    __shared__ uint8_t listed_sp[JOINT ? kDefer : 1];      // their species
-    __shared__ double sums[JOINT ? kMaxTiled * kWaveSums : 1];   // diagnostics per species and wavefront
     // Chunks in groups of kXcdGroup per XCD.  Workgroups are dealt to the
     // XCDs round-robin; a line of the field arrays spans four tiles along k,
     // and neighbouring tiles share their halos, so with neighbours on
@@ -300,12 +260,15 @@ __global__ void __launch_bounds__(kTBlock, sizeof(real) == 4 ? 4 : 2) k_push_til
         vb = (l / kXcdGroup * 8 + xcd) * kXcdGroup + l % kXcdGroup;
     }
     int m = 0;
-    while (!JOINT && m + 1 < args.ns && vb >= args.sp[m + 1].first) ++m;
-    const int4 *runs = JOINT ? args.runs + (size_t)vb * args.ns : args.sp[m].chunks + (vb - args.sp[m].first);
-    const int tile = runs->x;
+    while (m + 1 < args.ns && vb >= args.sp[m + 1].first) ++m;
+    const TiledSpecies<real> &sp = args.sp[m];
+    const Species<real> s = sp.s;
+    const StepConst<real> sc = sp.sc;
+    const int4 ch = sp.chunks[vb - sp.first];
+    const int tile = ch.x;
     const int tk = tile % tg.ntz, t2 = tile / tg.ntz;
     const int tj = t2 % tg.nty, ti = t2 / tg.nty;
-    const int i0 = ti * kTx - args.sp[m].ishift, j0 = tj * kTy, k0 = tk * kTz;
+    const int i0 = ti * kTx - sp.ishift, j0 = tj * kTy, k0 = tk * kTz;
     // Slots as 32-bit indices: the record arrays are addressed as scalar
     // base + one shared 32-bit byte offset (capacity keeps slot * size below
     // 2^32).  The first two rounds' records load while the tile is staged.
@@ -318,26 +281,18 @@ __global__ void __launch_bounds__(kTBlock, sizeof(real) == 4 ? 4 : 2) k_push_til
     // 2.67 ms from an aligned one (5.8 TB/s; 2.90 and 2.78 ms with cached
     // accesses, which cost the field sweeps 20 % at 256x128x128).  Push 5.36 ->
     // 4.73 ms at 512x256x256, 0.675 -> 0.62 ms at 256x128x128.
-    auto first_slot = [](const int4 &ch, uint32_t n) {   // the n-th particle of a run in the order of the rounds
-        const uint32_t count = (uint32_t)ch.z, end32 = (uint32_t)ch.y + count;
-        const uint32_t q = min(((uint32_t)ch.y + 31u) & ~31u, end32) + n;
+    const uint32_t count = (uint32_t)ch.z, end32 = (uint32_t)ch.y + count;
+    const uint32_t aligned = min(((uint32_t)ch.y + 31u) & ~31u, end32);
+    auto slot_of = [&](uint32_t n) {   // the n-th particle in the order of the rounds
+        const uint32_t q = aligned + n;
         return q < end32 ? q : q - count;
     };
+    uint32_t n = threadIdx.x;
     PRec<real> r1, r2;   // the records one and two rounds ahead
-    // a run's entry, in scalar registers (the compiler cannot know that nothing stores to it)
-    auto run_entry = [&](int r) {
-        const int4 v = runs[r];
-        return make_int4(v.x, __builtin_amdgcn_readfirstlane(v.y), __builtin_amdgcn_readfirstlane(v.z), 0);
-    };
-    auto load_first = [&](int m, const int4 &ch) {
-        if (threadIdx.x < (uint32_t)ch.z) load_rec32(args.sp[m].s, first_slot(ch, threadIdx.x), r1);
-        if (threadIdx.x + kTBlock < (uint32_t)ch.z) load_rec32(args.sp[m].s, first_slot(ch, threadIdx.x + kTBlock), r2);
-    };
-    load_first(m, run_entry(0));
+    if (n < count) load_rec32(s, slot_of(n), r1);
+    if (n + kTBlock < count) load_rec32(s, slot_of(n + kTBlock), r2);
     for (int w = threadIdx.x; w < kJWin; w += kTBlock) win[w] = 0.0;
     if (threadIdx.x == 0) nlisted = 0;
-    if (JOINT && threadIdx.x < kMaxTiled * kWaveSums) sums[threadIdx.x] = 0.0;
-    static_assert(kMaxTiled * kWaveSums <= kTBlock, "one sum per thread");
     {
         const int si = i0 - kHalo, sj = j0 - kHalo, sk = k0 - kHalo;
         real v[6][kStageIt];
@@ -354,129 +309,110 @@ __global__ void __launch_bounds__(kTBlock, sizeof(real) == 4 ? 4 : 2) k_push_til
     __syncthreads();
 
     DiagAcc da;
-    for (int run = 0; run < (JOINT ? args.ns : 1); ++run) {
-        if (JOINT) m = run;
-        const Species<real> s = args.sp[m].s;
-        const StepConst<real> sc = args.sp[m].sc;
-        const int4 ch = run_entry(run);
-        const uint32_t count = (uint32_t)ch.z;
-        auto slot_of = [&](uint32_t n) { return first_slot(ch, n); };
-        uint32_t n = threadIdx.x;
-        // start cell relative to the tile, and whether it lies in the window
-        int ri = 0, rj = 0, rk = 0;
-        bool in_win = false;
-        auto dep = [&](int, int, int, int base, real q, real pos[3], const real d[3], DiagAcc &acc_d) {
-            // one accumulator per branch: a shared one with per-lane atomics
-            // (path split once, two masked atomics per term) measured 2.5 % slower
-            if (in_win) {
-                LdsAcc<real> acc(win, ri, rj, rk);
-                deposit_path<real>(acc, q, pos, d);
-            } else {
-                GlobalAcc<real> acc{cur.jx, cur.jy, cur.jz, g.sx, g.sy, base, base};
-                deposit_path<real>(acc, q, pos, d);
-                acc_d.fallback += 1;
-            }
-        };
-        // software pipeline over the rounds of kTBlock particles: while one
-        // particle is pushed, the next round's record has its field nodes
-        // gathered and the record two rounds ahead is loading (the first two
-        // rounds' records were issued before the staging).  listed_q: the
-        // particle was listed for the pass after the rounds.
-        auto gather = [&](const PRec<real> &q, uint32_t slot, int &a, int &b, int &cc, bool &w, bool &listed_q,
-                          Corners<real> &nd) {
-            listed_q = false;
-            if (q.cell < 0) return;
-            a = cell_i(q.cell) - i0;
-            b = cell_j(q.cell) - j0;
-            cc = cell_k(q.cell) - k0;
-            w = (unsigned)(a + kHalo) < (unsigned)(kTx + 2 * kHalo) && (unsigned)(b + kHalo) < (unsigned)(kTy + 2 * kHalo) &&
-                (unsigned)(cc + kHalo) < (unsigned)(kTz + 2 * kHalo);
-            if (w) {
-                load_corners_stage(stage, a, b, cc, nd);
-                return;
-            }
-            const int at = atomicAdd(&nlisted, 1);
-            if (at < kDefer) {
-                listed[at] = slot;
-                if (JOINT) listed_sp[at] = (uint8_t)m;
-                listed_q = true;
-                return;
-            }
-            load_corners(f, cell_base(g, q.cell), g.sx, g.sy, nd);
-        };
-        int ri1 = 0, rj1 = 0, rk1 = 0;
-        bool w1 = false, l1 = false;
-        // The pipeline carries the next particle's E and Be (six values), not
-        // its 24 field nodes: the nodes' LDS reads are issued before the push of
-        // the current particle and interpolated after it, so the nodes are dead
-        // at the loop's end and only six values are copied there (about a
-        // hundred fewer register moves per round; push 0.5 % faster).
-        real e1[3] = {}, b1[3] = {};
-        if (n < count) {
-            Corners<real> nd;
-            gather(r1, slot_of(n), ri1, rj1, rk1, w1, l1, nd);
-            if (r1.cell >= 0 && !l1) interp_corners(nd, r1.o[0], r1.o[1], r1.o[2], e1, b1);
+    // start cell relative to the tile, and whether it lies in the window
+    int ri = 0, rj = 0, rk = 0;
+    bool in_win = false;
+    auto dep = [&](int, int, int, int base, real q, real pos[3], const real d[3], DiagAcc &acc_d) {
+        // one accumulator per branch: a shared one with per-lane atomics
+        // (path split once, two masked atomics per term) measured 2.5 % slower
+        if (in_win) {
+            LdsAcc<real> acc(win, ri, rj, rk);
+            deposit_path<real>(acc, q, pos, d);
+        } else {
+            GlobalAcc<real> acc{cur.jx, cur.jy, cur.jz, g.sx, g.sy, base, base};
+            deposit_path<real>(acc, q, pos, d);
+            acc_d.fallback += 1;
         }
-        // Each round stores the record of the round before it, right after
-        // issuing its own loads: gfx9 counts loads and stores in one vmcnt, so
-        // the loop's wait for those loads (one round later) then waits for
-        // stores that have had a whole push to complete, not for stores just
-        // issued.  The first round rewrites its own record unchanged, and free
-        // and listed slots are rewritten unchanged, which keeps the stores
-        // unconditional.
-        PRec<real> rs = r1;
-        uint32_t ps = slot_of(n);
-        const bool started = n < count;
-        for (; n < count; n += kTBlock) {
-            PRec<real> r = r1;
-            const real e[3] = {e1[0], e1[1], e1[2]}, b[3] = {b1[0], b1[1], b1[2]};
-            ri = ri1;
-            rj = rj1;
-            rk = rk1;
-            in_win = w1;
-            const bool is_listed = l1;
-            r1 = r2;
-            const bool more = n + kTBlock < count;
-            Corners<real> nd;
-            // The round's memory operations (the next particle's LDS reads, the
-            // record two rounds ahead, the previous record's store) are issued
-            // at a raised wavefront priority, so that they reach the memory
-            // system ahead of the other wavefronts' arithmetic: push 1.3 %
-            // faster at both 512x256x256 and 256x128x128 (priority 1 or 3, or
-            // raised also for the staging or the flush, measured less).
-            __builtin_amdgcn_s_setprio(2);
-            if (more) gather(r1, slot_of(n + kTBlock), ri1, rj1, rk1, w1, l1, nd);
-            if (n + 2 * kTBlock < count) load_rec32(s, slot_of(n + 2 * kTBlock), r2);
-            store_rec32(s, ps, rs);
-            __builtin_amdgcn_s_setprio(0);
-            if (r.cell >= 0 && !is_listed) advance_particle_eb<real, PUSHER>(g, e, b, r, sc, dep, da);
-            if (more && r1.cell >= 0 && !l1) interp_corners(nd, r1.o[0], r1.o[1], r1.o[2], e1, b1);
-            rs = r;
-            ps = slot_of(n);
+    };
+    // software pipeline over the rounds of kTBlock particles: while one
+    // particle is pushed, the next round's record has its field nodes
+    // gathered and the record two rounds ahead is loading (the first two
+    // rounds' records were issued before the staging).  listed_q: the
+    // particle was listed for the pass after the rounds.
+    auto gather = [&](const PRec<real> &q, uint32_t slot, int &a, int &b, int &cc, bool &w, bool &listed_q,
+                      Corners<real> &nd) {
+        listed_q = false;
+        if (q.cell < 0) return;
+        a = cell_i(q.cell) - i0;
+        b = cell_j(q.cell) - j0;
+        cc = cell_k(q.cell) - k0;
+        w = (unsigned)(a + kHalo) < (unsigned)(kTx + 2 * kHalo) && (unsigned)(b + kHalo) < (unsigned)(kTy + 2 * kHalo) &&
+            (unsigned)(cc + kHalo) < (unsigned)(kTz + 2 * kHalo);
+        if (w) {
+            load_corners_stage(stage, a, b, cc, nd);
+            return;
         }
-        if (JOINT && run + 1 < args.ns) load_first(run + 1, run_entry(run + 1));
-        if (started) store_rec32(s, ps, rs);
-        if (JOINT) {
-            add_sums(sums + m * kWaveSums, da);
-            da = DiagAcc();
+        const int at = atomicAdd(&nlisted, 1);
+        if (at < kDefer) {
+            listed[at] = slot;
+            listed_q = true;
+            return;
         }
+        load_corners(f, cell_base(g, q.cell), g.sx, g.sy, nd);
+    };
+    int ri1 = 0, rj1 = 0, rk1 = 0;
+    bool w1 = false, l1 = false;
+    // The pipeline carries the next particle's E and Be (six values), not
+    // its 24 field nodes: the nodes' LDS reads are issued before the push of
+    // the current particle and interpolated after it, so the nodes are dead
+    // at the loop's end and only six values are copied there (about a
+    // hundred fewer register moves per round; push 0.5 % faster).
+    real e1[3] = {}, b1[3] = {};
+    if (n < count) {
+        Corners<real> nd;
+        gather(r1, slot_of(n), ri1, rj1, rk1, w1, l1, nd);
+        if (r1.cell >= 0 && !l1) interp_corners(nd, r1.o[0], r1.o[1], r1.o[2], e1, b1);
     }
+    // Each round stores the record of the round before it, right after
+    // issuing its own loads: gfx9 counts loads and stores in one vmcnt, so
+    // the loop's wait for those loads (one round later) then waits for
+    // stores that have had a whole push to complete, not for stores just
+    // issued.  The first round rewrites its own record unchanged, and free
+    // and listed slots are rewritten unchanged, which keeps the stores
+    // unconditional.
+    PRec<real> rs = r1;
+    uint32_t ps = slot_of(n);
+    const bool started = n < count;
+    for (; n < count; n += kTBlock) {
+        PRec<real> r = r1;
+        const real e[3] = {e1[0], e1[1], e1[2]}, b[3] = {b1[0], b1[1], b1[2]};
+        ri = ri1;
+        rj = rj1;
+        rk = rk1;
+        in_win = w1;
+        const bool is_listed = l1;
+        r1 = r2;
+        const bool more = n + kTBlock < count;
+        Corners<real> nd;
+        // The round's memory operations (the next particle's LDS reads, the
+        // record two rounds ahead, the previous record's store) are issued
+        // at a raised wavefront priority, so that they reach the memory
+        // system ahead of the other wavefronts' arithmetic: push 1.3 %
+        // faster at both 512x256x256 and 256x128x128 (priority 1 or 3, or
+        // raised also for the staging or the flush, measured less).
+        __builtin_amdgcn_s_setprio(2);
+        if (more) gather(r1, slot_of(n + kTBlock), ri1, rj1, rk1, w1, l1, nd);
+        if (n + 2 * kTBlock < count) load_rec32(s, slot_of(n + 2 * kTBlock), r2);
+        store_rec32(s, ps, rs);
+        __builtin_amdgcn_s_setprio(0);
+        if (r.cell >= 0 && !is_listed) advance_particle_eb<real, PUSHER>(g, e, b, r, sc, dep, da);
+        if (more && r1.cell >= 0 && !l1) interp_corners(nd, r1.o[0], r1.o[1], r1.o[2], e1, b1);
+        rs = r;
+        ps = slot_of(n);
+    }
+    if (started) store_rec32(s, ps, rs);
     // the listed slots' rewrites complete before the pass below stores them
     // again (vmcnt 0; expcnt and lgkmcnt left at their maxima)
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
-    const int nl = min(nlisted, kDefer);
-    for (int run = 0; run < (JOINT ? args.ns : 1) && nl > 0; ++run) {
-        if (JOINT) m = run;
-        const Species<real> s = args.sp[m].s;
-        const StepConst<real> sc = args.sp[m].sc;
+    {
         auto gdep = [&](int, int, int, int base, real q, real pos[3], const real d[3], DiagAcc &acc_d) {
             GlobalAcc<real> acc{cur.jx, cur.jy, cur.jz, g.sx, g.sy, base, base};
             deposit_path<real>(acc, q, pos, d);
             acc_d.fallback += 1;
         };
+        const int nl = min(nlisted, kDefer);
         for (int e = threadIdx.x; e < nl; e += kTBlock) {
-            if (JOINT && listed_sp[e] != m) continue;
             const uint32_t q = listed[e];
             PRec<real> rr;
             load_rec32(s, q, rr);
@@ -484,10 +420,6 @@ __global__ void __launch_bounds__(kTBlock, sizeof(real) == 4 ? 4 : 2) k_push_til
             load_corners(f, cell_base(g, rr.cell), g.sx, g.sy, nn);
             advance_particle<real, PUSHER>(g, nn, rr, sc, gdep, da);
             store_rec32(s, q, rr);
-        }
-        if (JOINT) {
-            add_sums(sums + m * kWaveSums, da);
-            da = DiagAcc();
         }
     }
 
@@ -504,54 +436,7 @@ __global__ void __launch_bounds__(kTBlock, sizeof(real) == 4 ? 4 : 2) k_push_til
         flush_component<1>(cur.jy, v[1], g, wi0, wj0, wk0);
         flush_component<2>(cur.jz, v[2], g, wi0, wj0, wk0);
     }
-    if (!JOINT) {
-        diag_accumulate(args.sp[m].diag, da.q, da.e, da.n, da.fallback);
-        return;
-    }
-    __syncthreads();
-    const int r = threadIdx.x / 4, a = threadIdx.x % 4;
-    if (r >= args.ns) return;
-    double v = 0, n = 0;
-    for (int w = 0; w < kWaveSums; w += 4) {
-        const double *o = sums + r * kWaveSums + w;
-        v += o[a];
-        n += o[2] + o[3];
-    }
-    if (n != 0) atomicAdd(args.sp[r].diag + blockIdx.x % kDiagSlots * kDiagStride + a, v);
-}
-
-// The runs of the joint launch: tile t = blockIdx.x * kBlock + threadIdx.x of
-// every species is cut into as many parts as its particles together need
-// (parts[t], scanned by the caller), and part p takes the p-th piece of each.
-struct JointTiles {
-    const int *start[kMaxTiled];   // ntiles + 1 first slots
-    int ns, ntiles, chunk;
-    __device__ inline int parts(int t) const
-    {
-        int64_t n = 0;
-        for (int m = 0; m < ns; ++m) n += start[m][t + 1] - start[m][t];
-        return (int)((n + chunk - 1) / chunk);
-    }
-};
-
-__global__ void __launch_bounds__(kBlock) k_joint_parts(JointTiles jt, int *parts)
-{
-    const int t = blockIdx.x * kBlock + threadIdx.x;
-    if (t <= jt.ntiles) parts[t] = t < jt.ntiles ? jt.parts(t) : 0;
-}
-
-__global__ void __launch_bounds__(kBlock) k_joint_runs(JointTiles jt, const int *off, int4 *runs, int max_items, int *n)
-{
-    const int t = blockIdx.x * kBlock + threadIdx.x;
-    if (t == 0) *n = off[jt.ntiles];
-    if (t >= jt.ntiles) return;
-    const int np = jt.parts(t), o = off[t];
-    for (int p = 0; p < np && o + p < max_items; ++p)
-        for (int m = 0; m < jt.ns; ++m) {
-            const int s = jt.start[m][t], e = jt.start[m][t + 1], sz = (e - s + np - 1) / np;
-            const int at = min(s + p * sz, e);
-            runs[(size_t)(o + p) * jt.ns + m] = make_int4(t, at, min(sz, e - at), 0);
-        }
+    diag_accumulate(sp.diag, da.q, da.e, da.n, da.fallback);
 }
 
 // Photons with QED off move on straight lines (src/advance.cpp:173-183) and
@@ -737,13 +622,12 @@ hipError_t launch_push_global(hipStream_t st, const Grid &g, const Fields<real> 
 
 template <typename real>
 hipError_t launch_push_tiled(hipStream_t st, const Grid &g, const Fields<real> &f, const Current<real> &j,
-                             const TileGeom &tg, int ns, const Species<real> *s, const PushArgs *a, const int4 *runs,
-                             int nruns)
+                             const TileGeom &tg, int ns, const Species<real> *s, const PushArgs *a)
 {
     TiledArgs<real> args{};
     int total = 0;
     for (int m = 0; m < ns; ++m) {
-        if (a[m].nchunks <= 0 && !runs) continue;
+        if (a[m].nchunks <= 0) continue;
         TiledSpecies<real> &t = args.sp[args.ns++];
         t.s = s[m];
         t.sc = step_const<real>(g, a[m]);
@@ -753,29 +637,9 @@ hipError_t launch_push_tiled(hipStream_t st, const Grid &g, const Fields<real> &
         t.ishift = a[m].ishift;
         total += a[m].nchunks;
     }
-    args.runs = runs;
-    if (runs) total = nruns;
     if (total == 0) return hipSuccess;
-#define QK_PUSH(P, M) k_push_tiled<real, P, M><<<total, kTBlock, 0, st>>>(g, f, j, tg, args)
-    if (a[0].pusher == 1) { if (runs) QK_PUSH(1, true); else QK_PUSH(1, false); }
-    else { if (runs) QK_PUSH(0, true); else QK_PUSH(0, false); }
-#undef QK_PUSH
-    return hipGetLastError();
-}
-
-hipError_t launch_joint_runs(hipStream_t st, int ns, const int *const *start, int ntiles, int chunk, int *parts,
-                             int *off, int *scratch, int4 *runs, int max_items, int *n)
-{
-    JointTiles jt{};
-    for (int m = 0; m < ns; ++m) jt.start[m] = start[m];
-    jt.ns = ns;
-    jt.ntiles = ntiles;
-    jt.chunk = chunk;
-    k_joint_parts<<<blocks_for(ntiles + 1), kBlock, 0, st>>>(jt, parts);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    if ((e = launch_exclusive_scan(st, parts, off, ntiles, scratch)) != hipSuccess) return e;
-    k_joint_runs<<<blocks_for(ntiles), kBlock, 0, st>>>(jt, off, runs, max_items, n);
+    if (a[0].pusher == 1) k_push_tiled<real, 1><<<total, kTBlock, 0, st>>>(g, f, j, tg, args);
+    else k_push_tiled<real, 0><<<total, kTBlock, 0, st>>>(g, f, j, tg, args);
     return hipGetLastError();
 }
 
@@ -827,7 +691,7 @@ hipError_t launch_scale_charge(hipStream_t st, const Species<real> &s, int64_t n
                                                  const Current<real> &, const Species<real> &, const PushArgs &); \
     template hipError_t launch_push_tiled<real>(hipStream_t, const Grid &, const Fields<real> &,                \
                                                 const Current<real> &, const TileGeom &, int,                   \
-                                                const Species<real> *, const PushArgs *, const int4 *, int);    \
+                                                const Species<real> *, const PushArgs *);                       \
     template hipError_t launch_load_uniform<real>(hipStream_t, const Grid &, const Species<real> &, int64_t, int, \
                                                   double, double, uint64_t, int, int);                           \
     template hipError_t launch_compute_rho<real>(hipStream_t, const Grid &, const Species<real> &, int64_t,       \
