@@ -124,29 +124,50 @@ __device__ inline void load_corners_stage(const EB<real> *st, int ri, int rj, in
         }
 }
 
-// Component C of one field into its stage block, in two passes over a
-// thread's share of the block: the loads (load_component), then the LDS
-// writes (store_component).  Nodes outside the grid (never read by a
-// particle) are set to zero.  With the loads of all six blocks issued before
-// the first write, a thread waits for memory once while staging, not once
-// per block and share (the push measured 5 % faster at 256x128x128).
+// w / D for 0 <= w < kMost (entries of a window or stage block) with a 24-bit
+// multiplication: the general division's high multiplication takes four
+// times as long
+template <int D, int kMost>
+__device__ inline int small_div(int w)
+{
+    constexpr int M = (65536 + D - 1) / D;
+    static_assert((int64_t)kMost * (M * D - 65536) < 65536 && (int64_t)kMost * M < (1ll << 32), "w * M >> 16 is w / D");
+    return (int)(__umul24((unsigned)w, (unsigned)M) >> 16);
+}
+
+// node idx of an array (at most 2^30 nodes: cells are packed in 30 bits); in
+// FP32 its byte offset fits 32 bits, added to the base by the memory operation
+__device__ inline float &node_at(float *base, int idx) { return at32(base, (uint32_t)idx * 4u); }
+__device__ inline const float &node_at(const float *base, int idx) { return at32(base, (uint32_t)idx * 4u); }
+__device__ inline double &node_at(double *base, int idx) { return base[idx]; }
+__device__ inline const double &node_at(const double *base, int idx) { return base[idx]; }
+
+// Component C of E and of Be into the stage, in two passes over a thread's
+// share of the block: the loads (load_component), then the LDS writes
+// (store_component).  Indices are clamped into the grid (no particle reads the
+// nodes outside it), so that no load waits for a branch.  With the loads of
+// all three components issued before the first write, a thread waits for
+// memory once while staging, not once per block and share (the push measured
+// 5 % faster at 256x128x128).  With the branches and the general divisions
+// the push took 22.5 us at 64x32x32 and 98.6 us at 128x64x64, now 21.4 and 97.
 constexpr int kStageIt = (fsize(0) + kTBlock - 1) / kTBlock;   // every block has fsize(0) nodes
 
 template <int C, typename real>
-__device__ inline void load_component(real (&v)[kStageIt], const real *__restrict__ src, const Grid &g, int gi0,
-                                      int gj0, int gk0)
+__device__ inline void load_component(real (&e)[kStageIt], real (&b)[kStageIt], const real *__restrict__ E,
+                                      const real *__restrict__ B, const Grid &g, int gi0, int gj0, int gk0)
 {
     static_assert(fsize(C) == fsize(0), "stage blocks of equal size");
     constexpr int d1 = fdim(C, 1), d2 = fdim(C, 2);
 #pragma unroll
     for (int m = 0; m < kStageIt; ++m) {
-        const int w = threadIdx.x + m * kTBlock;
-        const int lk = w % d2, t = w / d2;
-        const int lj = t % d1, li = t / d1;
-        const int gi = gi0 + li, gj = gj0 + lj, gk = gk0 + lk;
-        const bool in = w < fsize(C) && (unsigned)gi < (unsigned)g.nx && (unsigned)gj < (unsigned)g.ny &&
-                        (unsigned)gk < (unsigned)g.nz;
-        v[m] = in ? src[gi * g.sx + gj * g.sy + gk] : real(0);
+        const int w = min((int)threadIdx.x + m * kTBlock, fsize(C) - 1);
+        const int t = small_div<d2, fsize(C)>(w), li = small_div<d1, fsize(C)>(t);
+        const int lk = w - t * d2, lj = t - li * d1;
+        const int i = min(max(gi0 + li, 0), g.nx - 1), j = min(max(gj0 + lj, 0), g.ny - 1),
+                  k = min(max(gk0 + lk, 0), g.nz - 1);
+        const int idx = (int)(__umul24((unsigned)i, (unsigned)g.sx) + __umul24((unsigned)j, (unsigned)g.sy)) + k;
+        e[m] = node_at(E, idx);
+        b[m] = node_at(B, idx);
     }
 }
 
@@ -161,26 +182,27 @@ __device__ inline void store_component(EB<real> *dst, const real (&e)[kStageIt],
 }
 
 // add component C of the current window to the grid: one global atomic per
-// nonzero entry inside the grid.  v holds the thread's share of the window
-// block (entry threadIdx.x + m kTBlock), read from LDS for all three
-// components before the first atomic.
+// nonzero entry.  v holds the thread's share of the window block (entry
+// threadIdx.x + m kTBlock), read from LDS for all three components before the
+// first atomic; base is the window's first node.  A particle that deposits is
+// is_inside (1 .. n - 3) and crosses one face per axis at most, so the nodes it
+// reaches lie in the grid (0 .. n - 1) and entries outside it hold zero.
 constexpr int kFlushIt = (jsize(0) + kTBlock - 1) / kTBlock;
 
 template <int C, typename real>
-__device__ inline void flush_component(real *__restrict__ dst, const double (&v)[kFlushIt], const Grid &g, int gi0,
-                                       int gj0, int gk0)
+__device__ inline void flush_component(real *__restrict__ dst, const double (&v)[kFlushIt], const Grid &g, int base)
 {
     static_assert(jsize(C) <= kFlushIt * kTBlock, "window block larger than the thread shares");
-    constexpr int d1 = jdim(C, 1), d2 = jdim(C, 2);
+    constexpr int d1 = jdim(C, 1), d2 = jdim(C, 2), most = kFlushIt * kTBlock;
 #pragma unroll
     for (int m = 0; m < kFlushIt; ++m) {
         const int w = threadIdx.x + m * kTBlock;
-        const int wk = w % d2, t = w / d2;
-        const int wj = t % d1, wi = t / d1;
-        const int gi = gi0 + wi, gj = gj0 + wj, gk = gk0 + wk;
-        if (w < jsize(C) && v[m] != 0.0 && (unsigned)gi < (unsigned)g.nx && (unsigned)gj < (unsigned)g.ny &&
-            (unsigned)gk < (unsigned)g.nz)
-            unsafeAtomicAdd(dst + gi * g.sx + gj * g.sy + gk, (real)v[m]);
+        const int t = small_div<d2, most>(w), wi = small_div<d1, most>(t);
+        const int wk = w - t * d2, wj = t - wi * d1;
+        if (v[m] != 0.0) {   // zero past the block's end
+            const int idx = base + (int)(__umul24((unsigned)wi, (unsigned)g.sx) + __umul24((unsigned)wj, (unsigned)g.sy)) + wk;
+            unsafeAtomicAdd(&node_at(dst, idx), (real)v[m]);
+        }
     }
 }
 
@@ -241,7 +263,7 @@ template <typename real, int PUSHER>
 __global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<real> f, Current<real> cur, TileGeom tg,
                                                                 TiledArgs<real> args)
 {
-    __shared__ double win[kJWin];
+    __shared__ alignas(16) double win[kJWin];
     __shared__ EB<real> stage[kFStage];
     __shared__ uint32_t listed[kDefer];
     __shared__ int nlisted;
@@ -291,20 +313,22 @@ __global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<
     PRec<real> r1, r2;   // the records one and two rounds ahead
     if (n < count) load_rec32(s, slot_of(n), r1);
     if (n + kTBlock < count) load_rec32(s, slot_of(n + kTBlock), r2);
-    for (int w = threadIdx.x; w < kJWin; w += kTBlock) win[w] = 0.0;
+    static_assert(kJWin % 2 == 0, "cleared in pairs");
+#pragma unroll
+    for (int m = 0; m < (kJWin / 2 + kTBlock - 1) / kTBlock; ++m) {
+        const int w = threadIdx.x + m * kTBlock;
+        if (w < kJWin / 2) ((double2 *)win)[w] = make_double2(0.0, 0.0);
+    }
     if (threadIdx.x == 0) nlisted = 0;
     {
         const int si = i0 - kHalo, sj = j0 - kHalo, sk = k0 - kHalo;
-        real v[6][kStageIt];
-        load_component<0>(v[0], f.ex, g, si, sj, sk);
-        load_component<1>(v[1], f.ey, g, si, sj, sk);
-        load_component<2>(v[2], f.ez, g, si, sj, sk);
-        load_component<0>(v[3], f.bex, g, si, sj, sk);
-        load_component<1>(v[4], f.bey, g, si, sj, sk);
-        load_component<2>(v[5], f.bez, g, si, sj, sk);
-        store_component<0>(stage, v[0], v[3]);
-        store_component<1>(stage, v[1], v[4]);
-        store_component<2>(stage, v[2], v[5]);
+        real e[3][kStageIt], b[3][kStageIt];
+        load_component<0>(e[0], b[0], f.ex, f.bex, g, si, sj, sk);
+        load_component<1>(e[1], b[1], f.ey, f.bey, g, si, sj, sk);
+        load_component<2>(e[2], b[2], f.ez, f.bez, g, si, sj, sk);
+        store_component<0>(stage, e[0], b[0]);
+        store_component<1>(stage, e[1], b[1]);
+        store_component<2>(stage, e[2], b[2]);
     }
     __syncthreads();
 
@@ -424,7 +448,7 @@ __global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<
     }
 
     {
-        const int wi0 = i0 - kHalo - 1, wj0 = j0 - kHalo - 1, wk0 = k0 - kHalo - 1;
+        const int base = (i0 - kHalo - 1) * g.sx + (j0 - kHalo - 1) * g.sy + k0 - kHalo - 1;
         double v[3][kFlushIt];
 #pragma unroll
         for (int m = 0; m < kFlushIt; ++m) {
@@ -432,9 +456,9 @@ __global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<
 #pragma unroll
             for (int c = 0; c < 3; ++c) v[c][m] = w < jsize(c) ? win[joff(c) + w] : 0.0;
         }
-        flush_component<0>(cur.jx, v[0], g, wi0, wj0, wk0);
-        flush_component<1>(cur.jy, v[1], g, wi0, wj0, wk0);
-        flush_component<2>(cur.jz, v[2], g, wi0, wj0, wk0);
+        flush_component<0>(cur.jx, v[0], g, base);
+        flush_component<1>(cur.jy, v[1], g, base);
+        flush_component<2>(cur.jz, v[2], g, base);
     }
     diag_accumulate(sp.diag, da.q, da.e, da.n, da.fallback);
 }

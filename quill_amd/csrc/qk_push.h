@@ -192,6 +192,18 @@ __device__ inline void rebin(int &i, int &j, int &k, real pos[3])
     k += ci[2];
 }
 
+// whether an offset has left [0, 1) or is -0: as unsigned integers, the bits
+// of the numbers in [0, 1) lie below those of 1, all others at or above
+__device__ inline bool left_cell(const float pos[3])
+{
+    return max(max(__float_as_uint(pos[0]), __float_as_uint(pos[1])), __float_as_uint(pos[2])) >= 0x3f800000u;
+}
+__device__ inline bool left_cell(const double pos[3])
+{
+    return max(max((uint32_t)__double2hiint(pos[0]), (uint32_t)__double2hiint(pos[1])),
+               (uint32_t)__double2hiint(pos[2])) >= 0x3ff00000u;
+}
+
 // gamma - 1 as u^2 / (gamma + 1): no cancellation for slow particles
 template <typename real>
 __device__ inline double kinetic(const real u[3], real gam)
@@ -243,12 +255,18 @@ __device__ inline void advance_particle_eb(const Grid &g, const real (&ei)[3], c
         return;
     }
     dep(i, j, k, base, r.q, pos, d, da);
-    rebin(i, j, k, pos);
+    // a particle that stayed in its cell has nothing to re-bin: half of the
+    // wavefronts of a thermal plasma have no lane that moves on
+    bool alive = true;
+    if (left_cell(pos)) {
+        rebin(i, j, k, pos);
+        alive = is_inside(g, i, j, k);
+        r.cell = pack_cell(i, j, k);
+    }
     r.o[0] = pos[0];
     r.o[1] = pos[1];
     r.o[2] = pos[2];
-    if (is_inside(g, i, j, k)) {
-        r.cell = pack_cell(i, j, k);
+    if (alive) {
         const double ke = kinetic(u, gam);
         da.q += (double)r.q;
         da.n += 1;
