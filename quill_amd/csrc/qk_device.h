@@ -259,36 +259,50 @@ __device__ inline void deposit_segment(Acc &acc, real q, real px, real py, real 
 // set_cell(wi, wj, wk) (offsets of the piece's cell from the start cell)
 // before each piece.  On return p holds the end point, advanced piece by
 // piece as the reference advances the particle.
-template <typename real, class Acc>
-__device__ inline void deposit_path(Acc &acc, real q, real p[3], const real d[3])
+template <typename real>
+struct Crossings {
+    int to[3];    // the end cell relative to the start cell
+    int n;        // faces crossed
+    real t[3];    // path fractions of the crossings, ascending
+    int ax[3];    // and their axes
+};
+
+template <typename real>
+__device__ inline Crossings<real> find_crossings(const real p[3], const real d[3])
 {
-    int c2[3];
+    Crossings<real> c{{}, 0, {real(1), real(1), real(1)}, {0, 1, 2}};
 #pragma unroll
-    for (int m = 0; m < 3; ++m) c2[m] = (int)floor(p[m] + d[m]);
-    const int nc = (c2[0] != 0) + (c2[1] != 0) + (c2[2] != 0);
-    real t[3] = {real(1), real(1), real(1)};
-    int ax[3] = {0, 1, 2};
+    for (int m = 0; m < 3; ++m) c.to[m] = (int)floor(p[m] + d[m]);
+    c.n = (c.to[0] != 0) + (c.to[1] != 0) + (c.to[2] != 0);
     // a wavefront without a crossing lane skips the fractions
-    if (nc > 0) {
+    if (c.n > 0) {
 #pragma unroll
         for (int m = 0; m < 3; ++m)   // non-crossing axes sort after every crossing one
-            t[m] = c2[m] != 0 ? (real(c2[m] > 0 ? 1 : 0) - p[m]) * qk_rcp(d[m]) : real(2);
+            c.t[m] = c.to[m] != 0 ? (real(c.to[m] > 0 ? 1 : 0) - p[m]) * qk_rcp(d[m]) : real(2);
         auto cswap = [&](int a, int b) {
-            if (t[a] > t[b]) {
-                const real tt = t[a]; t[a] = t[b]; t[b] = tt;
-                const int ta = ax[a]; ax[a] = ax[b]; ax[b] = ta;
+            if (c.t[a] > c.t[b]) {
+                const real tt = c.t[a]; c.t[a] = c.t[b]; c.t[b] = tt;
+                const int ta = c.ax[a]; c.ax[a] = c.ax[b]; c.ax[b] = ta;
             }
         };
         cswap(0, 1);
         cswap(1, 2);
         cswap(0, 1);
     }
-    int w[3] = {0, 0, 0};
-    real done = real(0);
+    return c;
+}
+
+// pieces first .. last of the path; w and done: the first one's cell and the
+// fraction before it
+template <typename real, class Acc>
+__device__ inline void deposit_pieces(Acc &acc, real q, real p[3], const real d[3], const Crossings<real> &c, int first,
+                                      int last, int w[3], real &done)
+{
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
-        if (n > nc) break;
-        const real upto = n < nc ? t[n] : real(1);
+        if (n < first) continue;
+        if (n > last || n > c.n) break;
+        const real upto = n < c.n ? c.t[n] : real(1);
         const real fr = upto - done;
         done = upto;
         const real s0 = d[0] * fr, s1 = d[1] * fr, s2 = d[2] * fr;
@@ -300,8 +314,41 @@ __device__ inline void deposit_path(Acc &acc, real q, real p[3], const real d[3]
         if (n < 3) {
 #pragma unroll
             for (int m = 0; m < 3; ++m)
-                if (ax[n] == m) w[m] = c2[m];
+                if (c.ax[n] == m) w[m] = c.to[m];
         }
+    }
+}
+
+template <typename real, class Acc>
+__device__ inline void deposit_path(Acc &acc, real q, real p[3], const real d[3])
+{
+    const Crossings<real> c = find_crossings<real>(p, d);
+    int w[3] = {0, 0, 0};
+    real done = real(0);
+    deposit_pieces(acc, q, p, d, c, 0, 3, w, done);
+}
+
+// The same, but the second piece of a path with one crossing is left to the
+// caller: pend(q, p, s, w), p and s its start (relative to cell w) and
+// displacement.  before(crosses) runs in between for every lane.
+template <typename real, class Acc, class Before, class Pend>
+__device__ inline void deposit_path_pending(Acc &acc, real q, real p[3], const real d[3], Before &&before, Pend &&pend)
+{
+    const Crossings<real> c = find_crossings<real>(p, d);
+    int w[3] = {0, 0, 0};
+    real done = real(0);
+    deposit_pieces(acc, q, p, d, c, 0, 0, w, done);
+    before(c.n == 1);
+    if (c.n == 1) {
+        const real fr = real(1) - done;
+        const real s[3] = {d[0] * fr, d[1] * fr, d[2] * fr};
+        const real at[3] = {p[0] - real(w[0]), p[1] - real(w[1]), p[2] - real(w[2])};
+        pend(q, at, s, w);
+        p[0] += s[0];
+        p[1] += s[1];
+        p[2] += s[2];
+    } else if (c.n > 1) {
+        deposit_pieces(acc, q, p, d, c, 1, 3, w, done);
     }
 }
 

@@ -34,11 +34,6 @@ constexpr int kT[3] = {kTx, kTy, kTz};
 #ifndef QK_TBLOCK
 #define QK_TBLOCK 512
 #endif
-#ifdef QK_TWAVES_EU
-#define QK_TATTR __attribute__((amdgpu_waves_per_eu(QK_TWAVES_EU)))
-#else
-#define QK_TATTR
-#endif
 constexpr int kTBlock = QK_TBLOCK;
 // out-of-window particles listed per workgroup and pushed after its rounds:
 // at most this many per chunk, the rest inline
@@ -90,6 +85,29 @@ struct LdsAcc {
         atomicAdd(win + joff(comp) + cur[comp] + (di * d1 + dj) * d2 + dk, (double)v);
     }
 };
+
+// The second piece of a path that crossed one face, kept by its lane until
+// another one comes to the same lane or the rounds end; then every lane of
+// the wavefront deposits its own.  Some 1 % of the particles of a thermal
+// plasma cross per step, so that every other wavefront would run the second
+// piece for a lane or two in each round.  FP32 push 592 -> 578 us at 256x128x128
+// (NDFX, Vay), 4.91 -> 4.84 ms at 512x256x256; in FP64, where the registers do
+// not limit it but the second piece is a smaller share, 150 -> 152 us at
+// 97x61x53, so there it is deposited at once.
+template <typename real>
+struct Pending {
+    real q, p[3], s[3];
+    int cell = -1;   // window index of its cell, a byte per axis; negative: none
+};
+
+template <typename real>
+__device__ inline void deposit_pending(double *win, Pending<real> &pd)
+{
+    LdsAcc<real> acc(win, (pd.cell >> 16) - kHalo - 1, (pd.cell >> 8 & 255) - kHalo - 1, (pd.cell & 255) - kHalo - 1);
+    acc.set_cell(0, 0, 0);
+    deposit_segment<real>(acc, pd.q, pd.p[0], pd.p[1], pd.p[2], pd.s[0], pd.s[1], pd.s[2]);
+    pd.cell = -1;
+}
 
 // E and Be of one node and component side by side in the field stage: one
 // 8-byte LDS read takes 5.6 clocks per wavefront and CU at random cells, two
@@ -260,7 +278,7 @@ struct TiledArgs {
 };
 
 template <typename real, int PUSHER>
-__global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<real> f, Current<real> cur, TileGeom tg,
+__global__ void __launch_bounds__(kTBlock) k_push_tiled(Grid g, Fields<real> f, Current<real> cur, TileGeom tg,
                                                                 TiledArgs<real> args)
 {
     __shared__ alignas(16) double win[kJWin];
@@ -333,6 +351,7 @@ __global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<
     __syncthreads();
 
     DiagAcc da;
+    Pending<real> pd;
     // start cell relative to the tile, and whether it lies in the window
     int ri = 0, rj = 0, rk = 0;
     bool in_win = false;
@@ -341,7 +360,22 @@ __global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<
         // (path split once, two masked atomics per term) measured 2.5 % slower
         if (in_win) {
             LdsAcc<real> acc(win, ri, rj, rk);
-            deposit_path<real>(acc, q, pos, d);
+            if (sizeof(real) == 8) {
+                deposit_path<real>(acc, q, pos, d);
+                return;
+            }
+            auto before = [&](bool crosses) {
+                if (__any(crosses && pd.cell >= 0) && pd.cell >= 0) deposit_pending(win, pd);
+            };
+            auto pend = [&](real pq, const real pp[3], const real ps[3], const int w[3]) {
+                pd.q = pq;
+                for (int m = 0; m < 3; ++m) {
+                    pd.p[m] = pp[m];
+                    pd.s[m] = ps[m];
+                }
+                pd.cell = (ri + w[0] + kHalo + 1) << 16 | (rj + w[1] + kHalo + 1) << 8 | (rk + w[2] + kHalo + 1);
+            };
+            deposit_path_pending<real>(acc, q, pos, d, before, pend);
         } else {
             GlobalAcc<real> acc{cur.jx, cur.jy, cur.jz, g.sx, g.sy, base, base};
             deposit_path<real>(acc, q, pos, d);
@@ -425,6 +459,7 @@ __global__ void __launch_bounds__(kTBlock) QK_TATTR k_push_tiled(Grid g, Fields<
         ps = slot_of(n);
     }
     if (started) store_rec32(s, ps, rs);
+    if (sizeof(real) == 4 && pd.cell >= 0) deposit_pending(win, pd);
     // the listed slots' rewrites complete before the pass below stores them
     // again (vmcnt 0; expcnt and lgkmcnt left at their maxima)
     __builtin_amdgcn_s_waitcnt(0x0F70);
