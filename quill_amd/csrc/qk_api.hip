@@ -165,7 +165,10 @@ struct qk_ctx {
     // QED: device slot counters of every species plus an overflow flag, and
     // their pinned host mirror; the global step index keys the random streams
     int *d_count = nullptr;
-    int *h_count = nullptr;
+    int *h_count = nullptr;         // pinned: values on their way to d_count
+    int dev_n[QK_MAX_SPECIES];      // what d_count holds as far as the host knows (-1: unknown)
+    QedCounts *h_qed = nullptr;     // pinned: [0] after the pairs from vacuum, [1] at the step's end
+    unsigned qed_seq = 0, qed_end = 0;   // last one launched; the step's end
     uint32_t step_index = 0;
     // merging: device accumulators, their pinned mirror, and the deletion
     // fractions of a merge due at the start of the next step
@@ -484,15 +487,15 @@ int merge_impl(qk_ctx *c, int mode, const double *ppd)
     return QK_OK;
 }
 
-// evaluate_merging_condition (src/main.cpp:1691-1748) on the counts of the
-// step just finished (h: that step's accumulators)
-void merge_condition(qk_ctx *c, const double *h)
+// evaluate_merging_condition (src/main.cpp:1691-1748) on the live
+// counts after the step just finished
+void merge_condition(qk_ctx *c, const double (&live)[QK_MAX_SPECIES])
 {
     const double crnp = c->p.crnp;
     const int nsp = QK_ION0 + c->p.n_ion;
     double cnt[QK_MAX_SPECIES] = {}, total = 0;
     for (int s = 0; s < nsp; ++s) {
-        cnt[s] = h[s * kDiagPerSpecies + 2];
+        cnt[s] = live[s];
         total += cnt[s];
     }
     c->merge_due = false;
@@ -511,33 +514,59 @@ void merge_condition(qk_ctx *c, const double *h)
     }
 }
 
-// QED slot counters: host -> device before kernels that append, device ->
-// host (with a stream sync) after them
+// QED slot counters to the device where the host has changed them since
 int qed_upload_counts(qk_ctx *c)
 {
-    for (int s = 0; s < QK_MAX_SPECIES; ++s) c->h_count[s] = (int)c->sp[s].n;
+    bool same = true;
+    for (int s = 0; s < QK_MAX_SPECIES; ++s) same = same && c->dev_n[s] == (int)c->sp[s].n;
+    if (same) return QK_OK;
+    for (int s = 0; s < QK_MAX_SPECIES; ++s) c->dev_n[s] = c->h_count[s] = (int)c->sp[s].n;
     c->h_count[QK_MAX_SPECIES] = 0;
     HIP_TRY(hipMemcpyAsync(c->d_count, c->h_count, (QK_MAX_SPECIES + 1) * sizeof(int), hipMemcpyHostToDevice,
                            c->stream));
     return QK_OK;
 }
 
-int qed_download_counts(qk_ctx *c)
+// The counters (and, with diag, the live counts) to h_qed[which], and the wait
+// for them.  The GPU stores them and the host polls: the host has the counts
+// while the GPU works on what was enqueued behind them, where a copy and a
+// stream synchronization emptied the queue twice per step.
+int qed_publish(qk_ctx *c, int which, const double *diag)
 {
-    HIP_TRY(hipMemcpyAsync(c->h_count, c->d_count, (QK_MAX_SPECIES + 1) * sizeof(int), hipMemcpyDeviceToHost,
-                           c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    if (c->h_count[QK_MAX_SPECIES]) return fail(QK_ERR_CAPACITY, "QED appends exceeded the reserved capacity");
-    for (int s = 0; s < QK_MAX_SPECIES; ++s)
-        if (c->sp[s].active) c->sp[s].n = c->h_count[s];
+    HIP_TRY(launch_publish_counts(c->stream, c->d_count, QK_MAX_SPECIES + 1, diag, QK_MAX_SPECIES, c->h_qed + which,
+                                  ++c->qed_seq));
     return QK_OK;
+}
+
+int qed_wait(qk_ctx *c, int which, unsigned seq)
+{
+    const QedCounts &h = c->h_qed[which];
+    HIP_TRY(wait_flag(c->stream, &h.flag, seq));
+    if (h.n[QK_MAX_SPECIES]) {
+        c->dev_n[0] = -1;   // the next upload clears the overflow flag
+        return fail(QK_ERR_CAPACITY, "QED appends exceeded the reserved capacity");
+    }
+    for (int s = 0; s < QK_MAX_SPECIES; ++s)
+        if (c->sp[s].active) c->dev_n[s] = (int)(c->sp[s].n = h.n[s]);
+    return QK_OK;
+}
+
+// whether species s can take `extra` more slots (see ensure_species)
+bool fits(const qk_ctx *c, int s, int64_t extra)
+{
+    const int64_t need = c->sp[s].n + extra;
+    if (need <= c->sp[s].cap) return true;
+    return c->p.capacity > 0 ? need <= c->p.capacity : need < ((int64_t)1 << 32) / (int64_t)c->rsize;
 }
 
 // The particle phase with QED on (src/main.cpp:2323-2324): birth_from_vacuum,
 // then padvance with photon emission for leptons and pair creation for
-// photons.  Capacity is reserved for the worst case (every lepton emits,
-// every photon converts) so that no append can fail; the new counts are
-// read back after the step.
+// photons.  Capacity is reserved for the worst case (every cell bears a pair,
+// every lepton emits, every photon converts) so that no append can fail.  The
+// particles that were there are pushed while the host waits for the number of
+// pairs born from vacuum, which follow in a launch of their own (mostly none
+// are); where there is no room for both worst cases at once, the host waits
+// first and reserves for what was born.
 template <typename real>
 int qed_particle_phase(qk_ctx *c, const Fields<real> &f, const Current<real> &jc)
 {
@@ -553,23 +582,8 @@ int qed_particle_phase(qk_ctx *c, const Fields<real> &f, const Current<real> &jc
         t.diag = c->diag_row + s * kDiagPerSpecies;
         return t;
     };
-    const int64_t ninner = std::max<int64_t>(0, (int64_t)(c->p.nx - 4) * (c->p.ny - 4) * (c->p.nz - 4));
-    if (ninner > 0) {
-        QK_TRY(ensure_species(c, QK_ELECTRON, ninner));
-        QK_TRY(ensure_species(c, QK_POSITRON, ninner));
-        QK_TRY(qed_upload_counts(c));
-        HIP_TRY(launch_vacuum_pairs<real>(c->stream, c->g, f, c->p.pusher, c->p.q_vac, qa, target(QK_ELECTRON),
-                                          target(QK_POSITRON)));
-        QK_TRY(qed_download_counts(c));
-    }
-    QK_TRY(ensure_species(c, QK_PHOTON, be.n + bp.n));
-    QK_TRY(ensure_species(c, QK_ELECTRON, bph.n));
-    QK_TRY(ensure_species(c, QK_POSITRON, bph.n));
-    QK_TRY(qed_upload_counts(c));
-    const int64_t n_ph0 = bph.n;   // photons emitted in this step are not visited
-    for (int s = 0; s < QK_MAX_SPECIES; ++s) {
-        SpeciesBuf &b = c->sp[s];
-        if (!b.active || b.n == 0 || s == QK_PHOTON) continue;
+    auto push_args = [&](int s, int64_t first, int64_t n) {
+        const SpeciesBuf &b = c->sp[s];
         PushArgs a{};
         a.pusher = c->p.pusher;
         a.kind = b.kind;
@@ -578,30 +592,65 @@ int qed_particle_phase(qk_ctx *c, const Fields<real> &f, const Current<real> &jc
         a.diag = c->diag_row + s * kDiagPerSpecies;
         a.energy_mode = b.energy_mode;
         a.nonfinite = c->diag_row + kRowNonfinite;
-        a.first = 0;
-        a.n = b.n;
-        const Species<real> v = view<real>(b.buf[b.cur]);
-        if (s == QK_ELECTRON || s == QK_POSITRON)
-            HIP_TRY(launch_push_qed_lepton<real>(c->stream, c->g, f, jc, v, a, qa, target(QK_PHOTON)));
-        else
-            HIP_TRY(launch_push_global<real>(c->stream, c->g, f, jc, v, a));
+        a.first = first;
+        a.n = n;
+        return a;
+    };
+    // electrons, positrons and photons from their slot `first` on
+    auto push = [&](const int64_t (&first)[3], const int64_t (&n)[3]) -> int {
+        const int sp[3] = {QK_ELECTRON, QK_POSITRON, QK_PHOTON};
+        Species<real> s[3];
+        PushArgs a[3];
+        for (int m = 0; m < 3; ++m) {
+            s[m] = view<real>(c->sp[sp[m]].buf[c->sp[sp[m]].cur]);
+            a[m] = push_args(sp[m], first[m], n[m]);
+        }
+        HIP_TRY(launch_qed_particles<real>(c->stream, c->g, f, jc, s, a, qa, target(QK_ELECTRON), target(QK_POSITRON),
+                                           target(QK_PHOTON)));
+        return QK_OK;
+    };
+    const int64_t ninner = std::max<int64_t>(0, (int64_t)(c->p.nx - 4) * (c->p.ny - 4) * (c->p.nz - 4));
+    const int64_t ne = be.n, np = bp.n, nph = bph.n;   // photons emitted in this step are not visited
+    const bool ahead = ninner > 0 && fits(c, QK_ELECTRON, ninner + nph) && fits(c, QK_POSITRON, ninner + nph) &&
+                       fits(c, QK_PHOTON, ne + np) && ensure_species(c, QK_ELECTRON, ninner + nph) == QK_OK &&
+                       ensure_species(c, QK_POSITRON, ninner + nph) == QK_OK &&
+                       ensure_species(c, QK_PHOTON, ne + np) == QK_OK;
+    if (!ahead) (void)hipGetLastError();
+    if (ninner > 0) {
+        QK_TRY(ensure_species(c, QK_ELECTRON, ninner));
+        QK_TRY(ensure_species(c, QK_POSITRON, ninner));
+        QK_TRY(qed_upload_counts(c));
+        HIP_TRY(launch_vacuum_pairs<real>(c->stream, c->g, f, c->p.pusher, c->p.q_vac, qa, target(QK_ELECTRON),
+                                          target(QK_POSITRON)));
+        QK_TRY(qed_publish(c, 0, nullptr));
+        const unsigned seq = c->qed_seq;
+        if (ahead) QK_TRY(push({0, 0, 0}, {ne, np, nph}));
+        QK_TRY(qed_wait(c, 0, seq));
+    }
+    const int64_t born_e = be.n - ne, born_p = bp.n - np;
+    if (!ahead) {
+        QK_TRY(ensure_species(c, QK_PHOTON, be.n + bp.n));
+        QK_TRY(ensure_species(c, QK_ELECTRON, nph));
+        QK_TRY(ensure_species(c, QK_POSITRON, nph));
+        QK_TRY(qed_upload_counts(c));
+        QK_TRY(push({0, 0, 0}, {be.n, bp.n, nph}));
+    } else if (born_e > 0 || born_p > 0) {
+        // the buffers may move: the counts after the launch above come first
+        QK_TRY(qed_publish(c, 0, nullptr));
+        QK_TRY(qed_wait(c, 0, c->qed_seq));
+        QK_TRY(ensure_species(c, QK_PHOTON, born_e + born_p));
+        QK_TRY(push({ne, np, 0}, {born_e, born_p, 0}));
+    }
+    for (int s = 0; s < QK_MAX_SPECIES; ++s) {
+        SpeciesBuf &b = c->sp[s];
+        const int64_t n = s == QK_ELECTRON ? ne + born_e : (s == QK_POSITRON ? np + born_p : (s == QK_PHOTON ? nph : b.n));
+        if (!b.active || n == 0) continue;
+        if (s >= QK_ION0)
+            HIP_TRY(launch_push_global<real>(c->stream, c->g, f, jc, view<real>(b.buf[b.cur]), push_args(s, 0, n)));
         ++b.steps_since_sort;
     }
-    if (n_ph0 > 0) {
-        PushArgs a{};
-        a.pusher = c->p.pusher;
-        a.kind = 1;
-        a.cmr = 0;
-        a.external_bz = c->p.external_bz;
-        a.diag = c->diag_row + QK_PHOTON * kDiagPerSpecies;
-        a.energy_mode = 1;
-        a.nonfinite = c->diag_row + kRowNonfinite;
-        a.first = 0;
-        a.n = n_ph0;
-        HIP_TRY(launch_photon_qed<real>(c->stream, c->g, f, jc, view<real>(bph.buf[bph.cur]), a, qa,
-                                        target(QK_ELECTRON), target(QK_POSITRON)));
-        ++bph.steps_since_sort;
-    }
+    QK_TRY(qed_publish(c, 1, c->diag_row));
+    c->qed_end = c->qed_seq;
     return QK_OK;
 }
 
@@ -1100,10 +1149,13 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
         }
         HIP_TRY(hipEventRecord(c->ev[3 * l + 2], c->stream));
         c->jcur ^= 1;
-        if (qed) QK_TRY(qed_download_counts(c));
+        if (qed) QK_TRY(qed_wait(c, 1, c->qed_end));
         if (c->p.merging) {
-            HIP_TRY(hipStreamSynchronize(c->stream));
-            merge_condition(c, hd + (size_t)l * kDiagLen);
+            double live[QK_MAX_SPECIES];
+            if (!qed) HIP_TRY(hipStreamSynchronize(c->stream));
+            for (int s = 0; s < QK_MAX_SPECIES; ++s)
+                live[s] = qed ? c->h_qed[1].live[s] : hd[(size_t)l * kDiagLen + s * kDiagPerSpecies + 2];
+            merge_condition(c, live);
         }
         ++c->step_index;
     }
@@ -1402,8 +1454,11 @@ int qk_create(const qk_params *params, qk_ctx **out)
         return bail(fail(QK_ERR_HIP, hipGetErrorString(e)));
     if (p.qed) {
         if ((e = hipMalloc(&c->d_count, (QK_MAX_SPECIES + 1) * sizeof(int))) != hipSuccess ||
-            (e = hipHostMalloc((void **)&c->h_count, (QK_MAX_SPECIES + 1) * sizeof(int))) != hipSuccess)
+            (e = hipHostMalloc((void **)&c->h_count, (QK_MAX_SPECIES + 1) * sizeof(int))) != hipSuccess ||
+            (e = hipHostMalloc((void **)&c->h_qed, 2 * sizeof(QedCounts))) != hipSuccess)
             return bail(fail(QK_ERR_HIP, hipGetErrorString(e)));
+        c->h_qed[0].flag = c->h_qed[1].flag = 0;
+        std::fill(c->dev_n, c->dev_n + QK_MAX_SPECIES, -1);
         // the species that QED appends to exist from the start
         for (int s : {QK_ELECTRON, QK_POSITRON, QK_PHOTON})
             if (int rc = ensure_species(c, s, 0)) return bail(rc);
@@ -1438,6 +1493,7 @@ int qk_destroy(qk_ctx *c)
     if (c->h_diag) note(hipHostFree(c->h_diag));
     if (c->d_count) note(hipFree(c->d_count));
     if (c->h_count) note(hipHostFree(c->h_count));
+    if (c->h_qed) note(hipHostFree(c->h_qed));
     if (c->d_merge) note(hipFree(c->d_merge));
     if (c->h_merge) note(hipHostFree(c->h_merge));
     for (void *m : c->tape.ckpt) note(hipFree(m));

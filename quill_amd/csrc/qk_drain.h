@@ -46,6 +46,25 @@ private:
     int before_ = -1;
 };
 
+// Until a kernel on st has stored `want` to the pinned flag f.  Should the
+// stream end without it, the launch failed.
+inline hipError_t wait_flag(hipStream_t st, const unsigned *flag, unsigned want)
+{
+    const std::atomic<unsigned> *f = (const std::atomic<unsigned> *)flag;
+    for (unsigned spins = 1; f->load(std::memory_order_acquire) != want; ++spins) {
+        if (spins % 65536 == 0) {
+            const hipError_t e = hipStreamQuery(st);
+            if (e == hipErrorNotReady) continue;
+            if (e != hipSuccess) return e;
+            return f->load(std::memory_order_acquire) == want ? hipSuccess : hipErrorLaunchFailure;
+        }
+#if defined(__x86_64__)
+        __builtin_ia32_pause();
+#endif
+    }
+    return hipSuccess;
+}
+
 class Drain {
 public:
     // Bytes per slot and most workers: 8 workers write fresh huge pages at
@@ -139,25 +158,8 @@ private:
     static constexpr size_t kFlagLine = 128, kFlagBytes = kFlagLine * 2 * kWorkers;
     unsigned *flag(int s) const { return (unsigned *)(pin_ + kFlagLine * s); }
 
-    // until slot s holds its block.  The flag comes with the launch; should
-    // the stream end without it, the launch failed.
-    hipError_t wait(hipStream_t st, int s)
-    {
-        const std::atomic<unsigned> *f = (const std::atomic<unsigned> *)flag(s);
-        const unsigned want = seq_[s];
-        for (unsigned spins = 1; f->load(std::memory_order_acquire) != want; ++spins) {
-            if (spins % 65536 == 0) {
-                const hipError_t e = hipStreamQuery(st);
-                if (e == hipErrorNotReady) continue;
-                if (e != hipSuccess) return e;
-                return f->load(std::memory_order_acquire) == want ? hipSuccess : hipErrorLaunchFailure;
-            }
-#if defined(__x86_64__)
-            __builtin_ia32_pause();
-#endif
-        }
-        return hipSuccess;
-    }
+    // until slot s holds its block
+    hipError_t wait(hipStream_t st, int s) { return wait_flag(st, flag(s), seq_[s]); }
 
     // helpers sleep between reads and live as long as the context
     void open_job(int nw, std::function<void(int)> work)

@@ -86,18 +86,27 @@ struct AppendTarget {
     double *diag;        // kDiagPerSpecies accumulators of the target species (first copy)
 };
 
-// electrons / positrons with photon emission (src/advance.cpp:253-359);
-// every current contribution a global atomic; emitted photons go to ph
+// electrons and positrons with photon emission (src/advance.cpp:253-359) and
+// photons with Breit-Wheeler pair creation (src/advance.cpp:155-252), slots
+// [first, first + n) of each, in one launch; every current contribution a
+// global atomic; emitted photons go to ph, pairs to el / po
 template <typename real>
-hipError_t launch_push_qed_lepton(hipStream_t st, const Grid &g, const Fields<real> &f, const Current<real> &j,
-                                  const Species<real> &s, const PushArgs &a, const QedArgs &q,
-                                  const AppendTarget<real> &ph);
-// photons with Breit-Wheeler pair creation (src/advance.cpp:155-252); the
-// pairs go to el / po
-template <typename real>
-hipError_t launch_photon_qed(hipStream_t st, const Grid &g, const Fields<real> &f, const Current<real> &j,
-                             const Species<real> &s, const PushArgs &a, const QedArgs &q,
-                             const AppendTarget<real> &el, const AppendTarget<real> &po);
+hipError_t launch_qed_particles(hipStream_t st, const Grid &g, const Fields<real> &f, const Current<real> &j,
+                                const Species<real> (&s)[3], const PushArgs (&a)[3], const QedArgs &q,
+                                const AppendTarget<real> &el, const AppendTarget<real> &po,
+                                const AppendTarget<real> &ph);
+// slot counters and live counts in pinned host memory, valid once flag holds
+// the sequence number of their launch
+struct QedCounts {
+    static constexpr int kMost = 8;
+    int n[kMost];
+    double live[kMost];
+    unsigned flag;
+};
+// the n slot counters and, with diag (a step's accumulators), the live counts
+// of nsp species to *out
+hipError_t launch_publish_counts(hipStream_t st, const int *count, int n, const double *diag, int nsp, QedCounts *out,
+                                 unsigned seq);
 // birth_from_vacuum (src/mc.cpp:142-196): one draw per cell 2 .. n-3
 template <typename real>
 hipError_t launch_vacuum_pairs(hipStream_t st, const Grid &g, const Fields<real> &f, int pusher, double q_vac,

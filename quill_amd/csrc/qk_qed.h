@@ -76,6 +76,10 @@ __device__ inline double qed_vacuum_rate(double e_s, const double e[3], const do
     const double pi = 3.14159265358979323846;
     const double f = 0.5 * (e[0] * e[0] + e[1] * e[1] + e[2] * e[2] - b[0] * b[0] - b[1] * b[1] - b[2] * b[2]);
     const double gg = e[0] * b[0] + e[1] * b[1] + e[2] * b[2];
+    // xi^2 <= 2 |f| + |gg|: below this the exponential is zero in FP64, as it is
+    // in nearly every cell of a laser's focus
+    const double low = pi / 746 * e_s;
+    if (2 * fabs(f) + fabs(gg) < low * low) return 0;
     const double a = sqrt(f * f + gg * gg);
     const double xi = sqrt(a + f), th = sqrt(fmax(a - f, 0.0));
     if (xi == 0) return 0;

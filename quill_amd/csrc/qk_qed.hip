@@ -1,10 +1,10 @@
 // qk_qed.hip -- the particle phase with QED on (src/advance.cpp:90-387 with
 // qed_enabled) and birth_from_vacuum (src/mc.cpp:142-196) on gfx950.
 //
-//   k_push_qed_lepton  electrons / positrons: push, chi at n+1/2, photon
+//   qed_lepton         electrons / positrons: push, chi at n+1/2, photon
 //                      emission with recoil (rewind half a step, re-gather,
 //                      re-push), deposit, re-bin
-//   k_photon_qed       photons: chi, Breit-Wheeler pair creation (both
+//   qed_photon         photons: chi, Breit-Wheeler pair creation (both
 //                      leptons pushed and deposited), straight flight
 //   k_vacuum_pairs     Schwinger pairs, one draw per cell
 //
@@ -16,6 +16,8 @@
 // Philox streams keyed by (seed, step, slot, stream tag): statistics match
 // the reference, individual events do not (get_rand is a sequential
 // lagged-Fibonacci generator).
+#include <algorithm>
+
 #include "qk_push.h"
 #include "qk_qed.h"
 
@@ -95,14 +97,12 @@ __device__ inline bool deposit_move(const Grid &g, const Current<real> &cur, int
 }
 
 template <typename real, int PUSHER>
-__global__ void __launch_bounds__(kBlock) k_push_qed_lepton(Grid g, Fields<real> f, Current<real> cur,
-                                                            Species<real> s, int64_t first, int64_t n,
-                                                            StepConst<real> sc, real e_s, QedArgs qa, uint32_t tag,
-                                                            AppendTarget<real> ph, double *diag)
+__device__ inline void qed_lepton(const Grid &g, const Fields<real> &f, const Current<real> &cur,
+                                  const Species<real> &s, int64_t p, int64_t end, const StepConst<real> &sc, real e_s,
+                                  const QedArgs &qa, uint32_t tag, const AppendTarget<real> &ph, double *diag)
 {
-    const int64_t p = first + (int64_t)blockIdx.x * kBlock + threadIdx.x;
     DiagAcc da, dph;
-    int cell = p < first + n ? s.cell[p] : -1;
+    int cell = p < end ? s.cell[p] : -1;
     if (cell >= 0 && !is_inside(g, cell_i(cell), cell_j(cell), cell_k(cell))) {
         s.cell[p] = -1;   // p_boundary (src/plist.cpp:73-102)
         cell = -1;
@@ -215,14 +215,13 @@ __device__ inline void pair_lepton(const Grid &g, const Current<real> &cur, cons
 }
 
 template <typename real, int PUSHER>
-__global__ void __launch_bounds__(kBlock) k_photon_qed(Grid g, Fields<real> f, Current<real> cur, Species<real> s,
-                                                       int64_t first, int64_t n, StepConst<real> sc, real e_s,
-                                                       QedArgs qa, AppendTarget<real> el, AppendTarget<real> po,
-                                                       double *diag)
+__device__ inline void qed_photon(const Grid &g, const Fields<real> &f, const Current<real> &cur,
+                                  const Species<real> &s, int64_t p, int64_t end, const StepConst<real> &sc, real e_s,
+                                  const QedArgs &qa, const AppendTarget<real> &el, const AppendTarget<real> &po,
+                                  double *diag)
 {
-    const int64_t p = first + (int64_t)blockIdx.x * kBlock + threadIdx.x;
     DiagAcc da, de, dp;
-    int cell = p < first + n ? s.cell[p] : -1;
+    int cell = p < end ? s.cell[p] : -1;
     if (cell >= 0 && !is_inside(g, cell_i(cell), cell_j(cell), cell_k(cell))) {
         s.cell[p] = -1;   // p_boundary (src/plist.cpp:73-102)
         cell = -1;
@@ -275,6 +274,56 @@ __global__ void __launch_bounds__(kBlock) k_photon_qed(Grid g, Fields<real> f, C
     diag_accumulate(po.diag, dp.q, dp.e, dp.n, 0.0);
 }
 
+// Electrons, positrons and photons in one launch, a range of workgroups each:
+// none of them visits what another appends in the same step, and each alone
+// leaves most of the chip idle (21, 21 and 19 us in turn at some 1e4 of each:
+// one wavefront's chain of gathers, spectra and global atomics).  With the
+// counts published instead of copied (qed_publish) and the
+// cells of zero vacuum rate left early, a cascade on 128^3 cells takes 46.4 ms for 200 steps, before 59.3.
+template <typename real>
+struct QedParts {
+    Species<real> s[3];
+    StepConst<real> sc[3];
+    int64_t first[3], end[3];
+    int blocks[3];
+    double *diag[3];
+};
+
+template <typename real, int PUSHER>
+__global__ void __launch_bounds__(kBlock) k_qed_particles(Grid g, Fields<real> f, Current<real> cur,
+                                                          QedParts<real> a, real e_s, QedArgs qa,
+                                                          AppendTarget<real> el, AppendTarget<real> po,
+                                                          AppendTarget<real> ph)
+{
+    int b = blockIdx.x;
+    for (int m = 0; m < 2; ++m) {   // uniform over the workgroup
+        if (b < a.blocks[m]) {
+            qed_lepton<real, PUSHER>(g, f, cur, a.s[m], a.first[m] + (int64_t)b * kBlock + threadIdx.x, a.end[m],
+                                     a.sc[m], e_s, qa, kTagEmit + m, ph, a.diag[m]);
+            return;
+        }
+        b -= a.blocks[m];
+    }
+    qed_photon<real, PUSHER>(g, f, cur, a.s[2], a.first[2] + (int64_t)b * kBlock + threadIdx.x, a.end[2], a.sc[2], e_s,
+                             qa, el, po, a.diag[2]);
+}
+
+// the slot counters, and the live counts that the step's pushes have summed
+// over the copies of the diagnostics, to pinned host memory; then the flag
+__global__ void __launch_bounds__(64) k_publish_counts(const int *count, int n, const double *diag, int nsp,
+                                                       QedCounts *out, unsigned seq)
+{
+    static_assert(kDiagSlots == 64, "a lane per copy");
+    const int t = threadIdx.x;
+    if (t < n) out->n[t] = count[t];
+    for (int s = 0; s < nsp && diag; ++s) {
+        const double v = wave_sum(diag[t * kDiagStride + s * kDiagPerSpecies + 2]);
+        if (t == 0) out->live[s] = v;
+    }
+    __threadfence_system();
+    if (t == 0) __hip_atomic_store(&out->flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 template <typename real, int PUSHER>
 __global__ void __launch_bounds__(kBlock) k_vacuum_pairs(Grid g, Fields<real> f, double q_vac, QedArgs qa,
                                                          AppendTarget<real> el, AppendTarget<real> po, int64_t ncells)
@@ -290,6 +339,7 @@ __global__ void __launch_bounds__(kBlock) k_vacuum_pairs(Grid g, Fields<real> f,
     gather_global(f, g, i, j, k, half, e, b);
     const double ed[3] = {e[0], e[1], e[2]}, bd[3] = {b[0], b[1], b[2]};
     const double rate = qed_vacuum_rate(qa.e_s, ed, bd) * g.dt * g.dx * g.dy * g.dz;
+    if (!(rate > 0)) return;
     const uint32_t cell = (uint32_t)((i * g.ny + j) * g.nz + k);
     if (!(qed_draw(qa.seed, qa.step, cell, kTagVacuum).acc < rate)) return;
     // both born at rest (g = 1), pushed back by dt / 2 (src/mc.cpp:170-176)
@@ -305,35 +355,35 @@ __global__ void __launch_bounds__(kBlock) k_vacuum_pairs(Grid g, Fields<real> f,
 }  // namespace
 
 template <typename real>
-hipError_t launch_push_qed_lepton(hipStream_t st, const Grid &g, const Fields<real> &f, const Current<real> &j,
-                                  const Species<real> &s, const PushArgs &a, const QedArgs &q,
-                                  const AppendTarget<real> &ph)
+hipError_t launch_qed_particles(hipStream_t st, const Grid &g, const Fields<real> &f, const Current<real> &j,
+                                const Species<real> (&s)[3], const PushArgs (&a)[3], const QedArgs &q,
+                                const AppendTarget<real> &el, const AppendTarget<real> &po,
+                                const AppendTarget<real> &ph)
 {
-    if (a.n <= 0) return hipSuccess;
-    const StepConst<real> sc = step_const<real>(g, a);
-    const uint32_t tag = kTagEmit + (a.cmr < 0 ? 0u : 1u);
-    if (a.pusher == 1)
-        k_push_qed_lepton<real, 1><<<blocks_for(a.n), kBlock, 0, st>>>(g, f, j, s, a.first, a.n, sc, (real)q.e_s, q,
-                                                                      tag, ph, a.diag);
+    QedParts<real> p{};
+    int64_t total = 0;
+    for (int m = 0; m < 3; ++m) {
+        p.s[m] = s[m];
+        p.sc[m] = step_const<real>(g, a[m]);
+        p.first[m] = a[m].first;
+        p.end[m] = a[m].first + std::max<int64_t>(a[m].n, 0);
+        p.blocks[m] = a[m].n > 0 ? (int)blocks_for(a[m].n) : 0;
+        p.diag[m] = a[m].diag;
+        total += p.blocks[m];
+    }
+    if (total == 0) return hipSuccess;
+    if (a[0].pusher == 1)
+        k_qed_particles<real, 1><<<(unsigned)total, kBlock, 0, st>>>(g, f, j, p, (real)q.e_s, q, el, po, ph);
     else
-        k_push_qed_lepton<real, 0><<<blocks_for(a.n), kBlock, 0, st>>>(g, f, j, s, a.first, a.n, sc, (real)q.e_s, q,
-                                                                      tag, ph, a.diag);
+        k_qed_particles<real, 0><<<(unsigned)total, kBlock, 0, st>>>(g, f, j, p, (real)q.e_s, q, el, po, ph);
     return hipGetLastError();
 }
 
-template <typename real>
-hipError_t launch_photon_qed(hipStream_t st, const Grid &g, const Fields<real> &f, const Current<real> &j,
-                             const Species<real> &s, const PushArgs &a, const QedArgs &q,
-                             const AppendTarget<real> &el, const AppendTarget<real> &po)
+hipError_t launch_publish_counts(hipStream_t st, const int *count, int n, const double *diag, int nsp, QedCounts *out,
+                                 unsigned seq)
 {
-    if (a.n <= 0) return hipSuccess;
-    const StepConst<real> sc = step_const<real>(g, a);
-    if (a.pusher == 1)
-        k_photon_qed<real, 1><<<blocks_for(a.n), kBlock, 0, st>>>(g, f, j, s, a.first, a.n, sc, (real)q.e_s, q, el,
-                                                                 po, a.diag);
-    else
-        k_photon_qed<real, 0><<<blocks_for(a.n), kBlock, 0, st>>>(g, f, j, s, a.first, a.n, sc, (real)q.e_s, q, el,
-                                                                 po, a.diag);
+    if (n > QedCounts::kMost || nsp > QedCounts::kMost) return hipErrorInvalidValue;
+    k_publish_counts<<<1, 64, 0, st>>>(count, n, diag, nsp, out, seq);
     return hipGetLastError();
 }
 
@@ -351,13 +401,11 @@ hipError_t launch_vacuum_pairs(hipStream_t st, const Grid &g, const Fields<real>
 }
 
 #define QK_INST(real)                                                                                          \
-    template hipError_t launch_push_qed_lepton<real>(hipStream_t, const Grid &, const Fields<real> &,          \
-                                                     const Current<real> &, const Species<real> &,             \
-                                                     const PushArgs &, const QedArgs &, const AppendTarget<real> &); \
-    template hipError_t launch_photon_qed<real>(hipStream_t, const Grid &, const Fields<real> &,               \
-                                                const Current<real> &, const Species<real> &, const PushArgs &, \
-                                                const QedArgs &, const AppendTarget<real> &,                   \
-                                                const AppendTarget<real> &);                                   \
+    template hipError_t launch_qed_particles<real>(hipStream_t, const Grid &, const Fields<real> &,            \
+                                                   const Current<real> &, const Species<real> (&)[3],          \
+                                                   const PushArgs (&)[3], const QedArgs &,                     \
+                                                   const AppendTarget<real> &, const AppendTarget<real> &,     \
+                                                   const AppendTarget<real> &);                                \
     template hipError_t launch_vacuum_pairs<real>(hipStream_t, const Grid &, const Fields<real> &, int, double, \
                                                   const QedArgs &, const AppendTarget<real> &,                 \
                                                   const AppendTarget<real> &);
