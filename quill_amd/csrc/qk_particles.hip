@@ -153,12 +153,14 @@ __device__ inline int small_div(int w)
     return (int)(__umul24((unsigned)w, (unsigned)M) >> 16);
 }
 
-// node idx of an array (at most 2^30 nodes: cells are packed in 30 bits); in
-// FP32 its byte offset fits 32 bits, added to the base by the memory operation
-__device__ inline float &node_at(float *base, int idx) { return at32(base, (uint32_t)idx * 4u); }
-__device__ inline const float &node_at(const float *base, int idx) { return at32(base, (uint32_t)idx * 4u); }
-__device__ inline double &node_at(double *base, int idx) { return base[idx]; }
-__device__ inline const double &node_at(const double *base, int idx) { return base[idx]; }
+// the node `rel` nodes after the one that first points to (which may lie before
+// the array, as a window's first node may); rel * sizeof(real) fits 32 bits
+// inside a window or stage, so the address is a scalar base and one register
+template <typename real>
+__device__ inline real &node_after(real *first, int rel)
+{
+    return at32(first, (uint32_t)rel * (uint32_t)sizeof(real));
+}
 
 // Component C of E and of Be into the stage, in two passes over a thread's
 // share of the block: the loads (load_component), then the LDS writes
@@ -176,16 +178,19 @@ __device__ inline void load_component(real (&e)[kStageIt], real (&b)[kStageIt], 
 {
     static_assert(fsize(C) == fsize(0), "stage blocks of equal size");
     constexpr int d1 = fdim(C, 1), d2 = fdim(C, 2);
+    // the block's first node inside the grid, and each node relative to it
+    const int ib = min(max(gi0, 0), g.nx - 1), jb = min(max(gj0, 0), g.ny - 1), kb = min(max(gk0, 0), g.nz - 1);
+    const int64_t first = (int64_t)ib * g.sx + (int64_t)jb * g.sy + kb;
 #pragma unroll
     for (int m = 0; m < kStageIt; ++m) {
         const int w = min((int)threadIdx.x + m * kTBlock, fsize(C) - 1);
         const int t = small_div<d2, fsize(C)>(w), li = small_div<d1, fsize(C)>(t);
         const int lk = w - t * d2, lj = t - li * d1;
-        const int i = min(max(gi0 + li, 0), g.nx - 1), j = min(max(gj0 + lj, 0), g.ny - 1),
-                  k = min(max(gk0 + lk, 0), g.nz - 1);
-        const int idx = (int)(__umul24((unsigned)i, (unsigned)g.sx) + __umul24((unsigned)j, (unsigned)g.sy)) + k;
-        e[m] = node_at(E, idx);
-        b[m] = node_at(B, idx);
+        const int i = min(max(li + (gi0 - ib), -ib), g.nx - 1 - ib), j = min(max(lj + (gj0 - jb), -jb), g.ny - 1 - jb),
+                  k = min(max(lk + (gk0 - kb), -kb), g.nz - 1 - kb);
+        const int rel = (int)(__umul24((unsigned)i, (unsigned)g.sx) + __umul24((unsigned)j, (unsigned)g.sy)) + k;
+        e[m] = node_after(E + first, rel);
+        b[m] = node_after(B + first, rel);
     }
 }
 
@@ -202,13 +207,13 @@ __device__ inline void store_component(EB<real> *dst, const real (&e)[kStageIt],
 // add component C of the current window to the grid: one global atomic per
 // nonzero entry.  v holds the thread's share of the window block (entry
 // threadIdx.x + m kTBlock), read from LDS for all three components before the
-// first atomic; base is the window's first node.  A particle that deposits is
+// first atomic; first is the window's first node.  A particle that deposits is
 // is_inside (1 .. n - 3) and crosses one face per axis at most, so the nodes it
 // reaches lie in the grid (0 .. n - 1) and entries outside it hold zero.
 constexpr int kFlushIt = (jsize(0) + kTBlock - 1) / kTBlock;
 
 template <int C, typename real>
-__device__ inline void flush_component(real *__restrict__ dst, const double (&v)[kFlushIt], const Grid &g, int base)
+__device__ inline void flush_component(real *__restrict__ dst, const double (&v)[kFlushIt], const Grid &g, int64_t first)
 {
     static_assert(jsize(C) <= kFlushIt * kTBlock, "window block larger than the thread shares");
     constexpr int d1 = jdim(C, 1), d2 = jdim(C, 2), most = kFlushIt * kTBlock;
@@ -218,8 +223,8 @@ __device__ inline void flush_component(real *__restrict__ dst, const double (&v)
         const int t = small_div<d2, most>(w), wi = small_div<d1, most>(t);
         const int wk = w - t * d2, wj = t - wi * d1;
         if (v[m] != 0.0) {   // zero past the block's end
-            const int idx = base + (int)(__umul24((unsigned)wi, (unsigned)g.sx) + __umul24((unsigned)wj, (unsigned)g.sy)) + wk;
-            unsafeAtomicAdd(&node_at(dst, idx), (real)v[m]);
+            const int rel = (int)(__umul24((unsigned)wi, (unsigned)g.sx) + __umul24((unsigned)wj, (unsigned)g.sy)) + wk;
+            unsafeAtomicAdd(&node_after(dst + first, rel), (real)v[m]);
         }
     }
 }
@@ -483,7 +488,7 @@ __global__ void __launch_bounds__(kTBlock) k_push_tiled(Grid g, Fields<real> f, 
     }
 
     {
-        const int base = (i0 - kHalo - 1) * g.sx + (j0 - kHalo - 1) * g.sy + k0 - kHalo - 1;
+        const int64_t first = (int64_t)(i0 - kHalo - 1) * g.sx + (j0 - kHalo - 1) * g.sy + k0 - kHalo - 1;
         double v[3][kFlushIt];
 #pragma unroll
         for (int m = 0; m < kFlushIt; ++m) {
@@ -491,9 +496,9 @@ __global__ void __launch_bounds__(kTBlock) k_push_tiled(Grid g, Fields<real> f, 
 #pragma unroll
             for (int c = 0; c < 3; ++c) v[c][m] = w < jsize(c) ? win[joff(c) + w] : 0.0;
         }
-        flush_component<0>(cur.jx, v[0], g, base);
-        flush_component<1>(cur.jy, v[1], g, base);
-        flush_component<2>(cur.jz, v[2], g, base);
+        flush_component<0>(cur.jx, v[0], g, first);
+        flush_component<1>(cur.jy, v[1], g, first);
+        flush_component<2>(cur.jz, v[2], g, first);
     }
     diag_accumulate(sp.diag, da.q, da.e, da.n, da.fallback);
 }
