@@ -15,6 +15,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <exception>
 #include <functional>
@@ -54,7 +55,10 @@ inline hipError_t wait_flag(hipStream_t st, const unsigned *flag, unsigned want)
     for (unsigned spins = 1; f->load(std::memory_order_acquire) != want; ++spins) {
         if (spins % 65536 == 0) {
             const hipError_t e = hipStreamQuery(st);
-            if (e == hipErrorNotReady) continue;
+            if (e == hipErrorNotReady) {
+                (void)hipGetLastError();   // not an error of a later launch
+                continue;
+            }
             if (e != hipSuccess) return e;
             return f->load(std::memory_order_acquire) == want ? hipSuccess : hipErrorLaunchFailure;
         }
@@ -63,6 +67,20 @@ inline hipError_t wait_flag(hipStream_t st, const unsigned *flag, unsigned want)
 #endif
     }
     return hipSuccess;
+}
+
+// Until event e is reached: polled for a while, then waited for.  The stream
+// synchronization sleeps after some microseconds and is woken late, which a
+// call of a few small steps notices.
+inline hipError_t wait_event(hipEvent_t e)
+{
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(400);
+    do {
+        const hipError_t r = hipEventQuery(e);
+        if (r != hipErrorNotReady) return r;
+        (void)hipGetLastError();
+    } while (std::chrono::steady_clock::now() < until);
+    return hipEventSynchronize(e);
 }
 
 class Drain {

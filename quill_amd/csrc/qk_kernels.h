@@ -128,6 +128,14 @@ hipError_t launch_merge_delete(hipStream_t st, const Species<real> &s, int64_t n
 template <typename real>
 hipError_t launch_scale_charge(hipStream_t st, const Species<real> &s, int64_t n, double a);
 
+// how a kernel tells the host that its result is complete: the last of
+// its workgroups (counted in arrived, left at zero) stores seq to flag
+struct ReadDone {
+    unsigned *arrived;   // device memory
+    unsigned *flag;      // pinned host memory
+    unsigned seq;
+};
+
 // ---- moving window (src/advance.cpp:389-454) --------------------------------
 
 // E, B and Be move one plane toward -x (F[i] = F[i + 1]); the plane nx - 1 is zeroed
@@ -135,11 +143,12 @@ template <typename real>
 hipError_t launch_shift_fields(hipStream_t st, const Grid &g, const Fields<real> &f);
 // packed cells of slots [0, n): plane i = 0 is erased, the rest move to i - 1
 hipError_t launch_shift_particles(hipStream_t st, int *cell, int64_t n);
-// *out = max(*out, max over planes [ilo, ihi) of E^2 + B^2) as the bits of a
-// non-negative double (get_max_w, src/low-level.cpp:512-532)
+// max over planes [ilo, ihi) (not empty) of E^2 + B^2 as the bits of a
+// non-negative double (get_max_w, src/low-level.cpp:512-532) to *out, pinned;
+// acc: a device word, zero before and after
 template <typename real>
 hipError_t launch_max_w(hipStream_t st, const Grid &g, const Fields<real> &f, int ilo, int ihi,
-                        unsigned long long *out);
+                        unsigned long long *acc, unsigned long long *out, const ReadDone &done);
 // fill_cell_by_particles (src/init.cpp:402-478) with T = 0 on ncells listed
 // cells (i j k triples), npic[0] x npic[1] x npic[2] particles each, written to
 // slots first, first + 1, ...; ids idbase[m] + particle index when s.id is set
@@ -239,13 +248,6 @@ hipError_t launch_compute_rho(hipStream_t st, const Grid &g, const Species<real>
 
 // slots per run of the live-particle counts
 constexpr int kLiveRun = 1024;
-// how a pack kernel tells the host that its block is complete: the last of
-// its workgroups (counted in arrived, left at zero) stores seq to flag
-struct ReadDone {
-    unsigned *arrived;   // device memory
-    unsigned *flag;      // pinned host memory
-    unsigned seq;
-};
 // out[3 m + c] = component c at node first + m, m in [0, n), n > 0
 template <typename real>
 hipError_t launch_pack_fields(hipStream_t st, const real *a, const real *b, const real *c, int64_t first, int n,
