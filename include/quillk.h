@@ -226,6 +226,11 @@ int qk_tangent_get(qk_ctx *ctx, double *dE, double *dB, double *const *dpart);
  * cells.  The state after the call is the state before it. */
 int qk_adjoint(qk_ctx *ctx, const double *lam_E, const double *lam_B, const double *const *lam_part,
                double *grad_E, double *grad_B, double *const *grad_part);
+/* The same with the rows of lam_part and grad_part in the order of the
+ * particles' ids, which must be 0 .. n - 1 in each species (track_ids); the
+ * rows of deleted particles are taken times zero. */
+int qk_adjoint_by_id(qk_ctx *ctx, const double *lam_E, const double *lam_B, const double *const *lam_part,
+                     double *grad_E, double *grad_B, double *const *grad_part);
 
 /* timing of the last qk_step call, measured with HIP events on the context's
  * stream: total milliseconds and the part spent in the particle kernels */

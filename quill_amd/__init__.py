@@ -33,7 +33,8 @@ EXPORTS = ["qk_create", "qk_destroy", "qk_last_error", "qk_set_fields", "qk_get_
            "qk_load_uniform_plasma", "qk_init_laser_cos", "qk_init_boundaries", "qk_step", "qk_sync",
            "qk_particle_count", "qk_get_particles", "qk_compute_rho", "qk_compute_rho_noalloc", "qk_last_timing",
            "qk_last_fallback", "qk_get_stream", "qk_pmerging", "qk_moving_window", "qk_max_w", "qk_fill_cells",
-           "qk_tape_begin", "qk_adjoint", "qk_add_laser_source", "qk_tangent_begin", "qk_tangent_get"]
+           "qk_tape_begin", "qk_adjoint", "qk_adjoint_by_id",
+           "qk_add_laser_source", "qk_tangent_begin", "qk_tangent_get"]
 
 
 class QuillError(RuntimeError):
@@ -107,6 +108,7 @@ def load_library(path=LIB_PATH):
     L.qk_fill_cells.argtypes = [vp, C.c_int, C.c_int64, ip, dp, ip, C.c_double, C.c_int32, i64p]
     L.qk_tape_begin.argtypes = [vp, C.c_int]
     L.qk_adjoint.argtypes = [vp, dp, dp, C.POINTER(dp), dp, dp, C.POINTER(dp)]
+    L.qk_adjoint_by_id.argtypes = L.qk_adjoint.argtypes
     L.qk_tangent_begin.argtypes = [vp, dp, dp, C.POINTER(dp)]
     L.qk_tangent_get.argtypes = [vp, dp, dp, C.POINTER(dp)]
     for name in EXPORTS:
@@ -338,7 +340,15 @@ class Region:
         slot order (tape_ids; the order added with the global deposit; zero
         for deleted particles).  Returns (grad_E0, grad_B0, {species: (n, 7)})
         at tape_begin, in the same order."""
-        L = load_library()
+        return self._adjoint(load_library().qk_adjoint, lam_E, lam_B, lam_parts)
+
+    def adjoint_by_id(self, lam_E=None, lam_B=None, lam_parts=None):
+        """adjoint() with the particles' rows in the order of their ids, which
+        must be 0 .. n - 1 in each species (track_ids); the rows of deleted
+        particles are taken times zero."""
+        return self._adjoint(load_library().qk_adjoint_by_id, lam_E, lam_B, lam_parts)
+
+    def _adjoint(self, call, lam_E, lam_B, lam_parts):
         shape = self.shape + (3,)
         lE = np.ascontiguousarray(lam_E, np.float64) if lam_E is not None else None
         lB = np.ascontiguousarray(lam_B, np.float64) if lam_B is not None else None
@@ -357,8 +367,8 @@ class Region:
                 lp[s] = _dp(a)
             grads[s] = np.zeros((n, 7))
             gp[s] = _dp(grads[s])
-        _check(L.qk_adjoint(self._h, _dp(lE) if lE is not None else None, _dp(lB) if lB is not None else None, lp,
-                            _dp(gE), _dp(gB), gp), "qk_adjoint")
+        _check(call(self._h, _dp(lE) if lE is not None else None, _dp(lB) if lB is not None else None, lp, _dp(gE),
+                    _dp(gB), gp), "qk_adjoint")
         return gE, gB, grads
 
     def tangent_begin(self, dE=None, dB=None, dparts=None):

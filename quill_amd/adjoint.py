@@ -93,31 +93,20 @@ class PICRun(torch.autograd.Function):
         r, E, B, outs = simulate(spec, E0, B0, parts, tape=True)
         ctx.region = r
         ctx.spec = spec
-        ctx.shapes = [tuple(P.shape) for P in parts]
         return (E, B, *outs)
 
     @staticmethod
     def backward(ctx, gE, gB, *gparts):
         spec, r = ctx.spec, ctx.region
-        # rows are ids (the order added); the library's adjoint works in the
-        # slot order after tape_begin
-        lam, order = {}, {s: r.tape_ids(s) for s in spec.species if s in r._tape_ids}
-        for s, g in zip(spec.species, gparts):
-            if g is not None and s in order:
-                lam[s] = (g.detach().cpu().double().numpy() * spec.alive[s][:, None])[order[s]]
+        # rows are ids (the order added)
+        lam = {s: g.detach().cpu().double().numpy() for s, g in zip(spec.species, gparts)
+               if g is not None and s in r._tape_ids}
         try:
-            gE0, gB0, gp = r.adjoint(gE.detach().cpu().double().numpy() if gE is not None else None,
-                                     gB.detach().cpu().double().numpy() if gB is not None else None, lam)
+            gE0, gB0, gp = r.adjoint_by_id(gE.detach().cpu().double().numpy() if gE is not None else None,
+                                           gB.detach().cpu().double().numpy() if gB is not None else None, lam)
         finally:
             r.close()
-        grads = []
-        for s, P in zip(spec.species, ctx.shapes):
-            if s in gp:
-                g = np.zeros(P)
-                g[order[s]] = gp[s]
-                grads.append(torch.from_numpy(g))
-            else:
-                grads.append(None)
+        grads = [torch.from_numpy(gp[s]) if s in gp else None for s in spec.species]
         return (None, torch.from_numpy(gE0), torch.from_numpy(gB0), *grads)
 
 

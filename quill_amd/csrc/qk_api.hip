@@ -119,6 +119,7 @@ struct Tape {
     void *fin = nullptr;          // the end state, restored after the adjoint
     double *lam = nullptr;        // 12 field adjoints: E, B, Be, J
     double *lpart = nullptr;      // 7 record adjoints per species
+    double *rows = nullptr;       // rows on their way from and to the caller's arrays
     // tangent-linear run along the recorded steps (qk_tangent_begin)
     bool tangent = false;
     double *tfield = nullptr;     // 15 FP64 arrays: E, B, Be, J (two buffers)
@@ -662,43 +663,32 @@ int qed_particle_phase(qk_ctx *c, const Fields<real> &f, const Current<real> &jc
 // the record arrays a snapshot keeps per species: cell, ox oy oz ux uy uz q
 size_t species_state_bytes(const qk_ctx *c, int64_t n) { return (size_t)n * (4 + 7 * c->rsize); }
 
-int tape_save(qk_ctx *c, void *dst)
+// the whole state to (save) or from a snapshot
+int tape_copy(qk_ctx *c, void *snap, bool save)
 {
-    char *d = (char *)dst;
-    HIP_TRY(hipMemcpyAsync(d, c->fmem, c->tape.field_bytes, hipMemcpyDeviceToDevice, c->stream));
-    d += c->tape.field_bytes;
+    WordCopies w{};
+    char *d = (char *)snap;
+    auto add = [&](void *state, size_t bytes) {
+        w.src[w.count] = (const uint32_t *)(save ? state : d);
+        w.dst[w.count] = (uint32_t *)(save ? d : state);
+        w.n[w.count++] = (int64_t)(bytes / 4);
+        d += bytes;
+    };
+    static_assert(1 + 8 * QK_MAX_SPECIES <= WordCopies::kMost, "an entry per array");
+    add(c->fmem, c->tape.field_bytes);
     for (int s = 0; s < QK_MAX_SPECIES; ++s) {
         const int64_t n = c->tape.n[s];
         if (n == 0) continue;
         const SoA &b = c->sp[s].buf[c->sp[s].cur];
-        HIP_TRY(hipMemcpyAsync(d, b.cell, (size_t)n * 4, hipMemcpyDeviceToDevice, c->stream));
-        d += (size_t)n * 4;
-        for (int a = 0; a < 7; ++a) {
-            HIP_TRY(hipMemcpyAsync(d, b.a[a], (size_t)n * c->rsize, hipMemcpyDeviceToDevice, c->stream));
-            d += (size_t)n * c->rsize;
-        }
+        add(b.cell, (size_t)n * 4);
+        for (int a = 0; a < 7; ++a) add(b.a[a], (size_t)n * c->rsize);
     }
+    HIP_TRY(launch_copy_words(c->stream, w));
     return QK_OK;
 }
 
-int tape_load(qk_ctx *c, const void *src)
-{
-    const char *d = (const char *)src;
-    HIP_TRY(hipMemcpyAsync(c->fmem, d, c->tape.field_bytes, hipMemcpyDeviceToDevice, c->stream));
-    d += c->tape.field_bytes;
-    for (int s = 0; s < QK_MAX_SPECIES; ++s) {
-        const int64_t n = c->tape.n[s];
-        if (n == 0) continue;
-        const SoA &b = c->sp[s].buf[c->sp[s].cur];
-        HIP_TRY(hipMemcpyAsync(b.cell, d, (size_t)n * 4, hipMemcpyDeviceToDevice, c->stream));
-        d += (size_t)n * 4;
-        for (int a = 0; a < 7; ++a) {
-            HIP_TRY(hipMemcpyAsync(b.a[a], d, (size_t)n * c->rsize, hipMemcpyDeviceToDevice, c->stream));
-            d += (size_t)n * c->rsize;
-        }
-    }
-    return QK_OK;
-}
+int tape_save(qk_ctx *c, void *dst) { return tape_copy(c, dst, true); }
+int tape_load(qk_ctx *c, const void *src) { return tape_copy(c, const_cast<void *>(src), false); }
 
 // views of a saved state: the fields (E, Be) and one species' records
 template <typename real>
@@ -758,10 +748,11 @@ void tape_free(qk_ctx *c)
     if (t.fin) (void)hipFree(t.fin);
     if (t.lam) (void)hipFree(t.lam);
     if (t.lpart) (void)hipFree(t.lpart);
+    if (t.rows) (void)hipFree(t.rows);
     if (t.tfield) (void)hipFree(t.tfield);
     if (t.tpart) (void)hipFree(t.tpart);
     t.seg = t.fin = nullptr;
-    t.lam = t.lpart = nullptr;
+    t.lam = t.lpart = t.rows = nullptr;
     t.tfield = t.tpart = nullptr;
     t.tangent = false;
     t.active = t.replay = t.dirty = false;
@@ -770,11 +761,29 @@ void tape_free(qk_ctx *c)
 
 template <typename real>
 int step_impl(qk_ctx *c, int nsteps, qk_diag *diag);
+int download_fields(qk_ctx *c, int nf, double *const *aos, void *const (*comp)[3], size_t rsize);
+int download_doubles(qk_ctx *c, double *dst, const double *src, int64_t n);
+
+// whether the ids of slots [0, n) name each row 0 .. n - 1 once
+int check_row_ids(qk_ctx *c, const int *id, int64_t n)
+{
+    if (!id) return fail(QK_ERR_STATE, "rows by id need track_ids");
+    int *seen = nullptr, bad = 0;
+    HIP_TRY(hipMalloc(&seen, ((size_t)n + 1) * sizeof(int)));
+    hipError_t e = launch_fill_int(c->stream, seen, (size_t)n + 1, 0);
+    if (e == hipSuccess) e = launch_check_ids(c->stream, id, n, seen, seen + n);
+    if (e == hipSuccess) e = hipMemcpyAsync(&bad, seen + n, sizeof(int), hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    const hipError_t e2 = hipFree(seen);
+    HIP_TRY(e);
+    HIP_TRY(e2);
+    return bad ? fail(QK_ERR_INVALID, "rows by id: the ids are not 0 .. n - 1") : QK_OK;
+}
 
 // the adjoint sweep of qk_adjoint (see there)
 template <typename real>
 int adjoint_impl(qk_ctx *c, const double *lam_E, const double *lam_B, const double *const *lam_part, double *grad_E,
-                 double *grad_B, double *const *grad_part)
+                 double *grad_B, double *const *grad_part, bool by_id)
 {
     Tape &t = c->tape;
     const int64_t nc = c->g.ncell;
@@ -801,27 +810,44 @@ int adjoint_impl(qk_ctx *c, const double *lam_E, const double *lam_B, const doub
     const int jcur_end = c->jcur;
     const uint32_t step_end = c->step_index;
     QK_TRY(tape_save(c, t.fin));
-    // seeds: fields AoS -> SoA, records AoS (x y z ux uy uz q) -> SoA
-    {
-        std::vector<double> h((size_t)nc * 12, 0.0);
-        for (int64_t m = 0; m < nc; ++m)
-            for (int a = 0; a < 3; ++a) {
-                if (lam_E) h[(size_t)a * nc + m] = lam_E[3 * m + a];
-                if (lam_B) h[(size_t)(3 + a) * nc + m] = lam_B[3 * m + a];
-            }
-        HIP_TRY(hipMemcpyAsync(t.lam, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
-        for (int s = 0; s < QK_MAX_SPECIES; ++s) {
-            const int64_t n = t.n[s];
-            if (n == 0) continue;
-            std::vector<double> hp((size_t)n * 7, 0.0);
-            if (lam_part && lam_part[s])
-                for (int64_t p = 0; p < n; ++p)
-                    for (int a = 0; a < 7; ++a) hp[(size_t)a * n + p] = lam_part[s][7 * p + a];
-            HIP_TRY(hipMemcpyAsync(lpart[s][0], hp.data(), hp.size() * sizeof(double), hipMemcpyHostToDevice,
-                                   c->stream));
+    // seeds: interleaved fields and rows go up in blocks of at most
+    // kRowBytes and are laid out by kernels
+    constexpr size_t kRowBytes = (size_t)64 << 20, kRow = 7 * sizeof(double), kNode = 3 * sizeof(double);
+    int64_t n_most = 0;
+    for (int s = 0; s < QK_MAX_SPECIES; ++s) n_most = std::max(n_most, t.n[s]);
+    const size_t row_bytes = std::min(kRowBytes, std::max((size_t)n_most * kRow, (size_t)nc * kNode));
+    const int64_t row_per = (int64_t)(row_bytes / kRow), node_per = (int64_t)(row_bytes / kNode);
+    if (!t.rows) HIP_TRY(hipMalloc(&t.rows, row_bytes));
+    const int *row_id[QK_MAX_SPECIES] = {};
+    for (int s = 0; s < QK_MAX_SPECIES && by_id; ++s)
+        if (t.n[s] > 0) {
+            row_id[s] = c->sp[s].buf[c->sp[s].cur].id;
+            QK_TRY(check_row_ids(c, row_id[s], t.n[s]));
         }
-        HIP_TRY(hipStreamSynchronize(c->stream));
+    HIP_TRY(launch_zero(c->stream, t.lam, (size_t)nc * 12));
+    for (int f = 0; f < 2; ++f) {
+        const double *src = f == 0 ? lam_E : lam_B;
+        for (int64_t m = 0; src && m < nc; m += node_per) {
+            const int64_t k = std::min(node_per, nc - m);
+            HIP_TRY(hipMemcpyAsync(t.rows, src + 3 * m, (size_t)k * kNode, hipMemcpyHostToDevice, c->stream));
+            HIP_TRY(launch_split_fields(c->stream, t.rows, lam + 3 * f, m, k));
+        }
     }
+    for (int s = 0; s < QK_MAX_SPECIES; ++s) {
+        const int64_t n = t.n[s];
+        if (n == 0) continue;
+        if (!lam_part || !lam_part[s]) {
+            HIP_TRY(launch_zero(c->stream, lpart[s][0], (size_t)n * 7));
+            continue;
+        }
+        for (int64_t r = 0; r < n; r += row_per) {
+            const int64_t k = std::min(row_per, n - r);
+            HIP_TRY(hipMemcpyAsync(t.rows, lam_part[s] + 7 * r, (size_t)k * kRow, hipMemcpyHostToDevice, c->stream));
+            HIP_TRY(launch_rows_in(c->stream, lpart[s], t.rows, row_id[s], c->sp[s].buf[c->sp[s].cur].cell, n, r, r + k));
+        }
+    }
+    // the caller's arrays are free again (and a failed copy is reported here)
+    HIP_TRY(hipStreamSynchronize(c->stream));
     // segments, last first
     t.replay = true;
     const int nseg = (T + t.every - 1) / t.every;
@@ -862,27 +888,18 @@ int adjoint_impl(qk_ctx *c, const double *lam_E, const double *lam_B, const doub
         HIP_TRY(launch_init_boundaries<double>(c->stream, c->p.solver, c->g, lf));
     }
     // results
-    {
-        std::vector<double> h((size_t)nc * 6);
-        HIP_TRY(hipMemcpyAsync(h.data(), t.lam, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        std::vector<std::vector<double>> hp(QK_MAX_SPECIES);
-        for (int s = 0; s < QK_MAX_SPECIES; ++s) {
-            if (t.n[s] == 0 || !grad_part || !grad_part[s]) continue;
-            hp[s].resize((size_t)t.n[s] * 7);
-            HIP_TRY(hipMemcpyAsync(hp[s].data(), lpart[s][0], hp[s].size() * sizeof(double), hipMemcpyDeviceToHost,
-                                   c->stream));
-        }
-        HIP_TRY(hipStreamSynchronize(c->stream));
-        for (int64_t m = 0; m < nc; ++m)
-            for (int a = 0; a < 3; ++a) {
-                if (grad_E) grad_E[3 * m + a] = h[(size_t)a * nc + m];
-                if (grad_B) grad_B[3 * m + a] = h[(size_t)(3 + a) * nc + m];
-            }
-        for (int s = 0; s < QK_MAX_SPECIES; ++s) {
-            if (hp[s].empty()) continue;
-            const int64_t n = t.n[s];
-            for (int64_t p = 0; p < n; ++p)
-                for (int a = 0; a < 7; ++a) grad_part[s][7 * p + a] = hp[s][(size_t)a * n + p];
+    for (int f = 0; f < 2; ++f) {
+        double *dst = f == 0 ? grad_E : grad_B;
+        void *const comp[1][3] = {{lam[3 * f], lam[3 * f + 1], lam[3 * f + 2]}};
+        if (dst) QK_TRY(download_fields(c, 1, &dst, comp, sizeof(double)));
+    }
+    for (int s = 0; s < QK_MAX_SPECIES; ++s) {
+        const int64_t n = t.n[s];
+        if (n == 0 || !grad_part || !grad_part[s]) continue;
+        for (int64_t r = 0; r < n; r += row_per) {
+            const int64_t k = std::min(row_per, n - r);
+            HIP_TRY(launch_rows_out(c->stream, lpart[s], t.rows, row_id[s], n, r, r + k));
+            QK_TRY(download_doubles(c, grad_part[s] + 7 * r, t.rows, 7 * k));
         }
     }
     QK_TRY(tape_load(c, t.fin));
@@ -1226,10 +1243,10 @@ int upload3(qk_ctx *c, const double *aos, void *d0, void *d1, void *d2)
     return QK_OK;
 }
 
-// widen n numbers of the region's precision to FP64
-void widen(const qk_ctx *c, const void *src, int64_t n, double *dst)
+// widen n numbers of rsize bytes to FP64
+void widen(size_t rsize, const void *src, int64_t n, double *dst)
 {
-    if (c->rsize == 8) {
+    if (rsize == 8) {
         std::memcpy(dst, src, (size_t)n * sizeof(double));
         return;
     }
@@ -1238,24 +1255,24 @@ void widen(const qk_ctx *c, const void *src, int64_t n, double *dst)
 }
 
 // up to four fields (three component arrays each) into interleaved FP64 arrays
-int download_fields(qk_ctx *c, int nf, double *const *aos, void *const (*comp)[3])
+int download_fields(qk_ctx *c, int nf, double *const *aos, void *const (*comp)[3], size_t rsize)
 {
     const int64_t n = c->g.ncell;
-    const size_t node = 3 * c->rsize, total = (size_t)nf * n * node;
+    const size_t node = 3 * rsize, total = (size_t)nf * n * node;
     const int64_t per = (int64_t)(Drain::slot_bytes(total) / node);   // nodes per block
     const int64_t nb = (n + per - 1) / per;                            // blocks per field
     auto launch = [&](int64_t b, void *slot, const ReadDone &done) {
         void *const *s = comp[b / nb];
         const int64_t first = b % nb * per;
         const int m = (int)std::min(per, n - first);
-        return c->rsize == 4 ? launch_pack_fields<float>(c->stream, (const float *)s[0], (const float *)s[1],
+        return rsize == 4 ? launch_pack_fields<float>(c->stream, (const float *)s[0], (const float *)s[1],
                                                          (const float *)s[2], first, m, (float *)slot, done)
                              : launch_pack_fields<double>(c->stream, (const double *)s[0], (const double *)s[1],
                                                           (const double *)s[2], first, m, (double *)slot, done);
     };
     auto take = [&](int64_t b, const void *slot) {
         const int64_t first = b % nb * per;
-        widen(c, slot, 3 * std::min(per, n - first), aos[b / nb] + 3 * first);
+        widen(rsize, slot, 3 * std::min(per, n - first), aos[b / nb] + 3 * first);
     };
     HIP_TRY(c->drain.run(c->p.device, c->stream, total, nf * nb, launch, take));
     return QK_OK;
@@ -1545,7 +1562,7 @@ int qk_get_fields(qk_ctx *c, double *E, double *B, double *J, double *Be)
     }
     const DeviceScope on(c->p.device);
     HIP_TRY(hipStreamSynchronize(c->stream));
-    if (nf > 0) QK_TRY(download_fields(c, nf, aos, comp));
+    if (nf > 0) QK_TRY(download_fields(c, nf, aos, comp, c->rsize));
     return QK_OK;
 }
 
@@ -2000,14 +2017,26 @@ int qk_tangent_get(qk_ctx *c, double *dE, double *dB, double *const *dpart)
     return QK_OK;
 }
 
-int qk_adjoint(qk_ctx *c, const double *lam_E, const double *lam_B, const double *const *lam_part, double *grad_E,
-               double *grad_B, double *const *grad_part)
+static int adjoint_call(qk_ctx *c, const double *lam_E, const double *lam_B, const double *const *lam_part, double *grad_E,
+                        double *grad_B, double *const *grad_part, bool by_id)
 {
     if (!c) return fail(QK_ERR_INVALID, "null context");
     if (!c->tape.active) return fail(QK_ERR_STATE, "no tape: call qk_tape_begin before the steps");
     if (c->tape.dirty) return fail(QK_ERR_STATE, "fields or particles changed outside qk_step since qk_tape_begin");
-    return c->rsize == 4 ? adjoint_impl<float>(c, lam_E, lam_B, lam_part, grad_E, grad_B, grad_part)
-                         : adjoint_impl<double>(c, lam_E, lam_B, lam_part, grad_E, grad_B, grad_part);
+    return c->rsize == 4 ? adjoint_impl<float>(c, lam_E, lam_B, lam_part, grad_E, grad_B, grad_part, by_id)
+                         : adjoint_impl<double>(c, lam_E, lam_B, lam_part, grad_E, grad_B, grad_part, by_id);
+}
+
+int qk_adjoint(qk_ctx *c, const double *lam_E, const double *lam_B, const double *const *lam_part, double *grad_E,
+               double *grad_B, double *const *grad_part)
+{
+    return adjoint_call(c, lam_E, lam_B, lam_part, grad_E, grad_B, grad_part, false);
+}
+
+int qk_adjoint_by_id(qk_ctx *c, const double *lam_E, const double *lam_B, const double *const *lam_part, double *grad_E,
+                     double *grad_B, double *const *grad_part)
+{
+    return adjoint_call(c, lam_E, lam_B, lam_part, grad_E, grad_B, grad_part, true);
 }
 
 int qk_last_timing(qk_ctx *c, double *ms_total, double *ms_particles, double *ms_fields)

@@ -178,6 +178,27 @@ template <typename real>
 hipError_t launch_adj_particles(hipStream_t st, const Grid &g, const Fields<real> &f, const Species<real> &s,
                                 int64_t n, const PushArgs &a, double *const lam[12], double *const lpart[7]);
 
+// rows of 7 doubles (x y z ux uy uz q) of rows [r0, r1) to the 7 arrays out,
+// and from them; id: the row of each slot (null: the slot), with which the
+// rows of slots whose cell is negative are taken times zero
+hipError_t launch_rows_in(hipStream_t st, double *const out[7], const double *rows, const int *id, const int *cell,
+                          int64_t n, int64_t r0, int64_t r1);
+hipError_t launch_rows_out(hipStream_t st, double *const in[7], double *rows, const int *id, int64_t n, int64_t r0,
+                           int64_t r1);
+// sets *bad unless id[0 .. n) is a permutation of 0 .. n - 1; seen: n zeros
+hipError_t launch_check_ids(hipStream_t st, const int *id, int64_t n, int *seen, int *bad);
+// component k of nodes [first, first + n) to c[k] from interleaved ones
+hipError_t launch_split_fields(hipStream_t st, const double *aos, double *const c[3], int64_t first, int64_t n);
+// dst[s][0 .. n[s]) = src[s][0 .. n[s]), s < count
+struct WordCopies {
+    static constexpr int kMost = 64;
+    const uint32_t *src[kMost];
+    uint32_t *dst[kMost];
+    int64_t n[kMost];
+    int count;
+};
+hipError_t launch_copy_words(hipStream_t st, const WordCopies &w);
+
 // the field-energy sum is spread over this many FP64 slots (one atomic per
 // workgroup lands on slot blockIdx mod kEnergySlots) and summed on the host
 constexpr int kEnergySlots = 256;
