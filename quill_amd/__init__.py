@@ -33,7 +33,7 @@ EXPORTS = ["qk_create", "qk_destroy", "qk_last_error", "qk_set_fields", "qk_get_
            "qk_load_uniform_plasma", "qk_init_laser_cos", "qk_init_boundaries", "qk_step", "qk_sync",
            "qk_particle_count", "qk_get_particles", "qk_compute_rho", "qk_compute_rho_noalloc", "qk_last_timing",
            "qk_last_fallback", "qk_get_stream", "qk_pmerging", "qk_moving_window", "qk_max_w", "qk_fill_cells",
-           "qk_tape_begin", "qk_adjoint", "qk_adjoint_by_id",
+           "qk_tape_begin", "qk_adjoint", "qk_adjoint_by_id", "qk_get_rows_by_id",
            "qk_add_laser_source", "qk_tangent_begin", "qk_tangent_get"]
 
 
@@ -109,6 +109,7 @@ def load_library(path=LIB_PATH):
     L.qk_tape_begin.argtypes = [vp, C.c_int]
     L.qk_adjoint.argtypes = [vp, dp, dp, C.POINTER(dp), dp, dp, C.POINTER(dp)]
     L.qk_adjoint_by_id.argtypes = L.qk_adjoint.argtypes
+    L.qk_get_rows_by_id.argtypes = [vp, C.c_int, C.c_int64, dp, ip]
     L.qk_tangent_begin.argtypes = [vp, dp, dp, C.POINTER(dp)]
     L.qk_tangent_get.argtypes = [vp, dp, dp, C.POINTER(dp)]
     for name in EXPORTS:
@@ -278,6 +279,13 @@ class Region:
         _check(load_library().qk_get_particles(self._h, species, cap, _dp(rec), _ip(ids), C.byref(n)),
                "qk_get_particles")
         return rec[:n.value], ids[:n.value]
+
+    def rows_by_id(self, species, n):
+        """(rows[n, 7] = x y z ux uy uz q of the live particles by id, mask of
+        the ids that are live); needs track_ids and ids in 0 .. n - 1."""
+        rows, live = np.zeros((n, 7)), np.zeros(n, np.int32)
+        _check(load_library().qk_get_rows_by_id(self._h, species, n, _dp(rows), _ip(live)), "qk_get_rows_by_id")
+        return rows, live != 0
 
     def compute_rho(self):
         rho = np.zeros(self.shape + (3,))

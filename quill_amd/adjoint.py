@@ -62,12 +62,7 @@ def simulate(spec, E0, B0, parts, tape=False):
         E, B, _, _ = r.get_fields()
         outs = []
         for s, P in zip(spec.species, parts):
-            rec, ids = r.particles(s)
-            out = np.zeros((len(P), 7))
-            alive = np.zeros(len(P), bool)
-            out[ids] = rec[:, [0, 1, 2, 3, 4, 5, 7]]
-            alive[ids] = True
-            spec.alive[s] = alive
+            out, spec.alive[s] = r.rows_by_id(s, len(P))
             outs.append(torch.from_numpy(out))
     except Exception:
         r.close()

@@ -484,6 +484,30 @@ __global__ void __launch_bounds__(kABlock) k_rows_out(RowArrays in, double *__re
     for (int a = 0; a < 7; ++a) row[a] = in.a[a][p];
 }
 
+// the state x y z ux uy uz q of the live slots to their rows (id) of [r0, r1),
+// with live[r - r0] = 1; *bad is set where an id lies outside [0, total)
+template <typename real>
+__global__ void __launch_bounds__(kABlock) k_state_rows(Species<real> s, int64_t n, int64_t total, int64_t r0, int64_t r1,
+                                                        double *__restrict__ rows, int *live, int *bad)
+{
+    const int64_t p = (int64_t)blockIdx.x * kABlock + threadIdx.x;
+    if (p >= n) return;
+    const int c = s.cell[p];
+    if (c < 0) return;
+    const int64_t r = s.id[p];
+    if (r < 0 || r >= total) *bad = 1;
+    if (r < r0 || r >= r1) return;
+    double *__restrict__ row = rows + 7 * (r - r0);
+    row[0] = cell_i(c) + (double)s.ox[p];
+    row[1] = cell_j(c) + (double)s.oy[p];
+    row[2] = cell_k(c) + (double)s.oz[p];
+    row[3] = s.ux[p];
+    row[4] = s.uy[p];
+    row[5] = s.uz[p];
+    row[6] = s.q[p];
+    live[r - r0] = 1;
+}
+
 // *bad is set unless id[0 .. n) is a permutation of 0 .. n - 1 (seen: n zeros)
 __global__ void __launch_bounds__(kABlock) k_check_ids(const int *id, int64_t n, int *seen, int *bad)
 {
@@ -543,6 +567,20 @@ hipError_t launch_rows_out(hipStream_t st, double *const in[7], double *rows, co
     k_rows_out<<<ablocks(n), kABlock, 0, st>>>(a, rows, id, n, r0, r1);
     return hipGetLastError();
 }
+
+template <typename real>
+hipError_t launch_state_rows(hipStream_t st, const Species<real> &s, int64_t n, int64_t total, int64_t r0, int64_t r1,
+                             double *rows, int *live, int *bad)
+{
+    if (n <= 0) return hipSuccess;
+    k_state_rows<real><<<ablocks(n), kABlock, 0, st>>>(s, n, total, r0, r1, rows, live, bad);
+    return hipGetLastError();
+}
+
+template hipError_t launch_state_rows<float>(hipStream_t, const Species<float> &, int64_t, int64_t, int64_t, int64_t,
+                                             double *, int *, int *);
+template hipError_t launch_state_rows<double>(hipStream_t, const Species<double> &, int64_t, int64_t, int64_t, int64_t,
+                                              double *, int *, int *);
 
 hipError_t launch_check_ids(hipStream_t st, const int *id, int64_t n, int *seen, int *bad)
 {

@@ -119,7 +119,6 @@ struct Tape {
     void *fin = nullptr;          // the end state, restored after the adjoint
     double *lam = nullptr;        // 12 field adjoints: E, B, Be, J
     double *lpart = nullptr;      // 7 record adjoints per species
-    double *rows = nullptr;       // rows on their way from and to the caller's arrays
     // tangent-linear run along the recorded steps (qk_tangent_begin)
     bool tangent = false;
     double *tfield = nullptr;     // 15 FP64 arrays: E, B, Be, J (two buffers)
@@ -191,6 +190,9 @@ struct qk_ctx {
     Drain drain;
     int *d_live = nullptr;
     size_t live_cap = 0;            // runs that fit
+    // rows of particles on their way from and to the caller's arrays
+    double *rows = nullptr;
+    size_t rows_cap = 0;            // bytes
     // laser sources at an x plane, per side (0: x-min, 1: x-max)
     InjSide inj[2];
     int window_shifts = 0;          // qk_moving_window calls so far
@@ -748,11 +750,10 @@ void tape_free(qk_ctx *c)
     if (t.fin) (void)hipFree(t.fin);
     if (t.lam) (void)hipFree(t.lam);
     if (t.lpart) (void)hipFree(t.lpart);
-    if (t.rows) (void)hipFree(t.rows);
     if (t.tfield) (void)hipFree(t.tfield);
     if (t.tpart) (void)hipFree(t.tpart);
     t.seg = t.fin = nullptr;
-    t.lam = t.lpart = t.rows = nullptr;
+    t.lam = t.lpart = nullptr;
     t.tfield = t.tpart = nullptr;
     t.tangent = false;
     t.active = t.replay = t.dirty = false;
@@ -763,6 +764,20 @@ template <typename real>
 int step_impl(qk_ctx *c, int nsteps, qk_diag *diag);
 int download_fields(qk_ctx *c, int nf, double *const *aos, void *const (*comp)[3], size_t rsize);
 int download_doubles(qk_ctx *c, double *dst, const double *src, int64_t n);
+
+// at least `bytes` at c->rows; callers move their rows in blocks of at most kRowBytes
+constexpr size_t kRowBytes = (size_t)64 << 20, kRow = 7 * sizeof(double);
+
+int ensure_rows(qk_ctx *c, size_t bytes)
+{
+    if (bytes <= c->rows_cap) return QK_OK;
+    if (c->rows) HIP_TRY(hipFree(c->rows));
+    c->rows = nullptr;
+    c->rows_cap = 0;
+    HIP_TRY(hipMalloc(&c->rows, bytes));
+    c->rows_cap = bytes;
+    return QK_OK;
+}
 
 // whether the ids of slots [0, n) name each row 0 .. n - 1 once
 int check_row_ids(qk_ctx *c, const int *id, int64_t n)
@@ -812,12 +827,12 @@ int adjoint_impl(qk_ctx *c, const double *lam_E, const double *lam_B, const doub
     QK_TRY(tape_save(c, t.fin));
     // seeds: interleaved fields and rows go up in blocks of at most
     // kRowBytes and are laid out by kernels
-    constexpr size_t kRowBytes = (size_t)64 << 20, kRow = 7 * sizeof(double), kNode = 3 * sizeof(double);
+    constexpr size_t kNode = 3 * sizeof(double);
     int64_t n_most = 0;
     for (int s = 0; s < QK_MAX_SPECIES; ++s) n_most = std::max(n_most, t.n[s]);
     const size_t row_bytes = std::min(kRowBytes, std::max((size_t)n_most * kRow, (size_t)nc * kNode));
     const int64_t row_per = (int64_t)(row_bytes / kRow), node_per = (int64_t)(row_bytes / kNode);
-    if (!t.rows) HIP_TRY(hipMalloc(&t.rows, row_bytes));
+    QK_TRY(ensure_rows(c, row_bytes));
     const int *row_id[QK_MAX_SPECIES] = {};
     for (int s = 0; s < QK_MAX_SPECIES && by_id; ++s)
         if (t.n[s] > 0) {
@@ -829,8 +844,8 @@ int adjoint_impl(qk_ctx *c, const double *lam_E, const double *lam_B, const doub
         const double *src = f == 0 ? lam_E : lam_B;
         for (int64_t m = 0; src && m < nc; m += node_per) {
             const int64_t k = std::min(node_per, nc - m);
-            HIP_TRY(hipMemcpyAsync(t.rows, src + 3 * m, (size_t)k * kNode, hipMemcpyHostToDevice, c->stream));
-            HIP_TRY(launch_split_fields(c->stream, t.rows, lam + 3 * f, m, k));
+            HIP_TRY(hipMemcpyAsync(c->rows, src + 3 * m, (size_t)k * kNode, hipMemcpyHostToDevice, c->stream));
+            HIP_TRY(launch_split_fields(c->stream, c->rows, lam + 3 * f, m, k));
         }
     }
     for (int s = 0; s < QK_MAX_SPECIES; ++s) {
@@ -842,8 +857,8 @@ int adjoint_impl(qk_ctx *c, const double *lam_E, const double *lam_B, const doub
         }
         for (int64_t r = 0; r < n; r += row_per) {
             const int64_t k = std::min(row_per, n - r);
-            HIP_TRY(hipMemcpyAsync(t.rows, lam_part[s] + 7 * r, (size_t)k * kRow, hipMemcpyHostToDevice, c->stream));
-            HIP_TRY(launch_rows_in(c->stream, lpart[s], t.rows, row_id[s], c->sp[s].buf[c->sp[s].cur].cell, n, r, r + k));
+            HIP_TRY(hipMemcpyAsync(c->rows, lam_part[s] + 7 * r, (size_t)k * kRow, hipMemcpyHostToDevice, c->stream));
+            HIP_TRY(launch_rows_in(c->stream, lpart[s], c->rows, row_id[s], c->sp[s].buf[c->sp[s].cur].cell, n, r, r + k));
         }
     }
     // the caller's arrays are free again (and a failed copy is reported here)
@@ -898,8 +913,8 @@ int adjoint_impl(qk_ctx *c, const double *lam_E, const double *lam_B, const doub
         if (n == 0 || !grad_part || !grad_part[s]) continue;
         for (int64_t r = 0; r < n; r += row_per) {
             const int64_t k = std::min(row_per, n - r);
-            HIP_TRY(launch_rows_out(c->stream, lpart[s], t.rows, row_id[s], n, r, r + k));
-            QK_TRY(download_doubles(c, grad_part[s] + 7 * r, t.rows, 7 * k));
+            HIP_TRY(launch_rows_out(c->stream, lpart[s], c->rows, row_id[s], n, r, r + k));
+            QK_TRY(download_doubles(c, grad_part[s] + 7 * r, c->rows, 7 * k));
         }
     }
     QK_TRY(tape_load(c, t.fin));
@@ -1507,6 +1522,7 @@ int qk_destroy(qk_ctx *c)
     for (int *p : sb)
         if (p) note(hipFree(p));
     if (c->h_sortinfo) note(hipHostFree(c->h_sortinfo));
+    if (c->rows) note(hipFree(c->rows));
     if (c->fmem) note(hipFree(c->fmem));
     if (c->mid) note(hipFree(c->mid));
     if (c->d_diag) note(hipFree(c->d_diag));
@@ -1694,6 +1710,36 @@ int qk_particle_count(qk_ctx *c, int s, int64_t *n)
     if (b.n == 0) return QK_OK;
     const DeviceScope on(c->p.device);
     QK_TRY(scan_live(c, b, *n, nullptr));
+    return QK_OK;
+}
+
+int qk_get_rows_by_id(qk_ctx *c, int s, int64_t n, double *rows, int32_t *live)
+{
+    if (!c) return fail(QK_ERR_INVALID, "null context");
+    if (!species_valid(c, s)) return fail(QK_ERR_INVALID, "invalid species");
+    if (n < 0 || (n > 0 && (!rows || !live))) return fail(QK_ERR_INVALID, "bad output buffers");
+    if (!c->p.track_ids) return fail(QK_ERR_STATE, "rows by id need track_ids");
+    if (n == 0) return QK_OK;
+    const DeviceScope on(c->p.device);
+    const SpeciesBuf &b = c->sp[s];
+    const int64_t per = std::min(n, (int64_t)(kRowBytes / (kRow + sizeof(int))));
+    QK_TRY(ensure_rows(c, (size_t)per * (kRow + sizeof(int)) + sizeof(int)));
+    int *const l = (int *)(c->rows + 7 * per);
+    int bad = 0;
+    for (int64_t r = 0; r < n; r += per) {
+        const int64_t k = std::min(per, n - r);
+        HIP_TRY(launch_zero(c->stream, c->rows, (size_t)per * 7));
+        HIP_TRY(launch_fill_int(c->stream, l, (size_t)per + 1, 0));
+        if (b.n > 0)
+            HIP_TRY(c->rsize == 4 ? launch_state_rows<float>(c->stream, view<float>(b.buf[b.cur]), b.n, n, r, r + k,
+                                                             c->rows, l, l + per)
+                                  : launch_state_rows<double>(c->stream, view<double>(b.buf[b.cur]), b.n, n, r, r + k,
+                                                              c->rows, l, l + per));
+        HIP_TRY(hipMemcpyAsync(live + r, l, (size_t)k * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(hipMemcpyAsync(&bad, l + per, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+        QK_TRY(download_doubles(c, rows + 7 * r, c->rows, 7 * k));
+        if (bad) return fail(QK_ERR_INVALID, "rows by id: an id lies outside 0 .. n - 1");
+    }
     return QK_OK;
 }
 

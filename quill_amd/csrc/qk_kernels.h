@@ -185,6 +185,11 @@ hipError_t launch_rows_in(hipStream_t st, double *const out[7], const double *ro
                           int64_t n, int64_t r0, int64_t r1);
 hipError_t launch_rows_out(hipStream_t st, double *const in[7], double *rows, const int *id, int64_t n, int64_t r0,
                            int64_t r1);
+// rows [r0, r1) of the live slots' state by id (of `total` rows), live[r - r0]
+// set to one where there is one; *bad set at an id outside [0, total)
+template <typename real>
+hipError_t launch_state_rows(hipStream_t st, const Species<real> &s, int64_t n, int64_t total, int64_t r0, int64_t r1,
+                             double *rows, int *live, int *bad);
 // sets *bad unless id[0 .. n) is a permutation of 0 .. n - 1; seen: n zeros
 hipError_t launch_check_ids(hipStream_t st, const int *id, int64_t n, int *seen, int *bad);
 // component k of nodes [first, first + n) to c[k] from interleaved ones

@@ -20,7 +20,8 @@ def _run(n, deposit, by_id, ids=None, steps=2):
     E, B = rng.uniform(-0.1, 0.1, SHAPE + (3,)), rng.uniform(-0.1, 0.1, SHAPE + (3,))
     lam = rng.normal(0, 1, (n, 7))
     lE, lB = rng.normal(0, 1, SHAPE + (3,)), rng.normal(0, 1, SHAPE + (3,))
-    ids = np.random.default_rng(9).permutation(n).astype(np.int32) if ids is None else ids
+    given = ids is not None
+    ids = ids if given else np.random.default_rng(9).permutation(n).astype(np.int32)
     print(f"adjoint rows {n} {deposit} {by_id}", flush=True)
     with qa.Region(*SHAPE, DX, DX, DX, 0.5 * DX, precision="fp64", deposit=deposit, track_ids=True) as r:
         r.set_fields(E, B)
@@ -28,7 +29,12 @@ def _run(n, deposit, by_id, ids=None, steps=2):
         r.init_boundaries()
         r.tape_begin(2)
         r.step(steps)
-        left = r.particles(0)[1]
+        rec, left = r.particles(0)
+        if given:
+            return r.adjoint_by_id(lE, lB, {0: lam})
+        rows, live = r.rows_by_id(0, n)
+        assert (np.flatnonzero(live) == np.sort(left)).all() and (rows[~live] == 0).all()
+        assert (rows[left] == rec[:, [0, 1, 2, 3, 4, 5, 7]]).all()
         if by_id:
             gE, gB, gp = r.adjoint_by_id(lE, lB, {0: lam})
             return gE, gB, gp[0], len(left)
@@ -48,6 +54,14 @@ def test_rows_by_id_are_rows_by_slot(n, deposit):
     for x, y in zip(a[:3], b[:3]):
         # FP64 sums in another order: some 1e3 terms per node
         assert np.abs(x - y).max() <= 1e-11 * np.abs(y).max()
+
+
+def test_ids_outside_the_rows_are_refused():
+    with qa.Region(*SHAPE, DX, DX, DX, 0.5 * DX, track_ids=True) as r:
+        r.add_particles(0, *[np.full(3, 5.5)] * 3, *[np.zeros(3)] * 3, np.full(3, -0.01), ids=np.array([0, 3, 1], np.int32))
+        with pytest.raises(qa.QuillError):
+            r.rows_by_id(0, 3)
+        assert (r.rows_by_id(0, 4)[1] == [True, True, False, True]).all()
 
 
 def test_other_ids_are_refused():
