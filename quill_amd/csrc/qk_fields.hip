@@ -504,9 +504,11 @@ __device__ inline bool pulse_at(const LaserFrame &L, double px, double py, doubl
     if (shift != 0) x -= L.b_sign ? shift : -shift;
     if (!(x < L.xs && x > -L.xs && y < L.ys && y > -L.ys && z < L.zs && z > -L.zs)) return false;
     const double xi = x + L.phase;
-    const double cx = cos(PI * x / 2 / L.xs), cy = cos(PI * y / 2 / L.ys), cz = cos(PI * z / 2 / L.zs);
-    const double sx = sin(PI * x / 2 / L.xs), sy = sin(PI * y / 2 / L.ys), sz = sin(PI * z / 2 / L.zs);
-    const double sxi = sin(xi), cxi = cos(xi);
+    double cx, sx, cy, sy, cz, sz, cxi, sxi;
+    sincos(PI * x / 2 / L.xs, &sx, &cx);
+    sincos(PI * y / 2 / L.ys, &sy, &cy);
+    sincos(PI * z / 2 / L.zs, &sz, &cz);
+    sincos(xi, &sxi, &cxi);
     const double tr = cy * cy * cz * cz;
     const double fy = L.a0y * tr * (cxi * cx * cx - PI / L.xs * sxi * cx * sx);
     const double fz = L.a0z * tr * (sxi * cx * cx + PI / L.xs * cxi * cx * sx);
@@ -565,13 +567,13 @@ __global__ void __launch_bounds__(kBX * kBY) k_laser_cos(Grid g, Fields<real> f,
 // wavefront per plane and row: one launch per sub-step for both sides.  Only differences along x cross the plane, and NDFX's smoothing of
 // the x component along x: component x is needed there only, and neither it
 // nor its own update is ever corrected.
-// Bound by the FP64 pulse (three sines and cosines per point and the
-// transverse ones).  Before, the pulse was evaluated on 18 planes of a stack
+// Bound by the FP64 pulse (four sines and cosines per point, taken in pairs).
+// Before, the pulse was evaluated on 18 planes of a stack
 // that the solver then swept whole, three launches per side and sub-step: a
 // sub-step took 66 us for two sides of 128 x 128 columns (five-point), now
-// 9.4 us; 17.6 us for one of 32 x 32 (FDTD), now 5.1 us.  With 64 x 4 columns
-// per workgroup (six points in turn per thread instead of at most two) it was
-// 21.7 us and 6.6 us.
+// 7.3 us; 17.6 us for one of 32 x 32 (FDTD), now 4.7 us (9.3 and 5.4 us with
+// sines and cosines apart).  With 64 x 4 columns per workgroup (six points in
+// turn per thread instead of at most two) it was 21.7 us and 6.6 us.
 template <int S>
 constexpr int kInjReach = S == 2 ? 2 : 1;
 
