@@ -362,23 +362,40 @@ int ensure_sort_buffers(qk_ctx *c)
     return QK_OK;
 }
 
-// Most particles per workgroup of the tiled push.  With at least half as many
-// tiles as the chip has CUs a tile is one chunk (kChunk).  Fewer tiles leave
-// CUs idle and run their particles in long serial rounds, so they are cut
-// into as many parts as give one workgroup per CU: 1.3 covers the tiles at
-// the box's faces, which hold less than the inner ones.  A second workgroup
-// per CU (FP32 only: two fit) pays for its own staging and flush, some four
-// rounds' time, only where the parts stay above half of kChunk.  Particle
-// phase at 128 tiles, 8 per cell: 36.8 -> 26.5 us (33.9 with four parts per
-// tile, 31.9 with 4096 per part), FP64 45.6 -> 30.3; 27 per cell: 57.0 ->
-// 47.1 us (51.9 at three parts, 62.5 at six); 27 tiles: 32.7 -> 15.4 us.  At
-// 432 tiles halves take 70 us against 61.
+// Most particles per workgroup of the tiled push.  With more than twice as
+// many tiles as the chip has CUs a tile is one chunk (kChunk).  Fewer tiles
+// leave CUs idle, or with one tile while others have two, and run their
+// particles in long serial rounds.
+//
+// Up to half as many tiles as CUs: cut into as many parts as give one workgroup
+// per CU; 1.3 covers the tiles at the box's faces, which hold less than the inner
+// ones.  A second workgroup per CU (FP32 only: two fit) pays for its own staging
+// and flush only where the parts stay above half of kChunk.  Particle phase at
+// 128 tiles, 8 per cell: 36.8 -> 26.5 us (33.9 with four parts per tile, 31.9
+// with 4096 per part), FP64 45.6 -> 30.3; 27 per cell: 57.0 -> 47.1 us (51.9 at
+// three parts, 62.5 at six); 27 tiles: 32.7 -> 15.4 us.
+//
+// From there to twice as many tiles as CUs: halves, where they fill the CUs
+// better and hold enough for their staging and flush: with 150 tiles 43.3 ->
+// 26.1 us, 250 43.0 -> 31.8, 432 61.0 -> 49.4, FP64 77.9 -> 75.1 (8 per cell);
+// but 27.3 -> 31.8 with 432 tiles and 2 per cell (20.5 us either way with 250).  FP64 has one
+// workgroup per CU and gains only beyond one tile per CU.  With 576 tiles
+// halves take 65 us against 71 at 8 per cell and 40 against 34 at 2, with 750
+// tiles 78 against 76.
 int chunk_size(const qk_ctx *c, int64_t n)
 {
-    constexpr int kCU = 256;
-    if (c->tg.ntiles > kCU / 2) return kChunk;
-    int64_t chunk = (13 * n / 10 + kCU - 1) / kCU;
-    if (c->rsize == 4 && chunk > kChunk / 2) chunk = (chunk + 1) / 2;
+    constexpr int kCU = 256, kHalfMean = 2048;
+    const int tiles = c->tg.ntiles;
+    if (tiles > 2 * kCU) return kChunk;
+    int64_t chunk;
+    if (tiles > kCU / 2) {
+        const bool halves = tiles > kCU ? n >= (int64_t)kHalfMean * tiles : c->rsize == 4;
+        if (!halves) return kChunk;
+        chunk = (13 * n / 10 / tiles + 1) / 2;
+    } else {
+        chunk = (13 * n / 10 + kCU - 1) / kCU;
+        if (c->rsize == 4 && chunk > kChunk / 2) chunk = (chunk + 1) / 2;
+    }
     return (int)std::min<int64_t>(std::max<int64_t>(chunk, kMinChunk), kChunk);
 }
 

@@ -29,8 +29,9 @@ constexpr int kDiagSlots = 64, kDiagStride = 32;
 // most particles per workgroup of the tiled kernel (a chunk never spans two
 // tiles; a tile is cut into equal chunks).  Twice the mean tile population at
 // 8 per cell, so a uniform plasma's tile is one chunk: 4096 measured 15 %
-// slower on the push, 2048 30 %, from staging tiles more than once.  A grid of
-// few tiles takes smaller chunks, at least kMinChunk (see chunk_size)
+// slower on the push, 2048 30 %, from staging tiles more than once; 6144 and
+// 5120 within 0.5 % of it at 512x256x256 and 256x128x128.  A grid of few tiles
+// takes smaller chunks, at least kMinChunk (see chunk_size)
 constexpr int kChunk = 8192, kMinChunk = 512;
 
 struct PushArgs {

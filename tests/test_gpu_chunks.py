@@ -31,3 +31,10 @@ def test_parts_match_global_deposit(shape, ppc):
         assert np.abs(a - b).max() <= 1e-12 * np.abs(b).max()
     assert out[1][1] == out[0][1]
     assert abs(out[1][2] - out[0][2]) <= 1e-12 * abs(out[0][2])
+
+
+@pytest.mark.parametrize("shape,ppc", [((72, 48, 40), 6), ((72, 48, 40), 3), ((64, 64, 64), 6), ((65, 64, 64), 6)])
+def test_halves_match_global_deposit(shape, ppc):
+    """Tiles in halves (270 and 512 tiles, with and without enough particles)
+    and one layer more than are cut."""
+    test_parts_match_global_deposit(shape, ppc)

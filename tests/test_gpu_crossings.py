@@ -1,7 +1,7 @@
 """Second pieces of crossing paths kept by their lane in the tiled push: FP32
 against the oracle where few and where most particles cross a face per step,
-some two or three, in one round per workgroup and in many; and tiles at the
-box's corners, where the staged nodes are clamped."""
+some two or three, in one round per workgroup and in many, tiles in halves (180
+tiles); and tiles at the box's corners, where the staged nodes are clamped."""
 import numpy as np
 import pytest
 
@@ -14,7 +14,7 @@ DX = 0.05 * 2 * np.pi
 
 
 @pytest.mark.parametrize("shape,ppc,sigma", [((8, 8, 8), 1, 0.02), ((9, 16, 17), 3, 0.5), ((24, 17, 16), 40, 0.02),
-                                             ((24, 17, 16), 40, 3.0)])
+                                             ((24, 17, 16), 40, 3.0), ((41, 48, 40), 3, 0.3)])
 def test_crossings_match_oracle(shape, ppc, sigma):
     rec, ids = oracle.synth_plasma(*shape, ppc, 0.02, sigma, 7)
     rec = rec.astype(np.float32).astype(np.float64)
