@@ -1394,6 +1394,14 @@ int download_particles(qk_ctx *c, const SpeciesBuf &b, const std::vector<int> &o
     return QK_OK;
 }
 
+// node charge of species b into rho[3 node + slot]
+template <typename real>
+hipError_t rho_species(qk_ctx *c, const SpeciesBuf &b, double *rho, int slot)
+{
+    return launch_compute_rho<real>(c->stream, c->g, view<real>(b.buf[b.cur]), b.n, rho, slot, c->tg, b.chunks, b.nchunks,
+                                    b.ishift, b.n_sorted);
+}
+
 // n doubles from device memory
 int download_doubles(qk_ctx *c, double *dst, const double *src, int64_t n)
 {
@@ -1798,8 +1806,8 @@ int qk_compute_rho(qk_ctx *c, double *rho)
     for (int t = 0; t < 3 && e == hipSuccess; ++t) {
         SpeciesBuf &b = c->sp[slots[t]];
         if (!b.active || b.n == 0) continue;
-        e = c->rsize == 4 ? launch_compute_rho<float>(c->stream, c->g, view<float>(b.buf[b.cur]), b.n, d, t)
-                          : launch_compute_rho<double>(c->stream, c->g, view<double>(b.buf[b.cur]), b.n, d, t);
+        e = c->rsize == 4 ? rho_species<float>(c, b, d, t)
+                          : rho_species<double>(c, b, d, t);
     }
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     const int rc = e == hipSuccess ? download_doubles(c, rho, d, 3 * (int64_t)c->g.ncell) : QK_OK;
@@ -1828,8 +1836,8 @@ int qk_compute_rho_noalloc(qk_ctx *c, double *rho)
     for (int t = 0; t < 3; ++t) {
         SpeciesBuf &b = c->sp[slots[t]];
         if (!b.active || b.n == 0) continue;
-        HIP_TRY(c->rsize == 4 ? launch_compute_rho<float>(c->stream, c->g, view<float>(b.buf[b.cur]), b.n, d, t)
-                              : launch_compute_rho<double>(c->stream, c->g, view<double>(b.buf[b.cur]), b.n, d, t));
+        HIP_TRY(c->rsize == 4 ? rho_species<float>(c, b, d, t)
+                              : rho_species<double>(c, b, d, t));
     }
     HIP_TRY(hipMemcpyAsync(rho, d, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));

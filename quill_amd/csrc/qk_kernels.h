@@ -268,8 +268,11 @@ hipError_t launch_inject(hipStream_t st, int solver, const Grid &g, const Solver
 template <typename real>
 hipError_t launch_load_uniform(hipStream_t st, const Grid &g, const Species<real> &s, int64_t first, int ppc,
                                double q, double sigma, uint64_t seed, int ilo, int ihi);
+// rho[3 node + slot] += node charge of slots [0, n); the first n_sorted of them
+// through the chunks of their last sort (as in PushArgs), nchunks = 0 for none
 template <typename real>
-hipError_t launch_compute_rho(hipStream_t st, const Grid &g, const Species<real> &s, int64_t n, double *rho, int slot);
+hipError_t launch_compute_rho(hipStream_t st, const Grid &g, const Species<real> &s, int64_t n, double *rho, int slot,
+                              const TileGeom &tg, const int4 *chunks, int nchunks, int ishift, int64_t n_sorted);
 
 // ---- results for the host (into pinned memory) ------------------------------
 
