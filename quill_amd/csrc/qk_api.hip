@@ -904,8 +904,14 @@ int adjoint_impl(qk_ctx *c, const double *lam_E, const double *lam_B, const doub
                 a.kind = 0;
                 a.cmr = c->sp[s].cmr;
                 a.external_bz = c->p.external_bz;
+                // the sort of qk_tape_begin, where there was one
+                const SpeciesBuf &b = c->sp[s];
+                a.chunks = b.chunks;
+                a.nchunks = b.nchunks;
+                a.ishift = b.ishift;
+                a.first = b.n_sorted;
                 HIP_TRY(launch_adj_particles<real>(c->stream, c->g, f, saved_species<real>(c, st, s), t.n[s], a, lam,
-                                                   lpart[s]));
+                                                   lpart[s], c->tg));
             }
         }
     }

@@ -174,10 +174,12 @@ hipError_t launch_tlm_particles(hipStream_t st, const Grid &g, const Fields<real
                                 double *const tpart[7]);
 // the adjoint of one species' push from its recorded state s and fields f
 // (E, Be) of the step: lpart = lx[3], lu[3], lq (FP64, per slot) go from after
-// the step to before it; lE and lBe receive the gather's node adjoints
+// the step to before it; lE and lBe receive the gather's node adjoints.  The
+// slots below a.first through the chunks of their last sort (a.nchunks > 0).
 template <typename real>
 hipError_t launch_adj_particles(hipStream_t st, const Grid &g, const Fields<real> &f, const Species<real> &s,
-                                int64_t n, const PushArgs &a, double *const lam[12], double *const lpart[7]);
+                                int64_t n, const PushArgs &a, double *const lam[12], double *const lpart[7],
+                                const TileGeom &tg);
 
 // rows of 7 doubles (x y z ux uy uz q) of rows [r0, r1) to the 7 arrays out,
 // and from them; id: the row of each slot (null: the slot), with which the
