@@ -147,6 +147,7 @@ struct qk_ctx {
     void *fmem = nullptr;           // all field arrays
     void *mid = nullptr;            // B at the step's end while the grid's B is half a step ahead (three arrays)
     bool no_mid = false;            // the memory for it is not there
+    bool b_ahead = false, b_held = false;   // the grid's B is half a step ahead; and mid holds the step's
     void *F[15] = {};               // ex ey ez bx by bz bex bey bez j0x j0y j0z j1x j1y j1z
     int jcur = 0;                   // current buffer deposited this step
     bool j_zero[2] = {true, true};  // which current buffers are known to be zero
@@ -1026,8 +1027,28 @@ int inject_impl(qk_ctx *c, int b_field, double frac, real *const *mid = nullptr,
     return QK_OK;
 }
 
+// The fields at the end of the last finished step, where a call failed with B
+// half a step ahead (step_all): B from mid, Be from that B.  Errors are not
+// reported, the caller has one.
 template <typename real>
-int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
+void settle_b(qk_ctx *c)
+{
+    c->b_ahead = false;
+    if (!c->b_held) return;   // neither particles nor sources: only the GPU itself can have failed
+    const size_t fb = ((size_t)c->g.ncell * sizeof(real) + 255) & ~(size_t)255;
+    WordCopies w{};
+    for (; w.count < 3; ++w.count) {
+        w.src[w.count] = (const uint32_t *)((char *)c->mid + w.count * fb);
+        w.dst[w.count] = (uint32_t *)c->F[3 + w.count];
+        w.n[w.count] = (int64_t)((size_t)c->g.ncell * sizeof(real) / 4);
+    }
+    (void)launch_copy_words(c->stream, w);
+    (void)launch_interpolate_be<real>(c->stream, c->g, fields_of<real>(c));
+    (void)hipStreamSynchronize(c->stream);
+}
+
+template <typename real>
+int step_all(qk_ctx *c, int nsteps, qk_diag *diag)
 {
     const Fields<real> f = fields_of<real>(c);
     // three events per step: before the particle phase (see `start`), between phases, after the field phase
@@ -1049,13 +1070,18 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
     // us at 256x128x128 and 29.6 -> 22.5 us at 128x64x64 in calls of four
     // steps; 64x32x32 with a laser source, 73 -> 60 us per step).  The B
     // between the two, at the step's end, is what Be, the laser sources'
-    // corrections and the field energy want: it is kept in `mid`.  Without
-    // charged particles nothing reads Be between two steps, and without a
-    // laser source nothing needs mid either (photons fly straight).  The tape
-    // keeps the state of every step, so there each half step runs by itself.
-    bool charged = qed || tp.active;
-    for (const SpeciesBuf &b : c->sp) charged = charged || (b.active && b.n > 0 && b.kind == 0);
-    const bool need_mid = charged || c->inj[0].nsrc > 0 || c->inj[1].nsrc > 0;
+    // corrections and the field energy want: it is kept in `mid`.  A call that
+    // fails on its way gets it back from there (settle_b): with particles a
+    // later step may find no room for its appends or its sort.  Without
+    // charged particles nothing reads Be between two steps, and without any
+    // particles and laser sources nothing needs mid either.  The tape keeps the
+    // state of every step, so there each half step runs by itself.
+    bool charged = qed || tp.active, any = charged;
+    for (const SpeciesBuf &b : c->sp) {
+        any = any || (b.active && b.n > 0);
+        charged = charged || (b.active && b.n > 0 && b.kind == 0);
+    }
+    const bool need_mid = any || c->inj[0].nsrc > 0 || c->inj[1].nsrc > 0;
     bool fuse_b = !tp.active;
     real *mid_b[3] = {};
     if (fuse_b && need_mid && nsteps > 1) {
@@ -1181,18 +1207,21 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
         // fields before fadvance (src/main.cpp:2327)
         if (charged) c->j_zero[c->jcur] = false;
         const bool no_j = !charged && c->j_zero[0] && c->j_zero[1], last = l + 1 == nsteps;
-        if (!fuse_b || l == 0) {
+        if (!c->b_ahead) {
             HIP_TRY(launch_maxwell_b<real>(c->stream, c->p.solver, c->g, c->coef, f, c->diag_row + kRowEnergy));
             QK_TRY(inject_impl<real>(c, 1, 0.0));
         }
         const DiagDrain dd{c->diag_row, hd + (size_t)l * kDiagLen, (int)kSpeciesLen, (int)(kDiagLen - kSpeciesLen)};
         HIP_TRY(launch_maxwell_e<real>(c->stream, c->p.solver, c->g, c->coef, f, no_j ? nullptr : &jc,
                                        no_j ? nullptr : &jn, dd));
+        c->b_ahead = false;   // E has caught up
         c->j_zero[c->jcur ^ 1] = true;
         QK_TRY(inject_impl<real>(c, 0, 0.5));
         if (fuse_b && !last) {
             double *next_en = c->d_diag + ((l + 1) & 1) * kDiagRow + kRowEnergy;
             HIP_TRY(launch_maxwell_b<real>(c->stream, c->p.solver, c->g, c->coef, f, next_en, true, mid));
+            c->b_ahead = true;
+            c->b_held = mid != nullptr;
             if (mid) QK_TRY(inject_impl<real>(c, 1, 1.0, mid, next_en));
         } else {
             HIP_TRY(launch_maxwell_b<real>(c->stream, c->p.solver, c->g, c->coef, f, nullptr));
@@ -1257,6 +1286,14 @@ int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
     c->have_step = true;
     c->diag_clear = true;
     return QK_OK;
+}
+
+template <typename real>
+int step_impl(qk_ctx *c, int nsteps, qk_diag *diag)
+{
+    const int rc = step_all<real>(c, nsteps, diag);
+    if (c->b_ahead) settle_b<real>(c);
+    return rc;
 }
 
 template <typename T>
