@@ -164,8 +164,8 @@ struct qk_ctx {
     size_t h_diag_cap = 0;          // steps that fit in h_diag
     std::vector<hipEvent_t> ev;     // timing events
     double ms_total = 0, ms_part = 0, ms_field = 0, fallback_frac = 0;
-    // QED: device slot counters of every species plus an overflow flag, and
-    // their pinned host mirror; the global step index keys the random streams
+    // QED: device slot counters of every species plus an overflow flag and the
+    // word that lets the push go ahead, and their pinned host mirror; the global step index keys the random streams
     int *d_count = nullptr;
     int *h_count = nullptr;         // pinned: values on their way to d_count
     int dev_n[QK_MAX_SPECIES];      // what d_count holds as far as the host knows (-1: unknown)
@@ -556,10 +556,10 @@ int qed_upload_counts(qk_ctx *c)
 // for them.  The GPU stores them and the host polls: the host has the counts
 // while the GPU works on what was enqueued behind them, where a copy and a
 // stream synchronization emptied the queue twice per step.
-int qed_publish(qk_ctx *c, int which, const double *diag)
+int qed_publish(qk_ctx *c, int which, const double *diag, const BornLimit &lim = BornLimit())
 {
     HIP_TRY(launch_publish_counts(c->stream, c->d_count, QK_MAX_SPECIES + 1, diag, QK_MAX_SPECIES, c->h_qed + which,
-                                  ++c->qed_seq));
+                                  ++c->qed_seq, lim));
     return QK_OK;
 }
 
@@ -587,11 +587,13 @@ bool fits(const qk_ctx *c, int s, int64_t extra)
 // The particle phase with QED on (src/main.cpp:2323-2324): birth_from_vacuum,
 // then padvance with photon emission for leptons and pair creation for
 // photons.  Capacity is reserved for the worst case (every cell bears a pair,
-// every lepton emits, every photon converts) so that no append can fail.  The
+// every lepton emits, every photon converts) before the first push, so that no
+// append can fail and a step that finds no room has moved nothing.  The
 // particles that were there are pushed while the host waits for the number of
 // pairs born from vacuum, which follow in a launch of their own (mostly none
-// are); where there is no room for both worst cases at once, the host waits
-// first and reserves for what was born.
+// are).  Where there is no room for both worst cases at once, or more are born
+// than the free photon slots can take the photons of (the kernel then returns
+// at once), the host waits first and reserves for what was born.
 template <typename real>
 int qed_particle_phase(qk_ctx *c, const Fields<real> &f, const Current<real> &jc)
 {
@@ -622,7 +624,7 @@ int qed_particle_phase(qk_ctx *c, const Fields<real> &f, const Current<real> &jc
         return a;
     };
     // electrons, positrons and photons from their slot `first` on
-    auto push = [&](const int64_t (&first)[3], const int64_t (&n)[3]) -> int {
+    auto push = [&](const int64_t (&first)[3], const int64_t (&n)[3], const int *go = nullptr) -> int {
         const int sp[3] = {QK_ELECTRON, QK_POSITRON, QK_PHOTON};
         Species<real> s[3];
         PushArgs a[3];
@@ -631,15 +633,15 @@ int qed_particle_phase(qk_ctx *c, const Fields<real> &f, const Current<real> &jc
             a[m] = push_args(sp[m], first[m], n[m]);
         }
         HIP_TRY(launch_qed_particles<real>(c->stream, c->g, f, jc, s, a, qa, target(QK_ELECTRON), target(QK_POSITRON),
-                                           target(QK_PHOTON)));
+                                           target(QK_PHOTON), go));
         return QK_OK;
     };
     const int64_t ninner = std::max<int64_t>(0, (int64_t)(c->p.nx - 4) * (c->p.ny - 4) * (c->p.nz - 4));
     const int64_t ne = be.n, np = bp.n, nph = bph.n;   // photons emitted in this step are not visited
-    const bool ahead = ninner > 0 && fits(c, QK_ELECTRON, ninner + nph) && fits(c, QK_POSITRON, ninner + nph) &&
-                       fits(c, QK_PHOTON, ne + np) && ensure_species(c, QK_ELECTRON, ninner + nph) == QK_OK &&
-                       ensure_species(c, QK_POSITRON, ninner + nph) == QK_OK &&
-                       ensure_species(c, QK_PHOTON, ne + np) == QK_OK;
+    bool ahead = ninner > 0 && fits(c, QK_ELECTRON, ninner + nph) && fits(c, QK_POSITRON, ninner + nph) &&
+                 fits(c, QK_PHOTON, ne + np) && ensure_species(c, QK_ELECTRON, ninner + nph) == QK_OK &&
+                 ensure_species(c, QK_POSITRON, ninner + nph) == QK_OK &&
+                 ensure_species(c, QK_PHOTON, ne + np) == QK_OK;
     if (!ahead) (void)hipGetLastError();
     if (ninner > 0) {
         QK_TRY(ensure_species(c, QK_ELECTRON, ninner));
@@ -647,10 +649,12 @@ int qed_particle_phase(qk_ctx *c, const Fields<real> &f, const Current<real> &jc
         QK_TRY(qed_upload_counts(c));
         HIP_TRY(launch_vacuum_pairs<real>(c->stream, c->g, f, c->p.pusher, c->p.q_vac, qa, target(QK_ELECTRON),
                                           target(QK_POSITRON)));
-        QK_TRY(qed_publish(c, 0, nullptr));
-        const unsigned seq = c->qed_seq;
-        if (ahead) QK_TRY(push({0, 0, 0}, {ne, np, nph}));
-        QK_TRY(qed_wait(c, 0, seq));
+        const int64_t room = bph.cap - nph;   // leptons that may emit
+        int *go = ahead ? c->d_count + QK_MAX_SPECIES + 1 : nullptr;
+        QK_TRY(qed_publish(c, 0, nullptr, {go, QK_ELECTRON, QK_POSITRON, room}));
+        if (ahead) QK_TRY(push({0, 0, 0}, {ne, np, nph}, go));
+        QK_TRY(qed_wait(c, 0, c->qed_seq));
+        ahead = ahead && be.n + bp.n <= room;
     }
     const int64_t born_e = be.n - ne, born_p = bp.n - np;
     if (!ahead) {
@@ -660,10 +664,6 @@ int qed_particle_phase(qk_ctx *c, const Fields<real> &f, const Current<real> &jc
         QK_TRY(qed_upload_counts(c));
         QK_TRY(push({0, 0, 0}, {be.n, bp.n, nph}));
     } else if (born_e > 0 || born_p > 0) {
-        // the buffers may move: the counts after the launch above come first
-        QK_TRY(qed_publish(c, 0, nullptr));
-        QK_TRY(qed_wait(c, 0, c->qed_seq));
-        QK_TRY(ensure_species(c, QK_PHOTON, born_e + born_p));
         QK_TRY(push({ne, np, 0}, {born_e, born_p, 0}));
     }
     for (int s = 0; s < QK_MAX_SPECIES; ++s) {
@@ -1562,7 +1562,7 @@ int qk_create(const qk_params *params, qk_ctx **out)
     if ((e = hipMalloc(&c->d_diag, 2 * kDiagRow * sizeof(double))) != hipSuccess)
         return bail(fail(QK_ERR_HIP, hipGetErrorString(e)));
     if (p.qed) {
-        if ((e = hipMalloc(&c->d_count, (QK_MAX_SPECIES + 1) * sizeof(int))) != hipSuccess ||
+        if ((e = hipMalloc(&c->d_count, (QK_MAX_SPECIES + 2) * sizeof(int))) != hipSuccess ||
             (e = hipHostMalloc((void **)&c->h_count, (QK_MAX_SPECIES + 1) * sizeof(int))) != hipSuccess ||
             (e = hipHostMalloc((void **)&c->h_qed, 2 * sizeof(QedCounts))) != hipSuccess)
             return bail(fail(QK_ERR_HIP, hipGetErrorString(e)));

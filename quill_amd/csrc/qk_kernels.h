@@ -90,12 +90,13 @@ struct AppendTarget {
 // electrons and positrons with photon emission (src/advance.cpp:253-359) and
 // photons with Breit-Wheeler pair creation (src/advance.cpp:155-252), slots
 // [first, first + n) of each, in one launch; every current contribution a
-// global atomic; emitted photons go to ph, pairs to el / po
+// global atomic; emitted photons go to ph, pairs to el / po.  With go, nothing
+// where that device word is zero (BornLimit)
 template <typename real>
 hipError_t launch_qed_particles(hipStream_t st, const Grid &g, const Fields<real> &f, const Current<real> &j,
                                 const Species<real> (&s)[3], const PushArgs (&a)[3], const QedArgs &q,
                                 const AppendTarget<real> &el, const AppendTarget<real> &po,
-                                const AppendTarget<real> &ph);
+                                const AppendTarget<real> &ph, const int *go);
 // slot counters and live counts in pinned host memory, valid once flag holds
 // the sequence number of their launch
 struct QedCounts {
@@ -104,10 +105,16 @@ struct QedCounts {
     double live[kMost];
     unsigned flag;
 };
+// *go (device) = whether the counters a and b stand at `most` or less together
+struct BornLimit {
+    int *go = nullptr;
+    int a = 0, b = 0;
+    int64_t most = 0;
+};
 // the n slot counters and, with diag (a step's accumulators), the live counts
 // of nsp species to *out
 hipError_t launch_publish_counts(hipStream_t st, const int *count, int n, const double *diag, int nsp, QedCounts *out,
-                                 unsigned seq);
+                                 unsigned seq, const BornLimit &lim);
 // birth_from_vacuum (src/mc.cpp:142-196): one draw per cell 2 .. n-3
 template <typename real>
 hipError_t launch_vacuum_pairs(hipStream_t st, const Grid &g, const Fields<real> &f, int pusher, double q_vac,

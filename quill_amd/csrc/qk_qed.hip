@@ -293,8 +293,9 @@ template <typename real, int PUSHER>
 __global__ void __launch_bounds__(kBlock) k_qed_particles(Grid g, Fields<real> f, Current<real> cur,
                                                           QedParts<real> a, real e_s, QedArgs qa,
                                                           AppendTarget<real> el, AppendTarget<real> po,
-                                                          AppendTarget<real> ph)
+                                                          AppendTarget<real> ph, const int *go)
 {
+    if (go && *go == 0) return;
     int b = blockIdx.x;
     for (int m = 0; m < 2; ++m) {   // uniform over the workgroup
         if (b < a.blocks[m]) {
@@ -311,11 +312,12 @@ __global__ void __launch_bounds__(kBlock) k_qed_particles(Grid g, Fields<real> f
 // the slot counters, and the live counts that the step's pushes have summed
 // over the copies of the diagnostics, to pinned host memory; then the flag
 __global__ void __launch_bounds__(64) k_publish_counts(const int *count, int n, const double *diag, int nsp,
-                                                       QedCounts *out, unsigned seq)
+                                                       QedCounts *out, unsigned seq, BornLimit lim)
 {
     static_assert(kDiagSlots == 64, "a lane per copy");
     const int t = threadIdx.x;
     if (t < n) out->n[t] = count[t];
+    if (t == 0 && lim.go) *lim.go = (int64_t)count[lim.a] + count[lim.b] <= lim.most;
     for (int s = 0; s < nsp && diag; ++s) {
         const double v = wave_sum(diag[t * kDiagStride + s * kDiagPerSpecies + 2]);
         if (t == 0) out->live[s] = v;
@@ -358,7 +360,7 @@ template <typename real>
 hipError_t launch_qed_particles(hipStream_t st, const Grid &g, const Fields<real> &f, const Current<real> &j,
                                 const Species<real> (&s)[3], const PushArgs (&a)[3], const QedArgs &q,
                                 const AppendTarget<real> &el, const AppendTarget<real> &po,
-                                const AppendTarget<real> &ph)
+                                const AppendTarget<real> &ph, const int *go)
 {
     QedParts<real> p{};
     int64_t total = 0;
@@ -373,17 +375,17 @@ hipError_t launch_qed_particles(hipStream_t st, const Grid &g, const Fields<real
     }
     if (total == 0) return hipSuccess;
     if (a[0].pusher == 1)
-        k_qed_particles<real, 1><<<(unsigned)total, kBlock, 0, st>>>(g, f, j, p, (real)q.e_s, q, el, po, ph);
+        k_qed_particles<real, 1><<<(unsigned)total, kBlock, 0, st>>>(g, f, j, p, (real)q.e_s, q, el, po, ph, go);
     else
-        k_qed_particles<real, 0><<<(unsigned)total, kBlock, 0, st>>>(g, f, j, p, (real)q.e_s, q, el, po, ph);
+        k_qed_particles<real, 0><<<(unsigned)total, kBlock, 0, st>>>(g, f, j, p, (real)q.e_s, q, el, po, ph, go);
     return hipGetLastError();
 }
 
 hipError_t launch_publish_counts(hipStream_t st, const int *count, int n, const double *diag, int nsp, QedCounts *out,
-                                 unsigned seq)
+                                 unsigned seq, const BornLimit &lim)
 {
     if (n > QedCounts::kMost || nsp > QedCounts::kMost) return hipErrorInvalidValue;
-    k_publish_counts<<<1, 64, 0, st>>>(count, n, diag, nsp, out, seq);
+    k_publish_counts<<<1, 64, 0, st>>>(count, n, diag, nsp, out, seq, lim);
     return hipGetLastError();
 }
 
@@ -405,7 +407,7 @@ hipError_t launch_vacuum_pairs(hipStream_t st, const Grid &g, const Fields<real>
                                                    const Current<real> &, const Species<real> (&)[3],          \
                                                    const PushArgs (&)[3], const QedArgs &,                     \
                                                    const AppendTarget<real> &, const AppendTarget<real> &,     \
-                                                   const AppendTarget<real> &);                                \
+                                                   const AppendTarget<real> &, const int *);                   \
     template hipError_t launch_vacuum_pairs<real>(hipStream_t, const Grid &, const Fields<real> &, int, double, \
                                                   const QedArgs &, const AppendTarget<real> &,                 \
                                                   const AppendTarget<real> &);

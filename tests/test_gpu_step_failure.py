@@ -46,3 +46,50 @@ def test_fields_after_a_failed_call(solver, source, precision):
     tol = 4 * np.finfo(np.float32 if precision == "fp32" else np.float64).eps
     for k in (0, 1, 3):
         assert np.abs(got[0][k] - got[1][k]).max() <= tol * np.abs(got[1][k]).max()
+
+
+def _vacuum(capacity):
+    """400 electrons at rest, and a pair from vacuum in each of 1728 cells
+    (rate x volume x dt = 4e7 at E = E_s)."""
+    n, ne = 16, 400
+    r = qa.Region(n, n, n, DX, DX, DX, 0.25 * DX, solver="five_point", pusher="vay", precision="fp64", qed=True,
+                  e_s=2000.0, q_vac=1e-9, seed=5, capacity=capacity)
+    E = np.zeros((n, n, n, 3))
+    E[..., 0] = 2000.0
+    r.set_fields(E, np.zeros_like(E))
+    pos = np.random.default_rng(6).uniform(5, 9, (3, ne))
+    r.add_particles(qa.ELECTRON, *pos, *np.zeros((3, ne)), np.full(ne, -1e-9))
+    r.init_boundaries()
+    return r
+
+
+def test_step_without_room_moves_nothing():
+    """The slots hold the photons of the electrons that were there (400), not
+    those of the pairs born as well (3856 leptons)."""
+    print("step failure, born pairs", flush=True)
+    with _vacuum(3000) as r:
+        before, fields = r.particles(qa.ELECTRON)[0], r.get_fields()
+        with pytest.raises(qa.QuillError, match="capacity"):
+            r.step(1)
+        assert (r.particles(qa.ELECTRON)[0][:len(before)] == before).all()
+        assert r.count(qa.PHOTON) == 0
+        for a, b in zip(r.get_fields(), fields):
+            assert (a == b).all()
+
+
+# slots for every photon before the pairs are counted (8000), and only after
+@pytest.mark.parametrize("capacity", [8000, 0])
+def test_every_lepton_is_pushed_once(capacity):
+    print(f"born pairs {capacity}", flush=True)
+    with _vacuum(capacity) as r:
+        d = r.step(1, diag=True)[0]
+        ue, up = (r.particles(s)[0][:, 3:6] for s in (qa.ELECTRON, qa.POSITRON))
+    assert d["n_e"] == len(ue) == 2128 and d["n_p"] == len(up) == 1728
+    dt = 0.25 * DX
+    # from rest, or born with half a step of the opposite sign; those that
+    # emitted a photon recoiled
+    recoiled = 0
+    for u, want in ((ue[:400], -1.0), (ue[400:], -0.5), (up, 0.5)):
+        recoiled += (~np.isclose(u[:, 0], want * 2000.0 * dt, rtol=1e-9, atol=0)).sum()
+        assert np.abs(u[:, 1:]).max() == 0
+    assert recoiled == d["n_ph"] < 2128
