@@ -140,7 +140,7 @@ int qk_particle_count(qk_ctx *ctx, int species, int64_t *n);
 int qk_get_particles(qk_ctx *ctx, int species, int64_t cap, double *rec10, int32_t *ids, int64_t *n_out);
 /* The state x y z ux uy uz q of the live particles by id (track_ids): row id of
  * rows (n x 7 doubles) and live[id] = 1; the rows of ids that no live particle
- * has are zero.  Every id must lie in 0 .. n - 1. */
+ * has are zero.  Every id must lie in 0 .. n - 1 and be one particle's only. */
 int qk_get_rows_by_id(qk_ctx *ctx, int species, int64_t n, double *rows, int32_t *live);
 /* compute_rho (src/fout.cpp:7-39): node charge of electrons, positrons and
  * photons in the three slots of rho (AoS [nx][ny][nz][3]) */

@@ -282,7 +282,7 @@ class Region:
 
     def rows_by_id(self, species, n):
         """(rows[n, 7] = x y z ux uy uz q of the live particles by id, mask of
-        the ids that are live); needs track_ids and ids in 0 .. n - 1."""
+        the ids that are live); needs track_ids and distinct ids in 0 .. n - 1."""
         rows, live = np.zeros((n, 7)), np.zeros(n, np.int32)
         _check(load_library().qk_get_rows_by_id(self._h, species, n, _dp(rows), _ip(live)), "qk_get_rows_by_id")
         return rows, live != 0

@@ -547,7 +547,8 @@ __global__ void __launch_bounds__(kABlock) k_rows_out(RowArrays in, double *__re
 }
 
 // the state x y z ux uy uz q of the live slots to their rows (id) of [r0, r1),
-// with live[r - r0] = 1; *bad is set where an id lies outside [0, total)
+// with live[r - r0] = 1 (zero before); *bad is set where an id lies outside
+// [0, total) or two live slots share one
 template <typename real>
 __global__ void __launch_bounds__(kABlock) k_state_rows(Species<real> s, int64_t n, int64_t total, int64_t r0, int64_t r1,
                                                         double *__restrict__ rows, int *live, int *bad)
@@ -559,6 +560,10 @@ __global__ void __launch_bounds__(kABlock) k_state_rows(Species<real> s, int64_t
     const int64_t r = s.id[p];
     if (r < 0 || r >= total) *bad = 1;
     if (r < r0 || r >= r1) return;
+    if (atomicExch(live + (r - r0), 1) != 0) {
+        *bad = 1;
+        return;   // the row is the other slot's
+    }
     double *__restrict__ row = rows + 7 * (r - r0);
     row[0] = cell_i(c) + (double)s.ox[p];
     row[1] = cell_j(c) + (double)s.oy[p];
@@ -567,7 +572,6 @@ __global__ void __launch_bounds__(kABlock) k_state_rows(Species<real> s, int64_t
     row[4] = s.uy[p];
     row[5] = s.uz[p];
     row[6] = s.q[p];
-    live[r - r0] = 1;
 }
 
 // *bad is set unless id[0 .. n) is a permutation of 0 .. n - 1 (seen: n zeros)

@@ -1812,7 +1812,7 @@ int qk_get_rows_by_id(qk_ctx *c, int s, int64_t n, double *rows, int32_t *live)
         HIP_TRY(hipMemcpyAsync(live + r, l, (size_t)k * sizeof(int), hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(hipMemcpyAsync(&bad, l + per, sizeof(int), hipMemcpyDeviceToHost, c->stream));
         QK_TRY(download_doubles(c, rows + 7 * r, c->rows, 7 * k));
-        if (bad) return fail(QK_ERR_INVALID, "rows by id: an id lies outside 0 .. n - 1");
+        if (bad) return fail(QK_ERR_INVALID, "rows by id: an id lies outside 0 .. n - 1, or two particles share it");
     }
     return QK_OK;
 }

@@ -196,7 +196,8 @@ hipError_t launch_rows_in(hipStream_t st, double *const out[7], const double *ro
 hipError_t launch_rows_out(hipStream_t st, double *const in[7], double *rows, const int *id, int64_t n, int64_t r0,
                            int64_t r1);
 // rows [r0, r1) of the live slots' state by id (of `total` rows), live[r - r0]
-// set to one where there is one; *bad set at an id outside [0, total)
+// set from zero to one where there is one; *bad set at an id outside [0, total)
+// and at one that two live slots have
 template <typename real>
 hipError_t launch_state_rows(hipStream_t st, const Species<real> &s, int64_t n, int64_t total, int64_t r0, int64_t r1,
                              double *rows, int *live, int *bad);
