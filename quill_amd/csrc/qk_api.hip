@@ -782,7 +782,7 @@ void tape_free(qk_ctx *c)
 template <typename real>
 int step_impl(qk_ctx *c, int nsteps, qk_diag *diag);
 int download_fields(qk_ctx *c, int nf, double *const *aos, void *const (*comp)[3], size_t rsize);
-int download_doubles(qk_ctx *c, double *dst, const double *src, int64_t n);
+int download_doubles(qk_ctx *c, double *dst, const double *src, int64_t n, int64_t of = 0);
 
 // at least `bytes` at c->rows; callers move their rows in blocks of at most kRowBytes
 constexpr size_t kRowBytes = (size_t)64 << 20, kRow = 7 * sizeof(double);
@@ -939,7 +939,7 @@ int adjoint_impl(qk_ctx *c, const double *lam_E, const double *lam_B, const doub
         for (int64_t r = 0; r < n; r += row_per) {
             const int64_t k = std::min(row_per, n - r);
             HIP_TRY(launch_rows_out(c->stream, lpart[s], c->rows, row_id[s], n, r, r + k));
-            QK_TRY(download_doubles(c, grad_part[s] + 7 * r, c->rows, 7 * k));
+            QK_TRY(download_doubles(c, grad_part[s] + 7 * r, c->rows, 7 * k, 7 * n));
         }
     }
     QK_TRY(tape_load(c, t.fin));
@@ -1339,8 +1339,9 @@ void widen(size_t rsize, const void *src, int64_t n, double *dst)
 int download_fields(qk_ctx *c, int nf, double *const *aos, void *const (*comp)[3], size_t rsize)
 {
     const int64_t n = c->g.ncell;
-    const size_t node = 3 * rsize, total = (size_t)nf * n * node;
-    const int64_t per = (int64_t)(Drain::slot_bytes(total) / node);   // nodes per block
+    const size_t node = 3 * rsize;
+    const bool shared = c->drain.shares((size_t)nf * n * node, Drain::kFields);
+    const int64_t per = (int64_t)(Drain::slot_bytes(shared) / node);   // nodes per block
     const int64_t nb = (n + per - 1) / per;                            // blocks per field
     auto launch = [&](int64_t b, void *slot, const ReadDone &done) {
         void *const *s = comp[b / nb];
@@ -1355,7 +1356,7 @@ int download_fields(qk_ctx *c, int nf, double *const *aos, void *const (*comp)[3
         const int64_t first = b % nb * per;
         widen(rsize, slot, 3 * std::min(per, n - first), aos[b / nb] + 3 * first);
     };
-    HIP_TRY(c->drain.run(c->p.device, c->stream, total, nf * nb, launch, take));
+    HIP_TRY(c->drain.run(c->p.device, c->stream, shared, nf * nb, launch, take));
     return QK_OK;
 }
 
@@ -1397,8 +1398,9 @@ int download_particles(qk_ctx *c, const SpeciesBuf &b, const std::vector<int> &o
     const Species<real> v = view<real>(src);
     const int nreal = src.a[7] ? 8 : 7;
     const bool has_id = src.id != nullptr;
-    const size_t row = 4 + (size_t)nreal * sizeof(real) + (has_id ? 4 : 0), total = (size_t)offs.back() * row;
-    const int64_t per = (int64_t)(Drain::slot_bytes(total) / row) / kLiveRun * kLiveRun;   // slots per block
+    const size_t row = 4 + (size_t)nreal * sizeof(real) + (has_id ? 4 : 0);
+    const bool shared = c->drain.shares((size_t)offs.back() * row, Drain::kRecords);
+    const int64_t per = (int64_t)(Drain::slot_bytes(shared) / row) / kLiveRun * kLiveRun;   // slots per block
     const int64_t nb = (b.n + per - 1) / per;
     // a slot holds `per` rows: the reals first (aligned), then cells and ids
     auto reals = [&](void *slot) { return (real *)slot; };
@@ -1433,7 +1435,7 @@ int download_particles(qk_ctx *c, const SpeciesBuf &b, const std::vector<int> &o
             else std::fill(ids + at, ids + at + m1, 0);
         }
     };
-    HIP_TRY(c->drain.run(c->p.device, c->stream, total, nb, launch, take));
+    HIP_TRY(c->drain.run(c->p.device, c->stream, shared, nb, launch, take));
     return QK_OK;
 }
 
@@ -1445,17 +1447,17 @@ hipError_t rho_species(qk_ctx *c, const SpeciesBuf &b, double *rho, int slot)
                                     b.ishift, b.n_sorted);
 }
 
-// n doubles from device memory
-int download_doubles(qk_ctx *c, double *dst, const double *src, int64_t n)
+// n doubles from device memory, a part of a result of `of` (0: all of it)
+int download_doubles(qk_ctx *c, double *dst, const double *src, int64_t n, int64_t of)
 {
-    const size_t total = (size_t)n * sizeof(double);
-    const int64_t per = (int64_t)(Drain::slot_bytes(total) / sizeof(double));
+    const bool shared = (size_t)std::max(n, of) * sizeof(double) > Drain::kNumbers;
+    const int64_t per = (int64_t)(Drain::slot_bytes(shared) / sizeof(double));
     auto count = [&](int64_t b) { return (size_t)std::min(per, n - b * per); };
     auto launch = [&](int64_t b, void *slot, const ReadDone &done) {
         return launch_copy_out(c->stream, src + b * per, (int)count(b), (double *)slot, done);
     };
     auto take = [&](int64_t b, const void *slot) { std::memcpy(dst + b * per, slot, count(b) * sizeof(double)); };
-    HIP_TRY(c->drain.run(c->p.device, c->stream, total, (n + per - 1) / per, launch, take));
+    HIP_TRY(c->drain.run(c->p.device, c->stream, shared, (n + per - 1) / per, launch, take));
     return QK_OK;
 }
 
@@ -1811,7 +1813,7 @@ int qk_get_rows_by_id(qk_ctx *c, int s, int64_t n, double *rows, int32_t *live)
                                                               c->rows, l, l + per));
         HIP_TRY(hipMemcpyAsync(live + r, l, (size_t)k * sizeof(int), hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(hipMemcpyAsync(&bad, l + per, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        QK_TRY(download_doubles(c, rows + 7 * r, c->rows, 7 * k));
+        QK_TRY(download_doubles(c, rows + 7 * r, c->rows, 7 * k, 7 * n));
         if (bad) return fail(QK_ERR_INVALID, "rows by id: an id lies outside 0 .. n - 1, or two particles share it");
     }
     return QK_OK;

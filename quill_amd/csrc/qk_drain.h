@@ -96,19 +96,45 @@ public:
     // 64x32x32 cells.  It has one slot, a small one (pinned allocations up to
     // 1 MiB cost 20 us, larger ones 340 us or more, and a short run reads
     // once), and sleeps in the stream's synchronization instead of polling.
+    //
+    // The workers' slots, their threads and their page faults in arrays of a
+    // few MB cost a context's first shared read 2 ms, with the caller's pool
+    // spinning 4 ms.  So a context shares its reads from where it has read
+    // kFields bytes, or kRecords for records.  First reads, ms, into fresh
+    // pages and into pages that the allocator had kept (spinning in brackets):
+    //                   MB   alone       shared                     pageable copies
+    //     fields         9   2.4, 1.0    3.2 (3.9), 2.8 (2.3)        2.7,  1.4
+    //                   24   4.8, 3.2    3.7 (6.1), 4.1 (5.3)        5.9,  4.4
+    //                   30   5.8, 3.9    4.0 (6.2), 4.7 (6.1)        7.4,  7.7
+    //     records       12   3.0, 2.0    3.3 (4.3), 3.6 (3.2)        5.5,  2.6
+    //                   24   5.7, 5.4    3.9 (6.4), 3.8 (6.7)       10.4,  6.8
+    //     node charges  24   2.9, 1.8    3.8 (5.5), 2.4 (3.9)        2.2,  2.1
+    //                   44   4.9, 4.6    4.4 (4.1), 1.7 (7.2)        5.2,  5.1
+    // and later ones: fields of 24 MB alone 4.7, 3.0, shared 1.5 (3.2), 1.8
+    // (3.7), but charges of 24 MB with the pool spinning 2.8, 1.7 and 2.3, 2.8:
+    // these, and rows by id, which are numbers too, are shared from kNumbers on.
     static constexpr size_t kShare = (size_t)8 << 20, kAloneSlot = (size_t)960 << 10;
+    static constexpr size_t kFields = (size_t)28 << 20, kRecords = (size_t)12 << 20, kNumbers = (size_t)40 << 20;
 
-    static size_t slot_bytes(size_t total) { return total < kShare ? kAloneSlot : kSlot; }
+    // whether to share a read of `total` bytes (in the slots' format)
+    bool shares(size_t total, size_t from)
+    {
+        if (total < kShare) return false;
+        read_ += total;
+        return read_ > from;
+    }
 
-    // launch(block, slot, done) -> hipError_t; take(block, slot).  `total` is
-    // the size of the whole read in the slots' format; `device` is current in
-    // the calling thread.  On return the stream is idle.
+    static size_t slot_bytes(bool shared) { return shared ? kSlot : kAloneSlot; }
+
+    // launch(block, slot, done) -> hipError_t; take(block, slot), a block of at
+    // most slot_bytes(shared).  `device` is current in the calling thread.  On
+    // return the stream is idle.
     template <class Launch, class Take>
-    hipError_t run(int device, hipStream_t st, size_t total, int64_t nblocks, Launch &&launch, Take &&take)
+    hipError_t run(int device, hipStream_t st, bool shared, int64_t nblocks, Launch &&launch, Take &&take)
     {
         if (nblocks <= 0) return hipSuccess;
-        const size_t slot = slot_bytes(total);
-        if (total < kShare) {
+        const size_t slot = slot_bytes(shared);
+        if (!shared) {
             if (hipError_t e = reserve(st, slot)) return e;
             void *at = pin_ + kFlagBytes;
             for (int64_t b = 0; b < nblocks; ++b) {
@@ -248,6 +274,7 @@ private:
 
     char *pin_ = nullptr;   // flags, then the workers' slots
     size_t cap_ = 0;
+    size_t read_ = 0;       // bytes of the reads of kShare or more
     unsigned *arrived_ = nullptr;   // workgroups of each slot's launch that are done
     unsigned seq_[2 * kWorkers] = {};
     std::mutex mu_;
