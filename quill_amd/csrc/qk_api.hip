@@ -93,6 +93,7 @@ struct SpeciesBuf {
     int4 *chunks = nullptr; // tiled-kernel work list
     int max_chunks = 0;     // capacity of chunks
     int nchunks = 0;        // host copy after the last sort
+    bool cut = false;       // tiles were cut into smaller chunks than kChunk (chunk_size)
     int steps_since_sort = 0;
     double fb_last = -1;    // window-fallback fraction of the last finished step (-1: unknown or re-sorted since)
     int ishift = 0;         // moving-window shifts since the last sort
@@ -147,6 +148,8 @@ struct qk_ctx {
     void *fmem = nullptr;           // all field arrays
     void *mid = nullptr;            // B at the step's end while the grid's B is half a step ahead (three arrays)
     bool no_mid = false;            // the memory for it is not there
+    void *wide = nullptr;           // FP32: FP64 part of the current where tiles are cut (three arrays)
+    bool wide_clear = false;        // whether it is zero
     bool b_ahead = false, b_held = false;   // the grid's B is half a step ahead; and mid holds the step's
     void *F[15] = {};               // ex ey ez bx by bz bex bey bez j0x j0y j0z j1x j1y j1z
     int jcur = 0;                   // current buffer deposited this step
@@ -372,17 +375,20 @@ int ensure_sort_buffers(qk_ctx *c)
 // per CU; 1.3 covers the tiles at the box's faces, which hold less than the inner
 // ones.  A second workgroup per CU (FP32 only: two fit) pays for its own staging
 // and flush only where the parts stay above half of kChunk.  Particle phase at
-// 128 tiles, 8 per cell: 36.8 -> 26.5 us (33.9 with four parts per tile, 31.9
-// with 4096 per part), FP64 45.6 -> 30.3; 27 per cell: 57.0 -> 47.1 us (51.9 at
-// three parts, 62.5 at six); 27 tiles: 32.7 -> 15.4 us.
+// 128 tiles, 8 per cell: 35.3 -> 22.6 us (with other kernels of the time 36.8 ->
+// 26.5, 33.9 with four parts per tile, 31.9 with 4096 per part; FP64 45.6 -> 30.3);
+// 27 per cell: 57.0 -> 38.7 us (57.0 -> 47.1, 51.9 at three parts, 62.5 at six);
+// 27 tiles: 31.4 -> 15.1 us.
 //
 // From there to twice as many tiles as CUs: halves, where they fill the CUs
-// better and hold enough for their staging and flush: with 150 tiles 43.3 ->
-// 26.1 us, 250 43.0 -> 31.8, 432 61.0 -> 49.4, FP64 77.9 -> 75.1 (8 per cell);
+// better and hold enough for their staging and flush: with 150 tiles 39.9 ->
+// 26.3 us, 250 43.6 -> 32.2, 432 57.8 -> 50.3, FP64 77.9 -> 75.1 (8 per cell);
 // but 27.3 -> 31.8 with 432 tiles and 2 per cell (20.5 us either way with 250).  FP64 has one
 // workgroup per CU and gains only beyond one tile per CU.  With 576 tiles
 // halves take 65 us against 71 at 8 per cell and 40 against 34 at 2, with 750
 // tiles 78 against 76.
+//
+// Where FP32 tiles are cut, their currents are summed in FP64 (see k_push_tiled).
 int chunk_size(const qk_ctx *c, int64_t n)
 {
     constexpr int kCU = 256, kHalfMean = 2048;
@@ -398,6 +404,14 @@ int chunk_size(const qk_ctx *c, int64_t n)
         if (c->rsize == 4 && chunk > kChunk / 2) chunk = (chunk + 1) / 2;
     }
     return (int)std::min<int64_t>(std::max<int64_t>(chunk, kMinChunk), kChunk);
+}
+
+// the FP64 part of an FP32 region's current
+Current<double> wide_of(const qk_ctx *c)
+{
+    const size_t n = c->g.ncell;
+    double *w = (double *)c->wide;
+    return w ? Current<double>{w, w + n, w + 2 * n} : Current<double>{};
 }
 
 // sort species s by (tile, cell), compacting free slots; builds its work list
@@ -421,11 +435,18 @@ int sort_species(qk_ctx *c, int s)
     sb.scratch = c->s_scratch;
     sb.max_chunks = b.max_chunks;
     sb.chunk = chunk_size(c, b.n);
+    if (c->rsize == 4 && sb.chunk < kChunk && !c->wide &&
+        hipMalloc(&c->wide, 3 * (size_t)c->g.ncell * sizeof(double)) != hipSuccess) {
+        (void)hipGetLastError();   // the tiles stay whole
+        c->wide = nullptr;
+        sb.chunk = kChunk;
+    }
     sb.info = c->h_sortinfo;
     HIP_TRY(launch_sort<real>(c->stream, c->tg, view<real>(b.buf[b.cur]), view<real>(b.buf[b.cur ^ 1]), b.n, sb));
     HIP_TRY(hipStreamSynchronize(c->stream));
     std::swap(b.tile_start, c->s_tile_start);   // the next sort's source
     b.cur ^= 1;
+    b.cut = sb.chunk < kChunk;
     b.n = c->h_sortinfo[0];
     b.n_sorted = b.n;
     b.nchunks = c->h_sortinfo[1];
@@ -1165,6 +1186,7 @@ int step_all(qk_ctx *c, int nsteps, qk_diag *diag)
         Species<real> ts[kMaxTiled];
         PushArgs ta[kMaxTiled];
         int nt = 0;
+        bool cut = false;
         for (int s = 0; s < QK_MAX_SPECIES && !qed; ++s) {
             SpeciesBuf &b = c->sp[s];
             if (!b.active || b.n == 0) continue;
@@ -1191,6 +1213,7 @@ int step_all(qk_ctx *c, int nsteps, qk_diag *diag)
                 a.ishift = b.ishift;
                 ts[nt] = v;
                 ta[nt++] = a;
+                cut = cut || b.cut;
                 a.first = b.n_sorted;   // the unsorted tail, if any
                 a.n = b.n - b.n_sorted;
             } else {
@@ -1200,7 +1223,10 @@ int step_all(qk_ctx *c, int nsteps, qk_diag *diag)
             HIP_TRY(launch_push_global<real>(c->stream, c->g, f, jc, v, a));
             ++b.steps_since_sort;
         }
-        if (nt > 0) HIP_TRY(launch_push_tiled<real>(c->stream, c->g, f, jc, c->tg, nt, ts, ta));
+        const Current<double> wide = wide_of(c), *const w = cut && sizeof(real) == 4 ? &wide : nullptr;
+        if (w && !c->wide_clear) HIP_TRY(launch_zero(c->stream, (double *)c->wide, 3 * (size_t)c->g.ncell));
+        if (w) c->wide_clear = false;
+        if (nt > 0) HIP_TRY(launch_push_tiled<real>(c->stream, c->g, f, jc, c->tg, nt, ts, ta, w));
         HIP_TRY(hipEventRecord(c->ev[3 * l + 1], c->stream));
         // fadvance (src/advance.cpp:13-18): B half, E, B half, interpolate_be.  The
         // first half step also sums compute_energy's field term, which sees the
@@ -1213,7 +1239,8 @@ int step_all(qk_ctx *c, int nsteps, qk_diag *diag)
         }
         const DiagDrain dd{c->diag_row, hd + (size_t)l * kDiagLen, (int)kSpeciesLen, (int)(kDiagLen - kSpeciesLen)};
         HIP_TRY(launch_maxwell_e<real>(c->stream, c->p.solver, c->g, c->coef, f, no_j ? nullptr : &jc,
-                                       no_j ? nullptr : &jn, dd));
+                                       no_j ? nullptr : &jn, dd, w));
+        if (w) c->wide_clear = true;
         c->b_ahead = false;   // E has caught up
         c->j_zero[c->jcur ^ 1] = true;
         QK_TRY(inject_impl<real>(c, 0, 0.5));
@@ -1601,6 +1628,7 @@ int qk_destroy(qk_ctx *c)
     if (c->rows) note(hipFree(c->rows));
     if (c->fmem) note(hipFree(c->fmem));
     if (c->mid) note(hipFree(c->mid));
+    if (c->wide) note(hipFree(c->wide));
     if (c->d_diag) note(hipFree(c->d_diag));
     if (c->h_diag) note(hipHostFree(c->h_diag));
     if (c->d_count) note(hipFree(c->d_count));

@@ -246,21 +246,25 @@ __global__ void __launch_bounds__(kSweep) k_maxwell_b(Grid g, SweepPlan sw, Coef
     }
 }
 
+// the current an E step takes: none, the FP32 or FP64 buffer, or that and the
+// FP64 part next to it (k_push_tiled)
+enum { kNoCurrent, kPlain, kWide };
+
 // E step with the current of this step; also clears the other current
 // buffer, which the next step deposits into (replaces the J reset of
-// src/advance.cpp:112-123 without a separate pass).  CUR false: both current
+// src/advance.cpp:112-123 without a separate pass).  kNoCurrent: both current
 // buffers are known to be zero (no charged particles), 36 instead of 60 B per
 // cell (92 us instead of 200 at 301x203x199, the sweep order included).  The last workgroup also hands the step's diagnostics over, complete
 // by now: the accumulators go to pinned host memory and are cleared for the
 // step after next.
-template <int S, bool CUR, typename real>
+template <int S, int CUR, typename real>
 __global__ void __launch_bounds__(kSweep) k_maxwell_e(Grid g, SweepPlan sw, Coef<real> cf, real *__restrict__ ex,
                                                       real *__restrict__ ey, real *__restrict__ ez,
                                                       const real *__restrict__ bx, const real *__restrict__ by,
-                                                      const real *__restrict__ bz, const real *__restrict__ jx,
-                                                      const real *__restrict__ jy, const real *__restrict__ jz,
+                                                      const real *__restrict__ bz, real *__restrict__ jx,
+                                                      real *__restrict__ jy, real *__restrict__ jz,
                                                       real *__restrict__ njx, real *__restrict__ njy,
-                                                      real *__restrict__ njz, DiagDrain dd)
+                                                      real *__restrict__ njz, DiagDrain dd, Current<double> wide)
 {
     if (dd.n > 0 && blockIdx.x == gridDim.x - 1) {
         // eight threads per accumulator, each summing every eighth copy
@@ -286,15 +290,24 @@ __global__ void __launch_bounds__(kSweep) k_maxwell_e(Grid g, SweepPlan sw, Coef
     int i, j, k;
     if (!sweep_cell(g, sw, i, j, k)) return;
     const int id = i * g.sx + j * g.sy + k;
-    const real c0 = CUR ? jx[id] * cf.d[0] : real(0), c1 = CUR ? jy[id] * cf.d[1] : real(0),
-               c2 = CUR ? jz[id] * cf.d[2] : real(0);
+    auto current = [&](real *j, double *w) -> real {
+        if (CUR == kNoCurrent) return real(0);
+        real v = j[id];
+        if (CUR == kWide) {
+            v = (real)((double)v + w[id]);
+            w[id] = 0.0;
+            j[id] = v;   // read back as the step's J
+        }
+        return v;
+    };
+    const real c0 = current(jx, wide.jx) * cf.d[0], c1 = current(jy, wide.jy) * cf.d[1], c2 = current(jz, wide.jz) * cf.d[2];
     if (e_updates<S, 0>(g, i, j, k))
         ex[id] += cf.dtd[1] * diff<S, 2, 1, false>(g, cf, bz, i, j, k) - cf.dtd[2] * diff<S, 1, 2, false>(g, cf, by, i, j, k) - c0;
     if (e_updates<S, 1>(g, i, j, k))
         ey[id] += -cf.dtd[0] * diff<S, 2, 0, false>(g, cf, bz, i, j, k) + cf.dtd[2] * diff<S, 0, 2, false>(g, cf, bx, i, j, k) - c1;
     if (e_updates<S, 2>(g, i, j, k))
         ez[id] += cf.dtd[0] * diff<S, 1, 0, false>(g, cf, by, i, j, k) - cf.dtd[1] * diff<S, 0, 1, false>(g, cf, bx, i, j, k) - c2;
-    if (CUR) {
+    if (CUR != kNoCurrent) {
         njx[id] = real(0);
         njy[id] = real(0);
         njz[id] = real(0);
@@ -749,17 +762,31 @@ hipError_t launch_maxwell_b(hipStream_t st, int solver, const Grid &g, const Sol
 
 template <typename real>
 hipError_t launch_maxwell_e(hipStream_t st, int solver, const Grid &g, const SolverCoef &c, const Fields<real> &f,
-                            const Current<real> *j, const Current<real> *jn, const DiagDrain &dd)
+                            const Current<real> *j, const Current<real> *jn, const DiagDrain &dd,
+                            const Current<double> *wide)
 {
     const Coef<real> cf = make_coef<real>(g, c);
     const SweepPlan sw = sweep_plan(g);
     const dim3 grid((unsigned)(sw.per * g.nx));
     const Current<real> none{nullptr, nullptr, nullptr}, a = j ? *j : none, b = j ? *jn : none;
-#define QK_E(S, C) k_maxwell_e<S, C, real><<<grid, kSweep, 0, st>>>(g, sw, cf, f.ex, f.ey, f.ez, f.bx, f.by, f.bz, a.jx, \
-                                                                   a.jy, a.jz, b.jx, b.jy, b.jz, dd)
-    if (solver == 0) { if (j) QK_E(0, true); else QK_E(0, false); }
-    else if (solver == 1) { if (j) QK_E(1, true); else QK_E(1, false); }
-    else { if (j) QK_E(2, true); else QK_E(2, false); }
+    const Current<double> w = wide ? *wide : Current<double>{};
+    if (wide && (!j || sizeof(real) != 4)) return hipErrorInvalidValue;
+    auto launch = [&](auto kernel) {
+        kernel<<<grid, kSweep, 0, st>>>(g, sw, cf, f.ex, f.ey, f.ez, f.bx, f.by, f.bz, a.jx, a.jy, a.jz, b.jx, b.jy, b.jz,
+                                        dd, w);
+    };
+#define QK_E(C)                                              \
+    if (solver == 0) launch(k_maxwell_e<0, C, real>);        \
+    else if (solver == 1) launch(k_maxwell_e<1, C, real>);   \
+    else launch(k_maxwell_e<2, C, real>)
+    if constexpr (sizeof(real) == 4) {
+        if (wide) {
+            QK_E(kWide);
+            return hipGetLastError();
+        }
+    }
+    if (j) { QK_E(kPlain); }
+    else { QK_E(kNoCurrent); }
 #undef QK_E
     return hipGetLastError();
 }
@@ -874,7 +901,8 @@ hipError_t launch_inject(hipStream_t st, int solver, const Grid &g, const Solver
     template hipError_t launch_maxwell_b<real>(hipStream_t, int, const Grid &, const SolverCoef &, const Fields<real> &, \
                                                double *, bool, real *const *);                                  \
     template hipError_t launch_maxwell_e<real>(hipStream_t, int, const Grid &, const SolverCoef &, const Fields<real> &, \
-                                               const Current<real> *, const Current<real> *, const DiagDrain &); \
+                                               const Current<real> *, const Current<real> *, const DiagDrain &, \
+                                               const Current<double> *);                                        \
     template hipError_t launch_interpolate_be<real>(hipStream_t, const Grid &, const Fields<real> &, const real *const *); \
     template hipError_t launch_init_boundaries<real>(hipStream_t, int, const Grid &, const Fields<real> &);     \
     template hipError_t launch_laser_cos<real>(hipStream_t, const Grid &, const Fields<real> &, const double *); \

@@ -60,11 +60,13 @@ hipError_t launch_push_global(hipStream_t st, const Grid &g, const Fields<real> 
                               const Species<real> &s, const PushArgs &a);
 // one workgroup per chunk of a cell tile: the current is accumulated in an
 // LDS window around the tile and flushed to global memory once; the chunks
-// of all ns species (at most kMaxTiled, one pusher) in one launch
+// of all ns species (at most kMaxTiled, one pusher) in one launch.  With wide
+// (FP32) the windows go to these FP64 arrays instead of j
 constexpr int kMaxTiled = 6;
 template <typename real>
 hipError_t launch_push_tiled(hipStream_t st, const Grid &g, const Fields<real> &f, const Current<real> &j,
-                             const TileGeom &tg, int ns, const Species<real> *s, const PushArgs *a);
+                             const TileGeom &tg, int ns, const Species<real> *s, const PushArgs *a,
+                             const Current<double> *wide);
 
 // ---- QED -------------------------------------------------------------------
 
@@ -234,10 +236,12 @@ struct DiagDrain {
     int nspread = 0, n = 0;
 };
 // E step; j (may be null: both buffers are zero) the step's current, jn the
-// buffer to clear for the next
+// buffer to clear for the next.  With wide (FP32), that part of the current
+// is added to j first, and cleared
 template <typename real>
 hipError_t launch_maxwell_e(hipStream_t st, int solver, const Grid &g, const SolverCoef &c, const Fields<real> &f,
-                            const Current<real> *j, const Current<real> *jn, const DiagDrain &dd = DiagDrain());
+                            const Current<real> *j, const Current<real> *jn, const DiagDrain &dd = DiagDrain(),
+                            const Current<double> *wide = nullptr);
 // Be from B, or from the three arrays b
 template <typename real>
 hipError_t launch_interpolate_be(hipStream_t st, const Grid &g, const Fields<real> &f, const real *const *b = nullptr);

@@ -211,11 +211,12 @@ __device__ inline void store_component(EB<real> *dst, const real (&e)[kStageIt],
 // threadIdx.x + m kTBlock), read from LDS for all three components before the
 // first atomic; first is the window's first node.  A particle that deposits is
 // is_inside (1 .. n - 3) and crosses one face per axis at most, so the nodes it
-// reaches lie in the grid (0 .. n - 1) and entries outside it hold zero.
+// reaches lie in the grid (0 .. n - 1) and entries outside it hold zero.  T:
+// the precision of the sums over the workgroups.
 constexpr int kFlushIt = (jsize(0) + kTBlock - 1) / kTBlock;
 
-template <int C, typename real>
-__device__ inline void flush_component(real *__restrict__ dst, const double (&v)[kFlushIt], const Grid &g, int64_t first)
+template <int C, typename T>
+__device__ inline void flush_component(T *__restrict__ dst, const double (&v)[kFlushIt], const Grid &g, int64_t first)
 {
     static_assert(jsize(C) <= kFlushIt * kTBlock, "window block larger than the thread shares");
     constexpr int d1 = jdim(C, 1), d2 = jdim(C, 2), most = kFlushIt * kTBlock;
@@ -226,7 +227,7 @@ __device__ inline void flush_component(real *__restrict__ dst, const double (&v)
         const int wk = w - t * d2, wj = t - wi * d1;
         if (v[m] != 0.0) {   // zero past the block's end
             const int rel = (int)(__umul24((unsigned)wi, (unsigned)g.sx) + __umul24((unsigned)wj, (unsigned)g.sy)) + wk;
-            unsafeAtomicAdd(&node_after(dst + first, rel), (real)v[m]);
+            unsafeAtomicAdd(&node_after(dst + first, rel), (T)v[m]);
         }
     }
 }
@@ -284,9 +285,18 @@ struct TiledArgs {
     int ns;
 };
 
-template <typename real, int PUSHER>
-__global__ void __launch_bounds__(kTBlock) k_push_tiled(Grid g, Fields<real> f, Current<real> cur, TileGeom tg,
-                                                                TiledArgs<real> args)
+//
+// WIDE: the windows are added to FP64 arrays, which the E step takes along.
+// Where tiles are cut into several chunks (chunk_size), a node's current would
+// otherwise be the FP32 sum of so many more parts: its error against FP64 (rms
+// of one step's J at 56x32x32 with 8 per cell) was 7.86e-8, with whole tiles
+// 7.49e-8, and two runs differed by 2.3e-8 and 4.5e-9; now 7.33e-8, and two
+// runs give the same bits.  It costs 1 us in the push and 0 to 2 us in the E
+// step (40.5 us per step instead of 39.8 at 64x32x32, 76.2 instead of 74.2 at
+// 96x48x48).
+template <typename real, int PUSHER, bool WIDE>
+__global__ void __launch_bounds__(kTBlock) k_push_tiled(Grid g, Fields<real> f, Current<real> cur, Current<double> wide,
+                                                        TileGeom tg, TiledArgs<real> args)
 {
     __shared__ alignas(16) double win[kJWin];
     __shared__ EB<real> stage[kFStage];
@@ -498,9 +508,15 @@ __global__ void __launch_bounds__(kTBlock) k_push_tiled(Grid g, Fields<real> f, 
 #pragma unroll
             for (int c = 0; c < 3; ++c) v[c][m] = w < jsize(c) ? win[joff(c) + w] : 0.0;
         }
-        flush_component<0>(cur.jx, v[0], g, first);
-        flush_component<1>(cur.jy, v[1], g, first);
-        flush_component<2>(cur.jz, v[2], g, first);
+        if (WIDE) {
+            flush_component<0>(wide.jx, v[0], g, first);
+            flush_component<1>(wide.jy, v[1], g, first);
+            flush_component<2>(wide.jz, v[2], g, first);
+        } else {
+            flush_component<0>(cur.jx, v[0], g, first);
+            flush_component<1>(cur.jy, v[1], g, first);
+            flush_component<2>(cur.jz, v[2], g, first);
+        }
     }
     diag_accumulate(sp.diag, da.q, da.e, da.n, da.fallback);
 }
@@ -740,7 +756,8 @@ hipError_t launch_push_global(hipStream_t st, const Grid &g, const Fields<real> 
 
 template <typename real>
 hipError_t launch_push_tiled(hipStream_t st, const Grid &g, const Fields<real> &f, const Current<real> &j,
-                             const TileGeom &tg, int ns, const Species<real> *s, const PushArgs *a)
+                             const TileGeom &tg, int ns, const Species<real> *s, const PushArgs *a,
+                             const Current<double> *wide)
 {
     TiledArgs<real> args{};
     int total = 0;
@@ -756,8 +773,17 @@ hipError_t launch_push_tiled(hipStream_t st, const Grid &g, const Fields<real> &
         total += a[m].nchunks;
     }
     if (total == 0) return hipSuccess;
-    if (a[0].pusher == 1) k_push_tiled<real, 1><<<total, kTBlock, 0, st>>>(g, f, j, tg, args);
-    else k_push_tiled<real, 0><<<total, kTBlock, 0, st>>>(g, f, j, tg, args);
+    const Current<double> w = wide ? *wide : Current<double>{};
+    auto launch = [&](auto kernel) { kernel<<<total, kTBlock, 0, st>>>(g, f, j, w, tg, args); };
+    if constexpr (sizeof(real) == 4) {
+        if (wide) {
+            if (a[0].pusher == 1) launch(k_push_tiled<real, 1, true>);
+            else launch(k_push_tiled<real, 0, true>);
+            return hipGetLastError();
+        }
+    }
+    if (a[0].pusher == 1) launch(k_push_tiled<real, 1, false>);
+    else launch(k_push_tiled<real, 0, false>);
     return hipGetLastError();
 }
 
@@ -817,7 +843,7 @@ hipError_t launch_scale_charge(hipStream_t st, const Species<real> &s, int64_t n
                                                  const Current<real> &, const Species<real> &, const PushArgs &); \
     template hipError_t launch_push_tiled<real>(hipStream_t, const Grid &, const Fields<real> &,                \
                                                 const Current<real> &, const TileGeom &, int,                   \
-                                                const Species<real> *, const PushArgs *);                       \
+                                                const Species<real> *, const PushArgs *, const Current<double> *); \
     template hipError_t launch_load_uniform<real>(hipStream_t, const Grid &, const Species<real> &, int64_t, int, \
                                                   double, double, uint64_t, int, int);                           \
     template hipError_t launch_compute_rho<real>(hipStream_t, const Grid &, const Species<real> &, int64_t,       \
