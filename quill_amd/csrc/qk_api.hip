@@ -1096,14 +1096,16 @@ int step_all(qk_ctx *c, int nsteps, qk_diag *diag)
     // later step may find no room for its appends or its sort.  Without
     // charged particles nothing reads Be between two steps, and without any
     // particles and laser sources nothing needs mid either.  The tape keeps the
-    // state of every step, so there each half step runs by itself.
+    // state of every step, so there each half step runs by itself, and so it
+    // does where the sources of both sides correct the same nodes.
     bool charged = qed || tp.active, any = charged;
     for (const SpeciesBuf &b : c->sp) {
         any = any || (b.active && b.n > 0);
         charged = charged || (b.active && b.n > 0 && b.kind == 0);
     }
     const bool need_mid = any || c->inj[0].nsrc > 0 || c->inj[1].nsrc > 0;
-    bool fuse_b = !tp.active;
+    bool fuse_b = !tp.active && (c->inj[0].nsrc == 0 || c->inj[1].nsrc == 0 ||
+                                 sides_apart(c->inj[0].plane, c->inj[1].plane));
     real *mid_b[3] = {};
     if (fuse_b && need_mid && nsteps > 1) {
         const size_t fb = ((size_t)c->g.ncell * sizeof(real) + 255) & ~(size_t)255;

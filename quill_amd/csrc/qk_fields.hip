@@ -6,8 +6,6 @@
 // Fields are structure-of-arrays, one array per component, [nx][ny][nz] with
 // k fastest; a thread owns one cell and consecutive lanes walk k, so every
 // stencil load of a wavefront is a coalesced run.
-#include <cstdlib>
-
 #include "qk_kernels.h"
 
 namespace qk {
@@ -176,6 +174,16 @@ __device__ inline real diff(const Grid &g, const Coef<real> &cf, const real *__r
     }
 }
 
+// rate of component C of B at cell (i,j,k); a half step adds half of it
+template <int S, int C, typename real>
+__device__ inline real b_rate(const Grid &g, const Coef<real> &cf, const real *__restrict__ ex, const real *__restrict__ ey,
+                              const real *__restrict__ ez, int i, int j, int k)
+{
+    if (C == 0) return -cf.dtd[1] * diff<S, 2, 1, true>(g, cf, ez, i, j, k) + cf.dtd[2] * diff<S, 1, 2, true>(g, cf, ey, i, j, k);
+    if (C == 1) return cf.dtd[0] * diff<S, 2, 0, true>(g, cf, ez, i, j, k) - cf.dtd[2] * diff<S, 0, 2, true>(g, cf, ex, i, j, k);
+    return cf.dtd[1] * diff<S, 0, 1, true>(g, cf, ex, i, j, k) - cf.dtd[0] * diff<S, 1, 0, true>(g, cf, ey, i, j, k);
+}
+
 // B at the step's end, between two half steps taken together
 template <typename real>
 struct Mid {
@@ -212,9 +220,9 @@ __global__ void __launch_bounds__(kSweep) k_maxwell_b(Grid g, SweepPlan sw, Coef
         if (energy && !TWICE) add_energy();
         const bool u0 = b_updates<S, 0>(g, i, j, k), u1 = b_updates<S, 1>(g, i, j, k), u2 = b_updates<S, 2>(g, i, j, k);
         real d0 = real(0), d1 = real(0), d2 = real(0);
-        if (u0) d0 = -cf.dtd[1] * diff<S, 2, 1, true>(g, cf, ez, i, j, k) + cf.dtd[2] * diff<S, 1, 2, true>(g, cf, ey, i, j, k);
-        if (u1) d1 = cf.dtd[0] * diff<S, 2, 0, true>(g, cf, ez, i, j, k) - cf.dtd[2] * diff<S, 0, 2, true>(g, cf, ex, i, j, k);
-        if (u2) d2 = cf.dtd[1] * diff<S, 0, 1, true>(g, cf, ex, i, j, k) - cf.dtd[0] * diff<S, 1, 0, true>(g, cf, ey, i, j, k);
+        if (u0) d0 = b_rate<S, 0>(g, cf, ex, ey, ez, i, j, k);
+        if (u1) d1 = b_rate<S, 1>(g, cf, ex, ey, ez, i, j, k);
+        if (u2) d2 = b_rate<S, 2>(g, cf, ex, ey, ez, i, j, k);
         if (u0) b0 += h * d0;
         if (u1) b1 += h * d1;
         if (u2) b2 += h * d2;
@@ -606,9 +614,11 @@ struct InjectSides {
 };
 
 // TURN: the corrections of a half step of B and of the next step's first one
-// (the same incident field) where both were taken together: the grid's B takes
-// them twice, mid once, and the energy of the fields between the two changes
-// with mid.
+// (the same incident field) where both were taken together: mid takes them
+// once, and the grid's B becomes mid after the second half step and its
+// corrections, in the order of two half steps taken apart (corrected twice
+// after both, FP32 runs came out 1 % further from FP64).  The energy of the
+// fields between the two changes with mid.
 template <int S, bool BF, bool TURN, typename real>
 __global__ void __launch_bounds__(kBX * kBY) k_inject(Grid g, Coef<real> cf, Fields<real> f, InjectSides sides,
                                                       Mid<real> mid, double *energy)
@@ -678,19 +688,25 @@ __global__ void __launch_bounds__(kBX * kBY) k_inject(Grid g, Coef<real> cf, Fie
         const int id = i * g.sx + j * g.sy + k;
         if (BF) {
             const real h = real(0.5);
-            auto correct = [&](real *F, real *at_mid, real d) {
+            auto correct = [&](real *F, real *at_mid, real d, real rate) {
                 if (!tot) d = -d;
-                real v = F[id] + d;
                 if (TURN) {
-                    v += d;
                     const real o = at_mid[id], w = o + d;
                     at_mid[id] = w;
                     en += (double)w * w - (double)o * o;
+                    real v = w;
+                    v += h * rate;
+                    F[id] = v + d;
+                } else {
+                    F[id] += d;
                 }
-                F[id] = v;
             };
-            if (b_updates<S, 1>(g, i, j, k)) correct(f.by, mid.b[1], h * (cf.dtd[0] * dx(2) - cf.dtd[2] * dt(2)));
-            if (b_updates<S, 2>(g, i, j, k)) correct(f.bz, mid.b[2], h * (cf.dtd[1] * dt(1) - cf.dtd[0] * dx(1)));
+            if (b_updates<S, 1>(g, i, j, k))
+                correct(f.by, mid.b[1], h * (cf.dtd[0] * dx(2) - cf.dtd[2] * dt(2)),
+                        TURN ? b_rate<S, 1>(g, cf, f.ex, f.ey, f.ez, i, j, k) : real(0));
+            if (b_updates<S, 2>(g, i, j, k))
+                correct(f.bz, mid.b[2], h * (cf.dtd[1] * dt(1) - cf.dtd[0] * dx(1)),
+                        TURN ? b_rate<S, 2>(g, cf, f.ex, f.ey, f.ez, i, j, k) : real(0));
         } else {
             if (e_updates<S, 1>(g, i, j, k)) {
                 const real d = -cf.dtd[0] * dx(2) + cf.dtd[2] * dt(2);
@@ -889,7 +905,8 @@ hipError_t launch_inject(hipStream_t st, int solver, const Grid &g, const Solver
     };
     // sides whose planes lie closer than the corrections reach follow each
     // other: in one launch they would update the same nodes
-    if (nsides == 2 && std::abs(a[0].plane - a[1].plane) < 2 * 2) {
+    if (nsides == 2 && !sides_apart(a[0].plane, a[1].plane)) {
+        if (mid) return hipErrorInvalidValue;   // each would set B to its own corrections
         grid.z = 1;
         const hipError_t e = one(a[0], a[0]);
         return e != hipSuccess ? e : one(a[1], a[1]);

@@ -271,10 +271,16 @@ struct InjectArgs {
     int side;                    // 0: total field at i >= plane; 1: at i < plane
     int plane;
 };
+// whether the sides' corrections reach no common node (two planes each way)
+inline bool sides_apart(int plane_a, int plane_b)
+{
+    const int d = plane_a - plane_b;
+    return d >= 4 || d <= -4;
+}
 // the corrections of one sub-step for nsides (1 or 2) sides: b_field = 1 after
 // a B half step (from E_inc), 0 after the E step (from B_inc).  With mid, after
-// two half steps taken together (launch_maxwell_b): B is corrected for both,
-// mid for the first, and energy for the change of mid.
+// two half steps taken together (launch_maxwell_b), the sides apart: B is
+// corrected for both, mid for the first, and energy for the change of mid.
 template <typename real>
 hipError_t launch_inject(hipStream_t st, int solver, const Grid &g, const SolverCoef &c, const Fields<real> &f,
                          int b_field, int nsides, const InjectArgs *a, real *const *mid = nullptr,
