@@ -128,7 +128,9 @@ int qk_init_boundaries(qk_ctx *ctx);
 
 /* nsteps of the loop body of src/main.cpp:2319-2332: birth_from_vacuum,
  * padvance, compute_N, compute_energy, fadvance.  diag (may be NULL) receives
- * one record per step. */
+ * one record per step.  A call that finds no room for its particles on the way
+ * (QK_ERR_CAPACITY) leaves the fields of the last finished step and no particle
+ * moved since; pairs that the failed step drew from vacuum are there. */
 int qk_step(qk_ctx *ctx, int nsteps, qk_diag *diag);
 /* wait for all queued work of the context */
 int qk_sync(qk_ctx *ctx);
@@ -178,8 +180,10 @@ int qk_pmerging(qk_ctx *ctx, int mode, const double *ppd);
 
 /* spatial_region::moving_window (src/advance.cpp:389-454): erase the
  * particles of the plane i = 0, move E, B, Be and every particle one cell
- * toward -x (x -= 1), zero the plane nx - 1.  J is left as it is.  The caller
- * decides when (check_moving_window, src/main.cpp:1953-1978) and refills the
+ * toward -x (x -= 1), zero the plane nx - 1.  J is left as it is.  The call
+ * returns with the work queued on the context's stream: every later call on the
+ * context comes after it, qk_sync waits for it, and a failure on the GPU may be
+ * reported by a later call.  The caller decides when (check_moving_window, src/main.cpp:1953-1978) and refills the
  * front (add_moving_window_particles, :1750-1835), as main() does. */
 int qk_moving_window(qk_ctx *ctx);
 /* spatial_region::get_max_w (src/low-level.cpp:512-532): the largest
@@ -191,8 +195,12 @@ int qk_max_w(qk_ctx *ctx, int ilo, int ihi, double *max_w);
  * u = (ux0, 0, 0), charge density / (npic product) (negative for cmr < 0).
  * Cells outside is_inside are skipped (place() deletes their particles).
  * With track_ids, the particles of the m-th listed cell get the ids
- * first_id + m x npt + (ip npic[1] + jp) npic[2] + kp.  *added (may be NULL)
- * receives the number stored. */
+ * first_id + m x npt + (ip npic[1] + jp) npic[2] + kp.  The new slots follow
+ * each other by groups of 64 stored cells, within a group all cells' first particles,
+ * then all their second ones: the order in which qk_get_particles gives them
+ * until the next sort.  *added (may be NULL) receives the number stored.  Like
+ * qk_moving_window the call may return with its work queued (the arrays passed
+ * in are free again). */
 int qk_fill_cells(qk_ctx *ctx, int species, int64_t ncells, const int32_t *cells, const double *density,
                   const int32_t npic[3], double ux0, int32_t first_id, int64_t *added);
 
