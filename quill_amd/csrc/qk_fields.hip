@@ -618,7 +618,8 @@ struct InjectSides {
 // once, and the grid's B becomes mid after the second half step and its
 // corrections, in the order of two half steps taken apart (corrected twice
 // after both, FP32 runs came out 1 % further from FP64).  The energy of the
-// fields between the two changes with mid.
+// fields between the two changes with mid.  9.4 us where a sub-step takes 7.7
+// (two sides of 128 x 128 columns), 5.2 and 4.8 us (one of 32 x 32).
 template <int S, bool BF, bool TURN, typename real>
 __global__ void __launch_bounds__(kBX * kBY) k_inject(Grid g, Coef<real> cf, Fields<real> f, InjectSides sides,
                                                       Mid<real> mid, double *energy)

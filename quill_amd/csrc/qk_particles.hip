@@ -291,9 +291,9 @@ struct TiledArgs {
 // otherwise be the FP32 sum of so many more parts: its error against FP64 (rms
 // of one step's J at 56x32x32 with 8 per cell) was 7.86e-8, with whole tiles
 // 7.49e-8, and two runs differed by 2.3e-8 and 4.5e-9; now 7.33e-8, and two
-// runs give the same bits.  It costs 1 us in the push and 0 to 2 us in the E
-// step (40.5 us per step instead of 39.8 at 64x32x32, 76.2 instead of 74.2 at
-// 96x48x48).
+// runs give the same bits.  The push takes 22.1 us instead of 21.6
+// at 64x32x32, the E step 4.7 instead of 4.4 (a step 40.5 instead of 39.8 us, at
+// 96x48x48 76.2 instead of 74.2).
 template <typename real, int PUSHER, bool WIDE>
 __global__ void __launch_bounds__(kTBlock) k_push_tiled(Grid g, Fields<real> f, Current<real> cur, Current<double> wide,
                                                         TileGeom tg, TiledArgs<real> args)
