@@ -1,6 +1,6 @@
 """Read-backs on both sides of the sizes from which helper threads share them,
-and again in the same context, which then shares smaller ones too: fields, node charges, records and rows by id are the same
-numbers either way."""
+and again in the same context, which then shares smaller ones too: fields,
+node charges, records and rows by id are the same numbers either way."""
 import numpy as np
 import pytest
 
